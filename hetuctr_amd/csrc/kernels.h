@@ -73,6 +73,26 @@ struct TableView {
   version_t *upd;                // [n_cached]
 };
 
+// How many columns of a row a lane moves at a time, as a template argument of the row kernels:
+//   4      16-byte vectors: the width is a multiple of four and the caller's pointer 16-byte aligned,
+//   kOdd4  vectors of four floats at any 4-byte address (gfx950 loads and stores them in one instruction): every other
+//          width from four on, and rows at pointers that are not 16-byte aligned.  The last lane of a row starts at
+//          column W - 4, so it shares up to three columns with the lane before: both read them, and where a row is
+//          updated in place only the lane before writes them,
+//   1      rows of less than four floats.
+// Against one float per lane (what every width but multiples of four took before), rows of 37 floats, 195 k keys of 39
+// Zipf fields on an MI355X: a training step 148 -> 86 us (the push alone was 103 us of
+// the 148).
+constexpr int kOdd4 = -4;
+template <int VEC> constexpr uint32_t kCols = VEC < 0 ? (uint32_t)-VEC : (uint32_t)VEC;
+inline int row_vec(uint32_t width, const void *p) {
+  return width < 4 ? 1 : (width % 4 == 0 && (uintptr_t)p % 16 == 0) ? 4 : kOdd4;
+}
+// the column a lane that is due at column c < width really starts at
+template <int VEC> __device__ __forceinline__ uint32_t lane_col(uint32_t c, uint32_t width) {
+  return VEC == kOdd4 ? min(c, width - 4) : c;
+}
+
 // ---- preprocess ---------------------------------------------------------------------------------
 // ids -> sort keys; flags ids outside [0, id_max) in *err (and sorts them as id 0)
 // comp_keys is the batch's copy of the ids as well (the reference's d_idx); nlong (optional) is zeroed;

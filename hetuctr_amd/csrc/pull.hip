@@ -13,9 +13,25 @@ constexpr int kBlock = 256;
 static_assert(kBlock == kRunListBlock, "the gather's blocks list runs chunk by chunk");
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// Rows travel in vectors of kCols<VEC> columns per lane: 4 (the width is a multiple of four and every pointer 16-byte
+// aligned), kOdd4 (any other width from 4 on: see kernels.h) or 1 (rows of less than four floats).
 template <int VEC> struct RowVec;
 template <> struct RowVec<4> { typedef floatx4 T; };
+template <> struct RowVec<kOdd4> { typedef floatx4 T __attribute__((aligned(4))); };
 template <> struct RowVec<1> { typedef float T; };
+// row[0 .. kCols) = v, without the columns the lane before writes too
+template <int VEC> __device__ __forceinline__ void store_own(embed_t *row, typename RowVec<VEC>::T v, uint32_t shared) {
+  typedef typename RowVec<VEC>::T V;
+  if constexpr (VEC == kOdd4) {
+    if (shared) {
+#pragma unroll
+      for (uint32_t k = 1; k < 4; k++)
+        if (k >= shared) row[k] = v[k];
+      return;
+    }
+  }
+  *(V *)row = v;
+}
 
 // The queries of a step (csrc/core/generate_query.cu:91-106): per unique key its id and the version of the local copy
 // (invalid if the key is not resident here), written where the key's owner reads its queries: place u + delta[owner]
@@ -122,17 +138,18 @@ __global__ __launch_bounds__(kBlock) void apply_remote_all(const OwnerShard *__r
         for (int a = 0; a < kAhead; a++)
           if (o[a] != kNoSlot) ver[o[a]] += load_once(rg_cnt + k0 + a * kGroups);
       }
-      for (uint32_t col = gl * VEC; col < W; col += LPR * VEC) {
+      for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+        const uint32_t col = lane_col<VEC>(c, W);
         V cur[kAhead], add[kAhead];
 #pragma unroll
         for (int a = 0; a < kAhead; a++) {
           if (o[a] == kNoSlot) continue;
           cur[a] = *(const V *)(emb + (size_t)o[a] * W + col);
-          add[a] = load_once((const V *)(rg_val + (size_t)(k0 + a * kGroups) * W + col)); // read once: keep it out of the caches
+          add[a] = __builtin_nontemporal_load((const V *)(rg_val + (size_t)(k0 + a * kGroups) * W + col)); // read once: keep it out of the caches
         }
 #pragma unroll
         for (int a = 0; a < kAhead; a++)
-          if (o[a] != kNoSlot) *(V *)(emb + (size_t)o[a] * W + col) = cur[a] + add[a];
+          if (o[a] != kNoSlot) store_own<VEC>(emb + (size_t)o[a] * W + col, cur[a] + add[a], c - col);
       }
     }
     __syncthreads(); // the next source may push to the same rows
@@ -348,7 +365,8 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
     for (int a = 0; a < kPackAhead; a++)
       if (o[a] != kNoSlot) *dst_ver[a] = S.t.ver[o[a]];
   }
-  for (uint32_t col = gl * VEC; col < W; col += LPR * VEC) {
+  for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+    const uint32_t col = lane_col<VEC>(c, W);
     V v[kPackAhead];
 #pragma unroll
     for (int a = 0; a < kPackAhead; a++)
@@ -457,19 +475,21 @@ __global__ __launch_bounds__(kBlock) void remote_emit(TableView t, BatchView c, 
 
 // one group per unique rank of the current batch
 template <int VEC, int LPR>
-__global__ __launch_bounds__(kBlock) void refresh(TableView t, BatchView c, PullArgs a) {
+__global__ __launch_bounds__(kBlock) void refresh(TableView t, BatchView b, PullArgs a) {
   typedef typename RowVec<VEC>::T V;
   constexpr int kGroups = kBlock / LPR;
-  const uint32_t U = *c.d_U, gl = threadIdx.x % LPR, W = t.width;
+  const uint32_t U = *b.d_U, gl = threadIdx.x % LPR, W = t.width;
   for (uint32_t u = blockIdx.x * kGroups + threadIdx.x / LPR; u < U; u += gridDim.x * kGroups) {
-    const slot_t o = c.uoff[u];
+    const slot_t o = b.uoff[u];
     const bool got = a.got[u] != 0;
     if (!got || o == kNoSlot || (uint32_t)o >= t.n_cached) continue; // (an owned row that came back is reported by remote_emit)
     const uint32_t k = a.ret_i[u];
     if (gl == 0) t.ver[o] = a.in_ver[k];
-    for (uint32_t col = gl * VEC; col < W; col += LPR * VEC)
+    for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+      const uint32_t col = lane_col<VEC>(c, W);
       *(V *)(t.emb + (size_t)o * W + col) =
           *(const V *)(a.in_val + (size_t)k * W + col) + *(const V *)(t.pend + (size_t)o * W + col);
+    }
   }
 }
 
@@ -483,13 +503,13 @@ constexpr int kRows = HCTR_GATHER_ROWS;
 // kStream: dst is written with nontemporal stores (a compile-time choice: merged into one store by the compiler, a
 // run-time one loses the hint)
 template <int VEC, int LPR, bool kLocalOnly, bool kStream>
-__global__ __launch_bounds__(kBlock) void gather(TableView t, BatchView c, PullArgs a) {
+__global__ __launch_bounds__(kBlock) void gather(TableView t, BatchView b, PullArgs a) {
   typedef typename RowVec<VEC>::T V;
   constexpr int kGroups = kBlock / LPR;
-  const uint32_t n = c.n, W = t.width;
+  const uint32_t n = b.n, W = t.width;
   if (blockIdx.x < a.list_chunks) { // the batch's run lists for its push one step later, before the block's own rows
     __shared__ uint32_t cnt[kRunLists], base[kRunLists];
-    for (uint32_t chunk = blockIdx.x; chunk < a.list_chunks; chunk += gridDim.x) list_runs_chunk(c, chunk, cnt, base);
+    for (uint32_t chunk = blockIdx.x; chunk < a.list_chunks; chunk += gridDim.x) list_runs_chunk(b, chunk, cnt, base);
   }
   const uint32_t j0 = (blockIdx.x * kGroups + threadIdx.x / LPR) * kRows;
   if (j0 >= n) return;
@@ -499,17 +519,18 @@ __global__ __launch_bounds__(kBlock) void gather(TableView t, BatchView c, PullA
 #pragma unroll
   for (int k = 0; k < kRows; k++) {
     const uint32_t j = min(j0 + k, n - 1);
-    const uint32_t u = c.rank_sorted[j];
-    const uint32_t i = c.sorted_arg[j];
+    const uint32_t u = b.rank_sorted[j];
+    const uint32_t i = b.sorted_arg[j];
     if (kLocalOnly) {
-      src[k] = t.emb + (size_t)c.uoff[u] * W;
+      src[k] = t.emb + (size_t)b.uoff[u] * W;
     } else {
       const uint32_t r = a.src_row[u];
       src[k] = (r & kReturnedRow) ? a.in_val + (size_t)(r & ~kReturnedRow) * W : t.emb + (size_t)r * W;
     }
     dst[k] = a.dst + (size_t)i * W;
   }
-  for (uint32_t col = gl * VEC; col < W; col += LPR * VEC) {
+  for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+    const uint32_t col = lane_col<VEC>(c, W);
     V v[kRows];
 #pragma unroll
     for (int k = 0; k < kRows; k++) v[k] = *(const V *)(src[k] + col);
@@ -542,7 +563,8 @@ __global__ __launch_bounds__(kBlock) void gather_direct(TableView t, const K *__
     const uint32_t i = min(i0 + k, n - 1);
     src[k] = t.emb + (size_t)t.slot[(uint64_t)(keys[i] & id_mask)] * W; // one shard: every id is resident
   }
-  for (uint32_t col = gl * VEC; col < W; col += LPR * VEC) {
+  for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+    const uint32_t col = lane_col<VEC>(c, W);
     V v[kRows];
 #pragma unroll
     for (int k = 0; k < kRows; k++) v[k] = *(const V *)(src[k] + col);
@@ -561,27 +583,28 @@ __global__ __launch_bounds__(kBlock) void gather_direct(TableView t, const K *__
 // row instead of `bag`.  Works in batch order, through the inverse index of the batch.
 constexpr int kPoolAhead = 8;
 template <int VEC, int LPR, bool kLocalOnly>
-__global__ __launch_bounds__(kBlock) void gather_pooled(TableView t, BatchView c, PullArgs a, uint32_t bag,
+__global__ __launch_bounds__(kBlock) void gather_pooled(TableView t, BatchView batch, PullArgs a, uint32_t bag,
                                                         uint32_t n_bags) {
   typedef typename RowVec<VEC>::T V;
   constexpr int kGroups = kBlock / LPR;
   if (blockIdx.x < a.list_chunks) { // the batch's run lists, as in gather
     __shared__ uint32_t cnt[kRunLists], base[kRunLists];
-    for (uint32_t chunk = blockIdx.x; chunk < a.list_chunks; chunk += gridDim.x) list_runs_chunk(c, chunk, cnt, base);
+    for (uint32_t chunk = blockIdx.x; chunk < a.list_chunks; chunk += gridDim.x) list_runs_chunk(batch, chunk, cnt, base);
   }
   const uint32_t b = blockIdx.x * kGroups + threadIdx.x / LPR;
   if (b >= n_bags) return;
   const uint32_t gl = threadIdx.x % LPR, W = t.width;
   const uint32_t i0 = b * bag;
-  for (uint32_t col = gl * VEC; col < W; col += LPR * VEC) {
+  for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+    const uint32_t col = lane_col<VEC>(c, W);
     V acc;
     for (uint32_t h0 = 0; h0 < bag; h0 += kPoolAhead) {
       const embed_t *src[kPoolAhead];
 #pragma unroll
       for (int k = 0; k < kPoolAhead; k++) {
-        const uint32_t u = c.idx_map[i0 + min(h0 + k, bag - 1)];
+        const uint32_t u = batch.idx_map[i0 + min(h0 + k, bag - 1)];
         if (kLocalOnly) {
-          src[k] = t.emb + (size_t)c.uoff[u] * W;
+          src[k] = t.emb + (size_t)batch.uoff[u] * W;
         } else {
           const uint32_t r = a.src_row[u];
           src[k] = (r & kReturnedRow) ? a.in_val + (size_t)(r & ~kReturnedRow) * W : t.emb + (size_t)r * W;
@@ -612,7 +635,8 @@ __global__ __launch_bounds__(kBlock) void gather_pooled_direct(TableView t, cons
   const uint32_t gl = threadIdx.x % LPR, W = t.width;
   const uint32_t i0 = b * bag;
   const K id_mask = (K)(((uint64_t)1 << id_bits) - 1);
-  for (uint32_t col = gl * VEC; col < W; col += LPR * VEC) {
+  for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+    const uint32_t col = lane_col<VEC>(c, W);
     V acc;
     for (uint32_t h0 = 0; h0 < bag; h0 += kPoolAhead) {
       const embed_t *src[kPoolAhead];
@@ -639,30 +663,26 @@ __global__ __launch_bounds__(kBlock) void plain_copy(const uint4 *__restrict__ s
 }
 
 inline int lanes_for(uint32_t width, int vec) {
-  const uint32_t lanes = (width + vec - 1) / vec;
+  const uint32_t per = vec == 1 ? 1 : 4, lanes = (width + per - 1) / per;
   return lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
 }
 
-// expands F<VEC, LPR>(args...) over the supported (VEC, LPR) pairs
-#define HCTR_DISPATCH_ROW(vec4, lpr, CALL) \
-  do {                                     \
-    if (vec4) {                            \
-      switch (lpr) {                       \
-        case 4: CALL(4, 4); break;         \
-        case 8: CALL(4, 8); break;         \
-        case 16: CALL(4, 16); break;       \
-        case 32: CALL(4, 32); break;       \
-        default: CALL(4, 64); break;       \
-      }                                    \
-    } else {                               \
-      switch (lpr) {                       \
-        case 4: CALL(1, 4); break;         \
-        case 8: CALL(1, 8); break;         \
-        case 16: CALL(1, 16); break;       \
-        case 32: CALL(1, 32); break;       \
-        default: CALL(1, 64); break;       \
-      }                                    \
-    }                                      \
+// expands F<VEC, LPR>(args...) over the (VEC, LPR) pairs; a row of less than four floats takes at most four lanes
+#define HCTR_DISPATCH_ROW(vec, lpr, CALL)         \
+  do {                                            \
+    if ((vec) == 4) HCTR_DISPATCH_LPR(4, lpr, CALL); \
+    else if ((vec) == kOdd4) HCTR_DISPATCH_LPR(kOdd4, lpr, CALL); \
+    else CALL(1, 4);                              \
+  } while (0)
+#define HCTR_DISPATCH_LPR(V, lpr, CALL) \
+  do {                                  \
+    switch (lpr) {                      \
+      case 4: CALL(V, 4); break;        \
+      case 8: CALL(V, 8); break;        \
+      case 16: CALL(V, 16); break;      \
+      case 32: CALL(V, 32); break;      \
+      default: CALL(V, 64); break;      \
+    }                                   \
   } while (0)
 
 } // namespace
@@ -679,7 +699,7 @@ void launch_build_queries(hipStream_t s, const TableView &t, const KeyLayout &kl
 size_t query_tiles(uint32_t q) { return std::max<size_t>(1, div_up(q, kBlock)); }
 
 uint32_t owner_push_rows_per_block(uint32_t width) {
-  const int lpr = lanes_for(width, width % 4 == 0 ? 4 : 1);
+  const int lpr = lanes_for(width, row_vec(width, nullptr));
   return kApplyBatches * kApplyAhead * (kBlock / lpr);
 }
 
@@ -705,13 +725,13 @@ static uint32_t guessed_blocks(uint32_t guess, uint32_t most, uint32_t per_block
 void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width,
                        uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess) {
   const uint32_t tiles = guessed_blocks(queries_guess, queries_max, kBlock);
-  const bool vec4 = width % 4 == 0;
-  const int lpr = lanes_for(width, vec4 ? 4 : 1);
+  const int vec = row_vec(width, nullptr);
+  const int lpr = lanes_for(width, vec);
   if (push_blocks) {
     const uint32_t rpb = owner_push_rows_per_block(width);
 #define CALL(V, L) \
   hipLaunchKernelGGL((apply_remote_all<V, L>), dim3(push_blocks, nshards), dim3(kBlock), 0, s, shards_dev, nsrc, rpb)
-    HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+    HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   }
   hipLaunchKernelGGL(decide_count, dim3(tiles, nshards), dim3(kBlock), 0, s, shards_dev, nsrc);
@@ -721,7 +741,7 @@ void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards,
 #define CALL(V, L)                                                                                                     \
   hipLaunchKernelGGL((pack_rows<V, L>), dim3(guessed_blocks(queries_guess, queries_max, kPackAhead * (kBlock / L)), nshards), \
                      dim3(kBlock), 0, s, shards_dev, nsrc)
-    HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+    HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   }
   HCTR_HIP(hipGetLastError());
@@ -734,19 +754,19 @@ void launch_refresh(hipStream_t s, const TableView &t, const BatchView &cur, uin
   hipLaunchKernelGGL(got_tile_sums, dim3(tiles), dim3(kBlock), 0, s, a.got, cur.d_U, tile_sums);
   hipLaunchKernelGGL(remote_emit, dim3(tiles), dim3(kBlock), 0, s, t, cur, a.got, tile_sums, a.ret_i, a.src_row, stats,
                      host_stats);
-  const bool vec4 = t.width % 4 == 0;
-  const int lpr = lanes_for(t.width, vec4 ? 4 : 1);
+  const int vec = row_vec(t.width, nullptr);
+  const int lpr = lanes_for(t.width, vec);
 #define CALL(V, L)                                                                                                      \
   hipLaunchKernelGGL((refresh<V, L>), dim3(guessed_blocks(unique_guess, unique_max, kBlock / L)), dim3(kBlock), 0, s, t, cur, a)
-  HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+  HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   HCTR_HIP(hipGetLastError());
 }
 
 void launch_gather(hipStream_t s, const TableView &t, const BatchView &cur, const PullArgs &a) {
   if (!cur.n) return;
-  const bool vec4 = t.width % 4 == 0 && ((uintptr_t)a.dst % 16) == 0;
-  const int lpr = lanes_for(t.width, vec4 ? 4 : 1);
+  const int vec = row_vec(t.width, a.dst);
+  const int lpr = lanes_for(t.width, vec);
   const bool local_only = a.got == nullptr;
 #define CALL(V, L)                                                                                               \
   do {                                                                                                           \
@@ -756,7 +776,7 @@ void launch_gather(hipStream_t s, const TableView &t, const BatchView &cur, cons
     else if (a.stream_stores) hipLaunchKernelGGL((gather<V, L, false, true>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a); \
     else hipLaunchKernelGGL((gather<V, L, false, false>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a);          \
   } while (0)
-  HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+  HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   HCTR_HIP(hipGetLastError());
 }
@@ -765,8 +785,8 @@ void launch_gather_direct(hipStream_t s, const TableView &t, const KeyLayout &kl
                           bool stream_stores) {
   if (!n) return;
   HCTR_CHECK(t.nrank == 1, "internal: the gather from the keys is for one shard");
-  const bool vec4 = t.width % 4 == 0 && ((uintptr_t)dst % 16) == 0;
-  const int lpr = lanes_for(t.width, vec4 ? 4 : 1);
+  const int vec = row_vec(t.width, dst);
+  const int lpr = lanes_for(t.width, vec);
 #define CALL(V, L)                                                                                                    \
   do {                                                                                                                \
     const unsigned blocks = div_up(n, (kBlock / L) * kRows);                                                          \
@@ -775,7 +795,7 @@ void launch_gather_direct(hipStream_t s, const TableView &t, const KeyLayout &kl
     else if (stream_stores) hipLaunchKernelGGL((gather_direct<V, L, uint32_t, true>), dim3(blocks), dim3(kBlock), 0, s, t, (const uint32_t *)keys, kl.id_bits, n, dst); \
     else hipLaunchKernelGGL((gather_direct<V, L, uint32_t, false>), dim3(blocks), dim3(kBlock), 0, s, t, (const uint32_t *)keys, kl.id_bits, n, dst); \
   } while (0)
-  HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+  HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   HCTR_HIP(hipGetLastError());
 }
@@ -785,15 +805,15 @@ void launch_gather_pooled_direct(hipStream_t s, const TableView &t, const KeyLay
   if (!n) return;
   HCTR_CHECK(t.nrank == 1, "internal: the gather from the keys is for one shard");
   const uint32_t n_bags = n / bag;
-  const bool vec4 = t.width % 4 == 0 && ((uintptr_t)dst % 16) == 0;
-  const int lpr = lanes_for(t.width, vec4 ? 4 : 1);
+  const int vec = row_vec(t.width, dst);
+  const int lpr = lanes_for(t.width, vec);
 #define CALL(V, L)                                                                                                    \
   do {                                                                                                                \
     const unsigned blocks = div_up(n_bags, kBlock / L);                                                               \
     if (kl.wide) hipLaunchKernelGGL((gather_pooled_direct<V, L, uint64_t>), dim3(blocks), dim3(kBlock), 0, s, t, (const uint64_t *)keys, kl.id_bits, dst, bag, n_bags); \
     else hipLaunchKernelGGL((gather_pooled_direct<V, L, uint32_t>), dim3(blocks), dim3(kBlock), 0, s, t, (const uint32_t *)keys, kl.id_bits, dst, bag, n_bags); \
   } while (0)
-  HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+  HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   HCTR_HIP(hipGetLastError());
 }
@@ -801,8 +821,8 @@ void launch_gather_pooled_direct(hipStream_t s, const TableView &t, const KeyLay
 void launch_gather_pooled(hipStream_t s, const TableView &t, const BatchView &cur, const PullArgs &a, uint32_t bag) {
   if (!cur.n) return;
   const uint32_t n_bags = cur.n / bag;
-  const bool vec4 = t.width % 4 == 0 && ((uintptr_t)a.dst % 16) == 0;
-  const int lpr = lanes_for(t.width, vec4 ? 4 : 1);
+  const int vec = row_vec(t.width, a.dst);
+  const int lpr = lanes_for(t.width, vec);
   const bool local_only = a.got == nullptr;
 #define CALL(V, L)                                                                                                  \
   do {                                                                                                              \
@@ -810,7 +830,7 @@ void launch_gather_pooled(hipStream_t s, const TableView &t, const BatchView &cu
     if (local_only) hipLaunchKernelGGL((gather_pooled<V, L, true>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a, bag, n_bags); \
     else hipLaunchKernelGGL((gather_pooled<V, L, false>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a, bag, n_bags);  \
   } while (0)
-  HCTR_DISPATCH_ROW(vec4, lpr, CALL);
+  HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
   HCTR_HIP(hipGetLastError());
 }

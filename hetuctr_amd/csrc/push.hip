@@ -24,6 +24,7 @@
 //  * short (<= kTinyRun): a group of LPR lanes (LPR*VEC floats = one row) owns a few consecutive unique keys
 //    and sums their runs, all first loads of the group issued together.
 #include <algorithm>
+#include <type_traits>
 #include "kernels.h"
 
 namespace hctr {
@@ -77,19 +78,7 @@ __device__ __forceinline__ uint32_t div_up_dev(uint32_t a, uint32_t b) { return 
 #define HCTR_GRAD_NT 1
 #endif
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-// A gradient row is read exactly once per step: it is loaded past the caches.  With sum-pooled bags (kPooled) a row
-// is read once per key of its bag, so there it is loaded the ordinary way and the repeats hit the cache.
-template <bool kPooled> __device__ __forceinline__ float4 grad_load(const float4 *p) {
-  if (HCTR_GRAD_NT && !kPooled) {
-    const f32x4 r = __builtin_nontemporal_load((const f32x4 *)p);
-    return make_float4(r.x, r.y, r.z, r.w);
-  }
-  return *p;
-}
-template <bool kPooled> __device__ __forceinline__ float grad_load(const float *p) {
-  if (HCTR_GRAD_NT && !kPooled) return __builtin_nontemporal_load(p);
-  return *p;
-}
+typedef f32x4 f32x4_any __attribute__((aligned(4))); // at any 4-byte address
 // The gradient row of batch position `pos`: the position itself, or with sum-pooled bags of `bag` consecutive
 // positions the row of the position's bag (every key of a bag receives the bag's gradient).
 // kPooled is a compile-time switch: the plain push must not pay for the division in its load pipelines.
@@ -97,26 +86,60 @@ template <bool kPooled> __device__ __forceinline__ uint32_t grad_row(uint32_t po
   return kPooled ? bag(pos) : pos;
 }
 
+// the columns a lane moves at a time (see kOdd4 in kernels.h); V: as they lie in memory
 template <int VEC> struct Vec;
-template <> struct Vec<4> {
-  typedef float4 T;
-  static __device__ __forceinline__ T zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
+struct Vec4Ops {
+  typedef f32x4 T;
+  static __device__ __forceinline__ T zero() { return (f32x4){0.f, 0.f, 0.f, 0.f}; }
   static __device__ __forceinline__ void add(T &a, const T &b) { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
-  static __device__ __forceinline__ T scale(const T &a, float s) { return make_float4(a.x * s, a.y * s, a.z * s, a.w * s); }
+  static __device__ __forceinline__ T scale(const T &a, float s) { return (f32x4){a.x * s, a.y * s, a.z * s, a.w * s}; }
+};
+template <> struct Vec<4> : Vec4Ops {
+  typedef f32x4 M;
+  static __device__ __forceinline__ void store(float *p, const T &a, uint32_t) { *(M *)p = a; }
   // a store past the caches: for rows another shard's kernel reads next
-  static __device__ __forceinline__ void store_away(T *p, const T &a) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    f4 v = {a.x, a.y, a.z, a.w};
-    __builtin_nontemporal_store(v, (f4 *)p);
+  static __device__ __forceinline__ void store_away(float *p, const T &a, uint32_t) { __builtin_nontemporal_store(a, (M *)p); }
+};
+template <> struct Vec<kOdd4> : Vec4Ops {
+  typedef f32x4_any M;
+  // without the first `shared` columns, which the lane before writes (and, in a row of more than one round of the
+  // group, may have updated before this lane reads them: what it computes for them is dropped)
+  static __device__ __forceinline__ void store(float *p, const T &a, uint32_t shared) {
+    if (!shared) {
+      *(M *)p = a;
+    } else {
+      if (shared < 2) p[1] = a.y;
+      if (shared < 3) p[2] = a.z;
+      p[3] = a.w;
+    }
+  }
+  static __device__ __forceinline__ void store_away(float *p, const T &a, uint32_t shared) {
+    if (!shared) {
+      __builtin_nontemporal_store(a, (M *)p);
+    } else {
+      if (shared < 2) __builtin_nontemporal_store(a.y, p + 1);
+      if (shared < 3) __builtin_nontemporal_store(a.z, p + 2);
+      __builtin_nontemporal_store(a.w, p + 3);
+    }
   }
 };
 template <> struct Vec<1> {
   typedef float T;
+  typedef float M;
   static __device__ __forceinline__ T zero() { return 0.f; }
   static __device__ __forceinline__ void add(T &a, const T &b) { a += b; }
   static __device__ __forceinline__ T scale(const T &a, float s) { return a * s; }
-  static __device__ __forceinline__ void store_away(T *p, const T &a) { __builtin_nontemporal_store(a, p); }
+  static __device__ __forceinline__ void store(float *p, const T &a, uint32_t) { *p = a; }
+  static __device__ __forceinline__ void store_away(float *p, const T &a, uint32_t) { __builtin_nontemporal_store(a, p); }
 };
+
+// A gradient row is read exactly once per step: it is loaded past the caches.  With sum-pooled bags (kPooled) a row
+// is read once per key of its bag, so there it is loaded the ordinary way and the repeats hit the cache.
+template <int VEC, bool kPooled> __device__ __forceinline__ typename Vec<VEC>::T grad_load(const embed_t *p) {
+  typedef typename Vec<VEC>::M M;
+  if (HCTR_GRAD_NT && !kPooled) return __builtin_nontemporal_load((const M *)p);
+  return *(const M *)p;
+}
 
 // The version / update counters of unique rank u and its entry among the pushed rows (gradient_index_kernel,
 // generate_query.cu:51-83).  type: the update type of generate_query.cu:18-25; q: the row's place among the pushed rows.
@@ -144,37 +167,38 @@ __device__ __forceinline__ void move_counters(const TableView &t, int id_bits, c
 // generate_query.cu:18-25.  The counters of the row move in the last blocks of the launch.
 template <int VEC, typename K>
 __device__ __forceinline__ void apply_row(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
-                                          uint32_t u, typename Vec<VEC>::T s, uint32_t col) {
+                                          uint32_t u, typename Vec<VEC>::T s, uint32_t col, uint32_t shared = 0) {
   typedef typename Vec<VEC>::T V;
+  typedef typename Vec<VEC>::M M;
   const slot_t o = p.uoff[u];
   const uint32_t W = t.width;
   if (t.nrank == 1) { // every key is owned and resident: type 1 only
-    V *e = (V *)(t.emb + (size_t)o * W + col);
-    V cur = *e;
+    embed_t *e = t.emb + (size_t)o * W + col;
+    V cur = *(const M *)e;
     Vec<VEC>::add(cur, s);
-    *e = cur;
+    Vec<VEC>::store(e, cur, shared);
     return;
   }
   const bool need = a.need[u] != 0;
   const int type = o == kNoSlot ? 0 : ((uint32_t)o >= t.n_cached ? 1 : (need ? 2 : 3));
   const uint32_t q = a.prefix[u];
   if (type != 0) {
-    V *e = (V *)(t.emb + (size_t)o * W + col);
-    V cur = *e;
+    embed_t *e = t.emb + (size_t)o * W + col;
+    V cur = *(const M *)e;
     Vec<VEC>::add(cur, s);
-    *e = cur;
+    Vec<VEC>::store(e, cur, shared);
   } else {
-    Vec<VEC>::store_away((V *)(a.g_val + (size_t)q * W + col), s);
+    Vec<VEC>::store_away(a.g_val + (size_t)q * W + col, s, shared);
   }
   if (type >= 2) {
-    V *g = (V *)(t.pend + (size_t)o * W + col);
-    V pg = *g;
+    embed_t *g = t.pend + (size_t)o * W + col;
+    V pg = *(const M *)g;
     Vec<VEC>::add(pg, s);
     if (type == 2) {
-      Vec<VEC>::store_away((V *)(a.g_val + (size_t)q * W + col), pg);
+      Vec<VEC>::store_away(a.g_val + (size_t)q * W + col, pg, shared);
       pg = Vec<VEC>::zero();
     }
-    *g = pg;
+    Vec<VEC>::store(g, pg, shared);
   }
 }
 
@@ -197,6 +221,7 @@ template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
 __device__ __forceinline__ void short_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
                                            uint32_t block, uint32_t U) {
   typedef typename Vec<VEC>::T V;
+  typedef typename Vec<VEC>::M M;
   constexpr int G = kRunsPerGroup;
   constexpr int kGroups = kPushBlock / LPR;
   const uint32_t W = t.width, n = p.n;
@@ -228,9 +253,9 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
   }
   const float neg_lr = t.neg_lr;
 
-  for (uint32_t c0 = 0; c0 < W; c0 += LPR * VEC) {
-    const uint32_t col = c0 + gl * VEC;
-    const bool active = col < W;
+  for (uint32_t c0 = 0; c0 < W; c0 += LPR * kCols<VEC>) {
+    const uint32_t due = c0 + gl * kCols<VEC>, col = lane_col<VEC>(due, W), shared = due - col;
+    const bool active = due < W;
     uint32_t len[G];
     bool mine[G];
     V e[G], pg[G];
@@ -245,13 +270,13 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 #pragma unroll
     for (int i = 0; i < G; i++) {
       e[i] = Vec<VEC>::zero();
-      if (mine[i] && (kSingle || type[i] != 0)) e[i] = *(const V *)(t.emb + (size_t)off[i] * W + col);
+      if (mine[i] && (kSingle || type[i] != 0)) e[i] = *(const M *)(t.emb + (size_t)off[i] * W + col);
     }
     if (!kSingle) {
 #pragma unroll
       for (int i = 0; i < G; i++) {
         pg[i] = Vec<VEC>::zero();
-        if (mine[i] && type[i] >= 2) pg[i] = *(const V *)(t.pend + (size_t)off[i] * W + col);
+        if (mine[i] && type[i] >= 2) pg[i] = *(const M *)(t.pend + (size_t)off[i] * W + col);
       }
     }
 #pragma unroll
@@ -263,7 +288,7 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 #pragma unroll
       for (int k = 0; k < kHead; k++) {
         v[i][k] = Vec<VEC>::zero();
-        if (mine[i] && (uint32_t)k < len[i]) v[i][k] = grad_load<kPooled>((const V *)(grad + (size_t)si[i][k] * W + col));
+        if (mine[i] && (uint32_t)k < len[i]) v[i][k] = grad_load<VEC, kPooled>(grad + (size_t)si[i][k] * W + col);
       }
     V acc[G];
 #pragma unroll
@@ -283,7 +308,7 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 #pragma unroll
         for (int k = 0; k < kTail; k++) sj[k] = grad_row<kPooled>(sorted_arg[min(j + k, rs[i + 1] - 1)], a.bag);
 #pragma unroll
-        for (int k = 0; k < kTail; k++) x[k] = grad_load<kPooled>((const V *)(grad + (size_t)sj[k] * W + col));
+        for (int k = 0; k < kTail; k++) x[k] = grad_load<VEC, kPooled>(grad + (size_t)sj[k] * W + col);
 #pragma unroll
         for (int k = 0; k < kTail; k++)
           if (j + k < rs[i + 1]) Vec<VEC>::add(acc[i], x[k]);
@@ -292,24 +317,24 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
       if (kSingle) {
         V r = e[i];
         Vec<VEC>::add(r, scaled);
-        *(V *)(t.emb + (size_t)off[i] * W + col) = r; // the version counters move in the last blocks of the launch
+        Vec<VEC>::store(t.emb + (size_t)off[i] * W + col, r, shared); // the version counters move in the last blocks of the launch
       } else {
         // the same updates as apply_row(), with the rows already here
         if (type[i] != 0) {
           V r = e[i];
           Vec<VEC>::add(r, scaled);
-          *(V *)(t.emb + (size_t)off[i] * W + col) = r;
+          Vec<VEC>::store(t.emb + (size_t)off[i] * W + col, r, shared);
         } else {
-          Vec<VEC>::store_away((V *)(a.g_val + (size_t)q[i] * W + col), scaled);
+          Vec<VEC>::store_away(a.g_val + (size_t)q[i] * W + col, scaled, shared);
         }
         if (type[i] >= 2) {
           V g = pg[i];
           Vec<VEC>::add(g, scaled);
           if (type[i] == 2) {
-            Vec<VEC>::store_away((V *)(a.g_val + (size_t)q[i] * W + col), g);
+            Vec<VEC>::store_away(a.g_val + (size_t)q[i] * W + col, g, shared);
             g = Vec<VEC>::zero();
           }
-          *(V *)(t.pend + (size_t)off[i] * W + col) = g;
+          Vec<VEC>::store(t.pend + (size_t)off[i] * W + col, g, shared);
         }
       }
     }
@@ -325,6 +350,7 @@ template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
 __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
                                             uint32_t *lds_idx, uint32_t block, uint32_t nblocks) {
   typedef typename Vec<VEC>::T V;
+  typedef typename Vec<VEC>::M M;
   constexpr int kGroups = kPushBlock / LPR;
   const uint32_t W = t.width;
   const uint32_t gl = threadIdx.x % LPR;
@@ -344,17 +370,17 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (uint32_t c0 = 0; c0 < W; c0 += LPR * VEC) {
-      const uint32_t col = c0 + gl * VEC;
-      const bool active = col < W;
+    for (uint32_t c0 = 0; c0 < W; c0 += LPR * kCols<VEC>) {
+      const uint32_t due = c0 + gl * kCols<VEC>, col = lane_col<VEC>(due, W), shared = due - col;
+      const bool active = due < W;
       const embed_t *gcol = grad + (active ? col : 0);
       V e = Vec<VEC>::zero();
-      if (kSingle && active) e = *(const V *)(t.emb + (size_t)off * W + col);
+      if (kSingle && active) e = *(const M *)(t.emb + (size_t)off * W + col);
       V acc = Vec<VEC>::zero();
       V xa[kBatch], xb[kBatch];
       auto fetch = [&](V(&x)[kBatch], uint32_t q0) { // rows q0 .. q0+kBatch-1 of the run (clamped to its end)
 #pragma unroll
-        for (int k = 0; k < kBatch; k++) x[k] = grad_load<kPooled>((const V *)(gcol + (size_t)my_idx[min(q0 + k, len - 1)] * W));
+        for (int k = 0; k < kBatch; k++) x[k] = grad_load<VEC, kPooled>(gcol + (size_t)my_idx[min(q0 + k, len - 1)] * W);
       };
       auto add = [&](const V(&x)[kBatch], uint32_t q0) {
 #pragma unroll
@@ -372,9 +398,9 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
       const V scaled = Vec<VEC>::scale(acc, neg_lr);
       if (kSingle) {
         Vec<VEC>::add(e, scaled);
-        *(V *)(t.emb + (size_t)off * W + col) = e; // versions: bump_versions
+        Vec<VEC>::store(t.emb + (size_t)off * W + col, e, shared); // versions: bump_versions
       } else {
-        apply_row<VEC, K>(t, id_bits, p, a, u, scaled, col);
+        apply_row<VEC, K>(t, id_bits, p, a, u, scaled, col, shared);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -402,7 +428,7 @@ constexpr int kTable = 16;     // runs per bundle at most
 constexpr int kSumBatch = HCTR_SUM_BATCH; // rows the summing wave reads from LDS in one go (two such batches are live)
 
 // the four floats of v to dst[0], dst[stride], dst[2 * stride], dst[3 * stride]
-__device__ __forceinline__ void store_transposed(float *dst, uint32_t stride, const float4 &v) {
+__device__ __forceinline__ void store_transposed(float *dst, uint32_t stride, const f32x4 &v) {
   dst[0] = v.x, dst[stride] = v.y, dst[2 * stride] = v.z, dst[3 * stride] = v.w;
 }
 __device__ __forceinline__ void store_transposed(float *, uint32_t, const float &) {} // generic path: never called
@@ -421,15 +447,21 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
                                           float *lds, uint4 *table, uint32_t *shared, float *row_stash, int c_lo,
                                           int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
   typedef typename Vec<VEC>::T V;
+  typedef typename Vec<VEC>::M M;
+  constexpr uint32_t C = kCols<VEC>;
   const uint32_t W = t.width;
-  const uint32_t CS = CSC ? (uint32_t)CSC : min((uint32_t)kSlice, (W + VEC - 1) / VEC * VEC);
-  uint32_t lanes = (CS + VEC - 1) / VEC; // loader lanes per row slice, rounded up to a power of two
+  uint32_t CS = CSC ? (uint32_t)CSC : min((uint32_t)kSlice, (W + C - 1) / C * C);
+  // the last slice of an odd width holds four columns at least, so that a lane that starts early stays inside its slice
+  // (some slice of 8..64 columns fits any width below 2^20)
+  if (VEC == kOdd4)
+    while (CS > 8 && W % CS != 0 && W % CS < 4) CS -= 4;
+  uint32_t lanes = (CS + C - 1) / C; // loader lanes per row slice, rounded up to a power of two
   lanes = lanes <= 1 ? 1 : lanes <= 2 ? 2 : lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
-  const uint32_t RPL = CSC ? (uint32_t)(kLoaders / (CSC / VEC)) : kLoaders / lanes;
+  const uint32_t RPL = CSC ? (uint32_t)(kLoaders / (CSC / C)) : kLoaders / lanes;
   const uint32_t CR = RPL * kRPT;                                   // rows per chunk
-  constexpr int kChunkRows = CSC ? kRPT * (kLoaders / (CSC / VEC)) : 1; // CR as a constant on the fast path
+  constexpr int kChunkRows = CSC ? kRPT * (int)(kLoaders / (CSC / C)) : 1; // CR as a constant on the fast path
   static_assert(!CSC || (kChunkRows % kSumBatch == 0 && kSumBatch % 4 == 0), "a chunk of the fast path is a whole number of sum batches");
-  static_assert(!CSC || kSlots * CSC * (kChunkRows + 4) <= kSlots * kRPT * kPushBlock * VEC, "ring slots of the fast path fit the LDS area");
+  static_assert(!CSC || kSlots * CSC * (kChunkRows + 4) <= kSlots * kRPT * kPushBlock * (int)C, "ring slots of the fast path fit the LDS area");
   const uint32_t slices = (W + CS - 1) / CS;
   // LDS layout of a ring slot.  Generic path: row-major [row][CS].  Fast path (CSC): column-major with the row
   // index fastest, [column place][pitch], pitch = rows + 4, so that the summing lane gets four consecutive rows of
@@ -525,13 +557,14 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
 
     if (!summer) {
       // ---------------- loaders ----------------
-      const uint32_t lcol = my_lane * VEC; // column inside the slice
-      const uint32_t col = slice * CS + lcol;
-      const bool in_slice = lcol < CS && my_row < RPL;
+      const uint32_t due = slice * CS + my_lane * C;   // first column of this lane's vector
+      const bool in_slice = my_lane * C < CS && my_row < RPL;
+      const uint32_t col = due < W ? lane_col<VEC>(due, W) : due;
+      const uint32_t lcol = col - slice * CS;          // ... inside the slice
       // Loads are unconditional and branch-free so that kDepth chunks stay in flight per thread: positions
       // past the end of a run re-read its last row (never summed), lanes outside the slice read column 0.
-      const embed_t *gbase = a.grad + ((in_slice && col < W) ? col : 0);
-      auto row_load = [&](uint32_t idx) -> V { return grad_load<kPooled>((const V *)(gbase + (size_t)idx * W)); };
+      const embed_t *gbase = a.grad + ((in_slice && due < W) ? col : 0);
+      auto row_load = [&](uint32_t idx) -> V { return grad_load<VEC, kPooled>(gbase + (size_t)idx * W); };
       // cursor of the index stage, 2 * kDepth chunks ahead of the LDS stage; past the end of the stream it
       // stays on the last run
       uint32_t cj = 0, cc = 0;
@@ -574,7 +607,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
         for (int q = 0; q < kRPT; q++) {
           if (in_slice) {
             if (CSC) store_transposed(sp + my_lane * pitch + (q * RPL + my_row), (CSC / 4) * pitch, val[k][q]);
-            else *(V *)(sp + (q * RPL + my_row) * CS + lcol) = val[k][q];
+            else *(M *)(sp + (q * RPL + my_row) * CS + lcol) = val[k][q];
           }
           val[k][q] = row_load(idx[k][q]); // chunk + kDepth
         }
@@ -710,7 +743,7 @@ template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
 __global__ __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR_PUSH_WAVES, 8))) void push_fused(TableView t, int id_bits, BatchView p, PushArgs a, uint32_t U) {
   // one LDS area for whichever role the block plays: the row ring of the long role or the index staging of the
   // medium role (one slice of kLongRun indices per group)
-  constexpr int kRingWords = kSlots * kRPT * kPushBlock * VEC;
+  constexpr int kRingWords = kSlots * kRPT * kPushBlock * (int)kCols<VEC>;
   constexpr int kStageWords = (kPushBlock / LPR) * (int)kLongRun;
   __shared__ __align__(16) float lds[kRingWords > kStageWords ? kRingWords : kStageWords];
   __shared__ uint4 run_table[kTable];
@@ -721,13 +754,24 @@ __global__ __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR
     // blocks feed each of them (the blocks of a saturated memory system get equal shares of it, and a chain
     // advances with the share of the block that feeds it), then tickets of the other long runs.
     uint32_t *tk = p.d_nlong + kTicketBase;
-    if (VEC == 4 && t.width % kSlice == 0) {
-      long_role<VEC, K, (VEC == 4 ? kGiantSlice : 0), kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kGiantClasses,
-                                                      blockIdx.x, kLongBlocks, tk);
-      long_role<VEC, K, (VEC == 4 ? kSlice : 0), kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, kGiantClasses, kLongBuckets,
-                                                 blockIdx.x, kLongBlocks, tk + kTicketLanes);
+    // Widths that are whole slices take the fast layout of the ring: 64 (the longest runs 32) columns, or 32, or rows
+    // of 32 and 16 floats as one slice.
+    auto all_runs = [&](auto csc) {
+      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kLongBuckets,
+                                                       blockIdx.x, kLongBlocks, tk);
+    };
+    constexpr int kOneSlice = VEC != 1 && LPR <= 8 ? LPR * 4 : 0, kNarrow = VEC != 1 && LPR > 8 ? kGiantSlice : 0;
+    if (kOneSlice && t.width == (uint32_t)kOneSlice) {
+      all_runs(std::integral_constant<int, kOneSlice>());
+    } else if (kNarrow && t.width % kSlice == 0) {
+      long_role<VEC, K, kNarrow, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kGiantClasses,
+                                          blockIdx.x, kLongBlocks, tk);
+      long_role<VEC, K, (kNarrow ? kSlice : 0), kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, kGiantClasses,
+                                                         kLongBuckets, blockIdx.x, kLongBlocks, tk + kTicketLanes);
+    } else if (kNarrow && t.width % kGiantSlice == 0) {
+      all_runs(std::integral_constant<int, kNarrow>());
     } else {
-      long_role<VEC, K, 0, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kLongBuckets, blockIdx.x, kLongBlocks, tk);
+      all_runs(std::integral_constant<int, 0>());
     }
   } else if (blockIdx.x < kLongBlocks + kMedBlocks) { // medium runs take long per block: they start early
     medium_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, (uint32_t *)lds, blockIdx.x - kLongBlocks, kMedBlocks);
@@ -780,12 +824,16 @@ void launch_push_t(hipStream_t st, const TableView &t, int id_bits, const BatchV
 template <int VEC, typename K, bool kSingle, bool kPooled>
 void launch_push_p(hipStream_t ps, const TableView &t, int id_bits, const BatchView &p, uint32_t U,
                    const PushArgs &a) {
-  const uint32_t lanes = (t.width + VEC - 1) / VEC;
-  if (lanes <= 4) launch_push_t<VEC, 4, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-  else if (lanes <= 8) launch_push_t<VEC, 8, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-  else if (lanes <= 16) launch_push_t<VEC, 16, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-  else if (lanes <= 32) launch_push_t<VEC, 32, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-  else launch_push_t<VEC, 64, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+  const uint32_t lanes = (t.width + kCols<VEC> - 1) / kCols<VEC>;
+  if constexpr (VEC == 1) { // rows of less than four floats
+    launch_push_t<VEC, 4, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+  } else {
+    if (lanes <= 4) launch_push_t<VEC, 4, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+    else if (lanes <= 8) launch_push_t<VEC, 8, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+    else if (lanes <= 16) launch_push_t<VEC, 16, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+    else if (lanes <= 32) launch_push_t<VEC, 32, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+    else launch_push_t<VEC, 64, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+  }
 }
 
 template <int VEC, typename K, bool kSingle>
@@ -819,14 +867,17 @@ void launch_place_rows(hipStream_t s, const KeyLayout &kl, const BatchView &prev
 void launch_push(hipStream_t ps, const TableView &t, const KeyLayout &kl, const BatchView &prev, uint32_t n_unique,
                  const PushArgs &a) {
   if (!prev.n || !n_unique) return;
-  const bool vec4 = t.width % 4 == 0 && ((uintptr_t)a.grad % 16) == 0;
-  if (vec4) {
-    if (kl.wide) launch_push_k<4, uint64_t>(ps, t, kl.id_bits, prev, n_unique, a);
-    else launch_push_k<4, uint32_t>(ps, t, kl.id_bits, prev, n_unique, a);
-  } else {
-    if (kl.wide) launch_push_k<1, uint64_t>(ps, t, kl.id_bits, prev, n_unique, a);
-    else launch_push_k<1, uint32_t>(ps, t, kl.id_bits, prev, n_unique, a);
+#define PUSH(VEC)                                                                         \
+  do {                                                                                    \
+    if (kl.wide) launch_push_k<VEC, uint64_t>(ps, t, kl.id_bits, prev, n_unique, a);      \
+    else launch_push_k<VEC, uint32_t>(ps, t, kl.id_bits, prev, n_unique, a);              \
+  } while (0)
+  switch (row_vec(t.width, a.grad)) {
+    case 4: PUSH(4); break;
+    case kOdd4: PUSH(kOdd4); break;
+    default: PUSH(1); break;
   }
+#undef PUSH
   HCTR_HIP(hipGetLastError());
 }
 

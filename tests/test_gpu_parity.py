@@ -617,3 +617,31 @@ def test_push_pull_twice_without_preprocess(nrank):
         assert_close(out[r], ref[r], 1e-5, "dst rank %d after" % r)
     p.compare_state(1e-5, "after")
     p.close()
+
+
+@pytest.mark.parametrize("nrank", [1, 2])
+@pytest.mark.parametrize("width", [1, 3, 4, 5, 7, 16, 18, 31, 32, 37, 61, 65, 67, 96, 130, 160, 193, 259])
+def test_row_widths_between_the_vector_sizes(width, nrank):
+    # widths whose last vector of a row overlaps the one before (every remainder, one slice and several, a last slice of
+    # one to three columns), the narrowest rows, and widths that are whole slices of 16 and 32 columns; keys skewed enough
+    # for runs of every length
+    say("row width", width, "shards", nrank)
+    rng = np.random.default_rng(9000 + 2 * width + nrank)
+    length, n = 6_000, 9_000
+    root = rng.integers(0, nrank, size=length).astype(np.uint8)
+    storage = []
+    for r in range(nrank):
+        own, other = np.where(root == r)[0], np.where(root != r)[0]
+        storage.append(np.concatenate([other[::3], own]).astype(np.int64))
+    p = Pair(nrank, length, width, root, storage, init=("Uniform", -0.01, 0.01), lr=0.05, bounds=(2, 2) if nrank > 1 else (0, 0))
+    draw = zipf_sampler(length, 1.2, rng)
+    prev_n = 0
+    for step in range(3):
+        p.preprocess([draw(n) for _ in range(nrank)], device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(prev_n, width)).astype(np.float32) if prev_n else None
+                                for _ in range(nrank)])
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst rank %d step %d" % (r, step))
+        p.compare_state(1e-5, "step %d" % step)
+        prev_n = n
+    p.close()
