@@ -7,6 +7,7 @@
 #include "radix_sort.h"
 #include "run_lists.h"
 #include "tile_sort.h"
+#include "unique_tile.h"
 
 namespace hctr {
 namespace {
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(kSortBlock) void make_keys(const index_t *__restric
 #ifndef HCTR_UNIQUE_ITEMS
 #define HCTR_UNIQUE_ITEMS 8
 #endif
-constexpr int kUBlock = 512, kUItems = HCTR_UNIQUE_ITEMS, kUTile = kUBlock * kUItems;
+constexpr int kUItems = HCTR_UNIQUE_ITEMS, kUTile = kUBlock * kUItems;
 inline unsigned unique_tiles(uint32_t n) { return div_up(n, kUTile); }
 
 // Heads (sorted positions that hold another key than the position before) are counted per chunk of sorted positions,
@@ -115,16 +116,12 @@ __global__ __launch_bounds__(kUBlock) void unique_emit(const K *__restrict__ sk,
                                                        const uint32_t *__restrict__ head_inner,
                                                        const K *__restrict__ head_first, const K *__restrict__ head_last,
                                                        uint32_t chunk, BatchView b, uint32_t *__restrict__ u_copy) {
-  constexpr int NW = kUBlock / kWave;
   constexpr uint32_t kTileU = ITEMS * kUBlock;
-  __shared__ uint32_t sm[NW + 1];
-  __shared__ uint32_t wsum[ITEMS * NW + 1];
   const uint32_t base = blockIdx.x * kTileU;
   const unsigned lane = lane_id();
-  const int w = threadIdx.x / kWave;
   // everything that comes from memory first: the keys of the tile, the key before every wave's first position and the
   // head counts of the chunks before the tile
-  K key[ITEMS], edge[ITEMS], pk[ITEMS];
+  K key[ITEMS], edge[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; k++) {
     const uint32_t j = base + k * kUBlock + threadIdx.x;
@@ -135,60 +132,7 @@ __global__ __launch_bounds__(kUBlock) void unique_emit(const K *__restrict__ sk,
   const uint32_t chunks_before = base / chunk;
   for (uint32_t i = threadIdx.x; i < chunks_before; i += kUBlock)
     s += head_inner[i] + ((i == 0 || head_first[i] != head_last[i - 1]) ? 1u : 0u);
-  bool head[ITEMS];
-  uint32_t before[ITEMS];
-#pragma unroll
-  for (int k = 0; k < ITEMS; k++) {
-    const uint32_t j = base + k * kUBlock + threadIdx.x;
-    const bool valid = j < n;
-    const K up = (K)__shfl_up(key[k], 1, kWave);
-    pk[k] = lane == 0 ? edge[k] : up;
-    head[k] = valid && (j == 0 || key[k] != pk[k]);
-    const uint64_t m = __ballot(head[k]);
-    before[k] = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) wsum[k * NW + w] = __popcll(m);
-  }
-  // the directory lookups of the heads travel while the ranks are worked out
-  const K id_mask = (K)(((uint64_t)1 << id_bits) - 1);
-  slot_t off[ITEMS];
-#pragma unroll
-  for (int k = 0; k < ITEMS; k++) off[k] = head[k] ? slot[(uint64_t)(key[k] & id_mask)] : kNoSlot;
-  uint32_t prefix;
-  block_exclusive_scan<kUBlock>(s, sm, prefix); // unique ranks before this tile
-  if (threadIdx.x < kWave) { // the wave totals, in item order, by one wave
-    uint32_t run = 0;
-    for (int i0 = 0; i0 < ITEMS * NW; i0 += kWave) {
-      const bool in = i0 + (int)lane < ITEMS * NW;
-      const uint32_t v = in ? wsum[i0 + lane] : 0u;
-      const uint32_t inc = wave_inclusive_scan(v);
-      if (in) wsum[i0 + lane] = run + inc - v;
-      run += __shfl(inc, kWave - 1, kWave);
-    }
-  }
-  __syncthreads();
-  K *ukey = (K *)b.ukey;
-#pragma unroll
-  for (int k = 0; k < ITEMS; k++) {
-    const uint32_t j = base + k * kUBlock + threadIdx.x;
-    if (j >= n) continue;
-    const uint32_t rank = prefix + wsum[k * NW + w] + before[k] + (head[k] ? 1u : 0u) - 1u;
-    const int r = (int)(key[k] >> id_bits);
-    if (head[k]) {
-      ukey[rank] = key[k];
-      b.run_start[rank] = j;
-      b.uoff[rank] = off[k];
-      const int r_prev = j == 0 ? -1 : (int)(pk[k] >> id_bits);
-      for (int i = r_prev + 1; i <= r; i++) b.bucket_lo[i] = rank;
-    }
-    b.rank_sorted[j] = rank;
-    if (j == n - 1) {
-      const uint32_t U = rank + 1;
-      *b.d_U = U;
-      if (u_copy) *u_copy = U;
-      b.run_start[U] = n;
-      for (int i = r + 1; i <= nrank; i++) b.bucket_lo[i] = U;
-    }
-  }
+  emit_unique_tile<K, ITEMS>(key, edge, s, base, n, id_bits, nrank, slot, b, u_copy);
 }
 
 // The inverse index in batch order (the reference's d_idx_map).  The hot path works in sorted order

@@ -59,6 +59,7 @@ struct Batch {
   bool planned = false; // the push plan (need, prefix, push_cnt) has been computed for the batch as it stands
   bool lists_ready = true;  // the run lists of the batch's push have been built (or the batch is empty)
   bool tile_sorted = false; // indexed by the tile-sorted passes (tile_sort.h)
+  bool one_block = false;   // indexed by one block in one launch (tile_sort.h)
   bool direct_gather = false; // one shard, small batch: the step's gather works from `comp` in batch order and does not
                               // wait for the index (the run lists are then built in front of the batch's push)
   bool comp_valid = false;    // comp holds the batch's sort keys in batch order
@@ -154,7 +155,8 @@ class Shard {
   bool pooled_from_keys = true;   // HETUCTR_POOLED_FROM_KEYS=0: pooled gathers of one shard go through the inverse index
   uint32_t direct_gather_max = 0; // keys: HCTR_DIRECT_GATHER_BYTES / bytes of a row, or HETUCTR_DIRECT_GATHER_MAX
   int tile_sort_mode = 1;                    // HETUCTR_TILE_SORT: 0 no batch takes the tile-sorted passes, 1 those of up
-                                             // to kTileSortMaxKeys keys, 2 every batch whose tiles they can hold
+                                             // to kTileSortMaxKeys keys (up to kOneBlockKeys: one block does it all), 2
+                                             // every batch whose tiles they can hold
   void plan_batch(Batch &b);  // enqueues the push plan of b; its counts reach the host when the stream has run it
   void enqueue_readback_preprocess();
   void finish_preprocess();                 // after the stream sync: mirrors -> host fields, error checks

@@ -303,7 +303,8 @@ void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scr
       // One shard and a small batch: the step's gather works from the keys in batch order and leaves the index off
       // the step's critical path (write_back); the keys are then made by a kernel of their own here as well.
       cur.direct_gather = cfg.nrank == 1 && flag != nullptr && cur.n <= direct_gather_max;
-      cur.keys_made = !cur.tile_sorted || (flag != nullptr && cur.n >= kKeysFirstFrom);
+      cur.one_block = tile_sort_mode == 1 && cur.n <= kOneBlockKeys && kl.max_digit_bits == 0;
+      cur.keys_made = !cur.tile_sorted || cur.one_block || (flag != nullptr && cur.n >= kKeysFirstFrom);
       cur.comp_valid = true; // either kernel leaves the sort keys in batch order (a gather from the keys reads them)
       if (!cur.keys_made)
         launch_tile_sort_keys(s, tv, kl, ids, nullptr, cur.n, tile_sort_buffers(), flag ? flag : err_ptr(),
@@ -328,7 +329,12 @@ TileSortBuffers Shard::tile_sort_buffers() const {
 void Shard::index_batch(uint32_t *u_out, int part) {
   hipStream_t s = group->stream;
   // part 1: the first launches of the sort; part 2: everything after them; 0: all of it
-  if (cur.n != 0) {
+  if (cur.n != 0 && cur.one_block) { // everything is one launch: it goes out with the first part
+    if (part != 2) {
+      StageScope st(*group, S_SORT);
+      launch_index_one_block(s, tv, kl, cur.comp.p, cur.view(), u_out ? u_out : &dst_->U);
+    }
+  } else if (cur.n != 0) {
     // head counts per chunk: one wave's share of a sort tile with the tile-sorted passes, else a tile of the unique pass
     const HeadChunks heads = head_chunks_in(sp.headws, cur.n, kl.wide, cur.tile_sorted ? (uint32_t)tile_items(cur.n) * kWave : 4096u);
     const void *sorted_keys = nullptr;

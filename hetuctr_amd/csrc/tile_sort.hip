@@ -10,6 +10,7 @@
 // their tile and in the new order, so block o, which produces positions [o * tile, (o + 1) * tile) of the new order, finds
 // the pieces that overlap its range and copies them.
 #include "tile_sort.h"
+#include "unique_tile.h"
 
 namespace hctr {
 namespace {
@@ -439,6 +440,54 @@ __global__ __launch_bounds__(kSortBlock) void regroup(const K *__restrict__ in_k
   }
 }
 
+// The index of a small batch by one block (see tile_sort.h): the keys stay in the block's registers and LDS from the first
+// pass to the unique keys.  A pass ranks on DBITS bits whether the last digit needs them or not (the bits above a key's
+// are zero), so that its ballots are straight-line code.
+template <typename K, int ITEMS, int DBITS>
+__global__ __launch_bounds__(kSortBlock) void index_one_block(const K *__restrict__ keys, uint32_t n, int bits, int id_bits,
+                                                               int nrank, const slot_t *__restrict__ slot, BatchView b,
+                                                               uint32_t *__restrict__ u_copy) {
+  using S = TileShape<K, ITEMS>;
+  static_assert(kSortBlock == kUBlock, "the block that sorts the keys lists the unique ones");
+  __shared__ __align__(16) uint32_t area[S::kAreaWords];
+  __shared__ uint32_t bin_start[kSortMaxBins];
+  __shared__ uint32_t sm[kWaves + 1];
+  const int w = threadIdx.x / kWave;
+  const unsigned lane = lane_id();
+  const K *skey = (const K *)area;
+  const uint32_t *sval = area + S::kTile * (sizeof(K) / 4);
+  K key[ITEMS];
+  uint32_t val[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; r++) {
+    val[r] = w * S::kSub + r * kWave + lane;
+    key[r] = val[r] < n ? keys[val[r]] : (K)0;
+  }
+  for (int shift = 0; shift < bits; shift += DBITS) {
+    tile_sort_by_digit<K, ITEMS, DBITS>(key, val, n, shift, DBITS, area, bin_start, sm); // ends with a barrier
+    if (shift + DBITS < bits) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; r++) {
+        const uint32_t e = w * S::kSub + r * kWave + lane;
+        if (e < n) {
+          key[r] = skey[e];
+          val[r] = sval[e];
+        }
+      }
+      __syncthreads(); // the area takes the digit counters of the next pass
+    }
+  }
+  K edge[ITEMS];
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++) {
+    const uint32_t j = k * kSortBlock + threadIdx.x;
+    key[k] = j < n ? skey[j] : (K)0;
+    edge[k] = (lane == 0 && j < n && j > 0) ? skey[j - 1] : (K)0;
+    if (j < n) b.sorted_arg[j] = sval[j];
+  }
+  emit_unique_tile<K, ITEMS>(key, edge, 0u, 0u, n, id_bits, nrank, slot, b, u_copy);
+}
+
 // digit widths and shifts of the passes: the bits are split evenly, as radix_sort_positions does
 struct DigitPlan {
   int passes;
@@ -488,6 +537,35 @@ DigitPlan plan_digits(const KeyLayout &kl) {
       default: CALL(K, I, 0); break;              \
     }                                             \
   } while (0)
+
+void launch_index_one_block(hipStream_t s, const TableView &t, const KeyLayout &kl, const void *keys, const BatchView &b,
+                            uint32_t *u_copy) {
+  if (!b.n) return;
+  HCTR_CHECK(b.n <= kOneBlockKeys, "internal: batch too large for one block");
+  const int bits = kl.total_bits < 1 ? 1 : kl.total_bits;
+  const bool nine = (bits + 8) / 9 == (bits + 9) / 10; // narrower digits where they take as many passes
+  const int items = (int)div_up(b.n, kSortBlock);
+#define ONE(K, I, D) \
+  hipLaunchKernelGGL((index_one_block<K, I, D>), dim3(1), dim3(kSortBlock), 0, s, (const K *)keys, b.n, bits, kl.id_bits, t.nrank, t.slot, b, u_copy)
+#define ONE_D(K, I)                \
+  do {                             \
+    if (nine) ONE(K, I, 9);        \
+    else ONE(K, I, 10);            \
+  } while (0)
+#define ONE_K(K)                       \
+  do {                                 \
+    if (items <= 2) ONE_D(K, 2);       \
+    else if (items <= 4) ONE_D(K, 4);  \
+    else if (items <= 8) ONE_D(K, 8);  \
+    else ONE_D(K, 16);                 \
+  } while (0)
+  if (kl.wide) ONE_K(uint64_t);
+  else ONE_K(uint32_t);
+#undef ONE_K
+#undef ONE_D
+#undef ONE
+  HCTR_HIP(hipGetLastError());
+}
 
 void launch_tile_sort_keys(hipStream_t s, const TableView &t, const KeyLayout &kl, const index_t *ids,
                            const void *made_keys, uint32_t n, const TileSortBuffers &b, uint32_t *err, uint32_t *nlong,

@@ -645,3 +645,31 @@ def test_row_widths_between_the_vector_sizes(width, nrank):
         p.compare_state(1e-5, "step %d" % step)
         prev_n = n
     p.close()
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("length", [3, 500, 5_000, 200_000])
+def test_batches_indexed_by_one_block(length, wide, monkeypatch):
+    # one launch of one block: 2, 4, 8, 16 keys per thread, full and ragged, up to the largest batch it takes and the first
+    # one it does not; one to three passes of 9 or 10 bits; all keys equal (length 3) to nearly all distinct; a shard of
+    # a group, whose owner buckets come from the same launch, beside a single one
+    if wide:
+        monkeypatch.setenv("HETUCTR_FORCE_WIDE_KEYS", "1")
+    say("one-block index, rows", length, "64-bit keys" if wide else "32-bit keys")
+    width = 4
+    for nrank in (1, 2):
+        rng = np.random.default_rng(length + nrank)
+        root = rng.integers(0, nrank, size=length).astype(np.uint8)
+        storage = [np.flatnonzero(root == r).astype(np.int64) for r in range(nrank)]
+        p = Pair(nrank, length, width, root, storage, init=("Zero", 0.0, 0.0), lr=0.5)
+        prev_n = [0] * nrank
+        for n in [1, 64, 511, 513, 1024, 1025, 2049, 4096, 4097, 8191, 8192, 8193, 2]:
+            ns = [n if r == 0 else max(n // 3, 1) for r in range(nrank)]
+            p.preprocess([rng.integers(0, length, size=k).astype(np.int64) for k in ns], device_keys=n % 2 == 0)
+            p.compare_ints(INT_ITEMS_PRE, "n %d" % n)
+            out, ref = p.push_pull([rng.integers(-2, 3, size=(k, width)).astype(np.float32) if k else None for k in prev_n])
+            for r in range(nrank):
+                assert_close(out[r], ref[r], 1e-5, "dst n %d rank %d" % (n, r))
+            prev_n = ns
+        p.compare_state(1e-5, "end")
+        p.close()
