@@ -133,19 +133,38 @@ HostStager::~HostStager() {
   if (pinned_) (void)hipHostFree(pinned_);
 }
 
-void HostStager::copy(void *dst, const void *src, size_t bytes, hipStream_t s, bool narrow_ids) {
-  if (!bytes) return;
+// a staging buffer of `bytes` bytes that nothing reads any more but, possibly, work on `reader`
+void HostStager::reserve(size_t bytes, hipStream_t reader) {
   // the transfers of the call before read the staging buffer: they have normally completed long ago
   if (sent_) HCTR_HIP(hipEventSynchronize(sent_));
   else HCTR_HIP(hipEventCreateWithFlags(&sent_, hipEventDisableTiming));
   if (bytes > cap_) {
-    if (pinned_) HCTR_HIP(hipHostFree(pinned_));
+    if (pinned_) {
+      HCTR_HIP(hipStreamSynchronize(reader)); // a kernel that was lent the buffer
+      HCTR_HIP(hipHostFree(pinned_));
+    }
     pinned_ = nullptr;
     cap_ = 0;
     const size_t want = bytes + bytes / 4;
     HCTR_HIP(hipHostMalloc((void **)&pinned_, want, hipHostMallocDefault));
     cap_ = want;
   }
+}
+
+const void *HostStager::lend(const void *src, size_t bytes, hipStream_t s, bool narrow_ids) {
+  reserve(bytes, s);
+  auto job = std::make_shared<Job>(src, pinned_, bytes, narrow_ids);
+  if (bytes >= kCrewFrom && host_copy_threads() > 1) crew().post(job);
+  while (job->take_piece()) {
+  }
+  for (size_t i = 0; i < job->pieces; i++) // pieces other threads are still copying
+    while (!job->done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
+  return pinned_;
+}
+
+void HostStager::copy(void *dst, const void *src, size_t bytes, hipStream_t s, bool narrow_ids) {
+  if (!bytes) return;
+  reserve(bytes, s);
   auto job = std::make_shared<Job>(src, pinned_, bytes, narrow_ids);
   const bool alone = bytes < kCrewFrom || host_copy_threads() == 1;
   if (!alone) crew().post(job);

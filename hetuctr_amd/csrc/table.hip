@@ -286,16 +286,21 @@ void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scr
       const bool visible = hipPointerGetAttributes(&attr, keys) == hipSuccess &&
                            (attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged);
       bool narrowed = false;
+      const index_t *ids = (const index_t *)keys;
       if (!visible) {
         (void)hipGetLastError(); // an unregistered host pointer leaves a sticky "invalid value"
         HCTR_CHECK(!scratch_area, "preprocess without allocations takes ids in device memory only (a transfer from "
                                   "pageable host memory needs a staging buffer)");
         // through pinned memory, as 32-bit ids when the table's ids fit (half the bytes on the bus)
         narrowed = tv.id_max <= 0xffffffffull;
-        cur.staged.reserve(n * sizeof(index_t));
-        stager.copy(cur.staged.p, keys, n * sizeof(index_t), s, narrowed);
+        if (n * sizeof(index_t) <= HostStager::kLendUpTo) { // a small batch: the key kernel reads the pinned memory itself
+          ids = (const index_t *)stager.lend(keys, n * sizeof(index_t), s, narrowed);
+        } else {
+          cur.staged.reserve(n * sizeof(index_t));
+          stager.copy(cur.staged.p, keys, n * sizeof(index_t), s, narrowed);
+          ids = cur.staged.as<index_t>();
+        }
       }
-      const index_t *ids = visible ? (const index_t *)keys : (const index_t *)cur.staged.as<index_t>();
       cur.tile_sorted = tile_sort_mode == 2 ? tile_sort_possible(cur.n) : (tile_sort_mode == 1 && tile_sort_fits(cur.n));
       // A call that returns as soon as the ids are read (flag: where it looks for a bad id) gets them read by the
       // lightest kernel there is when the batch is large: the sort keys alone.  Sorting a tile as well keeps the
