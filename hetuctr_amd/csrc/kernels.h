@@ -116,20 +116,29 @@ void launch_idx_map(hipStream_t s, const BatchView &b);
 void launch_list_long_runs(hipStream_t s, const BatchView &b);
 inline uint32_t run_list_chunks(uint32_t n) { return (n + 255) / 256; } // enough for any number of unique keys <= n
 
-// device-wide exclusive scan of n (<= *d_n if d_n != nullptr) 32-bit values; block_sums: div_up(n_max,2048)+1 words.
-// total (optional) receives the sum.
-void launch_exclusive_scan(hipStream_t s, const uint32_t *in, uint32_t *out, uint32_t n_max, const uint32_t *d_n,
-                           uint32_t *block_sums, uint32_t *total);
+// Kernels of a step that every shard of a loopback group launches alike serve up to kShardsPerLaunch shards with one
+// launch: blockIdx.y picks the shard, the records travel as kernel arguments.  (A launch costs a small batch more than
+// its work: one launch
+// per shard and kernel made a step of four shards of 53 k keys 73 launches and 365 us, one for all 35 and 280 us.)
+constexpr int kShardsPerLaunch = 8;
 
-// push plan of the previous batch (csrc/core/preprocess.cu:148-165): need[u] in {0,1}
-void launch_decide_update(hipStream_t s, const TableView &t, const KeyLayout &kl, const BatchView &prev,
-                          uint32_t *need);
-// pushed rows per owner from the scanned plan: cnt[d] = prefix[lo[d+1]] - prefix[lo[d]]
-void launch_bucket_counts(hipStream_t s, const BatchView &b, const uint32_t *prefix, const uint32_t *total,
-                          int nrank, uint64_t *cnt_out, uint64_t *host_out);
-// both also write their counts to host_out (pinned host memory), bucket_sizes the number of unique keys to host_U
-void launch_bucket_sizes(hipStream_t s, const BatchView &b, int nrank, uint64_t *cnt_out, uint64_t *host_out,
-                         uint32_t *host_U);
+// Push plan of a batch (csrc/core/preprocess.cu:148-182) for every record: need[u] in {0,1}, prefix[u] = pushed rows before
+// u, *total their number, and pushed rows per owner: prefix[lo[d+1]] - prefix[lo[d]] in cnt_out[0..nrank] and, pinned host
+// memory, host_out.
+struct PlanShard {
+  TableView t;
+  BatchView b;
+  uint32_t *need, *prefix, *total, *block_sums; // block_sums: scan_blocks(n) + 1 words
+  uint64_t *cnt_out, *host_out;
+};
+void launch_plans(hipStream_t s, const KeyLayout &kl, const PlanShard *shards, int count);
+// unique keys per owner of every record's batch, in cnt_out[0..nrank] and host_out, and their number in host_U
+struct BucketShard {
+  const uint32_t *bucket_lo, *d_U;
+  uint64_t *cnt_out, *host_out;
+  uint32_t *host_U;
+};
+void launch_bucket_sizes(hipStream_t s, int nrank, const BucketShard *shards, int count);
 
 // Division of a batch position by the bag size of sum-pooled lookups without a divide instruction: for any 32-bit
 // n and bag >= 2, n / bag == (((n - q) >> 1) + q) >> shift with q = high word of n * magic (the "round up, add back"
@@ -177,20 +186,26 @@ struct PushArgs {
   version_t *g_cnt;
   embed_t *g_val;
 };
-// pos[u] = prefix[u] + delta[owner of unique key u] for the n_unique unique keys of `prev`: the place of a pushed row in
-// a receive area shared by all owners, from its place in the shard's own plan (delta: nrank words in device memory)
-void launch_place_rows(hipStream_t s, const KeyLayout &kl, const BatchView &prev, uint32_t n_unique,
-                       const uint32_t *prefix, const uint32_t *delta, uint32_t *pos);
-// n_unique: number of unique keys of `prev` (host copy)
-void launch_push(hipStream_t s, const TableView &t, const KeyLayout &kl, const BatchView &prev, uint32_t n_unique,
-                 const PushArgs &a);
+// pos[u] = prefix[u] + delta[owner of unique key u] for the n_unique unique keys of every record's batch: the place of a
+// pushed row in a receive area shared by all owners, from its place in the shard's own plan (delta: nrank words in device
+// memory)
+struct PlaceShard {
+  const void *ukey;
+  uint32_t n_unique;
+  const uint32_t *prefix, *delta;
+  uint32_t *pos;
+};
+void launch_place_rows(hipStream_t s, const KeyLayout &kl, const PlaceShard *shards, int count);
+// the pushes of every record's batch (one shard's, or those of the shards of a group, all with the same bag size)
+struct PushShard {
+  TableView t;
+  BatchView b;
+  PushArgs a;
+  uint32_t n_unique;         // number of unique keys of the batch (host copy)
+};
+void launch_push(hipStream_t s, const KeyLayout &kl, const PushShard *shards, int count);
 
 // ---- query / owner side / pull -------------------------------------------------------------------------
-// id and local version of every unique key of the current batch, written to place (unique rank + delta[owner of the
-// key]) of q_idx / q_ver (delta: nrank words in device memory).  unique_max: no more unique keys than this (the batch's
-// size); how many there are the kernel reads from cur.d_U.
-void launch_build_queries(hipStream_t s, const TableView &t, const KeyLayout &kl, const BatchView &cur, uint32_t unique_max,
-                          const uint32_t *delta, index_t *q_idx, version_t *q_ver);
 // Owner side of a step: applying the received pushes (per target row in source order) and serving the received
 // queries (outdated flags, positions of the rows to return, rows packed, first returned row of every requester).
 // One entry per shard of the group; one set of launches serves them all.
@@ -266,13 +281,28 @@ struct PullArgs {
   bool stream_stores;        // write dst with nontemporal stores (see Shard::write_back)
   uint32_t list_chunks;      // the gather also builds the batch's run lists (run_lists.h): chunks of unique ranks, else 0
 };
+// One shard of a loopback group as the kernels on its own batch see it; the launches below serve all records.
+struct PullShard {
+  TableView t;
+  BatchView b;               // n != 0
+  PullArgs a;
+  // queries: id and local version of every unique key of the batch, written to place (unique rank + delta[owner of the
+  // key]) of q_idx / q_ver (delta: nrank words in device memory)
+  const uint32_t *delta;
+  index_t *q_idx;
+  version_t *q_ver;
+  // refresh: scratch of scan_blocks(n) words; five device words that read zero before the first call (the launch leaves
+  // them zero again); four words the device can write (hit / miss / refreshed counts of the step, error bits)
+  uint32_t *tile_sums, *stats, *host_stats;
+  uint32_t unique_guess;     // the grid of the row kernel is cut from it (how many keys are unique the kernels read)
+};
+void launch_build_queries(hipStream_t s, const KeyLayout &kl, const PullShard *shards, int count);
 // Index of every returned row per unique key (a.ret_i), where the gather reads each key's row (a.src_row), the counts of
-// the step and the refresh of the cached rows that came back.  tile_sums: scratch of scan_blocks(unique_max) words (unique_max: the batch's size; the number of unique keys is read from cur.d_U; unique_guess: the grid of the row kernel is cut from it);
-// stats: five device words that read zero before the first call (the launch leaves them zero again); host_stats: four
-// words the device can write (hit / miss / refreshed counts of the step, error bits)
-void launch_refresh(hipStream_t s, const TableView &t, const BatchView &cur, uint32_t unique_max, uint32_t unique_guess,
-                    const PullArgs &a,
-                    uint32_t *tile_sums, uint32_t *stats, uint32_t *host_stats);
+// the step and the refresh of the cached rows that came back.
+void launch_refresh(hipStream_t s, const PullShard *shards, int count);
+// every key's row into a.dst (may be null: nothing to gather), and the run lists of the batch (a.list_chunks)
+void launch_gather_group(hipStream_t s, const PullShard *shards, int count);
+// one shard, every row local
 void launch_gather(hipStream_t s, const TableView &t, const BatchView &cur, const PullArgs &a);
 // one shard: dst[i] = row of the id in keys[i] (the batch's sort keys in batch order), for all n positions; needs
 // nothing of the batch's index

@@ -3,6 +3,8 @@
 // Reference: csrc/core/preprocess.cu:11-182 (kernels generate_sort_kv, write_sort_result,
 // preprocess_batch_data, compute_idx_map, block_cvt_offset_to_shape, decide_update and the
 // cub RunLengthEncode / ExclusiveSum calls between them).
+#include <algorithm>
+
 #include "kernels.h"
 #include "radix_sort.h"
 #include "run_lists.h"
@@ -149,88 +151,101 @@ __global__ __launch_bounds__(kRunListBlock) void list_long_runs(BatchView b) {
   list_runs_chunk(b, blockIdx.x, cnt, base);
 }
 
-// ---- generic device-wide exclusive scan (two launches, no inter-block waiting) ----------------------
-__global__ __launch_bounds__(kBlock) void scan_block_sums(const uint32_t *__restrict__ in, uint32_t n_max,
-                                                          const uint32_t *__restrict__ d_n,
-                                                          uint32_t *__restrict__ block_sums) {
-  __shared__ uint32_t sm[kBlock / kWave + 1];
-  const uint32_t n = d_n ? min(*d_n, n_max) : n_max;
-  const uint32_t j0 = blockIdx.x * kTile + threadIdx.x * kItems;
-  uint32_t c = 0;
-#pragma unroll
-  for (int k = 0; k < kItems; k++) c += (j0 + k < n) ? in[j0 + k] : 0u;
-  uint32_t total;
-  block_exclusive_scan<kBlock>(c, sm, total);
-  if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
+// ---- push plan, three launches for all shards of a group (blockIdx.y = record) ------------------------------------
+struct PlanShards { PlanShard s[kShardsPerLaunch]; };
+struct BucketShards { BucketShard s[kShardsPerLaunch]; };
+// the records in pieces of one launch each: f(piece, records in it, keys of the largest batch among them)
+template <typename P, typename S, typename F> void for_shards(const S *shards, int count, F &&f) {
+  for (int i = 0; i < count; i += kShardsPerLaunch) {
+    P p = {};
+    const int m = std::min(kShardsPerLaunch, count - i);
+    uint32_t n = 0;
+    for (int k = 0; k < m; k++) {
+      p.s[k] = shards[i + k];
+      n = std::max(n, shards[i + k].b.n);
+    }
+    if (n) f(p, m, n);
+  }
 }
 
-__global__ __launch_bounds__(kBlock) void scan_emit(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
-                                                    uint32_t n_max, const uint32_t *__restrict__ d_n,
-                                                    const uint32_t *__restrict__ block_sums,
-                                                    uint32_t *__restrict__ total_out) {
+// need[u] of one tile of unique keys and the tile's sum
+template <typename K>
+__global__ __launch_bounds__(kBlock) void plan_decide(PlanShards shards, int id_bits) {
   __shared__ uint32_t sm[kBlock / kWave + 1];
-  const uint32_t n = d_n ? min(*d_n, n_max) : n_max;
+  const PlanShard &S = shards.s[blockIdx.y];
+  const uint32_t U = *S.b.d_U;
+  if (blockIdx.x * kTile >= U) return; // the grid is cut for the largest batch's keys
+  uint32_t c = 0;
+#pragma unroll
+  for (int k = 0; k < kItems; k++) {
+    const uint32_t u = blockIdx.x * kTile + k * kBlock + threadIdx.x;
+    if (u >= U) continue;
+    const int r = (int)(((const K *)S.b.ukey)[u] >> id_bits);
+    const slot_t o = S.b.uoff[u];
+    const version_t cnt = (version_t)(S.b.run_start[u + 1] - S.b.run_start[u]);
+    uint32_t nd;
+    if (r == S.t.rank) nd = 0;
+    else if (o == kNoSlot) nd = 1;
+    else nd = (S.t.upd[o] + cnt <= S.t.push_bound) ? 0 : 1;
+    S.need[u] = nd;
+    c += nd;
+  }
+  uint32_t total;
+  block_exclusive_scan<kBlock>(c, sm, total);
+  if (threadIdx.x == 0) S.block_sums[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(kBlock) void plan_scan(PlanShards shards) {
+  __shared__ uint32_t sm[kBlock / kWave + 1];
+  const PlanShard &S = shards.s[blockIdx.y];
+  const uint32_t U = *S.b.d_U;
+  if (blockIdx.x * kTile >= U) return;
   uint32_t s = 0;
-  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kBlock) s += block_sums[i];
+  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kBlock) s += S.block_sums[i];
   uint32_t prefix;
   block_exclusive_scan<kBlock>(s, sm, prefix);
   const uint32_t j0 = blockIdx.x * kTile + threadIdx.x * kItems;
   uint32_t v[kItems], c = 0;
 #pragma unroll
   for (int k = 0; k < kItems; k++) {
-    v[k] = (j0 + k < n) ? in[j0 + k] : 0u;
+    v[k] = (j0 + k < U) ? S.need[j0 + k] : 0u;
     c += v[k];
   }
   uint32_t total;
   uint32_t run = prefix + block_exclusive_scan<kBlock>(c, sm, total);
+  const bool last = (blockIdx.x + 1) * kTile >= U;
 #pragma unroll
   for (int k = 0; k < kItems; k++) {
-    if (j0 + k < n) out[j0 + k] = run;
+    if (j0 + k < U) S.prefix[j0 + k] = run;
     run += v[k];
   }
-  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) *total_out = run;
+  if (last && threadIdx.x == kBlock - 1) *S.total = run;
 }
 
-template <typename K>
-__global__ __launch_bounds__(kBlock) void decide_update(TableView t, int id_bits, BatchView p,
-                                                        uint32_t *__restrict__ need) {
-  const uint32_t u = blockIdx.x * kBlock + threadIdx.x;
-  if (u >= *p.d_U) return;
-  const K key = ((const K *)p.ukey)[u];
-  const int r = (int)(key >> id_bits);
-  const slot_t o = p.uoff[u];
-  const version_t cnt = (version_t)(p.run_start[u + 1] - p.run_start[u]);
-  uint32_t nd;
-  if (r == t.rank) nd = 0;
-  else if (o == kNoSlot) nd = 1;
-  else nd = (t.upd[o] + cnt <= t.push_bound) ? 0 : 1;
-  need[u] = nd;
-}
-
-__global__ void bucket_counts(BatchView b, const uint32_t *__restrict__ prefix, const uint32_t *__restrict__ total,
-                              int nrank, uint64_t *__restrict__ cnt_out, uint64_t *__restrict__ host_out) {
+__global__ void plan_counts(PlanShards shards, int nrank) {
+  const PlanShard &S = shards.s[blockIdx.x];
   const int d = threadIdx.x;
   if (d > nrank) return;
   uint64_t c = 0;
   if (d < nrank) {
-    const uint32_t U = *b.d_U;
-    const uint32_t lo = b.bucket_lo[d], hi = b.bucket_lo[d + 1];
-    const uint32_t a = lo >= U ? *total : prefix[lo];
-    const uint32_t e = hi >= U ? *total : prefix[hi];
+    const uint32_t U = *S.b.d_U;
+    const uint32_t lo = S.b.bucket_lo[d], hi = S.b.bucket_lo[d + 1];
+    const uint32_t a = lo >= U ? *S.total : S.prefix[lo];
+    const uint32_t e = hi >= U ? *S.total : S.prefix[hi];
     c = U ? (uint64_t)(e - a) : 0;
   }
-  cnt_out[d] = c;
-  host_out[d] = c; // pinned host memory: the caller sizes the push buffers from it, no copy in between
+  S.cnt_out[d] = c;
+  S.host_out[d] = c; // pinned host memory: the caller sizes the push buffers from it, no copy in between
 }
 
-__global__ void bucket_sizes(BatchView b, int nrank, uint64_t *__restrict__ cnt_out, uint64_t *__restrict__ host_out,
-                             uint32_t *__restrict__ host_U) {
+__global__ void bucket_sizes(BucketShards shards, int nrank) {
+  const BucketShard &S = shards.s[blockIdx.x];
   const int d = threadIdx.x;
   if (d > nrank) return;
-  const uint64_t c = d == nrank ? 0 : (uint64_t)(b.bucket_lo[d + 1] - b.bucket_lo[d]);
-  cnt_out[d] = c;
-  host_out[d] = c; // pinned host memory, like the number of unique keys beside it
-  if (d == 0) *host_U = *b.d_U;
+  const uint64_t c = d == nrank ? 0 : (uint64_t)(S.bucket_lo[d + 1] - S.bucket_lo[d]);
+  S.cnt_out[d] = c;
+  S.host_out[d] = c; // pinned host memory, like the number of unique keys beside it
+  if (d == 0) *S.host_U = *S.d_U;
 }
 
 } // namespace
@@ -300,37 +315,25 @@ void launch_list_long_runs(hipStream_t s, const BatchView &b) { // the class cou
   HCTR_HIP(hipGetLastError());
 }
 
-void launch_exclusive_scan(hipStream_t s, const uint32_t *in, uint32_t *out, uint32_t n_max, const uint32_t *d_n,
-                           uint32_t *block_sums, uint32_t *total) {
-  if (!n_max) {
-    if (total) HCTR_HIP(hipMemsetAsync(total, 0, sizeof(uint32_t), s));
-    return;
+void launch_plans(hipStream_t s, const KeyLayout &kl, const PlanShard *shards, int count) {
+  for_shards<PlanShards>(shards, count, [&](const PlanShards &p, int m, uint32_t n) {
+    const dim3 grid(div_up(n, kTile), m);
+    if (kl.wide) hipLaunchKernelGGL(plan_decide<uint64_t>, grid, dim3(kBlock), 0, s, p, kl.id_bits);
+    else hipLaunchKernelGGL(plan_decide<uint32_t>, grid, dim3(kBlock), 0, s, p, kl.id_bits);
+    hipLaunchKernelGGL(plan_scan, grid, dim3(kBlock), 0, s, p);
+    const int nrank = p.s[0].t.nrank;
+    hipLaunchKernelGGL(plan_counts, dim3(m), dim3(nrank + 1), 0, s, p, nrank);
+    HCTR_HIP(hipGetLastError());
+  });
+}
+
+void launch_bucket_sizes(hipStream_t s, int nrank, const BucketShard *shards, int count) {
+  for (int i = 0; i < count; i += kShardsPerLaunch) {
+    BucketShards a = {};
+    const int m = std::min(kShardsPerLaunch, count - i);
+    std::copy(shards + i, shards + i + m, a.s);
+    hipLaunchKernelGGL(bucket_sizes, dim3(m), dim3(nrank + 1), 0, s, a, nrank);
   }
-  const unsigned nb = div_up(n_max, kTile);
-  hipLaunchKernelGGL(scan_block_sums, dim3(nb), dim3(kBlock), 0, s, in, n_max, d_n, block_sums);
-  hipLaunchKernelGGL(scan_emit, dim3(nb), dim3(kBlock), 0, s, in, out, n_max, d_n, block_sums, total);
-  HCTR_HIP(hipGetLastError());
-}
-
-void launch_decide_update(hipStream_t s, const TableView &t, const KeyLayout &kl, const BatchView &prev,
-                          uint32_t *need) {
-  if (!prev.n) return;
-  if (kl.wide)
-    hipLaunchKernelGGL(decide_update<uint64_t>, dim3(div_up(prev.n, kBlock)), dim3(kBlock), 0, s, t, kl.id_bits, prev, need);
-  else
-    hipLaunchKernelGGL(decide_update<uint32_t>, dim3(div_up(prev.n, kBlock)), dim3(kBlock), 0, s, t, kl.id_bits, prev, need);
-  HCTR_HIP(hipGetLastError());
-}
-
-void launch_bucket_counts(hipStream_t s, const BatchView &b, const uint32_t *prefix, const uint32_t *total,
-                          int nrank, uint64_t *cnt_out, uint64_t *host_out) {
-  hipLaunchKernelGGL(bucket_counts, dim3(1), dim3(nrank + 1), 0, s, b, prefix, total, nrank, cnt_out, host_out);
-  HCTR_HIP(hipGetLastError());
-}
-
-void launch_bucket_sizes(hipStream_t s, const BatchView &b, int nrank, uint64_t *cnt_out, uint64_t *host_out,
-                         uint32_t *host_U) {
-  hipLaunchKernelGGL(bucket_sizes, dim3(1), dim3(nrank + 1), 0, s, b, nrank, cnt_out, host_out, host_U);
   HCTR_HIP(hipGetLastError());
 }
 

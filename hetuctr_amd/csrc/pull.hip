@@ -3,6 +3,8 @@
 // every key's row into the caller's output.
 // Reference: csrc/core/generate_query.cu:91-106, csrc/core/handle_query.cu:7-116,
 // csrc/core/writeback.cu:8-56.
+#include <algorithm>
+
 #include "kernels.h"
 #include "run_lists.h"
 
@@ -36,17 +38,19 @@ template <int VEC> __device__ __forceinline__ void store_own(embed_t *row, typen
 // The queries of a step (csrc/core/generate_query.cu:91-106): per unique key its id and the version of the local copy
 // (invalid if the key is not resident here), written where the key's owner reads its queries: place u + delta[owner]
 // of a receive area all owners share.
+// (This and the other kernels of a shard's own batch: blockIdx.y = record, see kShardsPerLaunch.)
+struct PullShards { PullShard s[kShardsPerLaunch]; };
 template <typename K>
-__global__ __launch_bounds__(kBlock) void build_queries(TableView t, int id_bits, BatchView c,
-                                                        const uint32_t *__restrict__ delta, index_t *__restrict__ q_idx,
-                                                        version_t *__restrict__ q_ver) {
+__global__ __launch_bounds__(kBlock) void build_queries(PullShards shards, int id_bits) {
+  const PullShard &S = shards.s[blockIdx.y];
+  const BatchView &c = S.b;
   const uint32_t u = blockIdx.x * kBlock + threadIdx.x;
-  if (u >= *c.d_U) return;
+  if (u >= c.n || u >= *c.d_U) return;
   const slot_t o = c.uoff[u];
   const K key = ((const K *)c.ukey)[u];
-  const uint32_t pos = u + delta[(uint32_t)(key >> id_bits)];
-  q_idx[pos] = (index_t)(key & (K)(((uint64_t)1 << id_bits) - 1));
-  q_ver[pos] = o != kNoSlot ? t.ver[o] : kInvalidVersion;
+  const uint32_t pos = u + S.delta[(uint32_t)(key >> id_bits)];
+  S.q_idx[pos] = (index_t)(key & (K)(((uint64_t)1 << id_bits) - 1));
+  S.q_ver[pos] = o != kNoSlot ? S.t.ver[o] : kInvalidVersion;
 }
 
 // ---- owner side: every kernel below serves ALL shards of a loopback group in one launch (blockIdx.y = shard), the
@@ -389,10 +393,11 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
 // counters back to zero for the next step: no clearing launch before, no copy after.
 constexpr uint32_t kReturnedRow = 0x80000000u;
 constexpr int kRItems = 8, kRTile = kBlock * kRItems; // 2048 keys: the tile scan_blocks() sizes the scratch for
-__global__ __launch_bounds__(kBlock) void got_tile_sums(const uint32_t *__restrict__ got, const uint32_t *__restrict__ d_U,
-                                                        uint32_t *__restrict__ tile_sums) {
+__global__ __launch_bounds__(kBlock) void got_tile_sums(PullShards shards) {
   __shared__ uint32_t sm[kBlock / kWave + 1];
-  const uint32_t U = *d_U; // the grid is cut for the batch's keys: the host has not seen the number of unique ones
+  const PullShard &S = shards.s[blockIdx.y];
+  const uint32_t *__restrict__ got = S.a.got;
+  const uint32_t U = *S.b.d_U; // the grid is cut for the batches' keys: the host has not seen the number of unique ones
   if (blockIdx.x * kRTile >= U) return;
   const uint32_t j0 = blockIdx.x * kRTile + threadIdx.x * kRItems;
   uint32_t c = 0;
@@ -400,13 +405,17 @@ __global__ __launch_bounds__(kBlock) void got_tile_sums(const uint32_t *__restri
   for (int k = 0; k < kRItems; k++) c += (j0 + k < U) ? got[j0 + k] : 0u;
   uint32_t total;
   block_exclusive_scan<kBlock>(c, sm, total);
-  if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
+  if (threadIdx.x == 0) S.tile_sums[blockIdx.x] = total;
 }
-__global__ __launch_bounds__(kBlock) void remote_emit(TableView t, BatchView c, const uint32_t *__restrict__ got,
-                                                      const uint32_t *__restrict__ tile_sums,
-                                                      uint32_t *__restrict__ ret_i, uint32_t *__restrict__ src_row,
-                                                      uint32_t *__restrict__ stats, uint32_t *__restrict__ host_stats) {
+__global__ __launch_bounds__(kBlock) void remote_emit(PullShards shards) {
   __shared__ uint32_t sm[kBlock / kWave + 1];
+  const PullShard &S = shards.s[blockIdx.y];
+  const TableView &t = S.t;
+  const BatchView &c = S.b;
+  const uint32_t *__restrict__ got = S.a.got;
+  const uint32_t *__restrict__ tile_sums = S.tile_sums;
+  uint32_t *__restrict__ ret_i = S.a.ret_i, *__restrict__ src_row = S.a.src_row, *__restrict__ stats = S.stats;
+  uint32_t *__restrict__ host_stats = S.host_stats;
   const uint32_t U = *c.d_U;
   const uint32_t tiles = (U + kRTile - 1) / kRTile; // of the grid's blocks (cut for the batch's keys) these have work
   if (blockIdx.x >= tiles) return;
@@ -475,8 +484,12 @@ __global__ __launch_bounds__(kBlock) void remote_emit(TableView t, BatchView c, 
 
 // one group per unique rank of the current batch
 template <int VEC, int LPR>
-__global__ __launch_bounds__(kBlock) void refresh(TableView t, BatchView b, PullArgs a) {
+__global__ __launch_bounds__(kBlock) void refresh(PullShards shards) {
   typedef typename RowVec<VEC>::T V;
+  const PullShard &S = shards.s[blockIdx.y];
+  const TableView &t = S.t;
+  const BatchView &b = S.b;
+  const PullArgs &a = S.a;
   constexpr int kGroups = kBlock / LPR;
   const uint32_t U = *b.d_U, gl = threadIdx.x % LPR, W = t.width;
   for (uint32_t u = blockIdx.x * kGroups + threadIdx.x / LPR; u < U; u += gridDim.x * kGroups) {
@@ -503,7 +516,7 @@ constexpr int kRows = HCTR_GATHER_ROWS;
 // kStream: dst is written with nontemporal stores (a compile-time choice: merged into one store by the compiler, a
 // run-time one loses the hint)
 template <int VEC, int LPR, bool kLocalOnly, bool kStream>
-__global__ __launch_bounds__(kBlock) void gather(TableView t, BatchView b, PullArgs a) {
+__device__ __forceinline__ void gather_rows(const TableView &t, const BatchView &b, const PullArgs &a) {
   typedef typename RowVec<VEC>::T V;
   constexpr int kGroups = kBlock / LPR;
   const uint32_t n = b.n, W = t.width;
@@ -541,6 +554,16 @@ __global__ __launch_bounds__(kBlock) void gather(TableView t, BatchView b, PullA
         else *(V *)(dst[k] + col) = v[k];
       }
   }
+}
+
+template <int VEC, int LPR, bool kStream>
+__global__ __launch_bounds__(kBlock) void gather(TableView t, BatchView b, PullArgs a) {
+  gather_rows<VEC, LPR, true, kStream>(t, b, a);
+}
+template <int VEC, int LPR, bool kStream>
+__global__ __launch_bounds__(kBlock) void gather_group(PullShards shards) {
+  const PullShard &S = shards.s[blockIdx.y];
+  gather_rows<VEC, LPR, false, kStream>(S.t, S.b, S.a);
 }
 
 // Gather in BATCH order straight from the batch's keys, for one shard: dst[i] = emb[slot[id of position i]].  It needs
@@ -687,13 +710,27 @@ inline int lanes_for(uint32_t width, int vec) {
 
 } // namespace
 
-void launch_build_queries(hipStream_t s, const TableView &t, const KeyLayout &kl, const BatchView &cur, uint32_t unique_max,
-                          const uint32_t *delta, index_t *q_idx, version_t *q_ver) {
-  if (!unique_max) return;
-  const dim3 grid(div_up(unique_max, kBlock)); // the kernel reads the number of unique keys itself
-  if (kl.wide) hipLaunchKernelGGL(build_queries<uint64_t>, grid, dim3(kBlock), 0, s, t, kl.id_bits, cur, delta, q_idx, q_ver);
-  else hipLaunchKernelGGL(build_queries<uint32_t>, grid, dim3(kBlock), 0, s, t, kl.id_bits, cur, delta, q_idx, q_ver);
-  HCTR_HIP(hipGetLastError());
+// the records in pieces of one launch each: f(piece, records in it, keys of the largest batch among them)
+template <typename F> static void for_shards(const PullShard *shards, int count, F &&f) {
+  for (int i = 0; i < count; i += kShardsPerLaunch) {
+    PullShards p = {};
+    const int m = std::min(kShardsPerLaunch, count - i);
+    uint32_t n = 0;
+    for (int k = 0; k < m; k++) {
+      p.s[k] = shards[i + k];
+      n = std::max(n, shards[i + k].b.n);
+    }
+    if (n) f(p, m, n);
+  }
+}
+
+void launch_build_queries(hipStream_t s, const KeyLayout &kl, const PullShard *shards, int count) {
+  for_shards(shards, count, [&](const PullShards &p, int m, uint32_t n) {
+    const dim3 grid(div_up(n, kBlock), m); // the kernel reads the numbers of unique keys itself
+    if (kl.wide) hipLaunchKernelGGL(build_queries<uint64_t>, grid, dim3(kBlock), 0, s, p, kl.id_bits);
+    else hipLaunchKernelGGL(build_queries<uint32_t>, grid, dim3(kBlock), 0, s, p, kl.id_bits);
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
 size_t query_tiles(uint32_t q) { return std::max<size_t>(1, div_up(q, kBlock)); }
@@ -747,34 +784,54 @@ void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards,
   HCTR_HIP(hipGetLastError());
 }
 
-void launch_refresh(hipStream_t s, const TableView &t, const BatchView &cur, uint32_t unique_max, uint32_t unique_guess,
-                    const PullArgs &a, uint32_t *tile_sums, uint32_t *stats, uint32_t *host_stats) {
-  if (!unique_max || !a.got) return;
-  const unsigned tiles = div_up(unique_max, kRTile); // for the batch's keys; the kernels read how many are unique
-  hipLaunchKernelGGL(got_tile_sums, dim3(tiles), dim3(kBlock), 0, s, a.got, cur.d_U, tile_sums);
-  hipLaunchKernelGGL(remote_emit, dim3(tiles), dim3(kBlock), 0, s, t, cur, a.got, tile_sums, a.ret_i, a.src_row, stats,
-                     host_stats);
-  const int vec = row_vec(t.width, nullptr);
-  const int lpr = lanes_for(t.width, vec);
-#define CALL(V, L)                                                                                                      \
-  hipLaunchKernelGGL((refresh<V, L>), dim3(guessed_blocks(unique_guess, unique_max, kBlock / L)), dim3(kBlock), 0, s, t, cur, a)
-  HCTR_DISPATCH_ROW(vec, lpr, CALL);
+void launch_refresh(hipStream_t s, const PullShard *shards, int count) {
+  for_shards(shards, count, [&](const PullShards &p, int m, uint32_t n) {
+    const dim3 tiles(div_up(n, kRTile), m); // for the batches' keys; the kernels read how many are unique
+    hipLaunchKernelGGL(got_tile_sums, tiles, dim3(kBlock), 0, s, p);
+    hipLaunchKernelGGL(remote_emit, tiles, dim3(kBlock), 0, s, p);
+    uint32_t guess = 0;
+    for (int k = 0; k < m; k++) guess = std::max(guess, p.s[k].unique_guess);
+    const uint32_t width = p.s[0].t.width;
+    const int vec = row_vec(width, nullptr), lpr = lanes_for(width, vec);
+#define CALL(V, L) hipLaunchKernelGGL((refresh<V, L>), dim3(guessed_blocks(guess, n, kBlock / L), m), dim3(kBlock), 0, s, p)
+    HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
-  HCTR_HIP(hipGetLastError());
+    HCTR_HIP(hipGetLastError());
+  });
+}
+
+void launch_gather_group(hipStream_t s, const PullShard *shards, int count) {
+  for_shards(shards, count, [&](const PullShards &p, int m, uint32_t n) {
+    const uint32_t width = p.s[0].t.width;
+    int vec = 4;
+    bool stream = true;
+    for (int k = 0; k < m; k++) { // one kernel for all: vectors that suit every output, the common kind of stores
+      if (row_vec(width, p.s[k].a.dst) != 4) vec = row_vec(width, p.s[k].a.dst);
+      stream = stream && p.s[k].a.stream_stores;
+    }
+    const int lpr = lanes_for(width, vec);
+#define CALL(V, L)                                                                                             \
+  do {                                                                                                         \
+    const dim3 grid(div_up(div_up(n, kRows), kBlock / L), m);                                                  \
+    if (stream) hipLaunchKernelGGL((gather_group<V, L, true>), grid, dim3(kBlock), 0, s, p);                   \
+    else hipLaunchKernelGGL((gather_group<V, L, false>), grid, dim3(kBlock), 0, s, p);                         \
+  } while (0)
+    HCTR_DISPATCH_ROW(vec, lpr, CALL);
+#undef CALL
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
 void launch_gather(hipStream_t s, const TableView &t, const BatchView &cur, const PullArgs &a) {
   if (!cur.n) return;
+  HCTR_CHECK(t.nrank == 1, "internal: the gather of local rows is for one shard");
   const int vec = row_vec(t.width, a.dst);
   const int lpr = lanes_for(t.width, vec);
-  const bool local_only = a.got == nullptr;
 #define CALL(V, L)                                                                                               \
   do {                                                                                                           \
     const unsigned blocks = div_up(div_up(cur.n, kRows), kBlock / L);                                            \
-    if (local_only && a.stream_stores) hipLaunchKernelGGL((gather<V, L, true, true>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a); \
-    else if (local_only) hipLaunchKernelGGL((gather<V, L, true, false>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a); \
-    else if (a.stream_stores) hipLaunchKernelGGL((gather<V, L, false, true>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a); \
-    else hipLaunchKernelGGL((gather<V, L, false, false>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a);          \
+    if (a.stream_stores) hipLaunchKernelGGL((gather<V, L, true>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a);  \
+    else hipLaunchKernelGGL((gather<V, L, false>), dim3(blocks), dim3(kBlock), 0, s, t, cur, a);                 \
   } while (0)
   HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL

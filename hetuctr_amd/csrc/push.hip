@@ -737,10 +737,8 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
 // all roles in one launch: the long chains start first, medium and short blocks fill the machine behind them, the
 // version counters of a single shard come last
 template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
-#ifndef HCTR_PUSH_WAVES
-#define HCTR_PUSH_WAVES 4
-#endif
-__global__ __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR_PUSH_WAVES, 8))) void push_fused(TableView t, int id_bits, BatchView p, PushArgs a, uint32_t U) {
+__device__ __forceinline__ void push_block(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a, uint32_t U,
+                                           uint32_t block) {
   // one LDS area for whichever role the block plays: the row ring of the long role or the index staging of the
   // medium role (one slice of kLongRun indices per group)
   constexpr int kRingWords = kSlots * kRPT * kPushBlock * (int)kCols<VEC>;
@@ -749,7 +747,7 @@ __global__ __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR
   __shared__ uint4 run_table[kTable];
   __shared__ uint32_t run_totals[3];
   __shared__ float row_stash[kTable * kWave]; // long role: the table rows of a bundle's runs (one slice, one lane each)
-  if (blockIdx.x < kLongBlocks) {
+  if (block < kLongBlocks) {
     // Every block first takes tickets of the longest runs, which are cut into narrower column slices so that more
     // blocks feed each of them (the blocks of a saturated memory system get equal shares of it, and a chain
     // advances with the share of the block that feeds it), then tickets of the other long runs.
@@ -758,27 +756,27 @@ __global__ __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR
     // of 32 and 16 floats as one slice.
     auto all_runs = [&](auto csc) {
       long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kLongBuckets,
-                                                       blockIdx.x, kLongBlocks, tk);
+                                                       block, kLongBlocks, tk);
     };
     constexpr int kOneSlice = VEC != 1 && LPR <= 8 ? LPR * 4 : 0, kNarrow = VEC != 1 && LPR > 8 ? kGiantSlice : 0;
     if (kOneSlice && t.width == (uint32_t)kOneSlice) {
       all_runs(std::integral_constant<int, kOneSlice>());
     } else if (kNarrow && t.width % kSlice == 0) {
       long_role<VEC, K, kNarrow, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kGiantClasses,
-                                          blockIdx.x, kLongBlocks, tk);
+                                          block, kLongBlocks, tk);
       long_role<VEC, K, (kNarrow ? kSlice : 0), kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, kGiantClasses,
-                                                         kLongBuckets, blockIdx.x, kLongBlocks, tk + kTicketLanes);
+                                                         kLongBuckets, block, kLongBlocks, tk + kTicketLanes);
     } else if (kNarrow && t.width % kGiantSlice == 0) {
       all_runs(std::integral_constant<int, kNarrow>());
     } else {
       all_runs(std::integral_constant<int, 0>());
     }
-  } else if (blockIdx.x < kLongBlocks + kMedBlocks) { // medium runs take long per block: they start early
-    medium_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, (uint32_t *)lds, blockIdx.x - kLongBlocks, kMedBlocks);
+  } else if (block < kLongBlocks + kMedBlocks) { // medium runs take long per block: they start early
+    medium_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, (uint32_t *)lds, block - kLongBlocks, kMedBlocks);
   } else {
     constexpr int kGroups = kPushBlock / LPR;
     const uint32_t short_blocks = div_up_dev(U, kGroups * kRunsPerGroup);
-    const uint32_t b = blockIdx.x - kLongBlocks - kMedBlocks;
+    const uint32_t b = block - kLongBlocks - kMedBlocks;
     if (b < short_blocks) {
       short_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, b, U);
     } else {
@@ -804,81 +802,108 @@ __global__ __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR
   }
 }
 
-template <typename K>
-__global__ __launch_bounds__(256) void place_rows(const K *__restrict__ ukey, uint32_t U, int id_bits,
-                                                  const uint32_t *__restrict__ prefix,
-                                                  const uint32_t *__restrict__ delta, uint32_t *__restrict__ pos) {
+#ifndef HCTR_PUSH_WAVES
+#define HCTR_PUSH_WAVES 4
+#endif
+#define HCTR_PUSH_BOUNDS __launch_bounds__(kPushBlock) __attribute__((amdgpu_waves_per_eu(HCTR_PUSH_WAVES, 8)))
+template <int VEC, int LPR, typename K, bool kPooled>
+__global__ HCTR_PUSH_BOUNDS void push_fused(TableView t, int id_bits, BatchView p, PushArgs a, uint32_t U) {
+  push_block<VEC, LPR, K, true, kPooled>(t, id_bits, p, a, U, blockIdx.x);
+}
+// The pushes of the shards of a group in one launch: neighbouring blocks are the same block of different shards, so that
+// every shard's long chains start first.
+struct PushShards { PushShard s[kShardsPerLaunch]; };
+template <int VEC, int LPR, typename K, bool kPooled>
+__global__ HCTR_PUSH_BOUNDS void push_group(PushShards shards, uint32_t count, int id_bits) {
+  const PushShard &S = shards.s[blockIdx.x % count];
+  push_block<VEC, LPR, K, false, kPooled>(S.t, id_bits, S.b, S.a, S.n_unique, blockIdx.x / count);
+}
+
+struct PlaceShards { PlaceShard s[kShardsPerLaunch]; };
+template <typename K> __global__ __launch_bounds__(256) void place_rows(PlaceShards shards, int id_bits) {
+  const PlaceShard &S = shards.s[blockIdx.y];
   const uint32_t u = blockIdx.x * 256 + threadIdx.x;
-  if (u < U) pos[u] = prefix[u] + delta[(uint32_t)(ukey[u] >> id_bits)];
+  if (u < S.n_unique) S.pos[u] = S.prefix[u] + S.delta[(uint32_t)(((const K *)S.ukey)[u] >> id_bits)];
 }
 
-template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
-void launch_push_t(hipStream_t st, const TableView &t, int id_bits, const BatchView &p, uint32_t U, const PushArgs &a) {
+template <int VEC, int LPR, typename K, bool kPooled>
+void launch_push_t(hipStream_t st, int id_bits, const PushShards &shards, int count) {
   constexpr int kGroups = kPushBlock / LPR;
-  const unsigned ver_blocks = div_up(U, kPushBlock); // the counters of every unique key
-  const unsigned rest = kMedBlocks + div_up(U, kGroups * kRunsPerGroup) + ver_blocks;
-  hipLaunchKernelGGL((push_fused<VEC, LPR, K, kSingle, kPooled>), dim3(kLongBlocks + rest), dim3(kPushBlock), 0, st, t, id_bits, p,
-                     a, U);
+  unsigned blocks = 0; // of the shard with the most: chains, medium runs, short runs, the counters of every unique key
+  for (int i = 0; i < count; i++) {
+    const uint32_t U = shards.s[i].n_unique;
+    blocks = std::max(blocks, kLongBlocks + kMedBlocks + div_up(U, kGroups * kRunsPerGroup) + div_up(U, kPushBlock));
+  }
+  const PushShard &S = shards.s[0];
+  if (S.t.nrank == 1)
+    hipLaunchKernelGGL((push_fused<VEC, LPR, K, kPooled>), dim3(blocks), dim3(kPushBlock), 0, st, S.t, id_bits, S.b, S.a, S.n_unique);
+  else
+    hipLaunchKernelGGL((push_group<VEC, LPR, K, kPooled>), dim3(blocks * count), dim3(kPushBlock), 0, st, shards, (uint32_t)count, id_bits);
 }
 
-template <int VEC, typename K, bool kSingle, bool kPooled>
-void launch_push_p(hipStream_t ps, const TableView &t, int id_bits, const BatchView &p, uint32_t U,
-                   const PushArgs &a) {
-  const uint32_t lanes = (t.width + kCols<VEC> - 1) / kCols<VEC>;
+template <int VEC, typename K, bool kPooled>
+void launch_push_p(hipStream_t st, int id_bits, const PushShards &shards, int count) {
   if constexpr (VEC == 1) { // rows of less than four floats
-    launch_push_t<VEC, 4, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+    launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
   } else {
-    if (lanes <= 4) launch_push_t<VEC, 4, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-    else if (lanes <= 8) launch_push_t<VEC, 8, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-    else if (lanes <= 16) launch_push_t<VEC, 16, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-    else if (lanes <= 32) launch_push_t<VEC, 32, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
-    else launch_push_t<VEC, 64, K, kSingle, kPooled>(ps, t, id_bits, p, U, a);
+    const uint32_t lanes = (shards.s[0].t.width + kCols<VEC> - 1) / kCols<VEC>;
+    if (lanes <= 4) launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
+    else if (lanes <= 8) launch_push_t<VEC, 8, K, kPooled>(st, id_bits, shards, count);
+    else if (lanes <= 16) launch_push_t<VEC, 16, K, kPooled>(st, id_bits, shards, count);
+    else if (lanes <= 32) launch_push_t<VEC, 32, K, kPooled>(st, id_bits, shards, count);
+    else launch_push_t<VEC, 64, K, kPooled>(st, id_bits, shards, count);
   }
 }
 
-template <int VEC, typename K, bool kSingle>
-void launch_push_v(hipStream_t ps, const TableView &t, int id_bits, const BatchView &p, uint32_t U,
-                   const PushArgs &a) {
-  if (a.bag.bag > 1) launch_push_p<VEC, K, kSingle, true>(ps, t, id_bits, p, U, a);
-  else launch_push_p<VEC, K, kSingle, false>(ps, t, id_bits, p, U, a);
-}
-
 template <int VEC, typename K>
-void launch_push_k(hipStream_t ps, const TableView &t, int id_bits, const BatchView &p, uint32_t U,
-                   const PushArgs &a) {
-  if (t.nrank == 1) launch_push_v<VEC, K, true>(ps, t, id_bits, p, U, a);
-  else launch_push_v<VEC, K, false>(ps, t, id_bits, p, U, a);
+void launch_push_k(hipStream_t st, int id_bits, const PushShards &shards, int count) {
+  if (shards.s[0].a.bag.bag > 1) launch_push_p<VEC, K, true>(st, id_bits, shards, count);
+  else launch_push_p<VEC, K, false>(st, id_bits, shards, count);
 }
 
 } // namespace
 
-void launch_place_rows(hipStream_t s, const KeyLayout &kl, const BatchView &prev, uint32_t n_unique,
-                       const uint32_t *prefix, const uint32_t *delta, uint32_t *pos) {
-  if (!n_unique) return;
-  if (kl.wide)
-    hipLaunchKernelGGL(place_rows<uint64_t>, dim3(div_up(n_unique, 256)), dim3(256), 0, s, (const uint64_t *)prev.ukey,
-                       n_unique, kl.id_bits, prefix, delta, pos);
-  else
-    hipLaunchKernelGGL(place_rows<uint32_t>, dim3(div_up(n_unique, 256)), dim3(256), 0, s, (const uint32_t *)prev.ukey,
-                       n_unique, kl.id_bits, prefix, delta, pos);
-  HCTR_HIP(hipGetLastError());
+void launch_place_rows(hipStream_t s, const KeyLayout &kl, const PlaceShard *shards, int count) {
+  for (int i = 0; i < count; i += kShardsPerLaunch) {
+    PlaceShards p = {};
+    const int m = std::min(kShardsPerLaunch, count - i);
+    uint32_t most = 0;
+    for (int k = 0; k < m; k++) {
+      p.s[k] = shards[i + k];
+      most = std::max(most, p.s[k].n_unique);
+    }
+    if (!most) continue;
+    const dim3 grid(div_up(most, 256), m);
+    if (kl.wide) hipLaunchKernelGGL(place_rows<uint64_t>, grid, dim3(256), 0, s, p, kl.id_bits);
+    else hipLaunchKernelGGL(place_rows<uint32_t>, grid, dim3(256), 0, s, p, kl.id_bits);
+    HCTR_HIP(hipGetLastError());
+  }
 }
 
-void launch_push(hipStream_t ps, const TableView &t, const KeyLayout &kl, const BatchView &prev, uint32_t n_unique,
-                 const PushArgs &a) {
-  if (!prev.n || !n_unique) return;
-#define PUSH(VEC)                                                                         \
-  do {                                                                                    \
-    if (kl.wide) launch_push_k<VEC, uint64_t>(ps, t, kl.id_bits, prev, n_unique, a);      \
-    else launch_push_k<VEC, uint32_t>(ps, t, kl.id_bits, prev, n_unique, a);              \
+void launch_push(hipStream_t s, const KeyLayout &kl, const PushShard *shards, int count) {
+  for (int i = 0; i < count;) {
+    PushShards p = {};
+    int m = 0, vec = 4;
+    for (; i < count && m < kShardsPerLaunch; i++) {
+      if (!shards[i].b.n || !shards[i].n_unique) continue;
+      p.s[m++] = shards[i];
+      const int v = row_vec(shards[i].t.width, shards[i].a.grad);
+      if (v != 4) vec = v; // vectors that suit every shard's gradient
+    }
+    if (!m) break;
+#define PUSH(VEC)                                                       \
+  do {                                                                  \
+    if (kl.wide) launch_push_k<VEC, uint64_t>(s, kl.id_bits, p, m);     \
+    else launch_push_k<VEC, uint32_t>(s, kl.id_bits, p, m);             \
   } while (0)
-  switch (row_vec(t.width, a.grad)) {
-    case 4: PUSH(4); break;
-    case kOdd4: PUSH(kOdd4); break;
-    default: PUSH(1); break;
-  }
+    switch (vec) {
+      case 4: PUSH(4); break;
+      case kOdd4: PUSH(kOdd4); break;
+      default: PUSH(1); break;
+    }
 #undef PUSH
-  HCTR_HIP(hipGetLastError());
+    HCTR_HIP(hipGetLastError());
+  }
 }
 
 } // namespace hctr

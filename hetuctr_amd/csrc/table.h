@@ -157,7 +157,7 @@ class Shard {
   int tile_sort_mode = 1;                    // HETUCTR_TILE_SORT: 0 no batch takes the tile-sorted passes, 1 those of up
                                              // to kTileSortMaxKeys keys (up to kOneBlockKeys: one block does it all), 2
                                              // every batch whose tiles they can hold
-  void plan_batch(Batch &b);  // enqueues the push plan of b; its counts reach the host when the stream has run it
+  bool plan_record(Batch &b, PlanShard &o); // this shard's part of a launch of plans; false: b is empty, nothing to plan
   void enqueue_readback_preprocess();
   void finish_preprocess();                 // after the stream sync: mirrors -> host fields, error checks
   // the same in two halves, for a preprocess whose push plan and index run on different streams
@@ -166,13 +166,17 @@ class Shard {
   void check_key_error();                   // raises if the ingested batch held a key outside [0, length)
   // the push of a step in two halves, so that a group can place every shard's pushed rows before any push kernel runs
   void begin_push(const float *grad, uint32_t bag = 1);  // which batch is pushed (none on an inference step), checks
-  void generate_gradient(const uint32_t *delta);         // the push kernel; delta: see Group::place_pushes
-  void generate_query(const uint32_t *delta); // delta: see Group::place_queries
+  bool push_record(PushShard &o);                        // what the push kernel needs of this shard; false: nothing
   // handleGradient + handleQuery: what the group's owner-side launches need of this shard (queries_max: no shard
   // receives more queries than this)
   void fill_owner_args(OwnerShard &o, uint64_t queries_max);
   void finish_handle_query();               // after the step: return counts and error flags from the pinned block
-  void write_back(float *dst, uint32_t bag = 1);
+  // several shards: what the query, refresh and gather launches need of this one (delta: see QueryArea::query_delta)
+  bool pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *delta);
+  PullArgs pull_args(float *dst) const;
+  uint32_t take_list_chunks();
+  void gather_bags(const PullArgs &a, uint32_t bag);
+  void write_back(float *dst, uint32_t bag = 1); // one shard
   bool direct_now(uint32_t bag) const; // this step's gather works from the keys and does not wait for the index
   void finish_push_pull();
 
@@ -195,7 +199,7 @@ class Shard {
   DevStat *dst_ = nullptr; // == dstat.p
   uint32_t *err_ptr() const { return &dst_->err; }
   // send side
-  const float *push_grad_ = nullptr; // arguments of the push between begin_push and generate_gradient
+  const float *push_grad_ = nullptr; // arguments of the push between begin_push and push_record
   uint32_t push_bag_ = 1;
   // receive side (owner role)
   DeviceBuf src_row, ret_seg_dev;
@@ -269,6 +273,9 @@ class Group {
   bool index_rest_pending = false;       // single shard: preprocess enqueued only the first launches of the index
   void enqueue_index_rest();
   void enqueue_index_all(int part);             // enqueues the others
+  void enqueue_bucket_sizes(bool empty);
+  // enqueues the push plans of one batch of each of the shards; the counts reach the host when the stream has run it
+  void plan_batches(const std::vector<Shard *> &shards, Batch Shard::*which);
   void flush_index();                    // waits for a pending index and takes its results over
   // owner-side arguments of every shard: pinned staging and the device copy the kernels read
   OwnerShard *owner_host = nullptr;

@@ -378,8 +378,18 @@ void Shard::index_batch(uint32_t *u_out, int part) {
     // index or never came (lists_ready)
     // (built behind the index instead, they make the index the longer of a small step's two chains: 78 us against 64)
   }
-  if (part == 1) return;
-  if (cfg.nrank > 1) launch_bucket_sizes(s, cur.view(), cfg.nrank, dst_->send_cnt, mirror->st.send_cnt, &mirror->st.U);
+}
+
+// several shards: queries per owner of every shard's batch, behind the indexes of all of them (empty: the empty batches too)
+void Group::enqueue_bucket_sizes(bool empty) {
+  if (nrank == 1) return;
+  std::vector<BucketShard> v;
+  for (Shard *m : members)
+    if (m->cur.n != 0 || empty) {
+      const BatchView b = m->cur.view();
+      v.push_back({b.bucket_lo, b.d_U, m->dst_->send_cnt, m->mirror->st.send_cnt, &m->mirror->st.U});
+    }
+  launch_bucket_sizes(stream, nrank, v.data(), (int)v.size());
 }
 
 // The push plan of a batch (csrc/core/preprocess.cu:148-182): which of its remote unique keys are pushed when it is
@@ -387,23 +397,34 @@ void Shard::index_batch(uint32_t *u_out, int part) {
 // of the cached rows as the push of the step before left them, and nothing changes either between the end of that
 // step and the preprocess call the reference computes the plan in: push_pull computes it for its current batch (beside
 // the owner-side work, on the second stream), and the next preprocess finds it done.
-void Shard::plan_batch(Batch &b) {
-  hipStream_t s = group->stream;
-  if (cfg.nrank == 1) return; // single shard: every key is owned, nothing is ever pushed
+bool Shard::plan_record(Batch &b, PlanShard &o) {
   if (b.n == 0) {
     for (int i = 0; i <= cfg.nrank; i++) mirror->st.push_cnt[i] = 0; // nothing in flight writes the block
-    return;
+    return false;
   }
   b.need.reserve((size_t)b.n * 4);
   b.prefix.reserve((size_t)b.n * 4);
   b.plan_total.reserve(4);
   plan_sums.reserve((scan_blocks(b.n) + 2) * 4); // its own: the index of the next batch may be running beside it
-  StageScope st(*group, S_PLAN);
-  launch_decide_update(s, tv, kl, b.view(), b.need.as<uint32_t>());
-  launch_exclusive_scan(s, b.need.as<uint32_t>(), b.prefix.as<uint32_t>(), b.n, b.dU.as<uint32_t>(),
-                        plan_sums.as<uint32_t>(), b.plan_total.as<uint32_t>());
-  launch_bucket_counts(s, b.view(), b.prefix.as<uint32_t>(), b.plan_total.as<uint32_t>(), cfg.nrank, dst_->push_cnt,
-                       mirror->st.push_cnt);
+  o.t = tv;
+  o.b = b.view();
+  o.need = b.need.as<uint32_t>();
+  o.prefix = b.prefix.as<uint32_t>();
+  o.total = b.plan_total.as<uint32_t>();
+  o.block_sums = plan_sums.as<uint32_t>();
+  o.cnt_out = dst_->push_cnt;
+  o.host_out = mirror->st.push_cnt;
+  return true;
+}
+
+void Group::plan_batches(const std::vector<Shard *> &shards, Batch Shard::*which) {
+  if (nrank == 1) return; // single shard: every key is owned, nothing is ever pushed
+  std::vector<PlanShard> v;
+  PlanShard r;
+  for (Shard *m : shards)
+    if (m->plan_record(m->*which, r)) v.push_back(r);
+  StageScope st(*this, S_PLAN);
+  if (!v.empty()) launch_plans(stream, members[0]->kl, v.data(), (int)v.size());
 }
 
 void Shard::enqueue_readback_preprocess() {
@@ -470,43 +491,26 @@ void Shard::begin_push(const float *grad, uint32_t bag) {
   HCTR_CHECK(prev.n % bag == 0, "pooled push: the previous batch is not a whole number of bags");
 }
 
-void Shard::generate_gradient(const uint32_t *delta) {
-  if (!prev_active) return;
-  hipStream_t s = group->stream;
-  PushArgs a;
-  a.grad = push_grad_;
-  a.bag = BagDiv(push_bag_);
-  a.need = nullptr;
-  a.prefix = nullptr;
-  a.g_idx = nullptr;
-  a.g_cnt = nullptr;
-  a.g_val = nullptr;
+bool Shard::push_record(PushShard &o) {
+  if (!prev_active) return false;
   if (!prev.lists_ready) { // no gather has seen this batch (a second preprocess came first, or a call without output)
-    launch_list_long_runs(s, prev.view());
+    launch_list_long_runs(group->stream, prev.view());
     prev.lists_ready = true;
   }
-  StageScope st(*group, S_PUSH);
+  o = PushShard();
+  o.t = tv;
+  o.b = prev.view();
+  o.n_unique = prev.U;
+  o.a.grad = push_grad_;
+  o.a.bag = BagDiv(push_bag_);
   if (cfg.nrank > 1) {
-    // the pushed rows go straight into the group's receive area: plan position -> position there
-    push_pos.reserve((size_t)std::max<uint32_t>(prev.U, 1) * 4);
-    launch_place_rows(s, kl, prev.view(), prev.U, prev.prefix.as<uint32_t>(), delta, push_pos.as<uint32_t>());
-    a.need = prev.need.as<uint32_t>();
-    a.prefix = push_pos.as<uint32_t>();
-    a.g_idx = group->rg_idx_all.as<index_t>();
-    a.g_cnt = group->rg_cnt_all.as<version_t>();
-    a.g_val = group->rg_val_all.as<embed_t>();
+    o.a.need = prev.need.as<uint32_t>();
+    o.a.prefix = push_pos.as<uint32_t>(); // the pushed rows go straight into the group's receive area (place_pushes)
+    o.a.g_idx = group->rg_idx_all.as<index_t>();
+    o.a.g_cnt = group->rg_cnt_all.as<version_t>();
+    o.a.g_val = group->rg_val_all.as<embed_t>();
   }
-  launch_push(s, tv, kl, prev.view(), prev.U, a);
-}
-
-// csrc/core/generate_query.cu:91-106
-void Shard::generate_query(const uint32_t *delta) {
-  if (cfg.nrank == 1) return; // a shard never finds its own rows outdated (handle_query.cu:47-54)
-  hipStream_t s = group->stream;
-  StageScope st(*group, S_QUERY);
-  // every query is written where its owner reads it: the group's receive area (see Group::place_queries)
-  launch_build_queries(s, tv, kl, cur.view(), cur.n, delta, group->rq_idx_all.as<index_t>(),
-                       group->rq_ver_all.as<version_t>());
+  return true;
 }
 
 // What the owner-side kernels need of this shard for the step (csrc/core/handle_query.cu:7-116): the received pushes
@@ -571,57 +575,77 @@ bool Shard::direct_now(uint32_t bag) const {
 }
 
 // csrc/core/writeback.cu:43-56
-void Shard::write_back(float *dst, uint32_t bag) {
-  hipStream_t s = group->stream;
-  PullArgs a;
-  a.got = nullptr;
-  a.ret_i = nullptr;
-  a.src_row = nullptr;
-  a.in_ver = nullptr;
-  a.in_val = nullptr;
+PullArgs Shard::pull_args(float *dst) const {
+  PullArgs a = {};
   a.dst = dst;
-  a.list_chunks = 0;
   // The gathered rows are not read again by this library: streamed past the caches they leave the table rows of the
   // batch there for the push that updates them next.  The one case where that loses is a batch of (almost) all
   // distinct keys, where the gather reads as many rows as it writes; the previous batch is the predictor.
   a.stream_stores = !(prev.n != 0 && (double)prev.U >= 0.9 * (double)prev.n);
-  if (cfg.nrank > 1 && cur.n == 0) {
+  return a;
+}
+
+// a gather follows that builds the batch's run lists on its way, in its first blocks (if nobody has): their number
+uint32_t Shard::take_list_chunks() {
+  if (cur.lists_ready || cur.n == 0) return 0;
+  cur.lists_ready = true;
+  return run_list_chunks(cur.n);
+}
+
+// several shards: this shard's part of the launches on the requesters' own batches; false: its batch is empty
+bool Shard::pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *delta) {
+  if (cur.n == 0) {
     memset(mirror->stats, 0, sizeof mirror->stats); // no keys: nothing came back (nothing in flight writes the block)
-  } else if (cfg.nrank > 1) {
-    // sized for the batch's keys: how many of them are unique the kernels read on the device (the host has not
-    // waited for the index); the scan scratch is the one the batch's index was given, its kernels are through
-    ret_i.reserve((size_t)cur.n * 4);
-    src_row.reserve((size_t)cur.n * 4);
-    StageScope st(*group, S_REFRESH);
-    a.got = got.as<uint32_t>();
-    a.ret_i = ret_i.as<uint32_t>();
-    a.src_row = src_row.as<uint32_t>();
-    a.in_ver = in_ver.as<version_t>();
-    a.in_val = in_val.as<embed_t>();
-    launch_refresh(s, tv, cur.view(), cur.n, prev.U ? prev.U : cur.n, a, sp.block_sums, stats.as<uint32_t>(), mirror->stats);
+    return false;
   }
-  if (dst != nullptr && direct_now(bag)) {
-    StageScope st(*group, S_GATHER);
-    HCTR_CHECK(cur.n % bag == 0, "pooled pull: the batch is not a whole number of bags");
+  HCTR_CHECK(dst == nullptr || cur.n % bag == 0, "pooled pull: the batch is not a whole number of bags");
+  // sized for the batch's keys: how many of them are unique the kernels read on the device (the host has not
+  // waited for the index); the scan scratch is the one the batch's index was given, its kernels are through
+  ret_i.reserve((size_t)cur.n * 4);
+  src_row.reserve((size_t)cur.n * 4);
+  o.t = tv;
+  o.b = cur.view();
+  o.a = pull_args(dst);
+  o.a.got = got.as<uint32_t>();
+  o.a.ret_i = ret_i.as<uint32_t>();
+  o.a.src_row = src_row.as<uint32_t>();
+  o.a.in_ver = in_ver.as<version_t>();
+  o.a.in_val = in_val.as<embed_t>();
+  if (dst != nullptr) o.a.list_chunks = take_list_chunks();
+  o.delta = delta;
+  o.q_idx = group->rq_idx_all.as<index_t>();
+  o.q_ver = group->rq_ver_all.as<version_t>();
+  o.tile_sums = sp.block_sums;
+  o.stats = stats.as<uint32_t>();
+  o.host_stats = mirror->stats;
+  o.unique_guess = prev.U ? prev.U : cur.n;
+  return true;
+}
+
+// one shard: every row is local
+void Shard::write_back(float *dst, uint32_t bag) {
+  if (dst == nullptr) return;
+  hipStream_t s = group->stream;
+  PullArgs a = pull_args(dst);
+  StageScope st(*group, S_GATHER);
+  HCTR_CHECK(cur.n % bag == 0, "pooled pull: the batch is not a whole number of bags");
+  if (direct_now(bag)) {
     if (bag > 1) launch_gather_pooled_direct(s, tv, kl, cur.comp.p, cur.n, dst, bag);
     else launch_gather_direct(s, tv, kl, cur.comp.p, cur.n, dst, a.stream_stores);
-  } else if (dst != nullptr) {
-    StageScope st(*group, S_GATHER);
-    if (!cur.lists_ready && cur.n != 0) { // the first blocks of the gather build the batch's run lists on their way
-      a.list_chunks = run_list_chunks(cur.n);
-      cur.lists_ready = true;
-    }
-    if (bag > 1) { // sum-pooled bags: in batch order, through the inverse index
-      HCTR_CHECK(cur.n % bag == 0, "pooled pull: the batch is not a whole number of bags");
-      if (!cur.idx_map_valid) {
-        launch_idx_map(s, cur.view());
-        cur.idx_map_valid = true;
-      }
-      launch_gather_pooled(s, tv, cur.view(), a, bag);
-    } else {
-      launch_gather(s, tv, cur.view(), a);
-    }
+    return;
   }
+  a.list_chunks = take_list_chunks();
+  if (bag > 1) gather_bags(a, bag);
+  else launch_gather(s, tv, cur.view(), a);
+}
+
+// sum-pooled bags: in batch order, through the inverse index
+void Shard::gather_bags(const PullArgs &a, uint32_t bag) {
+  if (!cur.idx_map_valid) {
+    launch_idx_map(group->stream, cur.view());
+    cur.idx_map_valid = true;
+  }
+  launch_gather_pooled(group->stream, tv, cur.view(), a, bag);
 }
 
 void Shard::finish_push_pull() {
@@ -889,7 +913,9 @@ void Group::place_pushes() {
     total += G;
   }
   HCTR_CHECK(total < 0xfffffff0ull, "more than 2^32 rows are pushed in one step");
-  if (!total) return;
+  bool any = false;
+  for (const Shard *m : members) any |= m->prev_active;
+  if (!any) return;
   const size_t W = members[0]->cfg.width;
   rg_idx_all.reserve(total * sizeof(index_t));
   rg_cnt_all.reserve(total * sizeof(version_t));
@@ -905,6 +931,16 @@ void Group::place_pushes() {
     }
   }
   HCTR_HIP(hipMemcpyAsync(push_delta_dev.p, push_delta_host, (size_t)R * R * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+  // plan position -> position in the area, for every shard's push kernel
+  std::vector<PlaceShard> v;
+  for (Shard *m : members)
+    if (m->prev_active) {
+      m->push_pos.reserve((size_t)std::max<uint32_t>(m->prev.U, 1) * 4);
+      v.push_back({m->prev.ukey.p, m->prev.U, m->prev.prefix.as<uint32_t>(), push_delta_dev.as<uint32_t>() + (size_t)R * m->cfg.rank,
+                   m->push_pos.as<uint32_t>()});
+    }
+  StageScope st(*this, S_PUSH);
+  launch_place_rows(stream, members[0]->kl, v.data(), (int)v.size());
 }
 
 // csrc/core/all2all.cu:18-46: every owner's receive buffer is the requesters' buckets for it, in source order.  The
@@ -989,6 +1025,7 @@ void Group::enqueue_index_all(int part) {
     }
     m->index_batch(nullptr, part);
   }
+  if (part != 1) enqueue_bucket_sizes(false);
 }
 
 // the launches of the index that preprocess left to the next call
@@ -1060,10 +1097,8 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     // a previous batch that no push_pull has seen yet (two preprocess calls in a row) is planned here, on the main
     // stream, and waited for (the plan sizes the push buffers)
     for (Shard *m : members)
-      if (!m->prev.planned) {
-        m->plan_batch(m->prev);
-        late.push_back(m);
-      }
+      if (!m->prev.planned) late.push_back(m);
+    plan_batches(late, &Shard::prev);
     {
       StreamSwitch on(*this, index_stream);
       if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
@@ -1091,12 +1126,15 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     return;
   }
   if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
+  std::vector<Shard *> unplanned;
   for (Shard *m : members) {
     m->swap_batches();
     m->preprocess_index(keys[m->cfg.rank], n[m->cfg.rank]);
-    if (!m->prev.planned) m->plan_batch(m->prev);
-    m->enqueue_readback_preprocess();
+    if (!m->prev.planned) unplanned.push_back(m);
   }
+  enqueue_bucket_sizes(true);
+  plan_batches(unplanned, &Shard::prev);
+  for (Shard *m : members) m->enqueue_readback_preprocess();
   if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
   sync_stream();
   float ms = 0.f;
@@ -1192,8 +1230,14 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
   for (Shard *m : members) m->begin_push(grads[m->cfg.rank], bag);
   place_pushes();
-  for (Shard *m : members)
-    m->generate_gradient(nrank > 1 ? push_delta_dev.as<uint32_t>() + (size_t)nrank * m->cfg.rank : nullptr);
+  {
+    std::vector<PushShard> pushes;
+    PushShard r;
+    for (Shard *m : members)
+      if (m->push_record(r)) pushes.push_back(r);
+    StageScope st(*this, S_PUSH);
+    launch_push(stream, members[0]->kl, pushes.data(), (int)pushes.size());
+  }
   if (time_calls) HCTR_HIP(hipEventRecord(ev_push, stream));
   if (nrank > 1) HCTR_HIP(hipEventRecord(ev_pushed, stream));
   enqueue_index_rest(); // the pushes are in their queue, now the rest of the current batches' index
@@ -1224,7 +1268,7 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
       // the push plans of the current batches, for the step in which they are the previous ones: after the pushes of
       // this step (they move the update counters the plan reads), beside everything else the step still does
       HCTR_HIP(hipStreamWaitEvent(stream, ev_pushed, 0));
-      for (Shard *m : members) m->plan_batch(m->cur);
+      plan_batches(members, &Shard::cur);
       HCTR_HIP(hipEventRecord(ev_plan, stream));
     }
   }
@@ -1239,11 +1283,36 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   }
   if (join_index || nrank > 1) HCTR_HIP(hipStreamWaitEvent(stream, ev_index, 0));
   if (nrank > 1) {
-    for (Shard *m : members) m->generate_query(query_delta_dev.as<uint32_t>() + (size_t)nrank * m->cfg.rank);
+    std::vector<PullShard> pulls;
+    std::vector<Shard *> pulling;
+    PullShard r;
+    for (Shard *m : members)
+      if (m->pull_record(r, dsts[m->cfg.rank], bag, query_delta_dev.as<uint32_t>() + (size_t)nrank * m->cfg.rank)) {
+        pulls.push_back(r);
+        pulling.push_back(m);
+      }
+    {
+      // csrc/core/generate_query.cu:91-106: every query is written where its owner reads it (Group::reserve_queries)
+      StageScope st(*this, S_QUERY);
+      launch_build_queries(stream, members[0]->kl, pulls.data(), (int)pulls.size());
+    }
     owner_side(queries_max);
     // the reference waits here for the return counts (hetu_gpu_table.cu:33); they stay on the device
+    {
+      StageScope st(*this, S_REFRESH);
+      launch_refresh(stream, pulls.data(), (int)pulls.size());
+    }
+    StageScope st(*this, S_GATHER);
+    size_t k = 0;
+    for (size_t i = 0; i < pulls.size(); i++) // those that want an output, bags one shard at a time
+      if (pulls[i].a.dst != nullptr) {
+        if (bag > 1) pulling[i]->gather_bags(pulls[i].a, bag);
+        else pulls[k++] = pulls[i];
+      }
+    launch_gather_group(stream, pulls.data(), (int)k);
+  } else {
+    members[0]->write_back(dsts[0], bag);
   }
-  for (Shard *m : members) m->write_back(dsts[m->cfg.rank], bag);
   if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
   if (nrank > 1) HCTR_HIP(hipStreamWaitEvent(stream, ev_plan, 0));
   sync_stream();

@@ -312,3 +312,41 @@ def test_many_shards(nrank):
         p.compare_state(1e-5, "step %d" % step)
         prev = sizes
     p.close()
+
+
+@pytest.mark.parametrize("nrank,width", [(8, 16), (9, 5), (17, 8)])
+def test_groups_of_more_shards_than_a_launch_serves(nrank, width):
+    # the kernels on the shards' own batches serve eight shards per launch: exactly eight, one more, two full launches and
+    # one; batches of very different sizes and empty ones side by side, in changing places; outputs and gradients of some
+    # shards off by four bytes; a step without gradients in between
+    say("group launches, shards", nrank, "width", width)
+    p, _ = update_pair(nrank, 4_000, width, bounds=(2, 3), init=("Uniform", -0.1, 0.1), lr=0.05, cache="third", seed=nrank)
+    rng = np.random.default_rng(nrank)
+    draw = zipf_sampler(4_000, 1.2, rng)
+    sizes = [0, 1, 300, 5_000, 40]
+    prev = [0] * nrank
+    for step in range(6):
+        ns = [sizes[(r + 2 * step) % len(sizes)] for r in range(nrank)]
+        keys = [draw(n) if n else np.zeros(0, np.int64) for n in ns]
+        p.preprocess(keys, device_keys=True)
+        p.compare_ints(INT_ITEMS_PRE, "step %d" % step)
+        grads = [None if step == 3 else rng.normal(0, 1e-2, size=(n, width)).astype(np.float32) for n in prev]
+        bufs, dst, gptr = [], [], []
+        for r in range(nrank):
+            off = (r + step) % 2
+            d = torch.full((ns[r] * width + 1,), float("nan"), device="cuda")
+            dst.append(d[off:off + ns[r] * width])
+            g = torch.zeros(prev[r] * width + 1, device="cuda")
+            if grads[r] is not None:
+                g[off:off + prev[r] * width].copy_(torch.from_numpy(grads[r].reshape(-1)))
+            gptr.append(0 if grads[r] is None or not prev[r] else g.data_ptr() + 4 * off)
+            bufs += [d, g]
+        torch.cuda.synchronize()
+        capi.group_push_pull(p.tables, gptr, [d.data_ptr() if d.numel() else 0 for d in dst])
+        ref = p.oracle.push_pull(grads)
+        p.compare_ints(INT_ITEMS_POST, "step %d" % step)
+        for r in range(nrank):
+            assert_close(dst[r].cpu().numpy().reshape(-1, width), ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        p.compare_state(1e-5, "step %d" % step)
+        prev = ns
+    p.close()
