@@ -93,21 +93,54 @@ template <int VEC> __device__ __forceinline__ uint32_t lane_col(uint32_t c, uint
   return VEC == kOdd4 ? min(c, width - 4) : c;
 }
 
+// Kernels of a step that every shard of a loopback group launches alike serve up to kShardsPerLaunch shards with one
+// launch: blockIdx.y picks the shard, the records travel as kernel arguments.  (A launch costs a small batch more than
+// its work: one launch
+// per shard and kernel made a step of four shards of 53 k keys 73 launches and 365 us; one for all, 25 and 183 us.)
+constexpr int kShardsPerLaunch = 8;
+// the records of one launch: one by itself, or up to kShardsPerLaunch
+template <typename S, int M> struct Records { S s[M]; };
+// f(records, how many of them, keys of the largest batch among them) for `count` records in pieces of one launch each
+template <typename S, typename F> void for_records(const S *shards, int count, F &&f) {
+  for (int i = 0; i < count; i += kShardsPerLaunch) {
+    const int m = count - i < kShardsPerLaunch ? count - i : kShardsPerLaunch;
+    uint32_t n = 0;
+    for (int k = 0; k < m; k++) n = shards[i + k].keys() > n ? shards[i + k].keys() : n;
+    if (!n) continue;
+    if (count == 1) {
+      Records<S, 1> p;
+      p.s[0] = shards[0];
+      f(p, m, n);
+    } else {
+      Records<S, kShardsPerLaunch> p = {};
+      for (int k = 0; k < m; k++) p.s[k] = shards[i + k];
+      f(p, m, n);
+    }
+  }
+}
+
 // ---- preprocess ---------------------------------------------------------------------------------
 // ids -> sort keys; flags ids outside [0, id_max) in *err (and sorts them as id 0)
 // comp_keys is the batch's copy of the ids as well (the reference's d_idx); nlong (optional) is zeroed;
 // sort_counts: the sort's scratch, which receives the per-tile counts of the first pass' digit
 // ids32: `keys` points to 32-bit ids (narrowed on their way from pageable host memory; one that did not fit is
 // 0xffffffff, which the range check flags like the id it stands for)
-void launch_make_keys(hipStream_t s, const TableView &t, const KeyLayout &kl, const index_t *keys, uint32_t n,
-                      void *comp_keys, uint32_t *err, uint32_t *nlong, uint32_t *sort_counts, bool ids32 = false);
+struct KeyShard {
+  TableView t;
+  const index_t *ids;
+  uint32_t n;
+  void *comp_keys;
+  uint32_t *err, *nlong, *sort_counts;
+  bool ids32;                // the same for all records of a launch, like the tile shape that goes with n
+  uint32_t keys() const { return n; }
+};
+void launch_make_keys(hipStream_t s, const KeyLayout &kl, const KeyShard *shards, int count);
 // sorted keys -> everything per unique key + inverse index.  heads: the head counts per chunk of sorted positions that
 // the last launch of the tile-sorted passes left (count_heads false), or storage for them (count_heads true: a launch
 // of its own counts them first, one chunk per tile of the unique pass).
 // u_copy (optional) receives the number of unique keys as well (b.d_U always does)
-struct HeadChunks;
-void launch_unique(hipStream_t s, const TableView &t, const KeyLayout &kl, const void *sorted_keys,
-                   const BatchView &b, const HeadChunks &heads, bool count_heads, uint32_t *u_copy);
+struct UniqueShard;
+void launch_unique(hipStream_t s, const KeyLayout &kl, const UniqueShard *shards, int count, bool count_heads);
 
 // batch-order inverse index from sorted_arg and rank_sorted (introspection; the hot path does not need it)
 void launch_idx_map(hipStream_t s, const BatchView &b);
@@ -115,12 +148,6 @@ void launch_idx_map(hipStream_t s, const BatchView &b);
 // way when PullArgs::list_chunks is set
 void launch_list_long_runs(hipStream_t s, const BatchView &b);
 inline uint32_t run_list_chunks(uint32_t n) { return (n + 255) / 256; } // enough for any number of unique keys <= n
-
-// Kernels of a step that every shard of a loopback group launches alike serve up to kShardsPerLaunch shards with one
-// launch: blockIdx.y picks the shard, the records travel as kernel arguments.  (A launch costs a small batch more than
-// its work: one launch
-// per shard and kernel made a step of four shards of 53 k keys 73 launches and 365 us, one for all 35 and 280 us.)
-constexpr int kShardsPerLaunch = 8;
 
 // Push plan of a batch (csrc/core/preprocess.cu:148-182) for every record: need[u] in {0,1}, prefix[u] = pushed rows before
 // u, *total their number, and pushed rows per owner: prefix[lo[d+1]] - prefix[lo[d]] in cnt_out[0..nrank] and, pinned host

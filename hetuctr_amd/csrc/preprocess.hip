@@ -22,12 +22,18 @@ constexpr int kTile = kBlock * kItems; // 2048: scan_blocks(n) sizes the scratch
 // of the batch's run counters, and the per-tile counts of the first sort pass' digit: a block works on one sort tile, so the sort
 // needs no counting launch of its own for that pass.  This is the one kernel that reads the caller's buffer: the
 // call may return when it is through.
-template <typename K, int ITEMS>
-__global__ __launch_bounds__(kSortBlock) void make_keys(const index_t *__restrict__ keys, uint32_t n, uint64_t id_max,
-                                                         int id_bits, int nrank, const worker_t *__restrict__ root,
-                                                         K *__restrict__ comp, uint32_t *__restrict__ err,
-                                                         uint32_t *__restrict__ nlong, int dbits,
-                                                         uint32_t *__restrict__ counts, bool ids32) {
+template <typename K, int ITEMS, int M> // M: records of the launch, blockIdx.y picks one
+__global__ __launch_bounds__(kSortBlock) void make_keys(Records<KeyShard, M> shards, int id_bits, int dbits) {
+  const KeyShard &S = shards.s[M == 1 ? 0 : blockIdx.y];
+  const index_t *__restrict__ keys = S.ids;
+  const uint32_t n = S.n;
+  const uint64_t id_max = S.t.id_max;
+  const int nrank = S.t.nrank;
+  const worker_t *__restrict__ root = S.t.root;
+  K *__restrict__ comp = (K *)S.comp_keys;
+  uint32_t *__restrict__ err = S.err, *__restrict__ nlong = S.nlong, *__restrict__ counts = S.sort_counts;
+  const bool ids32 = S.ids32;
+  if (M > 1 && blockIdx.x * (ITEMS * kSortBlock) >= n) return; // the grid is cut for the largest batch
   __shared__ uint32_t h[kSortMaxBins];
   const uint32_t nb = 1u << dbits, mask = nb - 1;
   if (counts)
@@ -112,12 +118,14 @@ __global__ __launch_bounds__(kUBlock) void head_count(const K *__restrict__ sk, 
 
 // One block per tile of ITEMS * kUBlock sorted positions; position j of a tile is handled by thread (j % kUBlock) in
 // round (j / kUBlock).  chunk: sorted positions per entry of the head counts (a divisor of the tile).
-template <typename K, int ITEMS>
-__global__ __launch_bounds__(kUBlock) void unique_emit(const K *__restrict__ sk, uint32_t n, int id_bits, int nrank,
-                                                       const slot_t *__restrict__ slot,
-                                                       const uint32_t *__restrict__ head_inner,
-                                                       const K *__restrict__ head_first, const K *__restrict__ head_last,
-                                                       uint32_t chunk, BatchView b, uint32_t *__restrict__ u_copy) {
+template <typename K, int ITEMS, int M>
+__global__ __launch_bounds__(kUBlock) void unique_emit(Records<UniqueShard, M> shards, int id_bits, uint32_t chunk) {
+  const UniqueShard &S = shards.s[M == 1 ? 0 : blockIdx.y];
+  const K *__restrict__ sk = (const K *)S.sorted_keys;
+  const uint32_t n = S.b.n;
+  const uint32_t *__restrict__ head_inner = S.heads.inner;
+  const K *__restrict__ head_first = (const K *)S.heads.first, *__restrict__ head_last = (const K *)S.heads.last;
+  if (M > 1 && blockIdx.x * (ITEMS * kUBlock) >= n) return;
   constexpr uint32_t kTileU = ITEMS * kUBlock;
   const uint32_t base = blockIdx.x * kTileU;
   const unsigned lane = lane_id();
@@ -134,7 +142,7 @@ __global__ __launch_bounds__(kUBlock) void unique_emit(const K *__restrict__ sk,
   const uint32_t chunks_before = base / chunk;
   for (uint32_t i = threadIdx.x; i < chunks_before; i += kUBlock)
     s += head_inner[i] + ((i == 0 || head_first[i] != head_last[i - 1]) ? 1u : 0u);
-  emit_unique_tile<K, ITEMS>(key, edge, s, base, n, id_bits, nrank, slot, b, u_copy);
+  emit_unique_tile<K, ITEMS>(key, edge, s, base, n, id_bits, S.t.nrank, S.t.slot, S.b, S.u_copy);
 }
 
 // The inverse index in batch order (the reference's d_idx_map).  The hot path works in sorted order
@@ -250,42 +258,41 @@ __global__ void bucket_sizes(BucketShards shards, int nrank) {
 
 } // namespace
 
-void launch_make_keys(hipStream_t s, const TableView &t, const KeyLayout &kl, const index_t *keys, uint32_t n,
-                      void *comp_keys, uint32_t *err, uint32_t *nlong, uint32_t *sort_counts, bool ids32) {
-  HCTR_CHECK(!ids32 || t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
-  if (!n) return;
-  const unsigned nblocks = (unsigned)sort_tiles(n);
+void launch_make_keys(hipStream_t s, const KeyLayout &kl, const KeyShard *shards, int count) {
   const int dbits = sort_first_digit_bits(kl.total_bits);
-#define CALL(I)                                                                                                       \
-  do {                                                                                                                \
-    if (kl.wide)                                                                                                      \
-      hipLaunchKernelGGL((make_keys<uint64_t, I>), dim3(nblocks), dim3(kSortBlock), 0, s, keys, n, t.id_max,          \
-                         kl.id_bits, t.nrank, t.root, (uint64_t *)comp_keys, err, nlong, dbits, sort_counts,  \
-                         ids32);         \
-    else                                                                                                              \
-      hipLaunchKernelGGL((make_keys<uint32_t, I>), dim3(nblocks), dim3(kSortBlock), 0, s, keys, n, t.id_max,          \
-                         kl.id_bits, t.nrank, t.root, (uint32_t *)comp_keys, err, nlong, dbits, sort_counts,  \
-                         ids32);         \
+  for_records(shards, count, [&](const auto &p, int m, uint32_t most) {
+    constexpr int M = sizeof p.s / sizeof p.s[0];
+    for (int k = 0; k < m; k++) {
+      HCTR_CHECK(!p.s[k].ids32 || p.s[k].t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
+      HCTR_CHECK(sort_tile(p.s[k].n) == sort_tile(most), "internal: batches of one launch differ in shape");
+    }
+    const dim3 grid((unsigned)sort_tiles(most), m);
+#define CALL(I)                                                                                                     \
+  do {                                                                                                              \
+    if (kl.wide) hipLaunchKernelGGL((make_keys<uint64_t, I, M>), grid, dim3(kSortBlock), 0, s, p, kl.id_bits, dbits); \
+    else hipLaunchKernelGGL((make_keys<uint32_t, I, M>), grid, dim3(kSortBlock), 0, s, p, kl.id_bits, dbits);       \
   } while (0)
-  HCTR_SORT_ITEMS_DISPATCH(n, CALL);
+    HCTR_SORT_ITEMS_DISPATCH(most, CALL);
 #undef CALL
-  HCTR_HIP(hipGetLastError());
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
-void launch_unique(hipStream_t s, const TableView &t, const KeyLayout &kl, const void *sorted_keys,
-                   const BatchView &b, const HeadChunks &heads, bool count_heads, uint32_t *u_copy) {
-  if (!b.n) return;
-  // the tile of the pass: that of the sort that left the head counts, or kUTile when they are counted here
-  const int items = count_heads ? kUItems : (int)(heads.chunk / kWave);
-  const uint32_t chunk = count_heads ? (uint32_t)kUTile : heads.chunk;
-  const unsigned nb = div_up(b.n, (size_t)items * kUBlock);
-#define EMIT(K, I)                                                                                                  \
-  hipLaunchKernelGGL((unique_emit<K, I>), dim3(nb), dim3(kUBlock), 0, s, (const K *)sorted_keys, b.n, kl.id_bits,   \
-                     t.nrank, t.slot, heads.inner, (const K *)heads.first, (const K *)heads.last, chunk, b, u_copy)
+void launch_unique(hipStream_t s, const KeyLayout &kl, const UniqueShard *shards, int count, bool count_heads) {
+  for_records(shards, count, [&](const auto &p, int m, uint32_t most) {
+    constexpr int M = sizeof p.s / sizeof p.s[0];
+    const HeadChunks &heads = p.s[0].heads;
+    // the tile of the pass: that of the sort that left the head counts, or kUTile when they are counted here
+    const int items = count_heads ? kUItems : (int)(heads.chunk / kWave);
+    const uint32_t chunk = count_heads ? (uint32_t)kUTile : heads.chunk;
+    HCTR_CHECK(!count_heads || m == 1, "internal: heads are counted for one batch at a time");
+    for (int k = 0; k < m; k++) HCTR_CHECK(p.s[k].heads.chunk == heads.chunk, "internal: batches of one launch differ in shape");
+    const unsigned nb = div_up(most, (size_t)items * kUBlock);
+#define EMIT(K, I) hipLaunchKernelGGL((unique_emit<K, I, M>), dim3(nb, m), dim3(kUBlock), 0, s, p, kl.id_bits, chunk)
 #define EMIT_K(K)                                                                                          \
   do {                                                                                                     \
     if (count_heads)                                                                                       \
-      hipLaunchKernelGGL(head_count<K>, dim3(nb), dim3(kUBlock), 0, s, (const K *)sorted_keys, b.n, heads.inner, \
+      hipLaunchKernelGGL(head_count<K>, dim3(nb), dim3(kUBlock), 0, s, (const K *)p.s[0].sorted_keys, most, heads.inner, \
                          (K *)heads.first, (K *)heads.last);                                              \
     switch (items) {                                                                                       \
       case 2: EMIT(K, 2); break;                                                                           \
@@ -296,11 +303,12 @@ void launch_unique(hipStream_t s, const TableView &t, const KeyLayout &kl, const
       default: throw Error("hetuCTR: internal: no unique pass for this tile shape");                       \
     }                                                                                                      \
   } while (0)
-  if (kl.wide) EMIT_K(uint64_t);
-  else EMIT_K(uint32_t);
+    if (kl.wide) EMIT_K(uint64_t);
+    else EMIT_K(uint32_t);
 #undef EMIT_K
 #undef EMIT
-  HCTR_HIP(hipGetLastError());
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
 void launch_idx_map(hipStream_t s, const BatchView &b) {

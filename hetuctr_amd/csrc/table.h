@@ -150,6 +150,13 @@ class Shard {
   // sort, unique, run lists of the ingested batch; u_out: where the number of unique keys goes besides the batch's
   // own device word (default: the device block that is read back after the call)
   void index_batch(uint32_t *u_out = nullptr, int part = 0);
+  // the host's part of ingest_keys, without its launch (Group::launch_keys)
+  void prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scratch_area = nullptr);
+  TileSortShard tile_sort_record() const;
+  HeadChunks heads() const;
+  const index_t *ids_ = nullptr; // of the prepared batch: where the key kernel reads them, and whether as 32-bit words
+  bool narrowed_ = false;
+  uint32_t *key_flag_ = nullptr; // ... and where it reports a key out of range
   TileSortBuffers tile_sort_buffers() const; // the index scratch as the tile-sorted passes take it
   HostStager stager;                         // ids that arrive in pageable host memory go through its pinned buffer
   bool pooled_from_keys = true;   // HETUCTR_POOLED_FROM_KEYS=0: pooled gathers of one shard go through the inverse index
@@ -273,6 +280,9 @@ class Group {
   bool index_rest_pending = false;       // single shard: preprocess enqueued only the first launches of the index
   void enqueue_index_rest();
   void enqueue_index_all(int part);             // enqueues the others
+  // the same stage of several shards' batches, one launch for all whose batches have the same shape
+  void launch_keys(Shard *const *shards, size_t count);
+  void index_batches(Shard *const *shards, size_t count, uint32_t *u_out, int part);
   void enqueue_bucket_sizes(bool empty);
   // enqueues the push plans of one batch of each of the shards; the counts reach the host when the stream has run it
   void plan_batches(const std::vector<Shard *> &shards, Batch Shard::*which);

@@ -259,7 +259,7 @@ void Shard::use_scratch_area(void *area, uint32_t n) {
 }
 
 // csrc/core/preprocess.cu:92-141
-void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scratch_area) {
+void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scratch_area) {
   HCTR_CHECK(n < 0xfffffff0ull, "a batch holds fewer than 2^32 keys");
   HCTR_CHECK(keys != nullptr || n == 0, "null key pointer");
   hipStream_t s = group->stream;
@@ -270,6 +270,9 @@ void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scr
   cur.lists_ready = n == 0;
   cur.direct_gather = false;
   cur.comp_valid = false;
+  cur.one_block = cur.tile_sorted = false;
+  ids_ = nullptr;
+  key_flag_ = flag ? flag : err_ptr();
   if (!scratch_area) cur.reserve(cur.n, cfg.nrank, kl.wide); // else: the caller has checked that the buffers hold n keys
   if (n == 0) { // :93-95
     cur.clear(s, cfg.nrank);
@@ -281,7 +284,6 @@ void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scr
     {
       // ids -> device copy (:98-99) and sort keys.  When the caller's pointer is device-visible the copy is
       // written by the same kernel that reads the ids; a pageable host buffer goes through a transfer first.
-      StageScope st(*group, S_KEYS);
       hipPointerAttribute_t attr;
       const bool visible = hipPointerGetAttributes(&attr, keys) == hipSuccess &&
                            (attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged);
@@ -311,14 +313,77 @@ void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scr
       cur.one_block = tile_sort_mode == 1 && cur.n <= kOneBlockKeys && kl.max_digit_bits == 0;
       cur.keys_made = !cur.tile_sorted || cur.one_block || (flag != nullptr && cur.n >= kKeysFirstFrom);
       cur.comp_valid = true; // either kernel leaves the sort keys in batch order (a gather from the keys reads them)
-      if (!cur.keys_made)
-        launch_tile_sort_keys(s, tv, kl, ids, nullptr, cur.n, tile_sort_buffers(), flag ? flag : err_ptr(),
-                              cur.dnlong.as<uint32_t>(), narrowed, cur.comp.p);
-      else
-        launch_make_keys(s, tv, kl, ids, cur.n, cur.comp.p, flag ? flag : err_ptr(), cur.dnlong.as<uint32_t>(),
-                         cur.tile_sorted ? nullptr : sp.sortws, narrowed);
+      ids_ = ids;
+      narrowed_ = narrowed;
     }
   }
+}
+
+// The shards whose batches are not empty, in pieces of at most one launch each: f(shards of one piece, how many), all alike
+// by same(a, b) (nearly always all of them are).  No memory is allocated: the call that allocates nothing passes here.
+template <typename Same, typename F> static void for_alike(Shard *const *shards, size_t count, Same &&same, F &&f) {
+  bool done[256] = {};
+  HCTR_CHECK(count <= 256, "internal: more shards than a group holds");
+  for (size_t i = 0; i < count; i++) {
+    if (done[i] || shards[i]->cur.n == 0) continue;
+    Shard *v[kShardsPerLaunch];
+    int m = 0;
+    for (size_t j = i; j < count && m < kShardsPerLaunch; j++) {
+      if (done[j] || shards[j]->cur.n == 0 || !same(*shards[i], *shards[j])) continue;
+      v[m++] = shards[j];
+      done[j] = true;
+    }
+    f(v, m);
+  }
+}
+
+// the first launch of the prepared batches: the one kernel that reads the callers' ids
+void Group::launch_keys(Shard *const *shards, size_t count) {
+  auto same = [](const Shard &a, const Shard &b) {
+    return a.cur.keys_made == b.cur.keys_made && a.cur.tile_sorted == b.cur.tile_sorted &&
+           (a.cur.keys_made ? sort_tile(a.cur.n) == sort_tile(b.cur.n) : tile_items(a.cur.n) == tile_items(b.cur.n));
+  };
+  for_alike(shards, count, same, [&](Shard *const *v, int m) {
+    StageScope st(*this, S_KEYS);
+    if (!v[0]->cur.keys_made) {
+      TileSortShard r[kShardsPerLaunch];
+      for (int k = 0; k < m; k++) r[k] = v[k]->tile_sort_record();
+      launch_tile_sort_keys(stream, v[0]->kl, r, m);
+    } else {
+      KeyShard r[kShardsPerLaunch];
+      for (int k = 0; k < m; k++)
+        r[k] = {v[k]->tv, v[k]->ids_, v[k]->cur.n, v[k]->cur.comp.p, v[k]->key_flag_, v[k]->cur.dnlong.as<uint32_t>(),
+                v[k]->cur.tile_sorted ? nullptr : v[k]->sp.sortws, v[k]->narrowed_};
+      launch_make_keys(stream, v[0]->kl, r, m);
+    }
+  });
+}
+
+void Shard::ingest_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scratch_area) {
+  prepare_keys(keys, n, flag, scratch_area);
+  Shard *self = this;
+  group->launch_keys(&self, 1);
+}
+
+TileSortShard Shard::tile_sort_record() const {
+  TileSortShard o = {};
+  o.t = tv;
+  o.ids = ids_;
+  o.made_keys = cur.keys_made ? cur.comp.p : nullptr;
+  o.n = cur.n;
+  o.b = tile_sort_buffers();
+  o.err = key_flag_;
+  o.nlong = cur.dnlong.as<uint32_t>();
+  o.ids32 = narrowed_;
+  o.keys_out = cur.comp.p;
+  o.sorted_arg = cur.sorted_arg.as<uint32_t>();
+  o.heads = heads();
+  return o;
+}
+
+// head counts per chunk: one wave's share of a sort tile with the tile-sorted passes, else a tile of the unique pass
+HeadChunks Shard::heads() const {
+  return head_chunks_in(sp.headws, cur.n, kl.wide, cur.tile_sorted ? (uint32_t)tile_items(cur.n) * kWave : 4096u);
 }
 
 TileSortBuffers Shard::tile_sort_buffers() const {
@@ -332,52 +397,70 @@ TileSortBuffers Shard::tile_sort_buffers() const {
 }
 
 void Shard::index_batch(uint32_t *u_out, int part) {
-  hipStream_t s = group->stream;
-  // part 1: the first launches of the sort; part 2: everything after them; 0: all of it
-  if (cur.n != 0 && cur.one_block) { // everything is one launch: it goes out with the first part
-    if (part != 2) {
-      StageScope st(*group, S_SORT);
-      launch_index_one_block(s, tv, kl, cur.comp.p, cur.view(), u_out ? u_out : &dst_->U);
+  Shard *self = this;
+  group->index_batches(&self, 1, u_out, part);
+}
+
+// part 1: the first launches of the sort; part 2: everything after them; 0: all of it
+void Group::index_batches(Shard *const *shards, size_t count, uint32_t *u_out, int part) {
+  hipStream_t s = stream;
+  auto u_of = [&](Shard *m) { return u_out ? u_out : &m->dst_->U; };
+  auto same = [](const Shard &a, const Shard &b) {
+    if (a.cur.one_block || b.cur.one_block) return a.cur.one_block == b.cur.one_block;
+    if (!a.cur.tile_sorted || !b.cur.tile_sorted) return &a == &b; // the three-launch passes take one batch at a time
+    return a.cur.keys_made == b.cur.keys_made && tile_items(a.cur.n) == tile_items(b.cur.n);
+  };
+  for_alike(shards, count, same, [&](Shard *const *v, int m) {
+    Shard &f = *v[0];
+    const KeyLayout &kl = f.kl;
+    if (f.cur.one_block) { // everything is one launch: it goes out with the first part
+      if (part == 2) return;
+      StageScope st(*this, S_SORT);
+      OneBlockShard r[kShardsPerLaunch];
+      for (int k = 0; k < m; k++) r[k] = {v[k]->tv, v[k]->cur.comp.p, v[k]->cur.view(), u_of(v[k])};
+      launch_index_one_block(s, kl, r, m);
+      return;
     }
-  } else if (cur.n != 0) {
-    // head counts per chunk: one wave's share of a sort tile with the tile-sorted passes, else a tile of the unique pass
-    const HeadChunks heads = head_chunks_in(sp.headws, cur.n, kl.wide, cur.tile_sorted ? (uint32_t)tile_items(cur.n) * kWave : 4096u);
-    const void *sorted_keys = nullptr;
+    UniqueShard unique[kShardsPerLaunch];
+    for (int k = 0; k < m; k++) unique[k] = {v[k]->tv, nullptr, v[k]->cur.view(), v[k]->heads(), u_of(v[k])};
     {
-      StageScope sort_scope(*group, S_SORT);
-      if (cur.tile_sorted) {
-        if (cur.keys_made && part != 2) // the sort's first launch, from the keys the call made before it returned
-          launch_tile_sort_keys(s, tv, kl, nullptr, cur.comp.p, cur.n, tile_sort_buffers(), nullptr, nullptr);
+      StageScope sort_scope(*this, S_SORT);
+      if (f.cur.tile_sorted) {
+        TileSortShard r[kShardsPerLaunch];
+        for (int k = 0; k < m; k++) r[k] = v[k]->tile_sort_record();
+        if (f.cur.keys_made && part != 2) // the sort's first launch, from the keys the call made before it returned
+          launch_tile_sort_keys(s, kl, r, m);
         const int from = part == 2 ? 1 + kEarlyTilePasses : 1, to = part == 1 ? 1 + kEarlyTilePasses : (1 << 30);
-        launch_tile_sort_passes(s, kl, cur.n, tile_sort_buffers(), cur.sorted_arg.as<uint32_t>(), heads, &sorted_keys,
-                                from, to);
+        const int passes = launch_tile_sort_passes(s, kl, r, m, from, to);
+        for (int k = 0; k < m; k++) unique[k].sorted_keys = r[k].b.keys[passes & 1];
       } else {
         const int from = part == 2 ? kEarlySortSteps : 0, to = part == 1 ? kEarlySortSteps : (1 << 30);
+        Batch &cur = f.cur;
         SortScratch sc;
-        sc.words = sp.sortws;
+        sc.words = f.sp.sortws;
         sc.n_cap = cur.n;
         if (kl.wide) {
           const uint64_t *sk;
-          radix_sort_positions<uint64_t>(s, cur.comp.as<uint64_t>(), cur.n, kl.total_bits, (uint64_t *)sp.ktmp0,
-                                         (uint64_t *)sp.ktmp1, sp.vtmp0, sp.vtmp1,
+          radix_sort_positions<uint64_t>(s, cur.comp.as<uint64_t>(), cur.n, kl.total_bits, (uint64_t *)f.sp.ktmp0,
+                                         (uint64_t *)f.sp.ktmp1, f.sp.vtmp0, f.sp.vtmp1,
                                          cur.sorted_arg.as<uint32_t>(), sc, &sk, true, from, to);
-          sorted_keys = sk;
+          unique[0].sorted_keys = sk;
         } else {
           const uint32_t *sk;
-          radix_sort_positions<uint32_t>(s, cur.comp.as<uint32_t>(), cur.n, kl.total_bits, (uint32_t *)sp.ktmp0,
-                                         (uint32_t *)sp.ktmp1, sp.vtmp0, sp.vtmp1,
+          radix_sort_positions<uint32_t>(s, cur.comp.as<uint32_t>(), cur.n, kl.total_bits, (uint32_t *)f.sp.ktmp0,
+                                         (uint32_t *)f.sp.ktmp1, f.sp.vtmp0, f.sp.vtmp1,
                                          cur.sorted_arg.as<uint32_t>(), sc, &sk, true, from, to);
-          sorted_keys = sk;
+          unique[0].sorted_keys = sk;
         }
       }
     }
     if (part == 1) return;
-    StageScope st(*group, S_UNIQUE);
-    launch_unique(s, tv, kl, sorted_keys, cur.view(), heads, !cur.tile_sorted, u_out ? u_out : &dst_->U);
+    StageScope st(*this, S_UNIQUE);
+    launch_unique(s, kl, unique, m, !f.cur.tile_sorted);
     // the run lists follow in the gather of the step, or before the batch's push if that gather did not look at the
     // index or never came (lists_ready)
     // (built behind the index instead, they make the index the longer of a small step's two chains: 78 us against 64)
-  }
+  });
 }
 
 // several shards: queries per owner of every shard's batch, behind the indexes of all of them (empty: the empty batches too)
@@ -1021,10 +1104,9 @@ void Group::enqueue_index_all(int part) {
     if (m->cur.n == 0) { // an empty batch (a shard that only serves): nothing to launch, nothing to read back
       m->mirror->st.U = 0;
       for (int i = 0; i <= nrank; i++) m->mirror->st.send_cnt[i] = 0;
-      continue;
     }
-    m->index_batch(nullptr, part);
   }
+  index_batches(members.data(), members.size(), nullptr, part);
   if (part != 1) enqueue_bucket_sizes(false);
 }
 
@@ -1102,7 +1184,8 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     {
       StreamSwitch on(*this, index_stream);
       if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
-      for (Shard *m : members) m->ingest_keys(keys[m->cfg.rank], n[m->cfg.rank], &m->mirror->key_err);
+      for (Shard *m : members) m->prepare_keys(keys[m->cfg.rank], n[m->cfg.rank], &m->mirror->key_err);
+      launch_keys(members.data(), members.size());
       if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
       HCTR_HIP(hipEventRecord(ev_keys, stream));
     }

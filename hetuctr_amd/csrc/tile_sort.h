@@ -88,9 +88,21 @@ struct TileSortBuffers {
 // starts from them and looks at neither ids, err nor nlong.
 // ids32: `ids` points to 32-bit ids (see launch_make_keys).  keys_out (optional, with ids): receives the sort keys in
 // batch order as well.
-void launch_tile_sort_keys(hipStream_t s, const TableView &t, const KeyLayout &kl, const index_t *ids,
-                           const void *made_keys, uint32_t n, const TileSortBuffers &b, uint32_t *err, uint32_t *nlong,
-                           bool ids32 = false, void *keys_out = nullptr);
+struct TileSortShard {
+  TableView t;
+  const index_t *ids;
+  const void *made_keys;
+  uint32_t n;                // one tile shape for all records of a launch
+  TileSortBuffers b;
+  uint32_t *err, *nlong;
+  bool ids32;
+  void *keys_out;
+  uint32_t *sorted_arg;
+  HeadChunks heads;
+  uint32_t keys() const { return n; }
+};
+// (every record or none has made_keys)
+void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count);
 // Batches of up to kOneBlockKeys keys: the whole index -- sort, unique keys, run starts, directory look-ups -- by ONE block
 // in one launch, from the batch's sort keys in batch order.  The passes above cost such a batch five launches of one or
 // two mostly idle blocks each, every one a chain of table look-ups and a launch gap.  A look-up of 3328 keys from a table of 34 M
@@ -101,12 +113,28 @@ void launch_tile_sort_keys(hipStream_t s, const TableView &t, const KeyLayout &k
 #endif
 constexpr uint32_t kOneBlockKeys = HCTR_ONE_BLOCK_KEYS;
 static_assert(kOneBlockKeys <= kTileItemsMax * kSortBlock, "one tile");
-void launch_index_one_block(hipStream_t s, const TableView &t, const KeyLayout &kl, const void *keys, const BatchView &b,
-                            uint32_t *u_copy);
+struct OneBlockShard {
+  TableView t;
+  const void *keys_in;
+  BatchView b;
+  uint32_t *u_copy;
+  uint32_t keys() const { return b.n; }
+};
+void launch_index_one_block(hipStream_t s, const KeyLayout &kl, const OneBlockShard *shards, int count);
+
 // Launches [from, to) of the 1..P that follow (P = passes of kl.total_bits), for callers that enqueue them in pieces.
-// The last one writes the sorted positions to sorted_arg, the sorted keys to *sorted_keys (one of b.keys) and `heads`.
+// The last one writes the sorted positions to sorted_arg, the sorted keys to b.keys[P & 1] and `heads`.
 // Returns P.
-int launch_tile_sort_passes(hipStream_t s, const KeyLayout &kl, uint32_t n, const TileSortBuffers &b,
-                            uint32_t *sorted_arg, const HeadChunks &heads, const void **sorted_keys, int from = 1,
+int launch_tile_sort_passes(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count, int from = 1,
                             int to = 1 << 30);
+
+// The unique pass (launch_unique): sorted keys, head counts (made by the last of these passes, or storage for them).
+struct UniqueShard {
+  TableView t;
+  const void *sorted_keys;
+  BatchView b;
+  HeadChunks heads;
+  uint32_t *u_copy;
+  uint32_t keys() const { return b.n; }
+};
 } // namespace hctr

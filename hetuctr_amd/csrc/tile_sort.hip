@@ -9,6 +9,8 @@
 // earlier tiles, then the pair's place among the tile's pairs with digit d -- (digit, tile) pieces are contiguous both in
 // their tile and in the new order, so block o, which produces positions [o * tile, (o + 1) * tile) of the new order, finds
 // the pieces that overlap its range and copies them.
+#include <algorithm>
+
 #include "tile_sort.h"
 #include "unique_tile.h"
 
@@ -154,14 +156,30 @@ __device__ __forceinline__ void store_sorted_tile(const uint32_t *area, const ui
 // is through.  (csrc/core/preprocess.cu:11-20 builds the reference's sort key.)
 // kFromKeys: the sort keys have been made already (make_keys, for a caller that wants its buffer back sooner than a
 // tile is sorted): `ids` then points to them, and nothing is checked or reset here.
-template <typename K, int ITEMS, int DBITS, bool kFromKeys>
-__global__ __launch_bounds__(kSortBlock) void keys_tile_sort(const void *__restrict__ ids_or_keys, uint32_t n,
-                                                              uint64_t id_max, int id_bits, int nrank,
-                                                              const worker_t *__restrict__ root, uint32_t *__restrict__ err,
-                                                              uint32_t *__restrict__ nlong, int dbits, uint32_t pitch,
-                                                              K *__restrict__ out_keys, uint32_t *__restrict__ out_vals,
-                                                              uint16_t *__restrict__ table, bool ids32,
-                                                              K *__restrict__ keys_out) {
+struct KeysJob {
+  const void *ids_or_keys;
+  uint32_t n, pitch;
+  const worker_t *root;
+  uint32_t *err, *nlong;
+  void *out_keys;
+  uint32_t *out_vals;
+  uint16_t *table;
+  void *keys_out;
+  bool ids32;
+  uint32_t keys() const { return n; }
+};
+template <typename K, int ITEMS, int DBITS, bool kFromKeys, int M> // M: records of the launch, blockIdx.y picks one
+__global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M> jobs, uint64_t id_max, int id_bits, int nrank,
+                                                              int dbits) {
+  const KeysJob &J = jobs.s[M == 1 ? 0 : blockIdx.y];
+  const void *__restrict__ ids_or_keys = J.ids_or_keys;
+  const uint32_t n = J.n, pitch = J.pitch;
+  const worker_t *__restrict__ root = J.root;
+  uint32_t *__restrict__ err = J.err, *__restrict__ nlong = J.nlong, *__restrict__ out_vals = J.out_vals;
+  K *__restrict__ out_keys = (K *)J.out_keys, *__restrict__ keys_out = (K *)J.keys_out;
+  uint16_t *__restrict__ table = J.table;
+  const bool ids32 = J.ids32;
+  if (M > 1 && blockIdx.x * TileShape<K, ITEMS>::kTile >= n) return; // the grid is cut for the largest batch
   using S = TileShape<K, ITEMS>;
   __shared__ __align__(16) uint32_t area[S::kAreaWords];
   __shared__ uint32_t bin_start[kSortMaxBins];
@@ -263,14 +281,29 @@ static_assert((kTileSortMaxTiles + 7) / 8 <= 2 * (kSortBlock / kCoarse) && (kTil
 // sorted by that digit: the block fetches one segment per tile -- whole lines even where a single (digit, tile) piece
 // is a pair or two -- and, holding them in tile order, sorts them stably by the digit, which is the order wanted; the
 // few digit values of a block take few ballots per key.
-template <typename K, int ITEMS, int DBITS, bool kLast>
-__global__ __launch_bounds__(kSortBlock) void regroup(const K *__restrict__ in_keys, const uint32_t *__restrict__ in_vals,
-                                                       const uint16_t *__restrict__ table_in, int shift_in, int dbits_in,
-                                                       uint32_t n, uint32_t tiles, uint32_t pitch,
-                                                       K *__restrict__ out_keys, uint32_t *__restrict__ out_vals,
-                                                       uint16_t *__restrict__ table_out, int shift, int dbits,
-                                                       uint32_t *__restrict__ head_inner, K *__restrict__ head_first,
-                                                       K *__restrict__ head_last) {
+struct RegroupJob {
+  const void *in_keys;
+  const uint32_t *in_vals;
+  const uint16_t *table_in;
+  uint32_t n, tiles, pitch;
+  void *out_keys;
+  uint32_t *out_vals;
+  uint16_t *table_out;
+  uint32_t *head_inner;
+  void *head_first, *head_last;
+  uint32_t keys() const { return n; }
+};
+template <typename K, int ITEMS, int DBITS, bool kLast, int M>
+__global__ __launch_bounds__(kSortBlock) void regroup(Records<RegroupJob, M> jobs, int shift_in, int dbits_in, int shift, int dbits) {
+  const RegroupJob &J = jobs.s[M == 1 ? 0 : blockIdx.y];
+  const K *__restrict__ in_keys = (const K *)J.in_keys;
+  const uint32_t *__restrict__ in_vals = J.in_vals;
+  const uint16_t *__restrict__ table_in = J.table_in;
+  const uint32_t n = J.n, tiles = J.tiles, pitch = J.pitch;
+  K *__restrict__ out_keys = (K *)J.out_keys, *__restrict__ head_first = (K *)J.head_first, *__restrict__ head_last = (K *)J.head_last;
+  uint32_t *__restrict__ out_vals = J.out_vals, *__restrict__ head_inner = J.head_inner;
+  uint16_t *__restrict__ table_out = J.table_out;
+  if (M > 1 && blockIdx.x >= tiles) return;
   using S = TileShape<K, ITEMS>;
   __shared__ __align__(16) uint32_t area[S::kAreaWords];
   __shared__ uint32_t bin_start[kSortMaxBins];
@@ -443,10 +476,18 @@ __global__ __launch_bounds__(kSortBlock) void regroup(const K *__restrict__ in_k
 // The index of a small batch by one block (see tile_sort.h): the keys stay in the block's registers and LDS from the first
 // pass to the unique keys.  A pass ranks on DBITS bits whether the last digit needs them or not (the bits above a key's
 // are zero), so that its ballots are straight-line code.
-template <typename K, int ITEMS, int DBITS>
-__global__ __launch_bounds__(kSortBlock) void index_one_block(const K *__restrict__ keys, uint32_t n, int bits, int id_bits,
-                                                               int nrank, const slot_t *__restrict__ slot, BatchView b,
-                                                               uint32_t *__restrict__ u_copy) {
+struct OneBlockJob {
+  const void *in;
+  const slot_t *slot;
+  BatchView b;
+  uint32_t *u_copy;
+};
+template <typename K, int ITEMS, int DBITS, int M>
+__global__ __launch_bounds__(kSortBlock) void index_one_block(Records<OneBlockJob, M> jobs, int bits, int id_bits, int nrank) {
+  const OneBlockJob &J = jobs.s[M == 1 ? 0 : blockIdx.y];
+  const K *__restrict__ keys = (const K *)J.in;
+  const BatchView &b = J.b;
+  const uint32_t n = b.n;
   using S = TileShape<K, ITEMS>;
   static_assert(kSortBlock == kUBlock, "the block that sorts the keys lists the unique ones");
   __shared__ __align__(16) uint32_t area[S::kAreaWords];
@@ -485,7 +526,7 @@ __global__ __launch_bounds__(kSortBlock) void index_one_block(const K *__restric
     edge[k] = (lane == 0 && j < n && j > 0) ? skey[j - 1] : (K)0;
     if (j < n) b.sorted_arg[j] = sval[j];
   }
-  emit_unique_tile<K, ITEMS>(key, edge, 0u, 0u, n, id_bits, nrank, slot, b, u_copy);
+  emit_unique_tile<K, ITEMS>(key, edge, 0u, 0u, n, id_bits, nrank, J.slot, b, J.u_copy);
 }
 
 // digit widths and shifts of the passes: the bits are split evenly, as radix_sort_positions does
@@ -538,15 +579,18 @@ DigitPlan plan_digits(const KeyLayout &kl) {
     }                                             \
   } while (0)
 
-void launch_index_one_block(hipStream_t s, const TableView &t, const KeyLayout &kl, const void *keys, const BatchView &b,
-                            uint32_t *u_copy) {
-  if (!b.n) return;
-  HCTR_CHECK(b.n <= kOneBlockKeys, "internal: batch too large for one block");
+void launch_index_one_block(hipStream_t s, const KeyLayout &kl, const OneBlockShard *shards, int count) {
   const int bits = kl.total_bits < 1 ? 1 : kl.total_bits;
   const bool nine = (bits + 8) / 9 == (bits + 9) / 10; // narrower digits where they take as many passes
-  const int items = (int)div_up(b.n, kSortBlock);
+  for_records(shards, count, [&](const auto &p, int m, uint32_t most) {
+    HCTR_CHECK(most <= kOneBlockKeys, "internal: batch too large for one block");
+    const int items = (int)div_up(most, kSortBlock); // of the largest batch: fits the others too
+    constexpr int M = sizeof p.s / sizeof p.s[0];
+    Records<OneBlockJob, M> jobs = {};
+    for (int k = 0; k < m; k++) jobs.s[k] = {p.s[k].keys_in, p.s[k].t.slot, p.s[k].b, p.s[k].u_copy};
+    const int nrank = p.s[0].t.nrank;
 #define ONE(K, I, D) \
-  hipLaunchKernelGGL((index_one_block<K, I, D>), dim3(1), dim3(kSortBlock), 0, s, (const K *)keys, b.n, bits, kl.id_bits, t.nrank, t.slot, b, u_copy)
+  hipLaunchKernelGGL((index_one_block<K, I, D, M>), dim3(1, m), dim3(kSortBlock), 0, s, jobs, bits, kl.id_bits, nrank)
 #define ONE_D(K, I)                \
   do {                             \
     if (nine) ONE(K, I, 9);        \
@@ -559,66 +603,78 @@ void launch_index_one_block(hipStream_t s, const TableView &t, const KeyLayout &
     else if (items <= 8) ONE_D(K, 8);  \
     else ONE_D(K, 16);                 \
   } while (0)
-  if (kl.wide) ONE_K(uint64_t);
-  else ONE_K(uint32_t);
+    if (kl.wide) ONE_K(uint64_t);
+    else ONE_K(uint32_t);
 #undef ONE_K
 #undef ONE_D
 #undef ONE
-  HCTR_HIP(hipGetLastError());
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
-void launch_tile_sort_keys(hipStream_t s, const TableView &t, const KeyLayout &kl, const index_t *ids,
-                           const void *made_keys, uint32_t n, const TileSortBuffers &b, uint32_t *err, uint32_t *nlong,
-                           bool ids32, void *keys_out) {
-  if (!n) return;
-  HCTR_CHECK(!ids32 || t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
-  HCTR_CHECK(tile_sort_possible(n), "internal: batch too large for the tile-sorted passes");
+static uint16_t *tile_table(const TileSortShard &o, int which) {
+  return (uint16_t *)o.b.tables + (which ? tile_table_pitch(o.n) * kSortMaxBins : 0);
+}
+
+void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count) {
   const DigitPlan p = plan_digits(kl);
-  const unsigned tiles = (unsigned)tile_count(n), pitch = (unsigned)tile_table_pitch(n);
-  uint16_t *table0 = (uint16_t *)b.tables;
-#define CALL(K, I, D)                                                                                                 \
-  do {                                                                                                                \
-    if (made_keys)                                                                                                    \
-      hipLaunchKernelGGL((keys_tile_sort<K, I, D, true>), dim3(tiles), dim3(kSortBlock), 0, s, made_keys, n, t.id_max, \
-                         kl.id_bits, t.nrank, t.root, err, nlong, p.dbits[0], pitch, (K *)b.keys[0], b.vals[0], table0, \
-                         false, (K *)nullptr);                                                                        \
-    else                                                                                                              \
-      hipLaunchKernelGGL((keys_tile_sort<K, I, D, false>), dim3(tiles), dim3(kSortBlock), 0, s, (const void *)ids, n, \
-                         t.id_max, kl.id_bits, t.nrank, t.root, err, nlong, p.dbits[0], pitch, (K *)b.keys[0],        \
-                         b.vals[0], table0, ids32, (K *)keys_out);                                                    \
+  for_records(shards, count, [&](const auto &r, int m, uint32_t most) {
+    constexpr int M = sizeof r.s / sizeof r.s[0];
+    Records<KeysJob, M> jobs = {};
+    const bool made = r.s[0].made_keys != nullptr;
+    for (int k = 0; k < m; k++) {
+      const TileSortShard &o = r.s[k];
+      HCTR_CHECK(!o.ids32 || o.t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
+      HCTR_CHECK(tile_sort_possible(o.n), "internal: batch too large for the tile-sorted passes");
+      HCTR_CHECK(tile_items(o.n) == tile_items(most) && (o.made_keys != nullptr) == made, "internal: batches of one launch differ in shape");
+      jobs.s[k] = {made ? o.made_keys : (const void *)o.ids, o.n, (uint32_t)tile_table_pitch(o.n), o.t.root, o.err, o.nlong, o.b.keys[0],
+                   o.b.vals[0], tile_table(o, 0), made ? nullptr : o.keys_out, o.ids32};
+    }
+    const TableView &t = r.s[0].t;
+    const dim3 grid((unsigned)tile_count(most), m);
+#define CALL(K, I, D)                                                                                                  \
+  do {                                                                                                                 \
+    if (made) hipLaunchKernelGGL((keys_tile_sort<K, I, D, true, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0]); \
+    else hipLaunchKernelGGL((keys_tile_sort<K, I, D, false, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0]); \
   } while (0)
-  HCTR_TILE_SORT_DISPATCH(kl.wide, n, p.dbits[0], CALL);
+    HCTR_TILE_SORT_DISPATCH(kl.wide, most, p.dbits[0], CALL);
 #undef CALL
-  HCTR_HIP(hipGetLastError());
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
-int launch_tile_sort_passes(hipStream_t s, const KeyLayout &kl, uint32_t n, const TileSortBuffers &b,
-                            uint32_t *sorted_arg, const HeadChunks &heads, const void **sorted_keys, int from, int to) {
+int launch_tile_sort_passes(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count, int from, int to) {
   const DigitPlan p = plan_digits(kl);
-  *sorted_keys = b.keys[p.passes & 1];
-  if (!n) return p.passes;
-  const unsigned tiles = (unsigned)tile_count(n), pitch = (unsigned)tile_table_pitch(n);
-  HCTR_CHECK(heads.chunk == (uint32_t)tile_items(n) * kWave, "internal: head chunks do not match the tile shape");
-  uint16_t *table[2] = {(uint16_t *)b.tables, (uint16_t *)b.tables + (size_t)pitch * kSortMaxBins};
   for (int j = std::max(from, 1); j <= p.passes && j < to; j++) {
     const int in = (j - 1) & 1, out = j & 1;
-    if (j < p.passes) {
-#define CALL(K, I, D)                                                                                                   \
-  hipLaunchKernelGGL((regroup<K, I, D, false>), dim3(tiles), dim3(kSortBlock), 0, s, (const K *)b.keys[in], b.vals[in], \
-                     table[in], p.shift[j - 1], p.dbits[j - 1], n, tiles, pitch, (K *)b.keys[out], b.vals[out],         \
-                     table[out], p.shift[j], p.dbits[j], (uint32_t *)nullptr, (K *)nullptr, (K *)nullptr)
-      HCTR_TILE_SORT_DISPATCH(kl.wide, n, p.dbits[j], CALL);
+    const bool last = j == p.passes;
+    for_records(shards, count, [&](const auto &r, int m, uint32_t most) {
+      constexpr int M = sizeof r.s / sizeof r.s[0];
+      Records<RegroupJob, M> jobs = {};
+      for (int k = 0; k < m; k++) {
+        const TileSortShard &o = r.s[k];
+        HCTR_CHECK(tile_items(o.n) == tile_items(most), "internal: batches of one launch differ in shape");
+        HCTR_CHECK(o.heads.chunk == (uint32_t)tile_items(o.n) * kWave, "internal: head chunks do not match the tile shape");
+        jobs.s[k] = {o.b.keys[in], o.b.vals[in], tile_table(o, in), o.n, (uint32_t)tile_count(o.n), (uint32_t)tile_table_pitch(o.n),
+                     o.b.keys[out], last ? o.sorted_arg : o.b.vals[out], last ? nullptr : tile_table(o, out), o.heads.inner,
+                     o.heads.first, o.heads.last};
+      }
+      const dim3 grid((unsigned)tile_count(most), m);
+      if (!last) {
+#define CALL(K, I, D)                                                                                                 \
+  hipLaunchKernelGGL((regroup<K, I, D, false, M>), grid, dim3(kSortBlock), 0, s, jobs, p.shift[j - 1], p.dbits[j - 1], \
+                     p.shift[j], p.dbits[j])
+        HCTR_TILE_SORT_DISPATCH(kl.wide, most, p.dbits[j], CALL);
 #undef CALL
-    } else {
-#define CALL(K, I, D)                                                                                                  \
-  hipLaunchKernelGGL((regroup<K, I, 0, true>), dim3(tiles), dim3(kSortBlock), 0, s, (const K *)b.keys[in], b.vals[in], \
-                     table[in], p.shift[j - 1], p.dbits[j - 1], n, tiles, pitch, (K *)b.keys[out], sorted_arg,         \
-                     (uint16_t *)nullptr, 0, 0, heads.inner, (K *)heads.first, (K *)heads.last)
-      HCTR_TILE_SORT_DISPATCH(kl.wide, n, 0, CALL);
+      } else {
+#define CALL(K, I, D) \
+  hipLaunchKernelGGL((regroup<K, I, 0, true, M>), grid, dim3(kSortBlock), 0, s, jobs, p.shift[j - 1], p.dbits[j - 1], 0, 0)
+        HCTR_TILE_SORT_DISPATCH(kl.wide, most, 0, CALL);
 #undef CALL
-    }
+      }
+      HCTR_HIP(hipGetLastError());
+    });
   }
-  HCTR_HIP(hipGetLastError());
   return p.passes;
 }
 
