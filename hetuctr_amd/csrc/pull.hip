@@ -16,7 +16,7 @@ static_assert(kBlock == kRunListBlock, "the gather's blocks list runs chunk by c
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Rows travel in vectors of kCols<VEC> columns per lane: 4 (the width is a multiple of four and every pointer 16-byte
-// aligned), kOdd4 (any other width from 4 on: see kernels.h) or 1 (rows of less than four floats).
+// aligned), kOdd4 (any other width from 4 on: see kernels.h) or 1.
 template <int VEC> struct RowVec;
 template <> struct RowVec<4> { typedef floatx4 T; };
 template <> struct RowVec<kOdd4> { typedef floatx4 T __attribute__((aligned(4))); };
@@ -690,12 +690,13 @@ inline int lanes_for(uint32_t width, int vec) {
   return lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
 }
 
-// expands F<VEC, LPR>(args...) over the (VEC, LPR) pairs; a row of less than four floats takes at most four lanes
+// expands F<VEC, LPR>(args...) over the (VEC, LPR) pairs; rows that move one float per lane have less than four or millions
 #define HCTR_DISPATCH_ROW(vec, lpr, CALL)         \
   do {                                            \
     if ((vec) == 4) HCTR_DISPATCH_LPR(4, lpr, CALL); \
     else if ((vec) == kOdd4) HCTR_DISPATCH_LPR(kOdd4, lpr, CALL); \
-    else CALL(1, 4);                              \
+    else if ((lpr) == 4) CALL(1, 4);              \
+    else CALL(1, 64);                             \
   } while (0)
 #define HCTR_DISPATCH_LPR(V, lpr, CALL) \
   do {                                  \

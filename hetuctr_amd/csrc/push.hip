@@ -39,9 +39,6 @@ namespace hctr {
 #ifndef HCTR_RPT
 #define HCTR_RPT 2
 #endif
-#ifndef HCTR_SLICE
-#define HCTR_SLICE 64
-#endif
 #ifndef HCTR_LONG_BLOCKS
 #define HCTR_LONG_BLOCKS 128
 #endif
@@ -57,7 +54,7 @@ constexpr int kRPT = HCTR_RPT;            // long role: rows per loader thread a
 #define HCTR_SLOTS 3
 #endif
 constexpr int kSlots = HCTR_SLOTS;        // long role: LDS ring slots
-constexpr int kSlice = HCTR_SLICE;        // long role: columns per block
+constexpr int kSlice = kSliceColumns;     // long role: columns per block
 constexpr int kLongBlocks = HCTR_LONG_BLOCKS;
 #ifndef HCTR_GIANT_SLICE
 #define HCTR_GIANT_SLICE 32
@@ -451,10 +448,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
   constexpr uint32_t C = kCols<VEC>;
   const uint32_t W = t.width;
   uint32_t CS = CSC ? (uint32_t)CSC : min((uint32_t)kSlice, (W + C - 1) / C * C);
-  // the last slice of an odd width holds four columns at least, so that a lane that starts early stays inside its slice
-  // (some slice of 8..64 columns fits any width below 2^20)
-  if (VEC == kOdd4)
-    while (CS > 8 && W % CS != 0 && W % CS < 4) CS -= 4;
+  if (VEC == kOdd4) CS = overlap_slice(W, CS); // row_vec() has made sure that one of them holds the last lane
   uint32_t lanes = (CS + C - 1) / C; // loader lanes per row slice, rounded up to a power of two
   lanes = lanes <= 1 ? 1 : lanes <= 2 ? 2 : lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
   const uint32_t RPL = CSC ? (uint32_t)(kLoaders / (CSC / C)) : kLoaders / lanes;
@@ -843,8 +837,9 @@ void launch_push_t(hipStream_t st, int id_bits, const PushShards &shards, int co
 
 template <int VEC, typename K, bool kPooled>
 void launch_push_p(hipStream_t st, int id_bits, const PushShards &shards, int count) {
-  if constexpr (VEC == 1) { // rows of less than four floats
-    launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
+  if constexpr (VEC == 1) { // rows of less than four floats, or of millions (row_vec)
+    if (shards.s[0].t.width < 4) launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
+    else launch_push_t<VEC, 64, K, kPooled>(st, id_bits, shards, count);
   } else {
     const uint32_t lanes = (shards.s[0].t.width + kCols<VEC> - 1) / kCols<VEC>;
     if (lanes <= 4) launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);

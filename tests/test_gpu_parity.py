@@ -673,3 +673,27 @@ def test_batches_indexed_by_one_block(length, wide, monkeypatch):
             prev_n = ns
         p.compare_state(1e-5, "end")
         p.close()
+
+
+@pytest.mark.parametrize("width", [2882881, 2882882, 2882883])
+def test_widest_odd_rows_with_long_runs(width):
+    # 2882880 is a multiple of every slice width of 8 to 64 columns: the last slice of these rows has one to three columns
+    # whatever the slice.  One key with more than 128 occurrences; gradients of small whole numbers, whose sums are exact
+    # in any order
+    import torch
+    say("row width", width)
+    n = 150
+    p = Pair(1, 4, width, np.zeros(4, np.uint8), [np.arange(4, dtype=np.int64)], lr=0.5, with_oracle=False)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(width)
+    keys = np.array([2] * 140 + [0] * 9 + [3], np.int64)
+    grad = torch.randint(-3, 4, (n, width), device="cuda", generator=gen, dtype=torch.int8).float()
+    out = torch.empty((n, width), device="cuda")
+    torch.cuda.synchronize()
+    t = p.tables[0]
+    for g in (0, grad.data_ptr()):
+        t.preprocess(keys.ctypes.data, n)
+        t.push_pull(g, out.data_ptr())
+    for i in (0, 139, 140, 148, 149):
+        assert torch.equal(out[i], grad[torch.from_numpy(keys == keys[i]).cuda()].sum(0) * -0.5), "row %d" % i
+    p.close()
