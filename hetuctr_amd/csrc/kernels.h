@@ -2,6 +2,7 @@
 // Reference stages are cited where the launcher is defined.
 #pragma once
 #include "common.h"
+#include "launch_cut.h"
 #include "row_slices.h"
 
 namespace hctr {

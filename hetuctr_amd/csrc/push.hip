@@ -804,13 +804,27 @@ template <int VEC, int LPR, typename K, bool kPooled>
 __global__ HCTR_PUSH_BOUNDS void push_fused(TableView t, int id_bits, BatchView p, PushArgs a, uint32_t U) {
   push_block<VEC, LPR, K, true, kPooled>(t, id_bits, p, a, U, blockIdx.x);
 }
-// The pushes of the shards of a group in one launch: neighbouring blocks are the same block of different shards, so that
-// every shard's long chains start first.
-struct PushShards { PushShard s[kShardsPerLaunch]; };
+// The pushes of the shards of a group in one launch.  The blocks every shard has alike come first, neighbouring blocks being
+// the same block of different shards, so that every shard's long chains start first; then come the shards' other blocks, as
+// many as each one's batch needs.
+struct PushShards {
+  PushShard s[kShardsPerLaunch];
+  BlockCut<kShardsPerLaunch> cut; // of the blocks behind the first kEachBlocks of every shard
+};
+constexpr uint32_t kEachBlocks = kLongBlocks + kMedBlocks;
 template <int VEC, int LPR, typename K, bool kPooled>
 __global__ HCTR_PUSH_BOUNDS void push_group(PushShards shards, uint32_t count, int id_bits) {
-  const PushShard &S = shards.s[blockIdx.x % count];
-  push_block<VEC, LPR, K, false, kPooled>(S.t, id_bits, S.b, S.a, S.n_unique, blockIdx.x / count);
+  uint32_t block = blockIdx.x, k;
+  if (block < kEachBlocks * count) {
+    k = block % count;
+    block /= count;
+  } else {
+    block -= kEachBlocks * count;
+    k = record_of(shards.cut, block);
+    block += kEachBlocks;
+  }
+  const PushShard &S = shards.s[k];
+  push_block<VEC, LPR, K, false, kPooled>(S.t, id_bits, S.b, S.a, S.n_unique, block);
 }
 
 struct PlaceShards { PlaceShard s[kShardsPerLaunch]; };
@@ -821,22 +835,24 @@ template <typename K> __global__ __launch_bounds__(256) void place_rows(PlaceSha
 }
 
 template <int VEC, int LPR, typename K, bool kPooled>
-void launch_push_t(hipStream_t st, int id_bits, const PushShards &shards, int count) {
-  constexpr int kGroups = kPushBlock / LPR;
-  unsigned blocks = 0; // of the shard with the most: chains, medium runs, short runs, the counters of every unique key
-  for (int i = 0; i < count; i++) {
-    const uint32_t U = shards.s[i].n_unique;
-    blocks = std::max(blocks, kLongBlocks + kMedBlocks + div_up(U, kGroups * kRunsPerGroup) + div_up(U, kPushBlock));
-  }
+void launch_push_t(hipStream_t st, int id_bits, PushShards &shards, int count) {
+  // short runs, and the counters of every unique key
+  auto need = [](const PushShard &S) { return div_up(S.n_unique, (kPushBlock / LPR) * kRunsPerGroup) + div_up(S.n_unique, kPushBlock); };
   const PushShard &S = shards.s[0];
-  if (S.t.nrank == 1)
-    hipLaunchKernelGGL((push_fused<VEC, LPR, K, kPooled>), dim3(blocks), dim3(kPushBlock), 0, st, S.t, id_bits, S.b, S.a, S.n_unique);
-  else
-    hipLaunchKernelGGL((push_group<VEC, LPR, K, kPooled>), dim3(blocks * count), dim3(kPushBlock), 0, st, shards, (uint32_t)count, id_bits);
+  if (S.t.nrank == 1) {
+    hipLaunchKernelGGL((push_fused<VEC, LPR, K, kPooled>), dim3(kEachBlocks + need(S)), dim3(kPushBlock), 0, st, S.t, id_bits, S.b, S.a, S.n_unique);
+    return;
+  }
+  for (int i = 0; i < count;) { // nearly always one launch
+    const int m = cut_blocks(shards.cut, count - i, kPushBlock, kEachBlocks, [&](int k) { return need(shards.s[i + k]); });
+    if (i) std::copy(shards.s + i, shards.s + i + m, shards.s);
+    hipLaunchKernelGGL((push_group<VEC, LPR, K, kPooled>), dim3(kEachBlocks * m + shards.cut.total()), dim3(kPushBlock), 0, st, shards, (uint32_t)m, id_bits);
+    i += m;
+  }
 }
 
 template <int VEC, typename K, bool kPooled>
-void launch_push_p(hipStream_t st, int id_bits, const PushShards &shards, int count) {
+void launch_push_p(hipStream_t st, int id_bits, PushShards &shards, int count) {
   if constexpr (VEC == 1) { // rows of less than four floats, or of millions (row_vec)
     if (shards.s[0].t.width < 4) launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
     else launch_push_t<VEC, 64, K, kPooled>(st, id_bits, shards, count);
@@ -851,7 +867,7 @@ void launch_push_p(hipStream_t st, int id_bits, const PushShards &shards, int co
 }
 
 template <int VEC, typename K>
-void launch_push_k(hipStream_t st, int id_bits, const PushShards &shards, int count) {
+void launch_push_k(hipStream_t st, int id_bits, PushShards &shards, int count) {
   if (shards.s[0].a.bag.bag > 1) launch_push_p<VEC, K, true>(st, id_bits, shards, count);
   else launch_push_p<VEC, K, false>(st, id_bits, shards, count);
 }
