@@ -96,29 +96,46 @@ template <int VEC> __device__ __forceinline__ uint32_t lane_col(uint32_t c, uint
 }
 
 // Kernels of a step that every shard of a loopback group launches alike serve up to kShardsPerLaunch shards with one
-// launch: blockIdx.y picks the shard, the records travel as kernel arguments.  (A launch costs a small batch more than
-// its work: one launch
-// per shard and kernel made a step of four shards of 53 k keys 73 launches and 365 us; one for all, 25 and 183 us.)
+// launch: the records travel as kernel arguments, and a block finds its own from where the records' blocks start.  (A
+// launch costs a small batch more than its work: one launch per shard and kernel made a step of four shards of 53 k keys 73
+// launches and 365 us; one for all, 22 and 183 us.)
 constexpr int kShardsPerLaunch = 8;
 // the records of one launch: one by itself, or up to kShardsPerLaunch
-template <typename S, int M> struct Records { S s[M]; };
-// f(records, how many of them, keys of the largest batch among them) for `count` records in pieces of one launch each
-template <typename S, typename F> void for_records(const S *shards, int count, F &&f) {
-  for (int i = 0; i < count; i += kShardsPerLaunch) {
-    const int m = count - i < kShardsPerLaunch ? count - i : kShardsPerLaunch;
-    uint32_t n = 0;
-    for (int k = 0; k < m; k++) n = shards[i + k].keys() > n ? shards[i + k].keys() : n;
-    if (!n) continue;
-    if (count == 1) {
-      Records<S, 1> p;
-      p.s[0] = shards[0];
-      f(p, m, n);
-    } else {
-      Records<S, kShardsPerLaunch> p = {};
-      for (int k = 0; k < m; k++) p.s[k] = shards[i + k];
-      f(p, m, n);
-    }
+template <typename S, int M> struct Records {
+  S s[M];
+  BlockCut<M> cut;
+};
+// the record this block works for; block, blocks: its number among that record's blocks, and how many they are
+template <typename S, int M>
+__device__ __forceinline__ const S &my_record(const Records<S, M> &r, uint32_t &block, uint32_t &blocks) {
+  block = blockIdx.x;
+  if constexpr (M == 1) {
+    blocks = gridDim.x;
+    return r.s[0];
+  } else {
+    const uint32_t k = record_of(r.cut, block);
+    blocks = r.cut.blocks[k];
+    return r.s[k];
   }
+}
+// f(records, how many of them) for records make(0) .. make(count - 1) in pieces of one launch each, of blocks(k) blocks of
+// `threads` threads for record k; the launch's grid is grid_of(records)
+template <typename S, int M, typename Make, typename Blocks, typename F>
+void launch_records(int count, uint32_t threads, Make &&make, Blocks &&blocks, F &&f) {
+  for (int i = 0; i < count;) {
+    Records<S, M> p = {};
+    const int m = cut_blocks(p.cut, count - i, threads, 0, [&](int k) { return blocks(i + k); });
+    for (int k = 0; k < m; k++) p.s[k] = make(i + k);
+    if (p.cut.total) f(p, m);
+    i += m;
+  }
+}
+template <typename R> dim3 grid_of(const R &records) { return dim3(records.cut.total); }
+// ... with kernels of their own for a single record
+template <typename S, typename Make, typename Blocks, typename F>
+void launch_one_or_records(int count, uint32_t threads, Make &&make, Blocks &&blocks, F &&f) {
+  if (count == 1) launch_records<S, 1>(count, threads, make, blocks, f);
+  else launch_records<S, kShardsPerLaunch>(count, threads, make, blocks, f);
 }
 
 // ---- preprocess ---------------------------------------------------------------------------------
@@ -133,9 +150,9 @@ struct KeyShard {
   uint32_t n;
   void *comp_keys;
   uint32_t *err, *nlong, *sort_counts;
-  bool ids32;                // the same for all records of a launch, like the tile shape that goes with n
-  uint32_t keys() const { return n; }
+  bool ids32;
 };
+// (batches of one tile shape)
 void launch_make_keys(hipStream_t s, const KeyLayout &kl, const KeyShard *shards, int count);
 // sorted keys -> everything per unique key + inverse index.  heads: the head counts per chunk of sorted positions that
 // the last launch of the tile-sorted passes left (count_heads false), or storage for them (count_heads true: a launch

@@ -22,9 +22,10 @@ constexpr int kTile = kBlock * kItems; // 2048: scan_blocks(n) sizes the scratch
 // of the batch's run counters, and the per-tile counts of the first sort pass' digit: a block works on one sort tile, so the sort
 // needs no counting launch of its own for that pass.  This is the one kernel that reads the caller's buffer: the
 // call may return when it is through.
-template <typename K, int ITEMS, int M> // M: records of the launch, blockIdx.y picks one
+template <typename K, int ITEMS, int M> // M: records of the launch
 __global__ __launch_bounds__(kSortBlock) void make_keys(Records<KeyShard, M> shards, int id_bits, int dbits) {
-  const KeyShard &S = shards.s[M == 1 ? 0 : blockIdx.y];
+  uint32_t tile, tiles;
+  const KeyShard &S = my_record(shards, tile, tiles);
   const index_t *__restrict__ keys = S.ids;
   const uint32_t n = S.n;
   const uint64_t id_max = S.t.id_max;
@@ -33,13 +34,12 @@ __global__ __launch_bounds__(kSortBlock) void make_keys(Records<KeyShard, M> sha
   K *__restrict__ comp = (K *)S.comp_keys;
   uint32_t *__restrict__ err = S.err, *__restrict__ nlong = S.nlong, *__restrict__ counts = S.sort_counts;
   const bool ids32 = S.ids32;
-  if (M > 1 && blockIdx.x * (ITEMS * kSortBlock) >= n) return; // the grid is cut for the largest batch
   __shared__ uint32_t h[kSortMaxBins];
   const uint32_t nb = 1u << dbits, mask = nb - 1;
   if (counts)
     for (uint32_t i = threadIdx.x; i < nb; i += kSortBlock) h[i] = 0;
-  if (blockIdx.x == 0 && threadIdx.x < kRunCounters && nlong) nlong[threadIdx.x] = 0; // counters of this batch
-  const uint32_t base = blockIdx.x * (ITEMS * kSortBlock);
+  if (tile == 0 && threadIdx.x < kRunCounters && nlong) nlong[threadIdx.x] = 0; // counters of this batch
+  const uint32_t base = tile * (ITEMS * kSortBlock);
   uint64_t id[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; k++) {
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kSortBlock) void make_keys(Records<KeyShard, M> sha
   }
   if (!counts) return; // the keys alone: another sort counts for itself
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < nb; i += kSortBlock) counts[(size_t)blockIdx.x * nb + i] = h[i];
+  for (uint32_t i = threadIdx.x; i < nb; i += kSortBlock) counts[(size_t)tile * nb + i] = h[i];
 }
 
 // The unique pass works on tiles of kUTile sorted positions; position j of a tile is handled by thread (j % kUBlock)
@@ -120,14 +120,14 @@ __global__ __launch_bounds__(kUBlock) void head_count(const K *__restrict__ sk, 
 // round (j / kUBlock).  chunk: sorted positions per entry of the head counts (a divisor of the tile).
 template <typename K, int ITEMS, int M>
 __global__ __launch_bounds__(kUBlock) void unique_emit(Records<UniqueShard, M> shards, int id_bits, uint32_t chunk) {
-  const UniqueShard &S = shards.s[M == 1 ? 0 : blockIdx.y];
+  uint32_t tile, tiles;
+  const UniqueShard &S = my_record(shards, tile, tiles);
   const K *__restrict__ sk = (const K *)S.sorted_keys;
   const uint32_t n = S.b.n;
   const uint32_t *__restrict__ head_inner = S.heads.inner;
   const K *__restrict__ head_first = (const K *)S.heads.first, *__restrict__ head_last = (const K *)S.heads.last;
-  if (M > 1 && blockIdx.x * (ITEMS * kUBlock) >= n) return;
   constexpr uint32_t kTileU = ITEMS * kUBlock;
-  const uint32_t base = blockIdx.x * kTileU;
+  const uint32_t base = tile * kTileU;
   const unsigned lane = lane_id();
   // everything that comes from memory first: the keys of the tile, the key before every wave's first position and the
   // head counts of the chunks before the tile
@@ -159,34 +159,22 @@ __global__ __launch_bounds__(kRunListBlock) void list_long_runs(BatchView b) {
   list_runs_chunk(b, blockIdx.x, cnt, base);
 }
 
-// ---- push plan, three launches for all shards of a group (blockIdx.y = record) ------------------------------------
-struct PlanShards { PlanShard s[kShardsPerLaunch]; };
-struct BucketShards { BucketShard s[kShardsPerLaunch]; };
-// the records in pieces of one launch each: f(piece, records in it, keys of the largest batch among them)
-template <typename P, typename S, typename F> void for_shards(const S *shards, int count, F &&f) {
-  for (int i = 0; i < count; i += kShardsPerLaunch) {
-    P p = {};
-    const int m = std::min(kShardsPerLaunch, count - i);
-    uint32_t n = 0;
-    for (int k = 0; k < m; k++) {
-      p.s[k] = shards[i + k];
-      n = std::max(n, shards[i + k].b.n);
-    }
-    if (n) f(p, m, n);
-  }
-}
+// ---- push plan, three launches for all shards of a group ----------------------------------------------------------
+typedef Records<PlanShard, kShardsPerLaunch> PlanShards;
+typedef Records<BucketShard, kShardsPerLaunch> BucketShards;
 
 // need[u] of one tile of unique keys and the tile's sum
 template <typename K>
 __global__ __launch_bounds__(kBlock) void plan_decide(PlanShards shards, int id_bits) {
   __shared__ uint32_t sm[kBlock / kWave + 1];
-  const PlanShard &S = shards.s[blockIdx.y];
+  uint32_t tile, tiles;
+  const PlanShard &S = my_record(shards, tile, tiles);
   const uint32_t U = *S.b.d_U;
-  if (blockIdx.x * kTile >= U) return; // the grid is cut for the largest batch's keys
+  if (tile * kTile >= U) return; // the grid is cut for the batches' keys
   uint32_t c = 0;
 #pragma unroll
   for (int k = 0; k < kItems; k++) {
-    const uint32_t u = blockIdx.x * kTile + k * kBlock + threadIdx.x;
+    const uint32_t u = tile * kTile + k * kBlock + threadIdx.x;
     if (u >= U) continue;
     const int r = (int)(((const K *)S.b.ukey)[u] >> id_bits);
     const slot_t o = S.b.uoff[u];
@@ -200,19 +188,20 @@ __global__ __launch_bounds__(kBlock) void plan_decide(PlanShards shards, int id_
   }
   uint32_t total;
   block_exclusive_scan<kBlock>(c, sm, total);
-  if (threadIdx.x == 0) S.block_sums[blockIdx.x] = total;
+  if (threadIdx.x == 0) S.block_sums[tile] = total;
 }
 
 __global__ __launch_bounds__(kBlock) void plan_scan(PlanShards shards) {
   __shared__ uint32_t sm[kBlock / kWave + 1];
-  const PlanShard &S = shards.s[blockIdx.y];
+  uint32_t tile, tiles;
+  const PlanShard &S = my_record(shards, tile, tiles);
   const uint32_t U = *S.b.d_U;
-  if (blockIdx.x * kTile >= U) return;
+  if (tile * kTile >= U) return;
   uint32_t s = 0;
-  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kBlock) s += S.block_sums[i];
+  for (uint32_t i = threadIdx.x; i < tile; i += kBlock) s += S.block_sums[i];
   uint32_t prefix;
   block_exclusive_scan<kBlock>(s, sm, prefix);
-  const uint32_t j0 = blockIdx.x * kTile + threadIdx.x * kItems;
+  const uint32_t j0 = tile * kTile + threadIdx.x * kItems;
   uint32_t v[kItems], c = 0;
 #pragma unroll
   for (int k = 0; k < kItems; k++) {
@@ -221,7 +210,7 @@ __global__ __launch_bounds__(kBlock) void plan_scan(PlanShards shards) {
   }
   uint32_t total;
   uint32_t run = prefix + block_exclusive_scan<kBlock>(c, sm, total);
-  const bool last = (blockIdx.x + 1) * kTile >= U;
+  const bool last = (tile + 1) * kTile >= U;
 #pragma unroll
   for (int k = 0; k < kItems; k++) {
     if (j0 + k < U) S.prefix[j0 + k] = run;
@@ -260,39 +249,45 @@ __global__ void bucket_sizes(BucketShards shards, int nrank) {
 
 void launch_make_keys(hipStream_t s, const KeyLayout &kl, const KeyShard *shards, int count) {
   const int dbits = sort_first_digit_bits(kl.total_bits);
-  for_records(shards, count, [&](const auto &p, int m, uint32_t most) {
+  auto make = [&](int k) {
+    HCTR_CHECK(!shards[k].ids32 || shards[k].t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
+    HCTR_CHECK(sort_tile(shards[k].n) == sort_tile(shards[0].n), "internal: batches of one launch differ in shape");
+    return shards[k];
+  };
+  auto blocks = [&](int k) { return (uint32_t)sort_tiles(shards[k].n); };
+  launch_one_or_records<KeyShard>(count, kSortBlock, make, blocks, [&](const auto &p, int) {
     constexpr int M = sizeof p.s / sizeof p.s[0];
-    for (int k = 0; k < m; k++) {
-      HCTR_CHECK(!p.s[k].ids32 || p.s[k].t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
-      HCTR_CHECK(sort_tile(p.s[k].n) == sort_tile(most), "internal: batches of one launch differ in shape");
-    }
-    const dim3 grid((unsigned)sort_tiles(most), m);
+    const dim3 grid = grid_of(p);
 #define CALL(I)                                                                                                     \
   do {                                                                                                              \
     if (kl.wide) hipLaunchKernelGGL((make_keys<uint64_t, I, M>), grid, dim3(kSortBlock), 0, s, p, kl.id_bits, dbits); \
     else hipLaunchKernelGGL((make_keys<uint32_t, I, M>), grid, dim3(kSortBlock), 0, s, p, kl.id_bits, dbits);       \
   } while (0)
-    HCTR_SORT_ITEMS_DISPATCH(most, CALL);
+    HCTR_SORT_ITEMS_DISPATCH(shards[0].n, CALL);
 #undef CALL
     HCTR_HIP(hipGetLastError());
   });
 }
 
 void launch_unique(hipStream_t s, const KeyLayout &kl, const UniqueShard *shards, int count, bool count_heads) {
-  for_records(shards, count, [&](const auto &p, int m, uint32_t most) {
+  HCTR_CHECK(!count_heads || count == 1, "internal: heads are counted for one batch at a time");
+  const HeadChunks &heads = shards[0].heads;
+  // the tile of the pass: that of the sort that left the head counts, or kUTile when they are counted here
+  const int items = count_heads ? kUItems : (int)(heads.chunk / kWave);
+  const uint32_t chunk = count_heads ? (uint32_t)kUTile : heads.chunk;
+  auto make = [&](int k) {
+    HCTR_CHECK(shards[k].heads.chunk == heads.chunk, "internal: batches of one launch differ in shape");
+    return shards[k];
+  };
+  auto blocks = [&](int k) { return div_up(shards[k].b.n, (size_t)items * kUBlock); };
+  launch_one_or_records<UniqueShard>(count, kUBlock, make, blocks, [&](const auto &p, int) {
     constexpr int M = sizeof p.s / sizeof p.s[0];
-    const HeadChunks &heads = p.s[0].heads;
-    // the tile of the pass: that of the sort that left the head counts, or kUTile when they are counted here
-    const int items = count_heads ? kUItems : (int)(heads.chunk / kWave);
-    const uint32_t chunk = count_heads ? (uint32_t)kUTile : heads.chunk;
-    HCTR_CHECK(!count_heads || m == 1, "internal: heads are counted for one batch at a time");
-    for (int k = 0; k < m; k++) HCTR_CHECK(p.s[k].heads.chunk == heads.chunk, "internal: batches of one launch differ in shape");
-    const unsigned nb = div_up(most, (size_t)items * kUBlock);
-#define EMIT(K, I) hipLaunchKernelGGL((unique_emit<K, I, M>), dim3(nb, m), dim3(kUBlock), 0, s, p, kl.id_bits, chunk)
+    const dim3 grid = grid_of(p);
+#define EMIT(K, I) hipLaunchKernelGGL((unique_emit<K, I, M>), grid, dim3(kUBlock), 0, s, p, kl.id_bits, chunk)
 #define EMIT_K(K)                                                                                          \
   do {                                                                                                     \
     if (count_heads)                                                                                       \
-      hipLaunchKernelGGL(head_count<K>, dim3(nb), dim3(kUBlock), 0, s, (const K *)p.s[0].sorted_keys, most, heads.inner, \
+      hipLaunchKernelGGL(head_count<K>, grid, dim3(kUBlock), 0, s, (const K *)p.s[0].sorted_keys, p.s[0].b.n, heads.inner, \
                          (K *)heads.first, (K *)heads.last);                                              \
     switch (items) {                                                                                       \
       case 2: EMIT(K, 2); break;                                                                           \
@@ -324,8 +319,10 @@ void launch_list_long_runs(hipStream_t s, const BatchView &b) { // the class cou
 }
 
 void launch_plans(hipStream_t s, const KeyLayout &kl, const PlanShard *shards, int count) {
-  for_shards<PlanShards>(shards, count, [&](const PlanShards &p, int m, uint32_t n) {
-    const dim3 grid(div_up(n, kTile), m);
+  auto make = [&](int k) { return shards[k]; };
+  auto blocks = [&](int k) { return div_up(shards[k].b.n, kTile); };
+  launch_records<PlanShard, kShardsPerLaunch>(count, kBlock, make, blocks, [&](const PlanShards &p, int m) {
+    const dim3 grid = grid_of(p);
     if (kl.wide) hipLaunchKernelGGL(plan_decide<uint64_t>, grid, dim3(kBlock), 0, s, p, kl.id_bits);
     else hipLaunchKernelGGL(plan_decide<uint32_t>, grid, dim3(kBlock), 0, s, p, kl.id_bits);
     hipLaunchKernelGGL(plan_scan, grid, dim3(kBlock), 0, s, p);
@@ -336,13 +333,11 @@ void launch_plans(hipStream_t s, const KeyLayout &kl, const PlanShard *shards, i
 }
 
 void launch_bucket_sizes(hipStream_t s, int nrank, const BucketShard *shards, int count) {
-  for (int i = 0; i < count; i += kShardsPerLaunch) {
-    BucketShards a = {};
-    const int m = std::min(kShardsPerLaunch, count - i);
-    std::copy(shards + i, shards + i + m, a.s);
-    hipLaunchKernelGGL(bucket_sizes, dim3(m), dim3(nrank + 1), 0, s, a, nrank);
-  }
-  HCTR_HIP(hipGetLastError());
+  auto make = [&](int k) { return shards[k]; };
+  launch_records<BucketShard, kShardsPerLaunch>(count, nrank + 1, make, [](int) { return 1u; }, [&](const BucketShards &p, int m) {
+    hipLaunchKernelGGL(bucket_sizes, dim3(m), dim3(nrank + 1), 0, s, p, nrank);
+    HCTR_HIP(hipGetLastError());
+  });
 }
 
 } // namespace hctr

@@ -804,33 +804,31 @@ template <int VEC, int LPR, typename K, bool kPooled>
 __global__ HCTR_PUSH_BOUNDS void push_fused(TableView t, int id_bits, BatchView p, PushArgs a, uint32_t U) {
   push_block<VEC, LPR, K, true, kPooled>(t, id_bits, p, a, U, blockIdx.x);
 }
-// The pushes of the shards of a group in one launch.  The blocks every shard has alike come first, neighbouring blocks being
-// the same block of different shards, so that every shard's long chains start first; then come the shards' other blocks, as
-// many as each one's batch needs.
-struct PushShards {
-  PushShard s[kShardsPerLaunch];
-  BlockCut<kShardsPerLaunch> cut; // of the blocks behind the first kEachBlocks of every shard
-};
+// The pushes of the shards of a group in one launch.  First come the blocks that every shard has (its chains, its medium runs
+// and as many more as the smallest batch needs), neighbouring blocks being the same block of different shards, so that every
+// shard's long chains start first; behind them the rest of the larger batches, a shard after the other.
+typedef Records<PushShard, kShardsPerLaunch> PushShards; // cut: of the rest
 constexpr uint32_t kEachBlocks = kLongBlocks + kMedBlocks;
 template <int VEC, int LPR, typename K, bool kPooled>
-__global__ HCTR_PUSH_BOUNDS void push_group(PushShards shards, uint32_t count, int id_bits) {
+__global__ HCTR_PUSH_BOUNDS void push_group(PushShards shards, uint32_t count, uint32_t common, int id_bits) {
   uint32_t block = blockIdx.x, k;
-  if (block < kEachBlocks * count) {
+  if (block < common * count) {
     k = block % count;
     block /= count;
   } else {
-    block -= kEachBlocks * count;
+    block -= common * count;
     k = record_of(shards.cut, block);
-    block += kEachBlocks;
+    block += common;
   }
   const PushShard &S = shards.s[k];
   push_block<VEC, LPR, K, false, kPooled>(S.t, id_bits, S.b, S.a, S.n_unique, block);
 }
 
-struct PlaceShards { PlaceShard s[kShardsPerLaunch]; };
+typedef Records<PlaceShard, kShardsPerLaunch> PlaceShards;
 template <typename K> __global__ __launch_bounds__(256) void place_rows(PlaceShards shards, int id_bits) {
-  const PlaceShard &S = shards.s[blockIdx.y];
-  const uint32_t u = blockIdx.x * 256 + threadIdx.x;
+  uint32_t block, blocks;
+  const PlaceShard &S = my_record(shards, block, blocks);
+  const uint32_t u = block * 256 + threadIdx.x;
   if (u < S.n_unique) S.pos[u] = S.prefix[u] + S.delta[(uint32_t)(((const K *)S.ukey)[u] >> id_bits)];
 }
 
@@ -846,7 +844,9 @@ void launch_push_t(hipStream_t st, int id_bits, PushShards &shards, int count) {
   for (int i = 0; i < count;) { // nearly always one launch
     const int m = cut_blocks(shards.cut, count - i, kPushBlock, kEachBlocks, [&](int k) { return need(shards.s[i + k]); });
     if (i) std::copy(shards.s + i, shards.s + i + m, shards.s);
-    hipLaunchKernelGGL((push_group<VEC, LPR, K, kPooled>), dim3(kEachBlocks * m + shards.cut.total()), dim3(kPushBlock), 0, st, shards, (uint32_t)m, id_bits);
+    const uint32_t least = *std::min_element(shards.cut.blocks, shards.cut.blocks + m), common = kEachBlocks + least;
+    cut_blocks(shards.cut, m, kPushBlock, common, [&](int k) { return need(shards.s[k]) - least; });
+    hipLaunchKernelGGL((push_group<VEC, LPR, K, kPooled>), dim3(common * m + shards.cut.total), dim3(kPushBlock), 0, st, shards, (uint32_t)m, common, id_bits);
     i += m;
   }
 }
@@ -875,20 +875,14 @@ void launch_push_k(hipStream_t st, int id_bits, PushShards &shards, int count) {
 } // namespace
 
 void launch_place_rows(hipStream_t s, const KeyLayout &kl, const PlaceShard *shards, int count) {
-  for (int i = 0; i < count; i += kShardsPerLaunch) {
-    PlaceShards p = {};
-    const int m = std::min(kShardsPerLaunch, count - i);
-    uint32_t most = 0;
-    for (int k = 0; k < m; k++) {
-      p.s[k] = shards[i + k];
-      most = std::max(most, p.s[k].n_unique);
-    }
-    if (!most) continue;
-    const dim3 grid(div_up(most, 256), m);
+  auto make = [&](int k) { return shards[k]; };
+  auto need = [&](int k) { return div_up(shards[k].n_unique, 256); };
+  launch_records<PlaceShard, kShardsPerLaunch>(count, 256, make, need, [&](const PlaceShards &p, int) {
+    const dim3 grid = grid_of(p);
     if (kl.wide) hipLaunchKernelGGL(place_rows<uint64_t>, grid, dim3(256), 0, s, p, kl.id_bits);
     else hipLaunchKernelGGL(place_rows<uint32_t>, grid, dim3(256), 0, s, p, kl.id_bits);
     HCTR_HIP(hipGetLastError());
-  }
+  });
 }
 
 void launch_push(hipStream_t s, const KeyLayout &kl, const PushShard *shards, int count) {

@@ -99,7 +99,6 @@ struct TileSortShard {
   void *keys_out;
   uint32_t *sorted_arg;
   HeadChunks heads;
-  uint32_t keys() const { return n; }
 };
 // (every record or none has made_keys)
 void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count);
@@ -118,7 +117,6 @@ struct OneBlockShard {
   const void *keys_in;
   BatchView b;
   uint32_t *u_copy;
-  uint32_t keys() const { return b.n; }
 };
 void launch_index_one_block(hipStream_t s, const KeyLayout &kl, const OneBlockShard *shards, int count);
 
@@ -135,6 +133,5 @@ struct UniqueShard {
   BatchView b;
   HeadChunks heads;
   uint32_t *u_copy;
-  uint32_t keys() const { return b.n; }
 };
 } // namespace hctr

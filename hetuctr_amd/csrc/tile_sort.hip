@@ -166,12 +166,12 @@ struct KeysJob {
   uint16_t *table;
   void *keys_out;
   bool ids32;
-  uint32_t keys() const { return n; }
 };
-template <typename K, int ITEMS, int DBITS, bool kFromKeys, int M> // M: records of the launch, blockIdx.y picks one
+template <typename K, int ITEMS, int DBITS, bool kFromKeys, int M> // M: records of the launch
 __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M> jobs, uint64_t id_max, int id_bits, int nrank,
                                                               int dbits) {
-  const KeysJob &J = jobs.s[M == 1 ? 0 : blockIdx.y];
+  uint32_t tile, tile_blocks;
+  const KeysJob &J = my_record(jobs, tile, tile_blocks);
   const void *__restrict__ ids_or_keys = J.ids_or_keys;
   const uint32_t n = J.n, pitch = J.pitch;
   const worker_t *__restrict__ root = J.root;
@@ -179,12 +179,11 @@ __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M>
   K *__restrict__ out_keys = (K *)J.out_keys, *__restrict__ keys_out = (K *)J.keys_out;
   uint16_t *__restrict__ table = J.table;
   const bool ids32 = J.ids32;
-  if (M > 1 && blockIdx.x * TileShape<K, ITEMS>::kTile >= n) return; // the grid is cut for the largest batch
   using S = TileShape<K, ITEMS>;
   __shared__ __align__(16) uint32_t area[S::kAreaWords];
   __shared__ uint32_t bin_start[kSortMaxBins];
   __shared__ uint32_t sm[kWaves + 1];
-  const uint32_t tile = blockIdx.x, tile_lo = tile * S::kTile;
+  const uint32_t tile_lo = tile * S::kTile;
   const uint32_t tile_n = min((uint32_t)S::kTile, n - tile_lo);
   const int w = threadIdx.x / kWave;
   const unsigned lane = lane_id();
@@ -200,7 +199,7 @@ __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M>
     }
   } else {
     const index_t *__restrict__ ids = (const index_t *)ids_or_keys;
-    if (blockIdx.x == 0 && threadIdx.x < kRunCounters && nlong) nlong[threadIdx.x] = 0; // counters of this batch
+    if (tile == 0 && threadIdx.x < kRunCounters && nlong) nlong[threadIdx.x] = 0; // counters of this batch
     uint64_t id[ITEMS];
 #pragma unroll
     for (int r = 0; r < ITEMS; r++) {
@@ -291,11 +290,11 @@ struct RegroupJob {
   uint16_t *table_out;
   uint32_t *head_inner;
   void *head_first, *head_last;
-  uint32_t keys() const { return n; }
 };
 template <typename K, int ITEMS, int DBITS, bool kLast, int M>
 __global__ __launch_bounds__(kSortBlock) void regroup(Records<RegroupJob, M> jobs, int shift_in, int dbits_in, int shift, int dbits) {
-  const RegroupJob &J = jobs.s[M == 1 ? 0 : blockIdx.y];
+  uint32_t tile, tile_blocks;
+  const RegroupJob &J = my_record(jobs, tile, tile_blocks);
   const K *__restrict__ in_keys = (const K *)J.in_keys;
   const uint32_t *__restrict__ in_vals = J.in_vals;
   const uint16_t *__restrict__ table_in = J.table_in;
@@ -303,7 +302,6 @@ __global__ __launch_bounds__(kSortBlock) void regroup(Records<RegroupJob, M> job
   K *__restrict__ out_keys = (K *)J.out_keys, *__restrict__ head_first = (K *)J.head_first, *__restrict__ head_last = (K *)J.head_last;
   uint32_t *__restrict__ out_vals = J.out_vals, *__restrict__ head_inner = J.head_inner;
   uint16_t *__restrict__ table_out = J.table_out;
-  if (M > 1 && blockIdx.x >= tiles) return;
   using S = TileShape<K, ITEMS>;
   __shared__ __align__(16) uint32_t area[S::kAreaWords];
   __shared__ uint32_t bin_start[kSortMaxBins];
@@ -311,7 +309,6 @@ __global__ __launch_bounds__(kSortBlock) void regroup(Records<RegroupJob, M> job
   __shared__ uint32_t coarse[kCoarse], fine[2 * kCoarse];
   __shared__ uint32_t found[6];
   __shared__ uint32_t wmax[kWaves];
-  const uint32_t tile = blockIdx.x;
   const uint32_t p0 = tile * S::kTile, tile_n = min((uint32_t)S::kTile, n - p0), p1 = p0 + tile_n;
   const uint32_t nb = 1u << dbits_in;
   const int w = threadIdx.x / kWave;
@@ -484,7 +481,8 @@ struct OneBlockJob {
 };
 template <typename K, int ITEMS, int DBITS, int M>
 __global__ __launch_bounds__(kSortBlock) void index_one_block(Records<OneBlockJob, M> jobs, int bits, int id_bits, int nrank) {
-  const OneBlockJob &J = jobs.s[M == 1 ? 0 : blockIdx.y];
+  uint32_t block, blocks;
+  const OneBlockJob &J = my_record(jobs, block, blocks);
   const K *__restrict__ keys = (const K *)J.in;
   const BatchView &b = J.b;
   const uint32_t n = b.n;
@@ -582,15 +580,16 @@ DigitPlan plan_digits(const KeyLayout &kl) {
 void launch_index_one_block(hipStream_t s, const KeyLayout &kl, const OneBlockShard *shards, int count) {
   const int bits = kl.total_bits < 1 ? 1 : kl.total_bits;
   const bool nine = (bits + 8) / 9 == (bits + 9) / 10; // narrower digits where they take as many passes
-  for_records(shards, count, [&](const auto &p, int m, uint32_t most) {
+  auto make = [&](int k) -> OneBlockJob { return {shards[k].keys_in, shards[k].t.slot, shards[k].b, shards[k].u_copy}; };
+  launch_one_or_records<OneBlockJob>(count, kSortBlock, make, [](int) { return 1u; }, [&](const auto &jobs, int m) {
+    constexpr int M = sizeof jobs.s / sizeof jobs.s[0];
+    uint32_t most = 1;
+    for (int k = 0; k < m; k++) most = std::max(most, jobs.s[k].b.n);
     HCTR_CHECK(most <= kOneBlockKeys, "internal: batch too large for one block");
     const int items = (int)div_up(most, kSortBlock); // of the largest batch: fits the others too
-    constexpr int M = sizeof p.s / sizeof p.s[0];
-    Records<OneBlockJob, M> jobs = {};
-    for (int k = 0; k < m; k++) jobs.s[k] = {p.s[k].keys_in, p.s[k].t.slot, p.s[k].b, p.s[k].u_copy};
-    const int nrank = p.s[0].t.nrank;
+    const int nrank = shards[0].t.nrank;
 #define ONE(K, I, D) \
-  hipLaunchKernelGGL((index_one_block<K, I, D, M>), dim3(1, m), dim3(kSortBlock), 0, s, jobs, bits, kl.id_bits, nrank)
+  hipLaunchKernelGGL((index_one_block<K, I, D, M>), grid_of(jobs), dim3(kSortBlock), 0, s, jobs, bits, kl.id_bits, nrank)
 #define ONE_D(K, I)                \
   do {                             \
     if (nine) ONE(K, I, 9);        \
@@ -618,26 +617,27 @@ static uint16_t *tile_table(const TileSortShard &o, int which) {
 
 void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count) {
   const DigitPlan p = plan_digits(kl);
-  for_records(shards, count, [&](const auto &r, int m, uint32_t most) {
-    constexpr int M = sizeof r.s / sizeof r.s[0];
-    Records<KeysJob, M> jobs = {};
-    const bool made = r.s[0].made_keys != nullptr;
-    for (int k = 0; k < m; k++) {
-      const TileSortShard &o = r.s[k];
-      HCTR_CHECK(!o.ids32 || o.t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
-      HCTR_CHECK(tile_sort_possible(o.n), "internal: batch too large for the tile-sorted passes");
-      HCTR_CHECK(tile_items(o.n) == tile_items(most) && (o.made_keys != nullptr) == made, "internal: batches of one launch differ in shape");
-      jobs.s[k] = {made ? o.made_keys : (const void *)o.ids, o.n, (uint32_t)tile_table_pitch(o.n), o.t.root, o.err, o.nlong, o.b.keys[0],
-                   o.b.vals[0], tile_table(o, 0), made ? nullptr : o.keys_out, o.ids32};
-    }
-    const TableView &t = r.s[0].t;
-    const dim3 grid((unsigned)tile_count(most), m);
+  const TileSortShard &f = shards[0];
+  const bool made = f.made_keys != nullptr;
+  auto make = [&](int k) -> KeysJob {
+    const TileSortShard &o = shards[k];
+    HCTR_CHECK(!o.ids32 || o.t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
+    HCTR_CHECK(tile_sort_possible(o.n), "internal: batch too large for the tile-sorted passes");
+    HCTR_CHECK(tile_items(o.n) == tile_items(f.n) && (o.made_keys != nullptr) == made, "internal: batches of one launch differ in shape");
+    return {made ? o.made_keys : (const void *)o.ids, o.n, (uint32_t)tile_table_pitch(o.n), o.t.root, o.err, o.nlong, o.b.keys[0],
+            o.b.vals[0], tile_table(o, 0), made ? nullptr : o.keys_out, o.ids32};
+  };
+  auto blocks = [&](int k) { return (uint32_t)tile_count(shards[k].n); };
+  launch_one_or_records<KeysJob>(count, kSortBlock, make, blocks, [&](const auto &jobs, int) {
+    constexpr int M = sizeof jobs.s / sizeof jobs.s[0];
+    const TableView &t = f.t;
+    const dim3 grid = grid_of(jobs);
 #define CALL(K, I, D)                                                                                                  \
   do {                                                                                                                 \
     if (made) hipLaunchKernelGGL((keys_tile_sort<K, I, D, true, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0]); \
     else hipLaunchKernelGGL((keys_tile_sort<K, I, D, false, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0]); \
   } while (0)
-    HCTR_TILE_SORT_DISPATCH(kl.wide, most, p.dbits[0], CALL);
+    HCTR_TILE_SORT_DISPATCH(kl.wide, f.n, p.dbits[0], CALL);
 #undef CALL
     HCTR_HIP(hipGetLastError());
   });
@@ -648,28 +648,28 @@ int launch_tile_sort_passes(hipStream_t s, const KeyLayout &kl, const TileSortSh
   for (int j = std::max(from, 1); j <= p.passes && j < to; j++) {
     const int in = (j - 1) & 1, out = j & 1;
     const bool last = j == p.passes;
-    for_records(shards, count, [&](const auto &r, int m, uint32_t most) {
-      constexpr int M = sizeof r.s / sizeof r.s[0];
-      Records<RegroupJob, M> jobs = {};
-      for (int k = 0; k < m; k++) {
-        const TileSortShard &o = r.s[k];
-        HCTR_CHECK(tile_items(o.n) == tile_items(most), "internal: batches of one launch differ in shape");
-        HCTR_CHECK(o.heads.chunk == (uint32_t)tile_items(o.n) * kWave, "internal: head chunks do not match the tile shape");
-        jobs.s[k] = {o.b.keys[in], o.b.vals[in], tile_table(o, in), o.n, (uint32_t)tile_count(o.n), (uint32_t)tile_table_pitch(o.n),
-                     o.b.keys[out], last ? o.sorted_arg : o.b.vals[out], last ? nullptr : tile_table(o, out), o.heads.inner,
-                     o.heads.first, o.heads.last};
-      }
-      const dim3 grid((unsigned)tile_count(most), m);
+    auto make = [&](int k) -> RegroupJob {
+      const TileSortShard &o = shards[k];
+      HCTR_CHECK(tile_items(o.n) == tile_items(shards[0].n), "internal: batches of one launch differ in shape");
+      HCTR_CHECK(o.heads.chunk == (uint32_t)tile_items(o.n) * kWave, "internal: head chunks do not match the tile shape");
+      return {o.b.keys[in], o.b.vals[in], tile_table(o, in), o.n, (uint32_t)tile_count(o.n), (uint32_t)tile_table_pitch(o.n),
+              o.b.keys[out], last ? o.sorted_arg : o.b.vals[out], last ? nullptr : tile_table(o, out), o.heads.inner,
+              o.heads.first, o.heads.last};
+    };
+    auto blocks = [&](int k) { return (uint32_t)tile_count(shards[k].n); };
+    launch_one_or_records<RegroupJob>(count, kSortBlock, make, blocks, [&](const auto &jobs, int) {
+      constexpr int M = sizeof jobs.s / sizeof jobs.s[0];
+      const dim3 grid = grid_of(jobs);
       if (!last) {
 #define CALL(K, I, D)                                                                                                 \
   hipLaunchKernelGGL((regroup<K, I, D, false, M>), grid, dim3(kSortBlock), 0, s, jobs, p.shift[j - 1], p.dbits[j - 1], \
                      p.shift[j], p.dbits[j])
-        HCTR_TILE_SORT_DISPATCH(kl.wide, most, p.dbits[j], CALL);
+        HCTR_TILE_SORT_DISPATCH(kl.wide, shards[0].n, p.dbits[j], CALL);
 #undef CALL
       } else {
 #define CALL(K, I, D) \
   hipLaunchKernelGGL((regroup<K, I, 0, true, M>), grid, dim3(kSortBlock), 0, s, jobs, p.shift[j - 1], p.dbits[j - 1], 0, 0)
-        HCTR_TILE_SORT_DISPATCH(kl.wide, most, 0, CALL);
+        HCTR_TILE_SORT_DISPATCH(kl.wide, shards[0].n, 0, CALL);
 #undef CALL
       }
       HCTR_HIP(hipGetLastError());

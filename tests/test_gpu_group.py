@@ -350,3 +350,37 @@ def test_groups_of_more_shards_than_a_launch_serves(nrank, width):
         p.compare_state(1e-5, "step %d" % step)
         prev = ns
     p.close()
+
+
+@pytest.mark.parametrize("sizes,width", [
+    # tile-sorted batches of one shape in more shards than a launch serves, one-block ones and an empty one among them
+    ([8193 + 431 * r for r in range(13)] + [8192, 40, 0, 2_500], 8),
+    # three shapes of the index side by side: four and two keys per thread of a sort tile, and one block
+    ([270_000, 9_000, 300], 5),
+    # one large batch beside many small ones: a launch's blocks belong to very different numbers of rows
+    ([120_000] + [60] * 8, 12)])
+def test_batches_of_unequal_shape_in_shared_launches(sizes, width):
+    nrank = len(sizes)
+    say("shared launches, keys per shard", sizes, "width", width)
+    p, _ = update_pair(nrank, 30_000, width, bounds=(1, 2), init=("Uniform", -0.1, 0.1), lr=0.05, cache="third", seed=nrank)
+    rng = np.random.default_rng(nrank)
+    draw = zipf_sampler(30_000, 1.1, rng)
+    prev = [0] * nrank
+    for step in range(4):
+        ns = [sizes[(r + 2 * step) % nrank] for r in range(nrank)]
+        keys = [draw(n) for n in ns]
+        # the ids of every other shard lie in host memory
+        dev = [None if (r + step) % 2 else torch.from_numpy(keys[r]).cuda() for r in range(nrank)]
+        torch.cuda.synchronize()
+        ptrs = [0 if not ns[r] else keys[r].ctypes.data if dev[r] is None else dev[r].data_ptr() for r in range(nrank)]
+        capi.group_preprocess(p.tables, ptrs, ns)
+        p.n = ns
+        p.oracle.preprocess(keys)
+        p.compare_ints(INT_ITEMS_PRE, "step %d" % step)
+        out, ref = p.push_pull([rng.normal(0, 1e-2, size=(n, width)).astype(np.float32) for n in prev])
+        p.compare_ints(INT_ITEMS_POST, "step %d" % step)
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        p.compare_state(1e-5, "step %d" % step)
+        prev = ns
+    p.close()

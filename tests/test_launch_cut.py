@@ -4,8 +4,8 @@ import subprocess
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hetuctr_amd", "csrc")
 
-# Records of 0 blocks to millions, in every place; every block of a launch must find its record and number, no block may be
-# left over, and a launch must stay below 2^32 threads (one that cannot goes alone).
+# Records of 0 blocks to millions, in every place: every block of a launch must find its record and number, no block may be left
+# over, and a launch must stay below 2^32 threads (a record that cannot goes alone).
 PROGRAM = r"""
 #include <cstdio>
 #include <cstdlib>
@@ -18,22 +18,21 @@ static const char *check(const std::vector<uint32_t> &need, uint32_t threads, ui
   for (int i = 0; i < (int)need.size();) {
     BlockCut<M> cut;
     for (auto &f : cut.first) f = 12345; // what the launch before left there
-    cut.first[0] = 0;
     const int m = cut_blocks(cut, (int)need.size() - i, threads, each, [&](int k) { return need[i + k]; });
     if (m < 1 || m > M) return "a launch serves no record, or too many";
     uint64_t sum = 0;
     for (int k = 0; k < m; k++) {
-      if (cut.blocks(k) != need[i + k]) return "a record has not the blocks it needs";
-      sum += need[i + k];
-    }
-    if (cut.total() != sum) return "blocks without a record";
-    if (m > 1 && (sum + (uint64_t)each * m) * threads >= (1ull << 32)) return "too many threads";
-    for (int k = 0; k < M; k++)
-      for (uint32_t b : {0u, 1u, need[k < m ? i + k : i] / 2, cut.blocks(k) - 1})
-        if (b < cut.blocks(k)) {
-          uint32_t block = cut.first[k] + b;
-          if (record_of(cut, block) != k || block != b) return "a block finds another record";
+      const uint32_t n = need[i + k];
+      if (cut.blocks[k] != n) return "a record has not the blocks it needs";
+      for (uint32_t b : {0u, 1u, n / 2, n - 1})
+        if (b < n) {
+          uint32_t block = (uint32_t)sum + b;
+          if ((int)record_of(cut, block) != k || block != b) return "a block finds another record";
         }
+      sum += n;
+    }
+    if (cut.total != sum) return "blocks without a record";
+    if (m > 1 && (sum + (uint64_t)each * m) * threads >= (1ull << 32)) return "too many threads";
     i += m;
     launches++;
   }
