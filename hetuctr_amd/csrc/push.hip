@@ -83,36 +83,48 @@ template <bool kPooled> __device__ __forceinline__ uint32_t grad_row(uint32_t po
   return kPooled ? bag(pos) : pos;
 }
 
-// the columns a lane moves at a time (see kOdd4 in kernels.h); V: as they lie in memory
-template <int VEC> struct Vec;
-struct Vec4Ops {
-  typedef f32x4 T;
-  static __device__ __forceinline__ T zero() { return (f32x4){0.f, 0.f, 0.f, 0.f}; }
+// The columns a lane moves at a time (see kOdd4 in kernels.h).  M: as they lie in memory.  T: as the lane computes with them, a
+// vector f32x4 or the four floats of a float4.  The medium role takes the latter: its two batches of vectors, each held in
+// four registers in a row, left one register too few, and a push with scratch memory took a batch of 53 k keys 22.2 us
+// instead of 20.4.  The short role takes vectors: 8.5 M uniform keys are pushed in 1027 us, with float4 in 1064.
+template <typename T4, typename Mem> struct Vec4 {
+  typedef T4 T;
+  typedef Mem M;
+  static __device__ __forceinline__ T zero() { return T{0.f, 0.f, 0.f, 0.f}; }
   static __device__ __forceinline__ void add(T &a, const T &b) { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
-  static __device__ __forceinline__ T scale(const T &a, float s) { return (f32x4){a.x * s, a.y * s, a.z * s, a.w * s}; }
+  static __device__ __forceinline__ T scale(const T &a, float s) { return T{a.x * s, a.y * s, a.z * s, a.w * s}; }
+  static __device__ __forceinline__ T load(const float *p) { return of(*(const M *)p); }
+  static __device__ __forceinline__ T load_once(const float *p) { return of(__builtin_nontemporal_load((const M *)p)); }
+  static __device__ __forceinline__ void store_all(float *p, const T &a) { *(M *)p = to(a); }
+  static __device__ __forceinline__ void store_all_away(float *p, const T &a) { __builtin_nontemporal_store(to(a), (M *)p); }
+
+ private:
+  static __device__ __forceinline__ T of(const f32x4 &v) { return T{v.x, v.y, v.z, v.w}; }
+  static __device__ __forceinline__ f32x4 to(const T &a) { return f32x4{a.x, a.y, a.z, a.w}; }
 };
-template <> struct Vec<4> : Vec4Ops {
-  typedef f32x4 M;
-  static __device__ __forceinline__ void store(float *p, const T &a, uint32_t) { *(M *)p = a; }
+template <int VEC, typename T4 = f32x4> struct Vec;
+template <typename T4> struct Vec<4, T4> : Vec4<T4, f32x4> {
+  typedef Vec4<T4, f32x4> B;
+  static __device__ __forceinline__ void store(float *p, const T4 &a, uint32_t) { B::store_all(p, a); }
   // a store past the caches: for rows another shard's kernel reads next
-  static __device__ __forceinline__ void store_away(float *p, const T &a, uint32_t) { __builtin_nontemporal_store(a, (M *)p); }
+  static __device__ __forceinline__ void store_away(float *p, const T4 &a, uint32_t) { B::store_all_away(p, a); }
 };
-template <> struct Vec<kOdd4> : Vec4Ops {
-  typedef f32x4_any M;
+template <typename T4> struct Vec<kOdd4, T4> : Vec4<T4, f32x4_any> {
+  typedef Vec4<T4, f32x4_any> B;
   // without the first `shared` columns, which the lane before writes (and, in a row of more than one round of the
   // group, may have updated before this lane reads them: what it computes for them is dropped)
-  static __device__ __forceinline__ void store(float *p, const T &a, uint32_t shared) {
+  static __device__ __forceinline__ void store(float *p, const T4 &a, uint32_t shared) {
     if (!shared) {
-      *(M *)p = a;
+      B::store_all(p, a);
     } else {
       if (shared < 2) p[1] = a.y;
       if (shared < 3) p[2] = a.z;
       p[3] = a.w;
     }
   }
-  static __device__ __forceinline__ void store_away(float *p, const T &a, uint32_t shared) {
+  static __device__ __forceinline__ void store_away(float *p, const T4 &a, uint32_t shared) {
     if (!shared) {
-      __builtin_nontemporal_store(a, (M *)p);
+      B::store_all_away(p, a);
     } else {
       if (shared < 2) __builtin_nontemporal_store(a.y, p + 1);
       if (shared < 3) __builtin_nontemporal_store(a.z, p + 2);
@@ -120,22 +132,22 @@ template <> struct Vec<kOdd4> : Vec4Ops {
     }
   }
 };
-template <> struct Vec<1> {
+template <typename T4> struct Vec<1, T4> {
   typedef float T;
-  typedef float M;
   static __device__ __forceinline__ T zero() { return 0.f; }
   static __device__ __forceinline__ void add(T &a, const T &b) { a += b; }
   static __device__ __forceinline__ T scale(const T &a, float s) { return a * s; }
+  static __device__ __forceinline__ T load(const float *p) { return *p; }
+  static __device__ __forceinline__ T load_once(const float *p) { return __builtin_nontemporal_load(p); }
+  static __device__ __forceinline__ void store_all(float *p, const T &a) { *p = a; }
   static __device__ __forceinline__ void store(float *p, const T &a, uint32_t) { *p = a; }
   static __device__ __forceinline__ void store_away(float *p, const T &a, uint32_t) { __builtin_nontemporal_store(a, p); }
 };
 
 // A gradient row is read exactly once per step: it is loaded past the caches.  With sum-pooled bags (kPooled) a row
 // is read once per key of its bag, so there it is loaded the ordinary way and the repeats hit the cache.
-template <int VEC, bool kPooled> __device__ __forceinline__ typename Vec<VEC>::T grad_load(const embed_t *p) {
-  typedef typename Vec<VEC>::M M;
-  if (HCTR_GRAD_NT && !kPooled) return __builtin_nontemporal_load((const M *)p);
-  return *(const M *)p;
+template <typename R, bool kPooled> __device__ __forceinline__ typename R::T grad_load(const embed_t *p) { // R: a Vec
+  return HCTR_GRAD_NT && !kPooled ? R::load_once(p) : R::load(p);
 }
 
 // The version / update counters of unique rank u and its entry among the pushed rows (gradient_index_kernel,
@@ -162,18 +174,17 @@ __device__ __forceinline__ void move_counters(const TableView &t, int id_bits, c
 
 // Applies the finished sum of unique rank u (already multiplied by -lr) to column(s) `col`.  Update types as in
 // generate_query.cu:18-25.  The counters of the row move in the last blocks of the launch.
-template <int VEC, typename K>
+template <typename R, typename K> // R: a Vec
 __device__ __forceinline__ void apply_row(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
-                                          uint32_t u, typename Vec<VEC>::T s, uint32_t col, uint32_t shared = 0) {
-  typedef typename Vec<VEC>::T V;
-  typedef typename Vec<VEC>::M M;
+                                          uint32_t u, typename R::T s, uint32_t col, uint32_t shared = 0) {
+  typedef typename R::T V;
   const slot_t o = p.uoff[u];
   const uint32_t W = t.width;
   if (t.nrank == 1) { // every key is owned and resident: type 1 only
     embed_t *e = t.emb + (size_t)o * W + col;
-    V cur = *(const M *)e;
-    Vec<VEC>::add(cur, s);
-    Vec<VEC>::store(e, cur, shared);
+    V cur = R::load(e);
+    R::add(cur, s);
+    R::store(e, cur, shared);
     return;
   }
   const bool need = a.need[u] != 0;
@@ -181,21 +192,21 @@ __device__ __forceinline__ void apply_row(const TableView &t, int id_bits, const
   const uint32_t q = a.prefix[u];
   if (type != 0) {
     embed_t *e = t.emb + (size_t)o * W + col;
-    V cur = *(const M *)e;
-    Vec<VEC>::add(cur, s);
-    Vec<VEC>::store(e, cur, shared);
+    V cur = R::load(e);
+    R::add(cur, s);
+    R::store(e, cur, shared);
   } else {
-    Vec<VEC>::store_away(a.g_val + (size_t)q * W + col, s, shared);
+    R::store_away(a.g_val + (size_t)q * W + col, s, shared);
   }
   if (type >= 2) {
     embed_t *g = t.pend + (size_t)o * W + col;
-    V pg = *(const M *)g;
-    Vec<VEC>::add(pg, s);
+    V pg = R::load(g);
+    R::add(pg, s);
     if (type == 2) {
-      Vec<VEC>::store_away(a.g_val + (size_t)q * W + col, pg, shared);
-      pg = Vec<VEC>::zero();
+      R::store_away(a.g_val + (size_t)q * W + col, pg, shared);
+      pg = R::zero();
     }
-    Vec<VEC>::store(g, pg, shared);
+    R::store(g, pg, shared);
   }
 }
 
@@ -218,7 +229,6 @@ template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
 __device__ __forceinline__ void short_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
                                            uint32_t block, uint32_t U) {
   typedef typename Vec<VEC>::T V;
-  typedef typename Vec<VEC>::M M;
   constexpr int G = kRunsPerGroup;
   constexpr int kGroups = kPushBlock / LPR;
   const uint32_t W = t.width, n = p.n;
@@ -267,13 +277,13 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 #pragma unroll
     for (int i = 0; i < G; i++) {
       e[i] = Vec<VEC>::zero();
-      if (mine[i] && (kSingle || type[i] != 0)) e[i] = *(const M *)(t.emb + (size_t)off[i] * W + col);
+      if (mine[i] && (kSingle || type[i] != 0)) e[i] = Vec<VEC>::load(t.emb + (size_t)off[i] * W + col);
     }
     if (!kSingle) {
 #pragma unroll
       for (int i = 0; i < G; i++) {
         pg[i] = Vec<VEC>::zero();
-        if (mine[i] && type[i] >= 2) pg[i] = *(const M *)(t.pend + (size_t)off[i] * W + col);
+        if (mine[i] && type[i] >= 2) pg[i] = Vec<VEC>::load(t.pend + (size_t)off[i] * W + col);
       }
     }
 #pragma unroll
@@ -285,7 +295,7 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 #pragma unroll
       for (int k = 0; k < kHead; k++) {
         v[i][k] = Vec<VEC>::zero();
-        if (mine[i] && (uint32_t)k < len[i]) v[i][k] = grad_load<VEC, kPooled>(grad + (size_t)si[i][k] * W + col);
+        if (mine[i] && (uint32_t)k < len[i]) v[i][k] = grad_load<Vec<VEC>, kPooled>(grad + (size_t)si[i][k] * W + col);
       }
     V acc[G];
 #pragma unroll
@@ -305,7 +315,7 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 #pragma unroll
         for (int k = 0; k < kTail; k++) sj[k] = grad_row<kPooled>(sorted_arg[min(j + k, rs[i + 1] - 1)], a.bag);
 #pragma unroll
-        for (int k = 0; k < kTail; k++) x[k] = grad_load<VEC, kPooled>(grad + (size_t)sj[k] * W + col);
+        for (int k = 0; k < kTail; k++) x[k] = grad_load<Vec<VEC>, kPooled>(grad + (size_t)sj[k] * W + col);
 #pragma unroll
         for (int k = 0; k < kTail; k++)
           if (j + k < rs[i + 1]) Vec<VEC>::add(acc[i], x[k]);
@@ -346,8 +356,8 @@ __device__ __forceinline__ void short_role(const TableView &t, int id_bits, cons
 template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
 __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
                                             uint32_t *lds_idx, uint32_t block, uint32_t nblocks) {
-  typedef typename Vec<VEC>::T V;
-  typedef typename Vec<VEC>::M M;
+  typedef Vec<VEC, float4> R;
+  typedef typename R::T V;
   constexpr int kGroups = kPushBlock / LPR;
   const uint32_t W = t.width;
   const uint32_t gl = threadIdx.x % LPR;
@@ -371,18 +381,18 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
       const uint32_t due = c0 + gl * kCols<VEC>, col = lane_col<VEC>(due, W), shared = due - col;
       const bool active = due < W;
       const embed_t *gcol = grad + (active ? col : 0);
-      V e = Vec<VEC>::zero();
-      if (kSingle && active) e = *(const M *)(t.emb + (size_t)off * W + col);
-      V acc = Vec<VEC>::zero();
+      V e = R::zero();
+      if (kSingle && active) e = R::load(t.emb + (size_t)off * W + col);
+      V acc = R::zero();
       V xa[kBatch], xb[kBatch];
       auto fetch = [&](V(&x)[kBatch], uint32_t q0) { // rows q0 .. q0+kBatch-1 of the run (clamped to its end)
 #pragma unroll
-        for (int k = 0; k < kBatch; k++) x[k] = grad_load<VEC, kPooled>(gcol + (size_t)my_idx[min(q0 + k, len - 1)] * W);
+        for (int k = 0; k < kBatch; k++) x[k] = grad_load<R, kPooled>(gcol + (size_t)my_idx[min(q0 + k, len - 1)] * W);
       };
       auto add = [&](const V(&x)[kBatch], uint32_t q0) {
 #pragma unroll
         for (int k = 0; k < kBatch; k++)
-          if (q0 + k < len) Vec<VEC>::add(acc, x[k]);
+          if (q0 + k < len) R::add(acc, x[k]);
       };
       fetch(xa, 0);
       for (uint32_t q = 0; q < len; q += 2 * kBatch) {
@@ -392,12 +402,12 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
         if (q + kBatch < len) add(xb, q + kBatch);
       }
       if (!active) continue;
-      const V scaled = Vec<VEC>::scale(acc, neg_lr);
+      const V scaled = R::scale(acc, neg_lr);
       if (kSingle) {
-        Vec<VEC>::add(e, scaled);
-        Vec<VEC>::store(t.emb + (size_t)off * W + col, e, shared); // versions: bump_versions
+        R::add(e, scaled);
+        R::store(t.emb + (size_t)off * W + col, e, shared); // versions: bump_versions
       } else {
-        apply_row<VEC, K>(t, id_bits, p, a, u, scaled, col, shared);
+        apply_row<R, K>(t, id_bits, p, a, u, scaled, col, shared);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -444,7 +454,6 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
                                           float *lds, uint4 *table, uint32_t *shared, float *row_stash, int c_lo,
                                           int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
   typedef typename Vec<VEC>::T V;
-  typedef typename Vec<VEC>::M M;
   constexpr uint32_t C = kCols<VEC>;
   const uint32_t W = t.width;
   uint32_t CS = CSC ? (uint32_t)CSC : min((uint32_t)kSlice, (W + C - 1) / C * C);
@@ -558,7 +567,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
       // Loads are unconditional and branch-free so that kDepth chunks stay in flight per thread: positions
       // past the end of a run re-read its last row (never summed), lanes outside the slice read column 0.
       const embed_t *gbase = a.grad + ((in_slice && due < W) ? col : 0);
-      auto row_load = [&](uint32_t idx) -> V { return grad_load<VEC, kPooled>(gbase + (size_t)idx * W); };
+      auto row_load = [&](uint32_t idx) -> V { return grad_load<Vec<VEC>, kPooled>(gbase + (size_t)idx * W); };
       // cursor of the index stage, 2 * kDepth chunks ahead of the LDS stage; past the end of the stream it
       // stays on the last run
       uint32_t cj = 0, cc = 0;
@@ -601,7 +610,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
         for (int q = 0; q < kRPT; q++) {
           if (in_slice) {
             if (CSC) store_transposed(sp + my_lane * pitch + (q * RPL + my_row), (CSC / 4) * pitch, val[k][q]);
-            else *(M *)(sp + (q * RPL + my_row) * CS + lcol) = val[k][q];
+            else Vec<VEC>::store_all(sp + (q * RPL + my_row) * CS + lcol, val[k][q]);
           }
           val[k][q] = row_load(idx[k][q]); // chunk + kDepth
         }
@@ -720,7 +729,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
         if (col_ok) {
           const float scaled = acc * neg_lr;
           if (direct) t.emb[(size_t)m.w * W + mycol] = row_stash[j * kWave + threadIdx.x] + scaled;
-          else apply_row<1, K>(t, id_bits, p, a, m.x, scaled, mycol);
+          else apply_row<Vec<1>, K>(t, id_bits, p, a, m.x, scaled, mycol);
         }
       }
     }
