@@ -151,8 +151,8 @@ def test_skewed_keys_long_runs(alpha, width):
 @pytest.mark.parametrize("nrank", [1, 2])
 @pytest.mark.parametrize("width", [128, 20])
 def test_gradient_and_output_pointers_off_by_four_bytes(width, nrank):
-    # width % 4 == 0 but neither pointer 16-byte aligned: both kernels must fall back to 4-byte lanes (a 64-lane group
-    # per row at width 128) and still match the oracle bit for bit; skewed keys, so every role of the push runs
+    # width % 4 == 0 but neither pointer 16-byte aligned: both kernels move four floats at 4-byte addresses and still match
+    # the oracle bit for bit; skewed keys, so every role of the push runs
     import torch
     say("unaligned grad / dst, width", width, "shards", nrank)
     rng = np.random.default_rng(700 + width + nrank)

@@ -50,6 +50,50 @@ def test_single_shard_pooled(bag, width, gather, monkeypatch):
     p.close()
 
 
+@pytest.mark.parametrize("gather", ["from the keys", "through the inverse index"])
+@pytest.mark.parametrize("nrank", [1, 2])
+@pytest.mark.parametrize("bag,width,off", [(2, 5, 0), (3, 7, 1), (10, 37, 0), (4, 67, 1), (3, 2, 0), (5, 64, 1)])
+def test_pooled_rows_of_odd_widths_and_unaligned_pointers(bag, width, off, nrank, gather, monkeypatch):
+    # rows whose last four-float vector overlaps the one before, and gradient and output pointers off by `off` floats, in
+    # both pooled gathers and the pooled push; keys skewed enough for runs of every length
+    if gather != "from the keys":
+        if nrank > 1:
+            pytest.skip("several shards have one gather")
+        monkeypatch.setenv("HETUCTR_POOLED_FROM_KEYS", "0")
+        monkeypatch.setenv("HETUCTR_DIRECT_GATHER_MAX", "0")
+    print("pooled, bag", bag, "width", width, "pointers off by", off, "shards", nrank, gather, flush=True)
+    rng = np.random.default_rng(100 * width + bag + nrank)
+    length, bags = 6_000, 2_500
+    root = rng.integers(0, nrank, size=length).astype(np.uint8)
+    storage = []
+    for r in range(nrank):
+        own, other = np.where(root == r)[0], np.where(root != r)[0]
+        storage.append(np.concatenate([other[::3], own]).astype(np.int64))
+    p = Pair(nrank, length, width, root, storage, init=("Uniform", -0.01, 0.01), lr=0.05, bounds=(2, 2) if nrank > 1 else (0, 0))
+    draw = zipf_sampler(length, 1.25, rng)
+    prev = 0
+    for step in range(3):
+        nb = bags - 3 * step
+        p.preprocess([draw(nb * bag) for _ in range(nrank)], device_keys=True)
+        grads = [rng.normal(0, 1e-3, size=(prev, width)).astype(np.float32) for _ in range(nrank)]
+        gbuf = [torch.zeros(prev * width + 1, device="cuda") for _ in range(nrank)]
+        dbuf = [torch.full((nb * width + 1,), float("nan"), device="cuda") for _ in range(nrank)]
+        for r in range(nrank):
+            gbuf[r][off:off + prev * width].copy_(torch.from_numpy(grads[r].reshape(-1)))
+        torch.cuda.synchronize()
+        capi.group_push_pull_pooled(p.tables, [g.data_ptr() + 4 * off if prev else 0 for g in gbuf],
+                                    [d.data_ptr() + 4 * off for d in dbuf], bag)
+        ref = p.oracle.push_pull_pooled([g if prev else None for g in grads], bag)
+        for r in range(nrank):
+            out = dbuf[r].cpu().numpy()
+            assert_close(out[off:off + nb * width].reshape(-1, width), ref[r], 1e-5, "rank %d step %d" % (r, step))
+            assert np.isnan(out[0 if off else -1])           # nothing written in front of the rows, or behind them
+        p.compare_state(1e-5, "step %d" % step)
+        p.compare_ints([capi.VERSION, capi.UPDATES], "step %d" % step)
+        prev = nb
+    p.close()
+
+
 def test_pooled_matches_the_plain_call_with_replicated_gradients():
     # the definition itself, on the GPU alone: same table state as hctr_push_pull with every bag's gradient repeated,
     # pooled rows = the plain rows added up in key order
