@@ -76,6 +76,9 @@ __device__ __forceinline__ uint32_t div_up_dev(uint32_t a, uint32_t b) { return 
 #endif
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef f32x4 f32x4_any __attribute__((aligned(4))); // at any 4-byte address
+// the vectors of a row as they lie in memory (never a template argument: that drops the alignment from the type)
+template <int VEC> struct RowMem { typedef f32x4 M; };
+template <> struct RowMem<kOdd4> { typedef f32x4_any M; };
 // The gradient row of batch position `pos`: the position itself, or with sum-pooled bags of `bag` consecutive
 // positions the row of the position's bag (every key of a bag receives the bag's gradient).
 // kPooled is a compile-time switch: the plain push must not pay for the division in its load pipelines.
@@ -83,13 +86,14 @@ template <bool kPooled> __device__ __forceinline__ uint32_t grad_row(uint32_t po
   return kPooled ? bag(pos) : pos;
 }
 
-// The columns a lane moves at a time (see kOdd4 in kernels.h).  M: as they lie in memory.  T: as the lane computes with them, a
+// The columns a lane moves at a time (see kOdd4 in kernels.h).  T: as the lane computes with them, a
 // vector f32x4 or the four floats of a float4.  The medium role takes the latter: its two batches of vectors, each held in
 // four registers in a row, left one register too few, and a push with scratch memory took a batch of 53 k keys 22.2 us
 // instead of 20.4.  The short role takes vectors: 8.5 M uniform keys are pushed in 1027 us, with float4 in 1064.
-template <typename T4, typename Mem> struct Vec4 {
+template <typename T4, int VEC> struct Vec4 {
   typedef T4 T;
-  typedef Mem M;
+  typedef typename RowMem<VEC>::M M;
+  static_assert(alignof(M) == (VEC == kOdd4 ? 4 : 16), "what the compiler may take for granted of a row's address");
   static __device__ __forceinline__ T zero() { return T{0.f, 0.f, 0.f, 0.f}; }
   static __device__ __forceinline__ void add(T &a, const T &b) { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
   static __device__ __forceinline__ T scale(const T &a, float s) { return T{a.x * s, a.y * s, a.z * s, a.w * s}; }
@@ -103,14 +107,14 @@ template <typename T4, typename Mem> struct Vec4 {
   static __device__ __forceinline__ f32x4 to(const T &a) { return f32x4{a.x, a.y, a.z, a.w}; }
 };
 template <int VEC, typename T4 = f32x4> struct Vec;
-template <typename T4> struct Vec<4, T4> : Vec4<T4, f32x4> {
-  typedef Vec4<T4, f32x4> B;
+template <typename T4> struct Vec<4, T4> : Vec4<T4, 4> {
+  typedef Vec4<T4, 4> B;
   static __device__ __forceinline__ void store(float *p, const T4 &a, uint32_t) { B::store_all(p, a); }
   // a store past the caches: for rows another shard's kernel reads next
   static __device__ __forceinline__ void store_away(float *p, const T4 &a, uint32_t) { B::store_all_away(p, a); }
 };
-template <typename T4> struct Vec<kOdd4, T4> : Vec4<T4, f32x4_any> {
-  typedef Vec4<T4, f32x4_any> B;
+template <typename T4> struct Vec<kOdd4, T4> : Vec4<T4, kOdd4> {
+  typedef Vec4<T4, kOdd4> B;
   // without the first `shared` columns, which the lane before writes (and, in a row of more than one round of the
   // group, may have updated before this lane reads them: what it computes for them is dropped)
   static __device__ __forceinline__ void store(float *p, const T4 &a, uint32_t shared) {
