@@ -282,8 +282,9 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
     if (scratch_area) use_scratch_area(scratch_area, cur.n);
     else reserve_batch_scratch(cur.n);
     {
-      // ids -> device copy (:98-99) and sort keys.  When the caller's pointer is device-visible the copy is
-      // written by the same kernel that reads the ids; a pageable host buffer goes through a transfer first.
+      // ids -> device copy (:98-99) and sort keys.  The copy is written by the same kernel that reads the ids, at the
+      // caller's pointer when it is device-visible; ids in pageable host memory are staged in pinned memory, which the
+      // kernel reads itself for a small batch and which goes through a transfer first for a larger one.
       hipPointerAttribute_t attr;
       const bool visible = hipPointerGetAttributes(&attr, keys) == hipSuccess &&
                            (attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged);
