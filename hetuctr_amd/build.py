@@ -19,7 +19,7 @@ HEADERS = ["common.h", "host_copy.h", "kernels.h", "radix_sort.h", "tile_sort.h"
 # packed-fp32 instruction selection is switched off for all device code; no fused multiply-add contraction, so
 # that "sum * -lr" then "row + that" rounds twice like the CPU restatement it is checked against (fused
 # operations are written explicitly where they are meant)
-HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fvisibility=hidden", "-Wall", "-Wno-unused-function",
+HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fvisibility=hidden", "-Wall", "-Wno-unused-function", "-Werror=align-mismatch",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # host code of the partitioner's sweeps: AVX2 (no fused multiply-add is formed: contraction is off above)
 EXTRA_FLAGS = {"partition.hip": ["-Xarch_host", "-march=x86-64-v3"], "host_copy.hip": ["-Xarch_host", "-march=x86-64-v3"]}

@@ -103,7 +103,8 @@ template <typename T4, int VEC> struct Vec4 {
   static __device__ __forceinline__ void store_all_away(float *p, const T &a) { __builtin_nontemporal_store(to(a), (M *)p); }
 
  private:
-  static __device__ __forceinline__ T of(const f32x4 &v) { return T{v.x, v.y, v.z, v.w}; }
+  // (by value: a reference to a row's vector would promise more alignment than it has)
+  static __device__ __forceinline__ T of(f32x4 v) { return T{v.x, v.y, v.z, v.w}; }
   static __device__ __forceinline__ f32x4 to(const T &a) { return f32x4{a.x, a.y, a.z, a.w}; }
 };
 template <int VEC, typename T4 = f32x4> struct Vec;
