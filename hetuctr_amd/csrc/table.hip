@@ -556,11 +556,12 @@ void Shard::check_key_error() {
 
 // csrc/core/generate_query.cu:85-89; inference rule of csrc/core/hetu_gpu_table.cu:14-21
 void Shard::begin_push(const float *grad, uint32_t bag) {
-  hipStream_t s = group->stream;
   if (grad == nullptr) {
+    // Nothing on the device reads a batch the host knows to be empty, and the next preprocess makes these buffers its
+    // own batch (or clears them, if that one is empty): the device side stays as it is.  Clearing it here was four
+    // fills in front of the gather of every look-up.
     prev.n = 0;
     prev.U = 0;
-    prev.clear(s, cfg.nrank);
     std::fill(prev.push_cnt.begin(), prev.push_cnt.end(), 0);
     std::fill(prev.pushrecv_cnt.begin(), prev.pushrecv_cnt.end(), 0);
   }
