@@ -57,15 +57,19 @@ __global__ __launch_bounds__(kSortBlock) void make_keys(Records<KeyShard, M> sha
       id[k] = 0;
     }
   }
-  if (bad) atomicOr(err, 1u);
   uint64_t owner[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; k++) owner[k] = nrank > 1 ? root[id[k]] : 0;
 #pragma unroll
   for (int k = 0; k < ITEMS; k++) {
     const uint32_t i = base + k * kSortBlock + threadIdx.x;
+    if (i < n) store_key(comp + i, (K)((owner[k] << id_bits) | id[k]), S.read);
+  }
+  tell_ids_read(S.read, tiles, bad, err);
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++) {
+    const uint32_t i = base + k * kSortBlock + threadIdx.x;
     const K c = (K)((owner[k] << id_bits) | id[k]);
-    if (i < n) comp[i] = c;
     if (counts) count_digit(h, (uint32_t)c & mask, i < n);
   }
   if (!counts) return; // the keys alone: another sort counts for itself

@@ -84,7 +84,7 @@ struct DevStat {
   uint32_t U;
   uint32_t err;
   uint32_t push_total;
-  uint32_t pad;
+  uint32_t read_count; // ReadSignal::count: zero between the launches that use it
   uint64_t send_cnt[257];
   uint64_t push_cnt[257];
 };
@@ -92,7 +92,9 @@ struct HostMirror {
   DevStat st;
   uint32_t stats[4];
   uint32_t ret_seg[258];
-  uint32_t key_err; // written by the kernel that reads the caller's ids when preprocess returns early (no copy)
+  // written by the kernel that reads the caller's ids when preprocess returns early (no copy): an id out of range, or
+  // the two at once (ReadSignal)
+  uint32_t key_err, ids_read;
 };
 
 class Group;
@@ -157,6 +159,8 @@ class Shard {
   const index_t *ids_ = nullptr; // of the prepared batch: where the key kernel reads them, and whether as 32-bit words
   bool narrowed_ = false;
   uint32_t *key_flag_ = nullptr; // ... and where it reports a key out of range
+  ReadSignal read_;              // ... or how it says that it has read them all
+  bool wait_ids_read(hipStream_t on); // waits for that, if it does say so; true: a key was out of range
   TileSortBuffers tile_sort_buffers() const; // the index scratch as the tile-sorted passes take it
   HostStager stager;                         // ids that arrive in pageable host memory go through its pinned buffer
   bool pooled_from_keys = true;   // HETUCTR_POOLED_FROM_KEYS=0: pooled gathers of one shard go through the inverse index
@@ -204,6 +208,7 @@ class Shard {
   } sp;
   DeviceBuf plan_sums, query_sums; // query_sums: flags per tile of received queries // plan_sums: scan scratch of the push plan (the index has block_sums to itself)
   DevStat *dst_ = nullptr; // == dstat.p
+  uint32_t read_seq_ = 0;
   uint32_t *err_ptr() const { return &dst_->err; }
   // send side
   const float *push_grad_ = nullptr; // arguments of the push between begin_push and push_record
@@ -310,6 +315,7 @@ class Group {
   std::vector<Shard *> members;
   double wait_seconds = 120.0;
   void sync_stream();
+  bool wait_ids_read(); // waits until the callers' ids have been read; true: a key was out of range
 
   // per-stage device time, accumulated over calls while stage_timing is on
   bool stage_timing = false;

@@ -99,6 +99,7 @@ struct TileSortShard {
   void *keys_out;
   uint32_t *sorted_arg;
   HeadChunks heads;
+  ReadSignal read;           // with ids
 };
 // (every record or none has made_keys)
 void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count);

@@ -166,6 +166,7 @@ struct KeysJob {
   uint16_t *table;
   void *keys_out;
   bool ids32;
+  ReadSignal read;
 };
 template <typename K, int ITEMS, int DBITS, bool kFromKeys, int M> // M: records of the launch
 __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M> jobs, uint64_t id_max, int id_bits, int nrank,
@@ -216,7 +217,6 @@ __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M>
         id[r] = 0;
       }
     }
-    if (bad) atomicOr(err, 1u);
     uint64_t owner[ITEMS];
 #pragma unroll
     for (int r = 0; r < ITEMS; r++) owner[r] = nrank > 1 ? root[id[r]] : 0;
@@ -225,8 +225,9 @@ __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M>
       key[r] = (K)((owner[r] << id_bits) | id[r]);
       val[r] = tile_lo + w * S::kSub + r * kWave + lane;
       // the sort keys in batch order as well, for a caller that works on the batch before it is sorted (optional)
-      if (keys_out && w * S::kSub + r * kWave + lane < tile_n) keys_out[val[r]] = key[r];
+      if (keys_out && w * S::kSub + r * kWave + lane < tile_n) store_key(keys_out + val[r], key[r], J.read);
     }
+    tell_ids_read(J.read, tile_blocks, bad, err); // the caller need not wait for the sort
   }
   tile_sort_by_digit<K, ITEMS, DBITS>(key, val, tile_n, 0, dbits, area, bin_start, sm);
   store_sorted_tile<K, ITEMS>(area, bin_start, tile, tile_n, dbits, pitch, out_keys, out_vals, table);
@@ -625,7 +626,7 @@ void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortSha
     HCTR_CHECK(tile_sort_possible(o.n), "internal: batch too large for the tile-sorted passes");
     HCTR_CHECK(tile_items(o.n) == tile_items(f.n) && (o.made_keys != nullptr) == made, "internal: batches of one launch differ in shape");
     return {made ? o.made_keys : (const void *)o.ids, o.n, (uint32_t)tile_table_pitch(o.n), o.t.root, o.err, o.nlong, o.b.keys[0],
-            o.b.vals[0], tile_table(o, 0), made ? nullptr : o.keys_out, o.ids32};
+            o.b.vals[0], tile_table(o, 0), made ? nullptr : o.keys_out, o.ids32, o.read};
   };
   auto blocks = [&](int k) { return (uint32_t)tile_count(shards[k].n); };
   launch_one_or_records<KeysJob>(count, kSortBlock, make, blocks, [&](const auto &jobs, int) {

@@ -697,3 +697,36 @@ def test_widest_odd_rows_with_long_runs(width):
     for i in (0, 139, 140, 148, 149):
         assert torch.equal(out[i], grad[torch.from_numpy(keys == keys[i]).cuda()].sum(0) * -0.5), "row %d" % i
     p.close()
+
+
+@pytest.mark.parametrize("n", [1, 8193, 1 << 18, (1 << 18) + 1, 1 << 21, (1 << 21) + 1])
+def test_ids_overwritten_on_another_stream_when_preprocess_returns(n):
+    # the kernel that reads the ids says so itself for batches of up to 256 of its blocks (262144 keys: 256 blocks of 1024;
+    # 2^21: 256 of 8192), behind it an event does; from then on the ids are the caller's, and a bad one has been seen
+    import torch
+    say("ids read,", n, "keys")
+    length, width = 50_000, 4
+    capi.seed(3)
+    t = capi.Table(0, 1, 0, "127.0.0.1", 39000, length, width, 0, 0, np.zeros(length, np.uint8),
+                   np.arange(length, dtype=np.int64), ("Uniform", -1.0, 1.0), 0.5, 0)
+    rows = torch.from_numpy(t.fetch(capi.EMBEDDING).reshape(length, width)).cuda()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    side = torch.cuda.Stream()
+    out = torch.empty((n, width), device="cuda")
+    for step in range(6):
+        ids = torch.randint(length, (n,), device="cuda", generator=gen)
+        want = ids.clone()
+        if step % 3 == 1:
+            ids[(n - 1) if step == 1 else n // 2] = length if step == 1 else -1
+        torch.cuda.synchronize()
+        if step % 3 == 1:
+            with pytest.raises(Exception, match="outside"):
+                t.preprocess(ids.data_ptr(), n)
+            continue
+        t.preprocess(ids.data_ptr(), n)
+        with torch.cuda.stream(side):
+            ids.fill_(7)
+        t.push_pull(0, out.data_ptr())
+        assert torch.equal(out, rows[want]), "step %d" % step
+    t.close()
