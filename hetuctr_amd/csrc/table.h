@@ -109,11 +109,6 @@ class Group;
 #define HCTR_EARLY_TILE_PASSES 1
 #endif
 constexpr int kEarlySortSteps = HCTR_EARLY_SORT_STEPS, kEarlyTilePasses = HCTR_EARLY_TILE_PASSES;
-// from this many keys on, a preprocess that returns early has its ids read by a kernel that only makes the sort keys
-#ifndef HCTR_KEYS_FIRST_FROM
-#define HCTR_KEYS_FIRST_FROM (1u << 20)
-#endif
-constexpr uint32_t kKeysFirstFrom = HCTR_KEYS_FIRST_FROM;
 // One shard: a batch whose output rows take up to this many bytes is gathered in batch order straight from its keys
 // (Batch::direct_gather).  Measured on an MI355X with 512-byte rows: 107 k keys 78 us per step against 92 with the gather
 // in sorted order behind the index, 426 k keys 165 against 174, 852 k keys 316 against 279 -- in batch order the

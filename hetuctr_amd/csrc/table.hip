@@ -306,14 +306,14 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
         }
       }
       cur.tile_sorted = tile_sort_mode == 2 ? tile_sort_possible(cur.n) : (tile_sort_mode == 1 && tile_sort_fits(cur.n));
-      // A call that returns as soon as the ids are read (flag: where it looks for a bad id) gets them read by the
-      // lightest kernel there is when the batch is large: the sort keys alone.  Sorting a tile as well keeps the
-      // caller -- whose next call starts the gradient push -- waiting several microseconds longer.
+      // The launch that sorts the tiles reads the ids itself, unless it is one block's (which a gather from the keys would
+      // wait for) or the three-launch passes' (which have none): it tells the caller that it has before it sorts (with a
+      // launch for the keys in front of it, steps of 1.2 and 1.4 M keys took 7 us longer).
       // One shard and a small batch: the step's gather works from the keys in batch order and leaves the index off
-      // the step's critical path (write_back); the keys are then made by a kernel of their own here as well.
+      // the step's critical path (write_back).
       cur.direct_gather = cfg.nrank == 1 && flag != nullptr && cur.n <= direct_gather_max;
       cur.one_block = tile_sort_mode == 1 && cur.n <= kOneBlockKeys && kl.max_digit_bits == 0;
-      cur.keys_made = !cur.tile_sorted || cur.one_block || (flag != nullptr && cur.n >= kKeysFirstFrom);
+      cur.keys_made = !cur.tile_sorted || cur.one_block;
       cur.comp_valid = true; // either kernel leaves the sort keys in batch order (a gather from the keys reads them)
       ids_ = ids;
       narrowed_ = narrowed;
@@ -376,7 +376,6 @@ TileSortShard Shard::tile_sort_record() const {
   TileSortShard o = {};
   o.t = tv;
   o.ids = ids_;
-  o.made_keys = cur.keys_made ? cur.comp.p : nullptr;
   o.n = cur.n;
   o.b = tile_sort_buffers();
   o.err = key_flag_;
@@ -385,7 +384,7 @@ TileSortShard Shard::tile_sort_record() const {
   o.keys_out = cur.comp.p;
   o.sorted_arg = cur.sorted_arg.as<uint32_t>();
   o.heads = heads();
-  if (!cur.keys_made) o.read = read_;
+  o.read = read_;
   return o;
 }
 
@@ -416,7 +415,7 @@ void Group::index_batches(Shard *const *shards, size_t count, uint32_t *u_out, i
   auto same = [](const Shard &a, const Shard &b) {
     if (a.cur.one_block || b.cur.one_block) return a.cur.one_block == b.cur.one_block;
     if (!a.cur.tile_sorted || !b.cur.tile_sorted) return &a == &b; // the three-launch passes take one batch at a time
-    return a.cur.keys_made == b.cur.keys_made && tile_items(a.cur.n) == tile_items(b.cur.n);
+    return tile_items(a.cur.n) == tile_items(b.cur.n);
   };
   for_alike(shards, count, same, [&](Shard *const *v, int m) {
     Shard &f = *v[0];
@@ -436,8 +435,6 @@ void Group::index_batches(Shard *const *shards, size_t count, uint32_t *u_out, i
       if (f.cur.tile_sorted) {
         TileSortShard r[kShardsPerLaunch];
         for (int k = 0; k < m; k++) r[k] = v[k]->tile_sort_record();
-        if (f.cur.keys_made && part != 2) // the sort's first launch, from the keys the call made before it returned
-          launch_tile_sort_keys(s, kl, r, m);
         const int from = part == 2 ? 1 + kEarlyTilePasses : 1, to = part == 1 ? 1 + kEarlyTilePasses : (1 << 30);
         const int passes = launch_tile_sort_passes(s, kl, r, m, from, to);
         for (int k = 0; k < m; k++) unique[k].sorted_keys = r[k].b.keys[passes & 1];

@@ -84,14 +84,11 @@ struct TileSortBuffers {
 
 // Launch 0: reads the caller's ids (and nothing reads them afterwards), checks their range (bit 0 of *err), resets the
 // batch's run counters (nlong, optional), writes the tiles sorted by the first digit into buffers 0.
-// made_keys (optional): the batch's sort keys in batch order, already made and checked by make_keys; the launch then
-// starts from them and looks at neither ids, err nor nlong.
-// ids32: `ids` points to 32-bit ids (see launch_make_keys).  keys_out (optional, with ids): receives the sort keys in
-// batch order as well.
+// ids32: `ids` points to 32-bit ids (see launch_make_keys).  keys_out: receives the sort keys in batch order as
+// well.
 struct TileSortShard {
   TableView t;
   const index_t *ids;
-  const void *made_keys;
   uint32_t n;                // one tile shape for all records of a launch
   TileSortBuffers b;
   uint32_t *err, *nlong;
@@ -99,9 +96,8 @@ struct TileSortShard {
   void *keys_out;
   uint32_t *sorted_arg;
   HeadChunks heads;
-  ReadSignal read;           // with ids
+  ReadSignal read;
 };
-// (every record or none has made_keys)
 void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count);
 // Batches of up to kOneBlockKeys keys: the whole index -- sort, unique keys, run starts, directory look-ups -- by ONE block
 // in one launch, from the batch's sort keys in batch order.  The passes above cost such a batch five launches of one or

@@ -154,10 +154,8 @@ __device__ __forceinline__ void store_sorted_tile(const uint32_t *area, const ui
 // Launch 0: ids -> sort keys (owner << id_bits | id), the range check, the reset of the batch's run counters, and the
 // tile sorted by the first digit.  This is the one kernel that reads the caller's buffer: the call may return when it
 // is through.  (csrc/core/preprocess.cu:11-20 builds the reference's sort key.)
-// kFromKeys: the sort keys have been made already (make_keys, for a caller that wants its buffer back sooner than a
-// tile is sorted): `ids` then points to them, and nothing is checked or reset here.
 struct KeysJob {
-  const void *ids_or_keys;
+  const index_t *ids;
   uint32_t n, pitch;
   const worker_t *root;
   uint32_t *err, *nlong;
@@ -168,12 +166,12 @@ struct KeysJob {
   bool ids32;
   ReadSignal read;
 };
-template <typename K, int ITEMS, int DBITS, bool kFromKeys, int M> // M: records of the launch
+template <typename K, int ITEMS, int DBITS, int M> // M: records of the launch
 __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M> jobs, uint64_t id_max, int id_bits, int nrank,
                                                               int dbits) {
   uint32_t tile, tile_blocks;
   const KeysJob &J = my_record(jobs, tile, tile_blocks);
-  const void *__restrict__ ids_or_keys = J.ids_or_keys;
+  const index_t *__restrict__ ids = J.ids;
   const uint32_t n = J.n, pitch = J.pitch;
   const worker_t *__restrict__ root = J.root;
   uint32_t *__restrict__ err = J.err, *__restrict__ nlong = J.nlong, *__restrict__ out_vals = J.out_vals;
@@ -190,45 +188,34 @@ __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M>
   const unsigned lane = lane_id();
   K key[ITEMS];
   uint32_t val[ITEMS];
-  if (kFromKeys) {
-    const K *__restrict__ keys = (const K *)ids_or_keys;
+  if (tile == 0 && threadIdx.x < kRunCounters && nlong) nlong[threadIdx.x] = 0; // counters of this batch
+  uint64_t id[ITEMS];
 #pragma unroll
-    for (int r = 0; r < ITEMS; r++) {
-      const uint32_t e = w * S::kSub + r * kWave + lane;
-      key[r] = e < tile_n ? keys[tile_lo + e] : (K)0;
-      val[r] = tile_lo + e;
-    }
-  } else {
-    const index_t *__restrict__ ids = (const index_t *)ids_or_keys;
-    if (tile == 0 && threadIdx.x < kRunCounters && nlong) nlong[threadIdx.x] = 0; // counters of this batch
-    uint64_t id[ITEMS];
-#pragma unroll
-    for (int r = 0; r < ITEMS; r++) {
-      const uint32_t e = w * S::kSub + r * kWave + lane;
-      // the caller's ids are read here and nowhere else (ids32: as narrowed on their way from pageable host memory)
-      id[r] = e >= tile_n ? 0 : ids32 ? (uint64_t)load_once(&((const uint32_t *)ids)[tile_lo + e]) : (uint64_t)load_once(&ids[tile_lo + e]);
-    }
-    bool bad = false;
-#pragma unroll
-    for (int r = 0; r < ITEMS; r++) {
-      const uint32_t e = w * S::kSub + r * kWave + lane;
-      if (e < tile_n && id[r] >= id_max) { // also catches negative ids
-        bad = true;
-        id[r] = 0;
-      }
-    }
-    uint64_t owner[ITEMS];
-#pragma unroll
-    for (int r = 0; r < ITEMS; r++) owner[r] = nrank > 1 ? root[id[r]] : 0;
-#pragma unroll
-    for (int r = 0; r < ITEMS; r++) {
-      key[r] = (K)((owner[r] << id_bits) | id[r]);
-      val[r] = tile_lo + w * S::kSub + r * kWave + lane;
-      // the sort keys in batch order as well, for a caller that works on the batch before it is sorted (optional)
-      if (keys_out && w * S::kSub + r * kWave + lane < tile_n) store_key(keys_out + val[r], key[r], J.read);
-    }
-    tell_ids_read(J.read, tile_blocks, bad, err); // the caller need not wait for the sort
+  for (int r = 0; r < ITEMS; r++) {
+    const uint32_t e = w * S::kSub + r * kWave + lane;
+    // the caller's ids are read here and nowhere else (ids32: as narrowed on their way from pageable host memory)
+    id[r] = e >= tile_n ? 0 : ids32 ? (uint64_t)load_once(&((const uint32_t *)ids)[tile_lo + e]) : (uint64_t)load_once(&ids[tile_lo + e]);
   }
+  bool bad = false;
+#pragma unroll
+  for (int r = 0; r < ITEMS; r++) {
+    const uint32_t e = w * S::kSub + r * kWave + lane;
+    if (e < tile_n && id[r] >= id_max) { // also catches negative ids
+      bad = true;
+      id[r] = 0;
+    }
+  }
+  uint64_t owner[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; r++) owner[r] = nrank > 1 ? root[id[r]] : 0;
+#pragma unroll
+  for (int r = 0; r < ITEMS; r++) {
+    key[r] = (K)((owner[r] << id_bits) | id[r]);
+    val[r] = tile_lo + w * S::kSub + r * kWave + lane;
+    // the sort keys in batch order as well, for a caller that works on the batch before it is sorted (optional)
+    if (keys_out && w * S::kSub + r * kWave + lane < tile_n) store_key(keys_out + val[r], key[r], J.read);
+  }
+  tell_ids_read(J.read, tile_blocks, bad, err); // the caller need not wait for the sort
   tile_sort_by_digit<K, ITEMS, DBITS>(key, val, tile_n, 0, dbits, area, bin_start, sm);
   store_sorted_tile<K, ITEMS>(area, bin_start, tile, tile_n, dbits, pitch, out_keys, out_vals, table);
 }
@@ -619,25 +606,21 @@ static uint16_t *tile_table(const TileSortShard &o, int which) {
 void launch_tile_sort_keys(hipStream_t s, const KeyLayout &kl, const TileSortShard *shards, int count) {
   const DigitPlan p = plan_digits(kl);
   const TileSortShard &f = shards[0];
-  const bool made = f.made_keys != nullptr;
   auto make = [&](int k) -> KeysJob {
     const TileSortShard &o = shards[k];
     HCTR_CHECK(!o.ids32 || o.t.id_max <= 0xffffffffull, "internal: narrowed ids and a table of 2^32 rows or more");
     HCTR_CHECK(tile_sort_possible(o.n), "internal: batch too large for the tile-sorted passes");
-    HCTR_CHECK(tile_items(o.n) == tile_items(f.n) && (o.made_keys != nullptr) == made, "internal: batches of one launch differ in shape");
-    return {made ? o.made_keys : (const void *)o.ids, o.n, (uint32_t)tile_table_pitch(o.n), o.t.root, o.err, o.nlong, o.b.keys[0],
-            o.b.vals[0], tile_table(o, 0), made ? nullptr : o.keys_out, o.ids32, o.read};
+    HCTR_CHECK(tile_items(o.n) == tile_items(f.n), "internal: batches of one launch differ in shape");
+    return {o.ids, o.n, (uint32_t)tile_table_pitch(o.n), o.t.root, o.err, o.nlong, o.b.keys[0],
+            o.b.vals[0], tile_table(o, 0), o.keys_out, o.ids32, o.read};
   };
   auto blocks = [&](int k) { return (uint32_t)tile_count(shards[k].n); };
   launch_one_or_records<KeysJob>(count, kSortBlock, make, blocks, [&](const auto &jobs, int) {
     constexpr int M = sizeof jobs.s / sizeof jobs.s[0];
     const TableView &t = f.t;
     const dim3 grid = grid_of(jobs);
-#define CALL(K, I, D)                                                                                                  \
-  do {                                                                                                                 \
-    if (made) hipLaunchKernelGGL((keys_tile_sort<K, I, D, true, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0]); \
-    else hipLaunchKernelGGL((keys_tile_sort<K, I, D, false, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0]); \
-  } while (0)
+#define CALL(K, I, D) \
+  hipLaunchKernelGGL((keys_tile_sort<K, I, D, M>), grid, dim3(kSortBlock), 0, s, jobs, t.id_max, kl.id_bits, t.nrank, p.dbits[0])
     HCTR_TILE_SORT_DISPATCH(kl.wide, f.n, p.dbits[0], CALL);
 #undef CALL
     HCTR_HIP(hipGetLastError());
