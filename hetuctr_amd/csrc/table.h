@@ -172,6 +172,7 @@ class Shard {
   void check_key_error();                   // raises if the ingested batch held a key outside [0, length)
   // the push of a step in two halves, so that a group can place every shard's pushed rows before any push kernel runs
   void begin_push(const float *grad, uint32_t bag = 1);  // which batch is pushed (none on an inference step), checks
+  void list_runs();
   bool push_record(PushShard &o);                        // what the push kernel needs of this shard; false: nothing
   // handleGradient + handleQuery: what the group's owner-side launches need of this shard (queries_max: no shard
   // receives more queries than this)
@@ -208,6 +209,7 @@ class Shard {
   // send side
   const float *push_grad_ = nullptr; // arguments of the push between begin_push and push_record
   uint32_t push_bag_ = 1;
+  bool trains_ = false;              // the last push_pull came with a gradient
   // receive side (owner role)
   DeviceBuf src_row, ret_seg_dev;
   std::vector<uint64_t> rq_seg, rg_seg, ret_seg; // R+1 prefix offsets per source / requester
@@ -342,6 +344,8 @@ class Group {
  private:
   void exchange_shapes();
   void push_pull_steps(const float *const *grads, float *const *dsts, uint32_t bag); // the body of push_pull_all
+  void finish_lists();
+  bool lists_running_ = false; // a preprocess has launched the run lists of the previous batch on the main stream
   bool index_joining_ = false; // push_pull has taken a pending index over and not yet read its results
   template <typename F> void collective(int rank, int op, F &&run_all);
   std::mutex mu_;

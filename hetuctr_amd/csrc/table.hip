@@ -573,6 +573,7 @@ void Shard::begin_push(const float *grad, uint32_t bag) {
   last_stats[3] = 0;
   push_grad_ = grad;
   push_bag_ = bag;
+  trains_ = grad != nullptr;
   if (!prev_active) return;
   uint64_t pushes = 0;
   for (int i = 0; i < cfg.nrank; i++) pushes += prev.push_cnt[i];
@@ -580,12 +581,16 @@ void Shard::begin_push(const float *grad, uint32_t bag) {
   HCTR_CHECK(prev.n % bag == 0, "pooled push: the previous batch is not a whole number of bags");
 }
 
+// the run lists of the batch that is pushed next, if no gather has built them
+void Shard::list_runs() {
+  if (prev.n == 0 || prev.lists_ready) return;
+  launch_list_long_runs(group->stream, prev.view());
+  prev.lists_ready = true;
+}
+
 bool Shard::push_record(PushShard &o) {
   if (!prev_active) return false;
-  if (!prev.lists_ready) { // no gather has seen this batch (a second preprocess came first, or a call without output)
-    launch_list_long_runs(group->stream, prev.view());
-    prev.lists_ready = true;
-  }
+  list_runs(); // (unless preprocess has)
   o = PushShard();
   o.t = tv;
   o.b = prev.view();
@@ -1169,10 +1174,18 @@ void Group::flush_index() {
   exchange_shapes();
 }
 
+// A preprocess without a push_pull since the one before: the buffers of the previous batch are about to become the current
+// batch's, on the other stream, and the kernel that lists its runs may still be at work on them.
+void Group::finish_lists() {
+  if (lists_running_) sync_stream();
+  lists_running_ = false;
+}
+
 void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
   HCTR_CHECK(complete(), "the loopback group named by (ip, port) is missing ranks");
   HCTR_HIP(hipSetDevice(device_id));
   flush_index(); // preprocess twice in a row: the earlier batch is indexed before it becomes the previous one
+  finish_lists();
   if (defer_index && !stage_timing && nrank == 1) {
     // One shard: everything is enqueued on the second stream, and the call returns as soon as the caller's ids have
     // been read.  Sorting and deduplicating them does not depend on the pending gradient push, which the next
@@ -1189,6 +1202,14 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     if (!m->read_.word) HCTR_HIP(hipEventRecord(ev_keys, stream));
     enqueue_index(m, 1);
     index_rest_pending = true;
+    if (m->trains_ && m->prev.n != 0 && !m->prev.lists_ready) {
+      // The next push_pull will probably push the previous batch, whose gather worked from the keys: its run lists are
+      // built now, on the main stream, while the host waits for the ids to be read (built in front of the push they
+      // are 4 us of kernel and a launch gap of a 53 k-key step; of 8.5 M keys 12 us).
+      StreamSwitch off(*this, on.saved);
+      m->list_runs();
+      lists_running_ = true;
+    }
     const bool bad_key = wait_ids_read();
     if (time_calls) {
       float ms = 0.f;
@@ -1274,6 +1295,7 @@ void Group::preprocess_noalloc(const int64_t *keys, size_t n) {
   HCTR_CHECK(!stage_timing, "stage timing takes events from a growing pool: switch it off for calls that may not allocate");
   HCTR_HIP(hipSetDevice(device_id));
   flush_index(); // an earlier deferred batch is indexed before it becomes the previous one
+  finish_lists();
   Shard *m = members[0];
   // after the swap the current batch lives in the buffers of the batch before the previous one
   HCTR_CHECK(m->prev.holds((uint32_t)n, 1, m->kl.wide),
@@ -1428,6 +1450,7 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
   if (nrank > 1) HCTR_HIP(hipStreamWaitEvent(stream, ev_plan, 0));
   sync_stream();
+  lists_running_ = false;
   collect_marks();
   if (nrank > 1)
     for (Shard *m : members) m->finish_plan(m->cur);

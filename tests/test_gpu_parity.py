@@ -730,3 +730,26 @@ def test_ids_overwritten_on_another_stream_when_preprocess_returns(n):
         t.push_pull(0, out.data_ptr())
         assert torch.equal(out, rows[want]), "step %d" % step
     t.close()
+
+
+@pytest.mark.parametrize("n", [700, 9_000, 60_000])
+def test_preprocess_again_while_the_run_lists_are_built(n):
+    # after a training step preprocess lists the runs of the batch before on the main stream; a second preprocess then makes
+    # that batch's buffers its own.  Nothing is fetched between the calls; small batches follow large ones
+    say("preprocess again,", n, "keys")
+    rng = np.random.default_rng(n)
+    length, width = 5_000, 8
+    p = single(length, width, lr=0.05)
+    draw = zipf_sampler(length, 1.2, rng)
+    prev_n = 0
+    for step in range(8):
+        for again in range(1 + step % 3):
+            k = n if (step + again) % 2 else n // 5
+            p.preprocess([draw(k)], device_keys=True)
+            prev_n, last = (last if step or again else 0), k
+        g = None if prev_n == 0 or step == 5 else rng.normal(0, 1e-3, size=(prev_n, width)).astype(np.float32)
+        out, ref = p.push_pull([g])
+        assert_close(out[0], ref[0], 1e-5, "dst step %d" % step)
+    p.compare_state(1e-5, "end")
+    p.compare_ints([capi.VERSION], "end")
+    p.close()
