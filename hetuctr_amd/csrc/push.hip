@@ -15,10 +15,10 @@
 //
 // One launch, three ranges of blocks, one per class of run length (the long chains are dispatched first and the
 // other blocks fill the machine behind them):
-//  * long (> kLongRun duplicates): bundles of runs are streamed by whole blocks, one column slice at a time.  Seven
-//    loader waves keep several 16-byte loads of gradient rows in flight each and stage them through a ring of
-//    LDS slots; the first wave adds the staged rows in order, one column per lane.  The serial chain costs a
-//    quarter of an LDS read and one add per duplicate while the memory latency is covered by the whole block.
+//  * long (> kLongRun duplicates): bundles of runs are streamed by whole blocks, one column slice at a time.  Six
+//    loader waves keep 16 vectors of gradient rows in flight per lane and stage them through two LDS slots; two waves
+//    take turns at adding the staged rows in order, one column per lane, each reading its rows from LDS into registers
+//    while the other one adds.  The serial chain costs one add per duplicate.
 //    The longest runs are started first and cut into narrower slices, i.e. fed by more blocks.
 //  * medium (kTinyRun < duplicates <= kLongRun): one group of LPR lanes per run, kBatch rows in flight.
 //  * short (<= kTinyRun): a group of LPR lanes (LPR*VEC floats = one row) owns a few consecutive unique keys
@@ -33,12 +33,6 @@ namespace hctr {
 #ifndef HCTR_TILE_BATCH
 #define HCTR_TILE_BATCH 8
 #endif
-#ifndef HCTR_DEPTH
-#define HCTR_DEPTH 8
-#endif
-#ifndef HCTR_RPT
-#define HCTR_RPT 2
-#endif
 #ifndef HCTR_LONG_BLOCKS
 #define HCTR_LONG_BLOCKS 128
 #endif
@@ -48,12 +42,7 @@ namespace hctr {
 constexpr int kPushBlock = 512;
 
 constexpr int kBatch = HCTR_TILE_BATCH;   // short role: gradient rows in flight per group past the first two
-constexpr int kDepth = HCTR_DEPTH;        // long role: chunks in flight per loader thread
-constexpr int kRPT = HCTR_RPT;            // long role: rows per loader thread and chunk
-#ifndef HCTR_SLOTS
-#define HCTR_SLOTS 3
-#endif
-constexpr int kSlots = HCTR_SLOTS;        // long role: LDS ring slots
+constexpr int kInFlight = 16;             // long role: rows in flight per loader thread
 constexpr int kSlice = kSliceColumns;     // long role: columns per block
 constexpr int kLongBlocks = HCTR_LONG_BLOCKS;
 #ifndef HCTR_GIANT_SLICE
@@ -425,25 +414,33 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
 // stream of chunks, so that the loads of the next run are in flight while the current one is summed.  Runs are
 // listed by length class, longest first; a bundle is 1..kTable runs of one class holding at least ~2048
 // occurrences.  Tickets (bundle, slice) are handed out through one counter per group of blocks that share slices;
-// the summing wave draws the next ticket and requests its run descriptors while the current bundle streams, so a
-// change of bundle costs only the refill of the load pipeline.
-// Wave 0 of the block only sums; the other 7 waves ("loaders") only move gradient rows global -> registers ->
-// LDS ring.  A row slice is read by CS/VEC loader lanes; one block-wide load covers RPL = 448 / (CS/VEC)
-// consecutive occurrences and a chunk is kRPT such loads (chunks never span two runs).  Loaders and the summing
-// wave meet at one barrier per chunk: barrier m says "chunk m is in LDS".  A slot is overwritten kSlots
-// barriers later, after the summing wave has passed the barrier that follows its reads.
-constexpr int kLoaders = kPushBlock - kWave;
+// the first wave draws the next ticket and fetches its run descriptors while the loaders of the current bundle wait
+// for their first rows, so a change of bundle costs only the refill of the load pipeline.
+// Fast path (slices of 16, 32 or 64 columns, CSC).  Two waves sum; the other six ("loaders") only move gradient rows global ->
+// registers -> LDS.  A row slice is read by CSC / 4 loader lanes, a chunk is 96 rows, or 192 where a slice has at most 32
+// columns and the two halves of a wave hold 96 rows each (chunks never span two runs).  Everyone meets at one barrier per
+// chunk: while chunk g - 1 is added by the wave that has it in registers, the other wave reads chunk g from its slot and the
+// loaders fill the other slot with chunk g + 1; the sums pass from wave to wave in LDS.  What bounds it: the chain of adds, 4.6
+// cycles per row (a lone wave's dependent v_add_f32), and per chunk a barrier, the hand-over and the change of halves, about
+// 400 cycles; with every block of a batch at it, the rows coming out of the last-level cache.  One wave that reads and
+// adds by turns spends 4 cycles per row on each.  Why rows lie in a slot as they come: written column by column, in 4-byte pieces, they
+// took the LDS longer than the adds (a chunk of 192 rows 1600 cycles with the adds left out).  A chain of 106 k rows is
+// summed in 290 us.  Bags of 10 ids x 64 floats, Zipf 1.4 (8.5 M keys): two steps 1757 -> 1580 us with what follows here; rows
+// of 37 floats, 195 k keys of 39 Zipf fields: 154 -> 140 us, since such widths take this path too.  More blocks at once do not
+// help (128 / 192 / 256: 1570 / 1584 / 1589 us, and rows of 37 floats 140 / 145 / 169).
+// Generic path (CSC 0; rows of less than four floats, and widths that leave one to three columns over): seven loader waves
+// and one that reads and adds, eight rows at a time, three slots.
 constexpr int kTable = 16;     // runs per bundle at most
-#ifndef HCTR_SUM_BATCH
-#define HCTR_SUM_BATCH 28
-#endif
-constexpr int kSumBatch = HCTR_SUM_BATCH; // rows the summing wave reads from LDS in one go (two such batches are live)
-
-// the four floats of v to dst[0], dst[stride], dst[2 * stride], dst[3 * stride]
-__device__ __forceinline__ void store_transposed(float *dst, uint32_t stride, const f32x4 &v) {
-  dst[0] = v.x, dst[stride] = v.y, dst[2 * stride] = v.z, dst[3 * stride] = v.w;
+constexpr int kHeldRows = 96;  // rows a lane of a summing wave holds
+constexpr int kSlotsFast = 2, kSlotsGeneric = 3; // LDS slots
+template <int CSC> constexpr int kRowSets = CSC == kWave ? 1 : 2;         // sets of rows in the lanes of a summing wave
+template <int CSC> constexpr int kChunkRows = kHeldRows * kRowSets<CSC>; // rows per chunk of the fast path
+constexpr int ring_floats(int cs) { return kSlotsFast * cs * (cs == kWave ? kHeldRows : 2 * kHeldRows + 1); }
+// the value of lane i in lane i + 32
+__device__ __forceinline__ float from_lower_half(float x) {
+  const uint32_t v = __float_as_uint(x);
+  return __uint_as_float(__builtin_amdgcn_permlane32_swap(v, v, false, false)[0]);
 }
-__device__ __forceinline__ void store_transposed(float *, uint32_t, const float &) {} // generic path: never called
 
 // a value that is the same in every lane, moved to a scalar register
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
@@ -456,31 +453,32 @@ __device__ __forceinline__ uint32_t bundle_runs(int cls, uint32_t shrink) {
 
 template <int VEC, typename K, int CSC, bool kPooled> // CSC: columns per slice if known at compile time, else 0
 __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
-                                          float *lds, uint4 *table, uint32_t *shared, float *row_stash, int c_lo,
+                                          float *lds, uint4 *tables, uint32_t *shared, float *row_stash, float *hand, int c_lo,
                                           int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
   typedef typename Vec<VEC>::T V;
   constexpr uint32_t C = kCols<VEC>;
+  constexpr int kSummers = CSC ? 2 : 1;
+  constexpr int kLoaders = kPushBlock - kSummers * kWave;
   const uint32_t W = t.width;
   uint32_t CS = CSC ? (uint32_t)CSC : min((uint32_t)kSlice, (W + C - 1) / C * C);
-  if (VEC == kOdd4) CS = overlap_slice(W, CS); // row_vec() has made sure that one of them holds the last lane
+  if (VEC == kOdd4 && !CSC) CS = overlap_slice(W, CS); // row_vec() has made sure that one of them holds the last lane
   uint32_t lanes = (CS + C - 1) / C; // loader lanes per row slice, rounded up to a power of two
   lanes = lanes <= 1 ? 1 : lanes <= 2 ? 2 : lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
   const uint32_t RPL = CSC ? (uint32_t)(kLoaders / (CSC / C)) : kLoaders / lanes;
-  const uint32_t CR = RPL * kRPT;                                   // rows per chunk
-  constexpr int kChunkRows = CSC ? kRPT * (int)(kLoaders / (CSC / C)) : 1; // CR as a constant on the fast path
-  static_assert(!CSC || (kChunkRows % kSumBatch == 0 && kSumBatch % 4 == 0), "a chunk of the fast path is a whole number of sum batches");
-  static_assert(!CSC || kSlots * CSC * (kChunkRows + 4) <= kSlots * kRPT * kPushBlock * (int)C, "ring slots of the fast path fit the LDS area");
+  constexpr int kSliceLanes = CSC ? CSC / (int)C : 1;
+  constexpr int kRPT = CSC ? kChunkRows<CSC> / (kLoaders / kSliceLanes) : 2; // rows per loader thread and chunk
+  constexpr int kDepth = kInFlight / kRPT;  // chunks in flight per loader thread
+  const uint32_t CR = RPL * kRPT;             // rows per chunk
+  static_assert(!CSC || kChunkRows<CSC> == kRPT * (kLoaders / kSliceLanes), "a chunk of the fast path is whole loads");
   const uint32_t slices = (W + CS - 1) / CS;
-  // LDS layout of a ring slot.  Generic path: row-major [row][CS].  Fast path (CSC): column-major with the row
-  // index fastest, [column place][pitch], pitch = rows + 4, so that the summing lane gets four consecutive rows of
-  // its column with one 16-byte read; column c sits at place (c % 4) * (CSC / 4) + c / 4, which makes both the
-  // loaders' 4-byte writes and the 16-byte reads free of bank conflicts (pitch % 8 == 4).
-  const uint32_t pitch = CR + 4;
-  const uint32_t slot_floats = CSC ? CS * pitch : CR * CS;
+  // A ring slot holds the rows of a chunk one after the other.  On the fast path the second set of rows lies one row further:
+  // the lanes that read it use the other half of the banks.
+  constexpr uint32_t kPad = CSC && kRowSets<CSC> > 1 ? 1 : 0;
+  const uint32_t slot_floats = (CR + kPad) * CS;
+  constexpr uint32_t slots = CSC ? kSlotsFast : kSlotsGeneric;
   const float neg_lr = t.neg_lr;
-  const bool summer = threadIdx.x < kWave;
-  const uint32_t lt = threadIdx.x - kWave; // loader thread number (meaningless on the summing wave)
-  const uint32_t my_row = lt / lanes, my_lane = lt % lanes;
+  const uint32_t wave = uni(threadIdx.x / kWave);
+  const bool summer = wave < (uint32_t)kSummers, lead = wave == 0; // the lead also draws the tickets
   const uint32_t *__restrict__ sorted_arg = p.sorted_arg;
 
   // tickets of this block's group: (bundle, slice) with the bundle changing slowest, so the longest runs go first
@@ -505,26 +503,24 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
   if (!nbundles) return;
   const uint32_t tickets = nbundles * n_sl;
 
-  // summing wave: draws a ticket and requests the descriptors of its runs (one lane per run)
-  uint4 pend = make_uint4(0, 0, 0, 0);
-  uint32_t pend_runs = 0, pend_slice = 0;
-  auto draw = [&]() {
+  // the lead wave draws a ticket and leaves its bundle in set `to`: descriptors of the runs (one lane per run), number of
+  // runs, chunks and the slice
+  auto draw = [&](uint32_t to) {
     uint32_t tk = 0;
     if (threadIdx.x == 0) tk = atomicAdd(counters + lane_id, 1u);
     tk = (uint32_t)__builtin_amdgcn_readfirstlane((int)tk);
-    pend_runs = 0;
     if (tk >= tickets) {
       // Every block of the group draws exactly one ticket past the end.  The block that draws the last of them
       // knows that nobody will touch the counter again in this launch and puts it back to zero, so that the same
       // batch can be pushed again (push_pull twice without a preprocess in between applies the gradient twice,
       // csrc/core/hetu_gpu_table.cu:9-41).
       if (threadIdx.x == 0 && tk == tickets + group_blocks - 1) atomicExch(counters + lane_id, 0u);
+      if (threadIdx.x == 0) shared[to * 4] = 0;
       return;
     }
     uint32_t bundle = tk / n_sl;
-    pend_slice = lane_id + (tk % n_sl) * share;
     int cls = 0;
-    uint32_t run0 = 0;
+    uint32_t run0 = 0, runs = 0;
     bool found = false;
 #pragma unroll
     for (int c = 0; c < kLongBuckets; c++) {
@@ -534,66 +530,74 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
           found = true;
           cls = c;
           run0 = bundle * bs;
-          pend_runs = min(bs, cnt[c] - run0);
+          runs = min(bs, cnt[c] - run0);
         } else {
           bundle -= nb;
         }
       }
     }
-    if (threadIdx.x < pend_runs) pend = p.long_list[(size_t)cls * p.long_cap + run0 + threadIdx.x];
-  };
-  // ... and makes them the block's current bundle: descriptors, number of runs, chunks and the slice
-  auto publish = [&]() {
-    uint32_t chunks = threadIdx.x < pend_runs ? (pend.z + CR - 1) / CR : 0u;
-    if (threadIdx.x < pend_runs) table[threadIdx.x] = pend; // rank, first position, length, offset
+    uint32_t chunks = 0;
+    if (threadIdx.x < runs) {
+      const uint4 m = p.long_list[(size_t)cls * p.long_cap + run0 + threadIdx.x]; // rank, first position, length, offset
+      chunks = (m.z + CR - 1) / CR;
+      tables[to * kTable + threadIdx.x] = m;
+    }
 #pragma unroll
     for (int d = kTable / 2; d; d >>= 1) chunks += __shfl_down(chunks, d);
     if (threadIdx.x == 0) {
-      shared[0] = pend_runs;
-      shared[1] = chunks;
-      shared[2] = pend_slice;
+      shared[to * 4] = runs;
+      shared[to * 4 + 1] = chunks;
+      shared[to * 4 + 2] = lane_id + (tk % n_sl) * share;
     }
   };
 
-  if (summer) draw();
-  for (;;) {
-    if (summer) publish();
-    __syncthreads();
-    const uint32_t J = uni(shared[0]), G = uni(shared[1]), slice = uni(shared[2]); // runs, chunks and slice of this bundle
+  __syncthreads(); // of the runs before these
+  if (lead) draw(0);
+  __syncthreads();
+  for (uint32_t cur = 0;; cur ^= 1) {
+    const uint4 *table = tables + cur * kTable;
+    const uint32_t J = uni(shared[cur * 4]), G = uni(shared[cur * 4 + 1]), slice = uni(shared[cur * 4 + 2]); // runs, chunks and slice of this bundle
     if (!J) break;
-    if (summer) draw(); // the requests stay in flight while this bundle streams
+    if (lead) draw(cur ^ 1); // while the loaders wait for the first rows of this bundle
 
     if (!summer) {
       // ---------------- loaders ----------------
+      uint32_t lt = threadIdx.x - kSummers * kWave; // loader thread number
+      asm volatile("" : "+v"(lt)); // what follows from it is worked out here and takes no registers of the summing waves
+      const uint32_t my_row = lt / lanes, my_lane = lt % lanes;
       const uint32_t due = slice * CS + my_lane * C;   // first column of this lane's vector
-      const bool in_slice = my_lane * C < CS && my_row < RPL;
+      const bool in_slice = CSC ? true : my_lane * C < CS && my_row < RPL;
       const uint32_t col = due < W ? lane_col<VEC>(due, W) : due;
       const uint32_t lcol = col - slice * CS;          // ... inside the slice
       // Loads are unconditional and branch-free so that kDepth chunks stay in flight per thread: positions
       // past the end of a run re-read its last row (never summed), lanes outside the slice read column 0.
       const embed_t *gbase = a.grad + ((in_slice && due < W) ? col : 0);
-      auto row_load = [&](uint32_t idx) -> V { return grad_load<Vec<VEC>, kPooled>(gbase + (size_t)idx * W); };
+      // The bag of a position is worked out here and not where the position is read: there it would wait for it.
+      auto row_load = [&](uint32_t pos) -> V {
+        return grad_load<Vec<VEC>, kPooled>((const embed_t *)((const char *)gbase + (uint64_t)grad_row<kPooled>(pos, a.bag) * (W * 4)));
+      };
       // cursor of the index stage, 2 * kDepth chunks ahead of the LDS stage; past the end of the stream it
       // stays on the last run
-      uint32_t cj = 0, cc = 0;
-      uint32_t clo, chi, cn;
-      {
-        const uint4 m = table[0];
-        clo = uni(m.y);
-        chi = clo + uni(m.z);
-        cn = (uni(m.z) + CR - 1) / CR;
-      }
+      uint32_t cj = 0, first = 0; // the run, and the first row of the next chunk in it
+      uint32_t clo, len;
+      auto open_run = [&]() {
+        const uint4 m = table[cj];
+        clo = uni(m.y), len = uni(m.z), first = 0;
+      };
+      open_run();
       auto next_chunk = [&](uint32_t(&dst)[kRPT]) {
+        const uint32_t from = min(first, len - 1), last = min(CR, len - from) - 1;
+        const uint32_t *pos = sorted_arg + clo + from;
 #pragma unroll
-        for (int q = 0; q < kRPT; q++) dst[q] = grad_row<kPooled>(sorted_arg[min(clo + cc * CR + q * RPL + my_row, chi - 1)], a.bag);
-        cc++;
-        if (cc >= cn && cj + 1 < J) {
-          cj++;
-          const uint4 m = table[cj];
-          clo = uni(m.y);
-          chi = clo + uni(m.z);
-          cn = (uni(m.z) + CR - 1) / CR;
-          cc = 0;
+        for (int q = 0; q < kRPT; q++) dst[q] = pos[min(q * RPL + my_row, last)];
+        first += CR;
+        if (first >= len) {
+          if (cj + 1 < J) {
+            cj++;
+            open_run();
+          } else {
+            first = len;
+          }
         }
       };
       uint32_t idx[kDepth][kRPT];
@@ -610,11 +614,12 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
       uint32_t slot = 0;
       auto step = [&](int k) {
         float *sp = lds + slot * slot_floats;
-        slot = slot + 1 == (uint32_t)kSlots ? 0 : slot + 1;
+        slot = slot + 1 == slots ? 0 : slot + 1;
 #pragma unroll
         for (int q = 0; q < kRPT; q++) {
           if (in_slice) {
-            if (CSC) store_transposed(sp + my_lane * pitch + (q * RPL + my_row), (CSC / 4) * pitch, val[k][q]);
+            // the fast path's lanes write where they are due, also the last one of a row, which starts before that
+            if (CSC) *(V *)(sp + (q * RPL + (q >= kRPT / 2 ? kPad : 0) + my_row) * CS + my_lane * C) = val[k][q];
             else Vec<VEC>::store_all(sp + (q * RPL + my_row) * CS + lcol, val[k][q]);
           }
           val[k][q] = row_load(idx[k][q]); // chunk + kDepth
@@ -631,115 +636,151 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
       }
 #pragma unroll
       for (int k = 0; k < kDepth; k++)
-        if (g0 + k < G) step(k); // uniform over the block: the summing wave makes the same number of barriers
+        if (g0 + k < G) step(k); // uniform over the block: the summing waves make the same number of barriers
+      if (CSC) __syncthreads();  // the last chunk is added behind this one
     } else {
-      // ---------------- summing wave: one column per lane, rows strictly in order ----------------
-      // the column this lane sums: lane = place in the fast path's layout
-      const uint32_t mycol = slice * CS + (CSC ? (threadIdx.x % (CSC ? CSC / 4 : 1)) * 4 + threadIdx.x / (CSC ? CSC / 4 : 1) : threadIdx.x);
-      const bool col_ok = threadIdx.x < CS && mycol < W;
+      // ---------------- summing waves: rows strictly in order ----------------
+      uint32_t lane = threadIdx.x % kWave;
+      asm volatile("" : "+v"(lane)); // what follows from it is worked out here and takes no registers of the loaders
+      constexpr uint32_t kHalves = CSC ? kRowSets<CSC> : 1;
+      // the place of the column this lane sums, and which rows of a chunk the lane holds
+      const uint32_t place = lane % (kWave / kHalves), half = lane / (kWave / kHalves);
+      const uint32_t mycol = slice * CS + place;
+      const bool col_ok = place < CS && mycol < W;
       const bool direct = t.nrank == 1; // every key is owned and resident; the version counters move elsewhere
-      uint32_t slot = 0;
-      if (direct) {
+      if (direct && wave == kSummers - 1) {
         // The table rows the sums are added to, for every run of the bundle at once and parked in LDS: requested
         // run by run, each would arrive a memory round trip after its run had been summed (a run of a few hundred
         // occurrences is summed in a fraction of one), and the loaders would wait behind the full ring meanwhile.
         // This wait happens once per bundle, while the loaders' first rows are on their way.
-        float rows[kTable];
+        float rows[kTable / kHalves];
 #pragma unroll
-        for (int j = 0; j < kTable; j++) {
+        for (uint32_t j = 0; j < kTable / kHalves; j++) {
           rows[j] = 0.f;
-          if ((uint32_t)j < J && col_ok) rows[j] = t.emb[(size_t)table[j].w * W + mycol];
+          if (j * kHalves + half < J && col_ok) rows[j] = t.emb[(size_t)table[j * kHalves + half].w * W + mycol];
         }
 #pragma unroll
-        for (int j = 0; j < kTable; j++) row_stash[j * kWave + threadIdx.x] = rows[j];
+        for (uint32_t j = 0; j < kTable / kHalves; j++) row_stash[(j * kHalves + half) * kWave + place] = rows[j];
       }
-      for (uint32_t j = 0; j < J; j++) {
-        const uint4 m = table[j];
-        const uint32_t L = m.z;
-        const uint32_t nfull = L / CR, nch = (L + CR - 1) / CR;
-        float acc = 0.f; // the reference starts every sum from 0
-        uint32_t c = 0;
-        if (CSC) {
-          // Full chunks, kSumBatch rows at a time, one batch ahead: the LDS reads of a batch are in flight while the
-          // previous batch is added.  Reading the first batch of a chunk passes that chunk's barrier, i.e. the wave
-          // is at most one barrier ahead of its adds, which the three ring slots allow.
-          constexpr int kBatches = kChunkRows / kSumBatch; // per chunk, even
-          static_assert(!CSC || kBatches % 2 == 0, "the two batch buffers alternate, a chunk starts on the first");
-          const uint32_t lane_off = (threadIdx.x < CS ? threadIdx.x : 0) * pitch;
-          const float *sp = lds;
-          auto open_chunk = [&]() { // passes the chunk's barrier
-            __syncthreads();
-            sp = lds + slot * slot_floats + lane_off;
-            slot = slot + 1 == (uint32_t)kSlots ? 0 : slot + 1;
-          };
-          auto read_batch = [&](int k, float(&dst)[kSumBatch]) { // batch k of the open chunk
-            const float4 *bp = (const float4 *)(sp + k * kSumBatch);
+      auto finish = [&](uint32_t u, uint32_t off, uint32_t j, float acc) { // the sum of run j of the bundle is complete
+        const float scaled = acc * neg_lr;
+        if (direct) t.emb[(size_t)off * W + mycol] = row_stash[j * kWave + place] + scaled;
+        else apply_row<Vec<1>, K>(t, id_bits, p, a, u, scaled, mycol);
+      };
+      if constexpr (CSC != 0) {
+        // this wave's chunks are every other one of the bundle
+        constexpr uint32_t kHeld = kHeldRows;
+        // where the column lies in a row of the ring: the last lane of a row at any address starts at column W - 4
+        const uint32_t due = mycol / 4 * 4, at = !col_ok ? 0 : place + (VEC == kOdd4 && due + 4 > W ? due + 4 - W : 0);
+        float x[kHeld];
+        uint32_t j = 0, c = wave, passed = 0; // chunk c of run j of the bundle is next
+        uint32_t rank, L, off;                // of that run
+        auto open_run = [&]() {
+          const uint4 m = table[j];
+          rank = uni(m.x), L = uni(m.z), off = uni(m.w);
+        };
+        auto settle = [&]() {
+          while (c * CR >= L && j + 1 < J) {
+            c -= (L + CR - 1) / CR;
+            j++;
+            open_run();
+          }
+        };
+        open_run();
+        settle();
+        if (wave) __syncthreads(), passed++;
+        for (uint32_t g = wave; g < G; g += 2) {
+          __syncthreads(); // chunk g is in the ring
+          const uint32_t rows = min(CR, L - c * CR);
+          const float *sp = lds + (g % slots) * slot_floats + at;
+          if (rows % 4) { // a last group of less than four rows is put aside
 #pragma unroll
-            for (int q = 0; q < kSumBatch / 4; q++) {
-              const float4 v = bp[q];
-              dst[4 * q] = v.x, dst[4 * q + 1] = v.y, dst[4 * q + 2] = v.z, dst[4 * q + 3] = v.w;
+            for (uint32_t q = 0; q < 3; q++) {
+              const uint32_t r = min(rows / 4 * 4 + q, CR - 1);
+              hand[(1 + wave * 3 + q) * kWave + lane] = sp[(r + (r >= kHeld ? kPad : 0)) * CS];
             }
-          };
-          auto add_batch = [&](const float(&x)[kSumBatch]) {
+          }
 #pragma unroll
-            for (int q = 0; q < kSumBatch; q++) acc += x[q];
-          };
-          if (nfull) {
-            float x0[kSumBatch], x1[kSumBatch];
-            open_chunk();
-            read_batch(0, x0);
-            // all chunks but the last: straight-line code, so that the waits for LDS data stay exact
-            for (uint32_t cc2 = 0; cc2 + 1 < nfull; cc2++) {
+          for (uint32_t q = 0; q < kHeld; q++) x[q] = sp[(half * (kHeld + kPad) + q) * CS];
+          __syncthreads(); // the other wave has added chunk g - 1; chunk g is in registers
+          float acc = 0.f; // the reference starts every sum from 0
+          if (c) acc = hand[place];
+          auto add4 = [&](uint32_t q) { acc += x[q], acc += x[q + 1], acc += x[q + 2], acc += x[q + 3]; };
+          auto add_held = [&](uint32_t n) { // the first n rows the lane holds, without those behind the last four
 #pragma unroll
-              for (int k = 0; k < kBatches; k += 2) {
-                read_batch(k + 1, x1);
-                add_batch(x0);
-                if (k + 2 < kBatches) {
-                  read_batch(k + 2, x0);
-                } else {
-                  open_chunk();
-                  read_batch(0, x0);
-                }
-                add_batch(x1);
+            for (uint32_t q = 0; q < kHeld; q += 4)
+              if (n >= q + 4) add4(q);
+          };
+          auto add_all = [&]() {
+#pragma unroll
+            for (uint32_t q = 0; q < kHeld; q += 4) add4(q);
+          };
+          if (rows < kHeld) {
+            add_held(rows);
+          } else {
+            add_all();
+            if (kHalves > 1 && rows > kHeld) {
+              acc = from_lower_half(acc);
+              if (rows == CR) add_all();
+              else add_held(rows - kHeld);
+            }
+          }
+          if (rows % 4) {
+            const float *rest = hand + (1 + wave * 3) * kWave + lane;
+            acc += rest[0];
+            if (rows % 4 > 1) acc += rest[kWave];
+            if (rows % 4 > 2) acc += rest[2 * kWave];
+          }
+          // the lanes that have added the last rows
+          const bool have = half == (rows > kHeld ? 1u : 0u);
+          if (c * CR + rows < L) {
+            if (have) hand[place] = acc;
+          } else if (have && col_ok) {
+            finish(rank, off, j, acc);
+          }
+          passed += 2;
+          c += 2;
+          settle();
+        }
+        if (passed < G + 1) __syncthreads();
+      } else {
+        uint32_t slot = 0;
+        for (uint32_t j = 0; j < J; j++) {
+          const uint4 m = table[j];
+          float acc = 0.f; // the reference starts every sum from 0
+          for (uint32_t c = 0; c * CR < m.z; c++) {
+            __syncthreads(); // barrier of this chunk
+            const float *sp = lds + slot * slot_floats + place;
+            slot = slot + 1 == slots ? 0 : slot + 1;
+            if (place < CS) {
+              const uint32_t rows = min(CR, m.z - c * CR);
+              uint32_t r = 0;
+              for (; r + 8 <= rows; r += 8) {
+                float x[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) x[q] = sp[(r + q) * CS];
+#pragma unroll
+                for (int q = 0; q < 8; q++) acc += x[q];
               }
-            }
-#pragma unroll
-            for (int k = 0; k < kBatches; k += 2) { // the last full chunk
-              read_batch(k + 1, x1);
-              add_batch(x0);
-              if (k + 2 < kBatches) read_batch(k + 2, x0);
-              add_batch(x1);
+              for (; r < rows; r++) acc += sp[r * CS];
             }
           }
-          c = nfull;
-        }
-        for (; c < nch; c++) { // generic path, and the partial last chunk of the fast path
-          __syncthreads();     // barrier of this chunk
-          const uint32_t rstride = CSC ? 1u : CS; // distance between two rows of this lane's column
-          const float *col_ptr = lds + slot * slot_floats + threadIdx.x * (CSC ? pitch : 1u);
-          slot = slot + 1 == (uint32_t)kSlots ? 0 : slot + 1;
-          if (threadIdx.x < CS) {
-            const uint32_t rows = min(CR, L - c * CR);
-            uint32_t r = 0;
-            for (; r + 8 <= rows; r += 8) {
-              float x[8];
-#pragma unroll
-              for (int q = 0; q < 8; q++) x[q] = col_ptr[(r + q) * rstride];
-#pragma unroll
-              for (int q = 0; q < 8; q++) acc += x[q];
-            }
-            for (; r < rows; r++) acc += col_ptr[r * rstride];
-          }
-        }
-        if (col_ok) {
-          const float scaled = acc * neg_lr;
-          if (direct) t.emb[(size_t)m.w * W + mycol] = row_stash[j * kWave + threadIdx.x] + scaled;
-          else apply_row<Vec<1>, K>(t, id_bits, p, a, m.x, scaled, mycol);
+          if (col_ok) finish(m.x, m.w, j, acc);
         }
       }
     }
     __syncthreads(); // everybody is done with the table and the ring
   }
+}
+
+// How many classes of long runs, from the longest on, are cut into slices of kGiantSlice columns, the others being cut into
+// slices of kSlice; negative: the width leaves one to three columns over in either, which no lane of four columns can serve.
+// Slices of kSlice columns are not worth it where the last one would be half empty.
+__device__ __forceinline__ int narrow_classes(uint32_t width) {
+  const uint32_t wide = width % kSlice, narrow = width % kGiantSlice;
+  const bool in_wide = wide == 0 || wide >= 4, in_narrow = narrow == 0 || narrow >= 4;
+  if (in_narrow && wide && wide <= kSlice / 2) return kLongBuckets;
+  return !in_wide ? -1 : in_narrow ? kGiantClasses : 0;
 }
 
 // all roles in one launch: the long chains start first, medium and short blocks fill the machine behind them, the
@@ -749,35 +790,36 @@ __device__ __forceinline__ void push_block(const TableView &t, int id_bits, cons
                                            uint32_t block) {
   // one LDS area for whichever role the block plays: the row ring of the long role or the index staging of the
   // medium role (one slice of kLongRun indices per group)
-  constexpr int kRingWords = kSlots * kRPT * kPushBlock * (int)kCols<VEC>;
+  constexpr int kRingWords = VEC == 1 ? kSlotsGeneric * 2 * kPushBlock
+                                      : std::max({ring_floats(64), ring_floats(32), ring_floats(16), kSlotsGeneric * 2 * kPushBlock * 4});
   constexpr int kStageWords = (kPushBlock / LPR) * (int)kLongRun;
   __shared__ __align__(16) float lds[kRingWords > kStageWords ? kRingWords : kStageWords];
-  __shared__ uint4 run_table[kTable];
-  __shared__ uint32_t run_totals[3];
+  __shared__ uint4 run_table[2 * kTable];
+  __shared__ uint32_t run_totals[2 * 4];
+  __shared__ float sums_at_hand[7 * kWave];  // long role: the sums one wave leaves to the other; up to three rows of each
   __shared__ float row_stash[kTable * kWave]; // long role: the table rows of a bundle's runs (one slice, one lane each)
   if (block < kLongBlocks) {
     // Every block first takes tickets of the longest runs, which are cut into narrower column slices so that more
     // blocks feed each of them (the blocks of a saturated memory system get equal shares of it, and a chain
     // advances with the share of the block that feeds it), then tickets of the other long runs.
     uint32_t *tk = p.d_nlong + kTicketBase;
-    // Widths that are whole slices take the fast layout of the ring: 64 (the longest runs 32) columns, or 32, or rows
-    // of 32 and 16 floats as one slice.
-    auto all_runs = [&](auto csc) {
-      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kLongBuckets,
-                                                       block, kLongBlocks, tk);
+    auto runs = [&](auto csc, int c_lo, int c_hi, uint32_t *counters) {
+      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, sums_at_hand, c_lo, c_hi, block,
+                                                       kLongBlocks, counters);
     };
     constexpr int kOneSlice = VEC != 1 && LPR <= 8 ? LPR * 4 : 0, kNarrow = VEC != 1 && LPR > 8 ? kGiantSlice : 0;
-    if (kOneSlice && t.width == (uint32_t)kOneSlice) {
-      all_runs(std::integral_constant<int, kOneSlice>());
-    } else if (kNarrow && t.width % kSlice == 0) {
-      long_role<VEC, K, kNarrow, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, 0, kGiantClasses,
-                                          block, kLongBlocks, tk);
-      long_role<VEC, K, (kNarrow ? kSlice : 0), kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, kGiantClasses,
-                                                         kLongBuckets, block, kLongBlocks, tk + kTicketLanes);
-    } else if (kNarrow && t.width % kGiantSlice == 0) {
-      all_runs(std::integral_constant<int, kNarrow>());
+    if constexpr (kOneSlice != 0) { // rows of up to 16 or 32 floats
+      runs(std::integral_constant<int, kOneSlice>(), 0, kLongBuckets, tk);
+    } else if constexpr (kNarrow != 0) {
+      const int narrow = narrow_classes(t.width);
+      if (narrow >= 0) {
+        if (narrow > 0) runs(std::integral_constant<int, kNarrow>(), 0, narrow, tk);
+        if (narrow < kLongBuckets) runs(std::integral_constant<int, kSlice>(), narrow, kLongBuckets, tk + kTicketLanes);
+      } else {
+        runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);
+      }
     } else {
-      all_runs(std::integral_constant<int, 0>());
+      runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);
     }
   } else if (block < kLongBlocks + kMedBlocks) { // medium runs take long per block: they start early
     medium_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, (uint32_t *)lds, block - kLongBlocks, kMedBlocks);

@@ -753,3 +753,30 @@ def test_preprocess_again_while_the_run_lists_are_built(n):
     p.compare_state(1e-5, "end")
     p.compare_ints([capi.VERSION], "end")
     p.close()
+
+
+@pytest.mark.parametrize("nrank", [1, 2])
+@pytest.mark.parametrize("width", [12, 16, 21, 32, 37, 64, 66, 80, 97, 128])
+def test_run_lengths_around_the_chunks_of_the_push(width, nrank):
+    # runs that end just before, at and behind the chunks of 96 and 192 rows, their halves and groups of four, in slices of 16,
+    # 32 and 64 columns, whole and partly filled, and (width 66) in the generic layout; sums bit for bit
+    say("runs around chunks", width, nrank)
+    rng = np.random.default_rng(13)
+    lens = [129, 130, 131, 159, 160, 189, 191, 192, 193, 194, 195, 196, 203, 287, 288, 289, 290, 383, 384, 385, 387, 575, 576,
+            577, 767, 768, 769, 1151, 1152, 1153, 2048, 4095, 4096, 4097, 4223, 4224, 4225, 4227, 4320, 4321]
+    length = 4 * len(lens)
+    root = (np.arange(length) % nrank).astype(np.uint8)
+    p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    prev_n = [0] * nrank
+    for step in range(2):
+        keys = [np.repeat(rng.permutation(length)[:len(lens)].astype(np.int64), lens) for _ in range(nrank)]
+        for k in keys:
+            rng.shuffle(k)
+        p.preprocess(keys, device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(n, width)).astype(np.float32) for n in prev_n])
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        p.compare_state(1e-5, "step %d" % step)
+        prev_n = [k.shape[0] for k in keys]
+    p.close()
