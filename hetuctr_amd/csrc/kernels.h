@@ -347,13 +347,16 @@ void launch_place_queries(hipStream_t s, OwnerShard *shards_dev, const OwnerShar
 // owner looks its requesters up there).  push_blocks: the most blocks a shard's received pushes need; queries_max: no
 // shard receives more queries than this; queries_guess: what the busiest shard probably receives (the grids are cut
 // from it; what a shard does receive, the kernels read from the records and stride over).
+// pulls: the requesters; their launches' share is the index of every returned row per unique key (a.ret_i), where the gather
+// reads each key's row (a.src_row) and the counts of the step.
+struct PullShard;
 void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width,
-                       uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess);
+                       uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess, const PullShard *pulls, int npulls);
 // requester: refresh cached rows that came back, then gather every key's row into dst
 struct PullArgs {
   const uint32_t *got;       // [U] or nullptr: nothing came back (nrank == 1)
-  uint32_t *ret_i;           // [U] index into the returned rows (written by launch_refresh)
-  uint32_t *src_row;         // [U] where the gather reads a key's row (written by launch_refresh): offset or returned row
+  uint32_t *ret_i;           // [U] index into the returned rows (written by launch_owner_side)
+  uint32_t *src_row;         // [U] where the gather reads a key's row (written by launch_owner_side): offset or returned row
   const version_t *in_ver;
   const embed_t *in_val;
   embed_t *dst;              // [n][width]
@@ -370,14 +373,13 @@ struct PullShard {
   const uint32_t *delta;
   index_t *q_idx;
   version_t *q_ver;
-  // refresh: scratch of scan_blocks(n) words; five device words that read zero before the first call (the launch leaves
-  // them zero again); four words the device can write (hit / miss / refreshed counts of the step, error bits)
-  uint32_t *tile_sums, *stats, *host_stats;
+  // refresh: scratch of 4 * scan_blocks(n) words; four words the device can write (hit / miss / refreshed counts of the step,
+  // error bits)
+  uint32_t *tile_counts, *host_stats;
   uint32_t unique_guess;     // the grid of the row kernel is cut from it (how many keys are unique the kernels read)
 };
 void launch_build_queries(hipStream_t s, const KeyLayout &kl, const PullShard *shards, int count);
-// Index of every returned row per unique key (a.ret_i), where the gather reads each key's row (a.src_row), the counts of
-// the step and the refresh of the cached rows that came back.
+// The refresh of the cached rows that came back.
 void launch_refresh(hipStream_t s, const PullShard *shards, int count);
 // every key's row into a.dst (may be null: nothing to gather), and the run lists of the batch (a.list_chunks)
 void launch_gather_group(hipStream_t s, const PullShard *shards, int count);

@@ -314,11 +314,138 @@ __global__ __launch_bounds__(kBlock) void scan_positions(const OwnerShard *__res
   }
 }
 
+// What comes back per unique key of the step, in two roles over tiles of kRTile keys.  They need the owners' flags only, so they
+// share the launches of place_returns and pack_rows, the flags and offsets being requested before the number of unique keys is
+// here.  (In launches of their own behind pack_rows they took 14 us and two gaps of a step of four shards of 53 k keys; two
+// steps 355 -> 337 us.)
+//  count_returned  returned rows per tile, and the counts of the step: keys cached and fresh enough, not stored here, cached
+//                  and refreshed; and whether an owned row came back as outdated (it never may)
+//  remote_emit     ret_i[u] = index of u's row among the returned rows (exclusive scan of the flags; a tile adds up the
+//                  sums of the tiles before it itself); src_row[u] = where the gather finds the row: the resident offset,
+//                  or (top bit set) that index.  The last tile adds up the counts of all tiles and hands them to the host
+//                  (pinned memory).
+// The counts were added up by device-scope atomics of every block of remote_emit, with a fence in front of the ticket that
+// named the last block.
+constexpr uint32_t kReturnedRow = 0x80000000u;
+constexpr int kRItems = 8, kRTile = kBlock * kRItems; // 2048 keys: the tile scan_blocks() sizes the scratch for
+struct TileCounts {
+  uint32_t returned, fresh, absent, refreshed; // top bit of the last: an owned row came back
+};
+constexpr uint32_t kOwnedCame = 0x80000000u;
+// the block's totals of four counts (top bit of the fourth: or), for its first thread; sm: 5 words that read zero
+__device__ __forceinline__ void block_totals(TileCounts &c, uint32_t *sm) {
+  uint32_t came = c.refreshed & kOwnedCame;
+  c.refreshed &= ~kOwnedCame;
+  for (int d = 32; d; d >>= 1) {
+    c.returned += __shfl_down(c.returned, d);
+    c.fresh += __shfl_down(c.fresh, d);
+    c.absent += __shfl_down(c.absent, d);
+    c.refreshed += __shfl_down(c.refreshed, d);
+    came |= __shfl_down(came, d);
+  }
+  __syncthreads(); // the zeros
+  if (threadIdx.x % kWave == 0) {
+    atomicAdd(&sm[0], c.returned);
+    atomicAdd(&sm[1], c.fresh);
+    atomicAdd(&sm[2], c.absent);
+    atomicAdd(&sm[3], c.refreshed); // at most 2^31 - 1 keys
+    atomicOr(&sm[4], came);
+  }
+  __syncthreads();
+  c = TileCounts{sm[0], sm[1], sm[2], sm[3] | sm[4]};
+}
+__device__ __forceinline__ void count_returned(const PullShards &shards, uint32_t tile) {
+  __shared__ uint32_t sm[5];
+  const PullShard &S = shards.s[record_of(shards.cut, tile)];
+  const uint32_t *__restrict__ got = S.a.got;
+  uint32_t g[kRItems];
+  slot_t o[kRItems];
+#pragma unroll
+  for (int k = 0; k < kRItems; k++) { // neighbouring threads count neighbouring keys; requested before U is here
+    const uint32_t j = min(tile * kRTile + k * kBlock + threadIdx.x, S.b.n - 1);
+    g[k] = got[j];
+    o[k] = S.b.uoff[j];
+  }
+  const uint32_t U = *S.b.d_U; // the grid is cut for the batches' keys: the host has not seen the number of unique ones
+  if (tile * kRTile >= U) return;
+  if (threadIdx.x < 5) sm[threadIdx.x] = 0;
+  TileCounts c = {0, 0, 0, 0};
+  uint32_t came = 0;
+#pragma unroll
+  for (int k = 0; k < kRItems; k++) {
+    if (tile * kRTile + k * kBlock + threadIdx.x >= U) continue;
+    c.returned += g[k];
+    if (o[k] == kNoSlot) c.absent++;
+    else if ((uint32_t)o[k] >= S.t.n_cached) came |= g[k] ? kOwnedCame : 0u;
+    else if (g[k]) c.refreshed++;
+    else c.fresh++;
+  }
+  c.refreshed |= came;
+  block_totals(c, sm);
+  if (threadIdx.x == 0) ((TileCounts *)S.tile_counts)[tile] = c;
+}
+__device__ __forceinline__ void remote_emit(const PullShards &shards, uint32_t tile) {
+  __shared__ uint32_t sm[kBlock / kWave + 1], tot[5];
+  const PullShard &S = shards.s[record_of(shards.cut, tile)];
+  const BatchView &c = S.b;
+  const uint32_t *__restrict__ got = S.a.got;
+  const TileCounts *__restrict__ counts = (const TileCounts *)S.tile_counts;
+  uint32_t *__restrict__ ret_i = S.a.ret_i, *__restrict__ src_row = S.a.src_row;
+  const uint32_t j0 = tile * kRTile + threadIdx.x * kRItems;
+  uint32_t g[kRItems], mine = 0;
+  slot_t o[kRItems];
+#pragma unroll
+  for (int k = 0; k < kRItems; k++) { // requested before U is here
+    g[k] = got[min(j0 + k, c.n - 1)];
+    o[k] = c.uoff[min(j0 + k, c.n - 1)];
+  }
+  uint32_t s = 0;
+  for (uint32_t i = threadIdx.x; i < tile; i += kBlock) s += counts[i].returned; // (past the last tile: not used)
+  const uint32_t U = *c.d_U;
+  const uint32_t tiles = (U + kRTile - 1) / kRTile; // of the grid's blocks (cut for the batch's keys) these have work
+  if (tile >= tiles) return;
+  uint32_t prefix;
+  block_exclusive_scan<kBlock>(s, sm, prefix); // its total: returned rows in the tiles before this one
+#pragma unroll
+  for (int k = 0; k < kRItems; k++) mine += j0 + k < U ? g[k] : 0u;
+  uint32_t total;
+  uint32_t run = prefix + block_exclusive_scan<kBlock>(mine, sm, total);
+#pragma unroll
+  for (int k = 0; k < kRItems; k++) {
+    if (j0 + k < U) {
+      ret_i[j0 + k] = run;
+      src_row[j0 + k] = o[k] == kNoSlot ? (kReturnedRow | run) : (uint32_t)o[k];
+    }
+    run += g[k];
+  }
+  if (tile == tiles - 1) {
+    if (threadIdx.x < 5) tot[threadIdx.x] = 0;
+    TileCounts sum = {0, 0, 0, 0};
+    for (uint32_t i = threadIdx.x; i < tiles; i += kBlock) {
+      const TileCounts n = counts[i];
+      sum.fresh += n.fresh, sum.absent += n.absent;
+      sum.refreshed = (sum.refreshed + (n.refreshed & ~kOwnedCame)) | (n.refreshed & kOwnedCame);
+    }
+    block_totals(sum, tot);
+    if (threadIdx.x == 0) {
+      S.host_stats[0] = sum.fresh;
+      S.host_stats[1] = sum.absent;
+      S.host_stats[2] = sum.refreshed & ~kOwnedCame;
+      S.host_stats[3] = sum.refreshed & kOwnedCame ? 8u : 0u;
+    }
+  }
+}
+
 // Where the rows an owner returns stand in the requesters' buffers: a requester's rows arrive in owner order
 // (csrc/core/all2all.cu:89-130), and how many rows an owner returns to a requester is only known on the device.
 // Thread (owner d, requester s): ret_delta of d for s = rows the owners before d return to s, minus the start of s'
 // segment in d's own return order.
-__global__ void place_returns(const OwnerShard *__restrict__ shards, int nrank) {
+// place_blocks of the launch's blocks do this, the others count_returned.
+__global__ __launch_bounds__(kBlock) void place_returns(const OwnerShard *__restrict__ shards, int nrank, PullShards pulls, uint32_t place_blocks) {
+  if (blockIdx.x >= place_blocks) {
+    count_returned(pulls, blockIdx.x - place_blocks);
+    return;
+  }
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (uint32_t)nrank * nrank) return;
   const int d = i / nrank, s = i % nrank;
@@ -333,8 +460,15 @@ __global__ void place_returns(const OwnerShard *__restrict__ shards, int nrank) 
 #define HCTR_PACK_AHEAD 2
 #endif
 constexpr int kPackAhead = HCTR_PACK_AHEAD;
+// The launch has a row of blocks per owner, the first pack_blocks of which do this; the rows behind them do remote_emit.
 template <int VEC, int LPR>
-__global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict__ shards, int nseg) {
+__global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict__ shards, int nseg, PullShards pulls, uint32_t pack_blocks) {
+  if (blockIdx.y >= (uint32_t)nseg) {
+    const uint32_t block = (blockIdx.y - nseg) * gridDim.x + blockIdx.x;
+    if (block < pulls.cut.total) remote_emit(pulls, block);
+    return;
+  }
+  if (blockIdx.x >= pack_blocks) return;
   typedef typename RowVec<VEC>::T V;
   constexpr int kGroups = kBlock / LPR;
   __shared__ uint32_t sseg[258], sdelta[257];
@@ -345,7 +479,7 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
   const uint32_t total = sseg[nseg]; // rows this shard returns: known on the device only, the grid is cut for the most
   const embed_t *__restrict__ emb = S.t.emb;
   const uint32_t gl = threadIdx.x % LPR, W = S.t.width;
-  for (uint32_t k0 = blockIdx.x * (kGroups * kPackAhead) + threadIdx.x / LPR; k0 < total; k0 += gridDim.x * (kGroups * kPackAhead)) {
+  for (uint32_t k0 = blockIdx.x * (kGroups * kPackAhead) + threadIdx.x / LPR; k0 < total; k0 += pack_blocks * (kGroups * kPackAhead)) {
   slot_t o[kPackAhead];
 #pragma unroll
   for (int a = 0; a < kPackAhead; a++) o[a] = k0 + a * kGroups < total ? S.ret_slot[k0 + a * kGroups] : kNoSlot;
@@ -383,107 +517,6 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
   }
 }
 
-// What comes back per unique key of the step, in two launches over tiles of kRTile keys:
-//  got_tile_sums   returned rows per tile
-//  remote_emit     ret_i[u] = index of u's row among the returned rows (exclusive scan of the flags; a tile adds up the
-//                  sums of the tiles before it itself); src_row[u] = where the gather finds the row: the resident offset,
-//                  or (top bit set) that index; and the counts of the step: [0] cached and fresh enough, [1] not stored
-//                  here, [2] cached and refreshed, [3] bit 3: an owned row came back as outdated (it never may).
-// Atomics on one address are served one after the other, so every thread counts its keys in registers and a block
-// adds its totals once.  The block that finishes last hands the totals to the host (pinned memory) and puts the device
-// counters back to zero for the next step: no clearing launch before, no copy after.
-constexpr uint32_t kReturnedRow = 0x80000000u;
-constexpr int kRItems = 8, kRTile = kBlock * kRItems; // 2048 keys: the tile scan_blocks() sizes the scratch for
-__global__ __launch_bounds__(kBlock) void got_tile_sums(PullShards shards) {
-  __shared__ uint32_t sm[kBlock / kWave + 1];
-  uint32_t tile, tiles_cut;
-  const PullShard &S = my_record(shards, tile, tiles_cut);
-  const uint32_t *__restrict__ got = S.a.got;
-  const uint32_t U = *S.b.d_U; // the grid is cut for the batches' keys: the host has not seen the number of unique ones
-  if (tile * kRTile >= U) return;
-  const uint32_t j0 = tile * kRTile + threadIdx.x * kRItems;
-  uint32_t c = 0;
-#pragma unroll
-  for (int k = 0; k < kRItems; k++) c += (j0 + k < U) ? got[j0 + k] : 0u;
-  uint32_t total;
-  block_exclusive_scan<kBlock>(c, sm, total);
-  if (threadIdx.x == 0) S.tile_sums[tile] = total;
-}
-__global__ __launch_bounds__(kBlock) void remote_emit(PullShards shards) {
-  __shared__ uint32_t sm[kBlock / kWave + 1];
-  uint32_t tile, tiles_cut;
-  const PullShard &S = my_record(shards, tile, tiles_cut);
-  const TableView &t = S.t;
-  const BatchView &c = S.b;
-  const uint32_t *__restrict__ got = S.a.got;
-  const uint32_t *__restrict__ tile_sums = S.tile_sums;
-  uint32_t *__restrict__ ret_i = S.a.ret_i, *__restrict__ src_row = S.a.src_row, *__restrict__ stats = S.stats;
-  uint32_t *__restrict__ host_stats = S.host_stats;
-  const uint32_t U = *c.d_U;
-  const uint32_t tiles = (U + kRTile - 1) / kRTile; // of the grid's blocks (cut for the batch's keys) these have work
-  if (tile >= tiles) return;
-  __shared__ uint32_t tot[4];
-  __shared__ bool last;
-  if (threadIdx.x < 4) tot[threadIdx.x] = 0;
-  uint32_t s = 0;
-  for (uint32_t i = threadIdx.x; i < tile; i += kBlock) s += tile_sums[i];
-  uint32_t prefix;
-  block_exclusive_scan<kBlock>(s, sm, prefix); // its total: returned rows in the tiles before this one
-  const uint32_t j0 = tile * kRTile + threadIdx.x * kRItems;
-  uint32_t g[kRItems], mine = 0;
-  slot_t o[kRItems];
-#pragma unroll
-  for (int k = 0; k < kRItems; k++) {
-    const bool in = j0 + k < U;
-    g[k] = in ? got[j0 + k] : 0u;
-    o[k] = in ? c.uoff[j0 + k] : 0;
-    mine += g[k];
-  }
-  uint32_t total;
-  uint32_t run = prefix + block_exclusive_scan<kBlock>(mine, sm, total);
-  uint32_t n0 = 0, n1 = 0, n2 = 0, bad = 0;
-#pragma unroll
-  for (int k = 0; k < kRItems; k++) {
-    if (j0 + k < U) {
-      ret_i[j0 + k] = run;
-      src_row[j0 + k] = o[k] == kNoSlot ? (kReturnedRow | run) : (uint32_t)o[k];
-      if (o[k] == kNoSlot) n1++;
-      else if ((uint32_t)o[k] < t.n_cached) {
-        if (g[k]) n2++;
-        else n0++;
-      } else if (g[k]) {
-        bad = 8u;
-      }
-    }
-    run += g[k];
-  }
-  for (int d = 32; d; d >>= 1) {
-    n0 += __shfl_down(n0, d);
-    n1 += __shfl_down(n1, d);
-    n2 += __shfl_down(n2, d);
-    bad |= __shfl_down(bad, d);
-  }
-  if (threadIdx.x % 64 == 0) {
-    atomicAdd(&tot[0], n0);
-    atomicAdd(&tot[1], n1);
-    atomicAdd(&tot[2], n2);
-    atomicOr(&tot[3], bad);
-  }
-  __syncthreads();
-  if (threadIdx.x < 3 && tot[threadIdx.x]) atomicAdd(&stats[threadIdx.x], tot[threadIdx.x]);
-  if (threadIdx.x == 3 && tot[3]) atomicOr(&stats[3], tot[3]);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    last = atomicAdd(&stats[4], 1u) == tiles - 1;
-  }
-  __syncthreads();
-  if (last && threadIdx.x < 4) {
-    __threadfence();
-    host_stats[threadIdx.x] = atomicExch(&stats[threadIdx.x], 0u);
-    if (threadIdx.x == 0) stats[4] = 0;
-  }
-}
 
 // One group per unique rank of the current batch, kRefreshRows of them after one another where the batch is large: a block's
 // start -- its record, how many keys there are -- costs as much as a row.  Four batches of 100 k unique keys, 128 floats: 18
@@ -763,7 +796,7 @@ static uint32_t guessed_blocks(uint32_t guess, uint32_t most, uint32_t per_block
 }
 
 void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width,
-                       uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess) {
+                       uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess, const PullShard *pulls, int npulls) {
   const uint32_t tiles = guessed_blocks(queries_guess, queries_max, kBlock);
   const int vec = row_vec(width, nullptr);
   const int lpr = lanes_for(width, vec);
@@ -776,26 +809,35 @@ void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards,
   }
   hipLaunchKernelGGL(decide_count, dim3(tiles, nshards), dim3(kBlock), 0, s, shards_dev, nsrc);
   hipLaunchKernelGGL(scan_positions, dim3(tiles, nshards), dim3(kBlock), 0, s, shards_dev, nsrc);
-  if (queries_max) {
-    hipLaunchKernelGGL(place_returns, dim3(div_up((uint32_t)(nsrc * nsrc), kBlock)), dim3(kBlock), 0, s, shards_dev, nsrc);
+  // the launches of several groups of requesters, the first of them with the owners' work
+  auto with_requesters = [&](bool owners, auto &&launch) {
+    // for the batches' keys; the kernels read how many are unique
+    for_shards(pulls, npulls, [](const PullShard &o) { return div_up(o.b.n, kRTile); }, [&](const PullShards &p, int) {
+      launch(p, owners);
+      owners = false;
+    });
+    if (owners) launch(PullShards{}, true); // nobody asked
+  };
+  with_requesters(queries_max != 0, [&](const PullShards &p, bool owners) {
+    const uint32_t place_blocks = owners ? div_up((uint32_t)(nsrc * nsrc), kBlock) : 0u;
+    hipLaunchKernelGGL(place_returns, dim3(place_blocks + p.cut.total), dim3(kBlock), 0, s, shards_dev, nsrc, p, place_blocks);
+  });
+  with_requesters(queries_max != 0, [&](const PullShards &p, bool owners) {
 #define CALL(V, L)                                                                                                     \
-  hipLaunchKernelGGL((pack_rows<V, L>), dim3(guessed_blocks(queries_guess, queries_max, kPackAhead * (kBlock / L)), nshards), \
-                     dim3(kBlock), 0, s, shards_dev, nsrc)
+  do {                                                                                                                 \
+    const uint32_t pack = owners ? guessed_blocks(queries_guess, queries_max, kPackAhead * (kBlock / L)) : 0u;         \
+    const uint32_t across = std::max(pack, 64u); /* few rows to pack: few idle blocks, and few rows of requesters */   \
+    hipLaunchKernelGGL((pack_rows<V, L>), dim3(across, nshards + div_up(p.cut.total, across)), dim3(kBlock), 0, s,     \
+                       shards_dev, nsrc, p, pack);                                                                     \
+  } while (0)
     HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
-  }
+  });
   HCTR_HIP(hipGetLastError());
 }
 
 void launch_refresh(hipStream_t s, const PullShard *shards, int count) {
   if (!count) return;
-  // for the batches' keys; the kernels read how many are unique
-  for_shards(shards, count, [](const PullShard &o) { return div_up(o.b.n, kRTile); }, [&](const PullShards &p, int) {
-    const dim3 tiles = grid_of(p);
-    hipLaunchKernelGGL(got_tile_sums, tiles, dim3(kBlock), 0, s, p);
-    hipLaunchKernelGGL(remote_emit, tiles, dim3(kBlock), 0, s, p);
-    HCTR_HIP(hipGetLastError());
-  });
   const uint32_t width = shards[0].t.width;
   const int vec = row_vec(width, nullptr), lpr = lanes_for(width, vec);
   const uint32_t groups = kBlock / lpr;

@@ -196,7 +196,7 @@ class Shard {
   bool prev_active = false; // false: inference step or no previous batch, nothing is pushed
   DeviceBuf root, slot, emb, ver, pend, upd, store_ids;
   // scratch shared by the stages
-  DeviceBuf ktmp0, ktmp1, vtmp0, vtmp1, sortws, block_sums, headws, dstat, stats;
+  DeviceBuf ktmp0, ktmp1, vtmp0, vtmp1, sortws, block_sums, headws, dstat;
   // where the index stages of the current batch find their scratch: the buffers above or pieces of the static array
   struct ScratchPtrs {
     void *ktmp0 = nullptr, *ktmp1 = nullptr;
@@ -292,7 +292,7 @@ class Group {
   // owner-side arguments of every shard: pinned staging and the device copy the kernels read
   OwnerShard *owner_host = nullptr;
   DeviceBuf owner_dev, ret_delta_dev;    // ret_delta_dev: nrank words per owner, see OwnerShard::ret_delta
-  void owner_side(uint64_t queries_max);
+  void owner_side(uint64_t queries_max, const std::vector<PullShard> &pulls);
   // Where every shard's pushed rows go: one receive area for the whole group (ids, counts, rows), cut into one piece
   // per owner and, inside it, per source; sized from the plans before any push kernel runs.  Every sender gets, per
   // owner, the distance between a row's place in its own plan and its place in the area (nrank words per sender).

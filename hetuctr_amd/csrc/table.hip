@@ -180,10 +180,8 @@ Shard::Shard(const hctr_config &c, const uint8_t *root_arr, const int64_t *stora
 
   dstat.reserve(sizeof(DevStat));
   dst_ = dstat.as<DevStat>();
-  stats.reserve(32);
   ret_seg_dev.reserve(2 * 258 * 4);
   HCTR_HIP(hipMemsetAsync(dstat.p, 0, dstat.bytes, s));
-  HCTR_HIP(hipMemsetAsync(stats.p, 0, 32, s));
   for (Batch *b : {&cur, &prev}) {
     b->reserve(1, c.nrank, kl.wide);
     b->clear(s, c.nrank);
@@ -228,7 +226,7 @@ void Shard::reserve_batch_scratch(uint32_t n) {
   vtmp0.reserve(m * 4);
   vtmp1.reserve(m * 4);
   sortws.reserve(index_table_words(m) * 4);
-  block_sums.reserve((scan_blocks(m) + 2) * 4);
+  block_sums.reserve((scan_blocks(m) + 2) * 16); // four words per tile in the refresh of a group
   headws.reserve(head_chunk_words(m) * 4);
   sp.ktmp0 = ktmp0.p;
   sp.ktmp1 = ktmp1.p;
@@ -709,8 +707,7 @@ bool Shard::pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *
   o.delta = delta;
   o.q_idx = group->rq_idx_all.as<index_t>();
   o.q_ver = group->rq_ver_all.as<version_t>();
-  o.tile_sums = sp.block_sums;
-  o.stats = stats.as<uint32_t>();
+  o.tile_counts = sp.block_sums;
   o.host_stats = mirror->stats;
   o.unique_guess = prev.U ? prev.U : cur.n;
   return true;
@@ -949,14 +946,14 @@ void Group::collect_marks() {
 }
 
 // handleGradient + handleQuery of every shard (csrc/core/hetu_gpu_table.cu:27-31): one set of launches for the group
-void Group::owner_side(uint64_t queries_max) {
+void Group::owner_side(uint64_t queries_max, const std::vector<PullShard> &pulls) {
   uint32_t push_blocks = 0;
   for (int r = 0; r < nrank; r++) push_blocks = std::max(push_blocks, owner_host[r].push_blocks);
   StageScope st(*this, S_OWNER);
   // the grids of the query kernels: from what the busiest owner received in the step before (the first step: the most)
   const uint32_t guess = queries_seen_ ? queries_guess_ : (uint32_t)queries_max;
   launch_owner_side(stream, owner_dev.as<OwnerShard>(), nrank, nrank, members[0]->cfg.width, push_blocks, (uint32_t)queries_max,
-                    guess);
+                    guess, pulls.data(), (int)pulls.size());
 }
 
 void Group::set_defer_index(bool on) {
@@ -1430,7 +1427,7 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
       StageScope st(*this, S_QUERY);
       launch_build_queries(stream, members[0]->kl, pulls.data(), (int)pulls.size());
     }
-    owner_side(queries_max);
+    owner_side(queries_max, pulls);
     // the reference waits here for the return counts (hetu_gpu_table.cu:33); they stay on the device
     {
       StageScope st(*this, S_REFRESH);
