@@ -63,11 +63,20 @@ __global__ __launch_bounds__(kBlock) void build_queries(PullShards shards, int i
 // between two splitters drawn from the longest segment, finds that id range in every other segment by binary search,
 // and walks the sources in order with a barrier between them.  Inside a source ids are distinct, so its rows are
 // applied in parallel, kAhead rows per group of LPR lanes at a time.
+//
+// A search is done by kProbes lanes at once, which cut what is left into kProbes + 1 pieces per round, and both ends of all ranges
+// are searched for side by side: 3 or 4 dependent loads for segments of 5 k rows where one lane per source, one end after the
+// other, took 24.  (Four shards of 53 k keys: 20.9 -> 17.2 us.)
+constexpr uint32_t kProbes = 16;
+// first position in [lo, hi) whose id is >= x; the kProbes neighbouring lanes of a group call it with the same arguments
 __device__ __forceinline__ uint32_t lower_bound_id(const index_t *__restrict__ a, uint32_t lo, uint32_t hi, index_t x) {
-  while (lo < hi) { // first position in [lo, hi) whose id is >= x
-    const uint32_t mid = lo + (hi - lo) / 2;
-    if (a[mid] < x) lo = mid + 1;
-    else hi = mid;
+  const uint32_t probe = threadIdx.x % kProbes, shift = threadIdx.x % kWave / kProbes * kProbes;
+  while (lo < hi) {
+    const uint32_t n = hi - lo, step = n <= kProbes ? 1 : (n - 1) / (kProbes + 1) + 1, at = (probe + 1) * step - 1;
+    const bool below = at < n && a[lo + at] < x;
+    const uint32_t c = __popc((uint32_t)(__ballot(below) >> shift) & ((1u << kProbes) - 1)); // ids ascend: the first c probes
+    if (c < kProbes) hi = min(hi, lo + (c + 1) * step - 1);
+    lo += c * step;
   }
   return lo;
 }
@@ -108,18 +117,16 @@ __global__ __launch_bounds__(kBlock) void apply_remote_all(const OwnerShard *__r
   const int longest = S.longest;
   const uint32_t big_lo = S.rg_seg[longest], big_hi = S.rg_seg[longest + 1];
   const uint32_t first = big_lo + blockIdx.x * rows_per_block, last = first + rows_per_block;
-  for (int s = threadIdx.x; s < nsrc; s += kBlock) {
-    const uint32_t a = S.rg_seg[s], b = S.rg_seg[s + 1];
-    if (s == longest) { // the splitters are this segment's own rows
-      lo[s] = first;
-      hi[s] = min(last, big_hi);
-    } else if (a == b) {
-      lo[s] = hi[s] = a;
-    } else {
-      // block 0 starts below every id, the last block ends above every id
-      lo[s] = blockIdx.x == 0 ? a : lower_bound_id(rg_idx, a, b, rg_idx[first]);
-      hi[s] = last >= big_hi ? b : lower_bound_id(rg_idx, lo[s], b, rg_idx[last]);
-    }
+  for (int q = threadIdx.x / kProbes; q < 2 * nsrc; q += kBlock / kProbes) { // lower and upper end for every source
+    const int s = q / 2;
+    const bool upper = q % 2;
+    const uint32_t a = S.rg_seg[s], b = S.rg_seg[s + 1], at = upper ? last : first;
+    uint32_t end;
+    if (s == longest) end = min(at, big_hi);           // the splitters are this segment's own rows
+    else if (upper && last >= big_hi) end = b;         // the last block ends above every id
+    else if (!upper && blockIdx.x == 0) end = a;       // block 0 starts below every id
+    else end = lower_bound_id(rg_idx, a, b, rg_idx[at]);
+    if (threadIdx.x % kProbes == 0) (upper ? hi : lo)[s] = end;
   }
   __syncthreads();
   const uint32_t gl = threadIdx.x % LPR;

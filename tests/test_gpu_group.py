@@ -384,3 +384,25 @@ def test_batches_of_unequal_shape_in_shared_launches(sizes, width):
         p.compare_state(1e-5, "step %d" % step)
         prev = ns
     p.close()
+
+
+@pytest.mark.parametrize("sizes", [(1, 2, 3), (16, 17, 18), (15, 33, 400), (289, 5000, 290), (5000, 0, 4999)])
+def test_pushes_of_unequal_length_to_one_owner(sizes):
+    # every source's range of ids between two rows of the longest segment is found by searches over segments of these lengths
+    print("pushed segments", sizes, flush=True)
+    rng = np.random.default_rng(3)
+    length, R, width = 24_000, len(sizes), 8
+    root = np.full(length, 2, np.uint8)                 # everything belongs to the last shard
+    storage = [np.zeros(0, np.int64), np.zeros(0, np.int64), np.arange(length, dtype=np.int64)]
+    p = Pair(R, length, width, root, storage, init=("Uniform", -0.01, 0.01), lr=0.05)
+    prev = [0] * R
+    for step in range(2):
+        keys = [rng.permutation(length)[:n].astype(np.int64) for n in sizes]
+        p.preprocess(keys, device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-2, size=(n, width)).astype(np.float32) for n in prev])
+        for r in range(R):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        p.compare_state(1e-5, "step %d" % step)
+        p.compare_ints(INT_ITEMS_POST, "step %d" % step)
+        prev = list(sizes)
+    p.close()
