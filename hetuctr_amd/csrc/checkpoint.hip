@@ -155,15 +155,8 @@ void Shard::load(const char *path) {
   file_to_device(in, upd.p, C * sizeof(version_t), st, s);
   // the batches in flight belong to the run that wrote the file, not to this one: start from empty ones
   for (Batch *b : {&cur, &prev}) {
-    b->n = 0;
-    b->U = 0;
-    b->idx_map_valid = false;
-    b->planned = false;
+    b->drop();
     b->clear(s, cfg.nrank);
-    std::fill(b->send_cnt.begin(), b->send_cnt.end(), 0);
-    std::fill(b->recv_cnt.begin(), b->recv_cnt.end(), 0);
-    std::fill(b->push_cnt.begin(), b->push_cnt.end(), 0);
-    std::fill(b->pushrecv_cnt.begin(), b->pushrecv_cnt.end(), 0);
   }
   prev_active = false;
   HCTR_HIP(hipStreamSynchronize(s));

@@ -75,6 +75,7 @@ struct Batch {
   void reserve(uint32_t n_keys, int nrank, bool wide);
   bool holds(uint32_t n_keys, int nrank, bool wide) const; // reserve() would not allocate
   void clear(hipStream_t s, int nrank); // make the device side an empty batch; does nothing if it already is
+  void drop(); // an empty batch to the host, whatever its buffers hold (they may be half made)
   BatchView view() const;
 };
 
@@ -137,6 +138,7 @@ class Shard {
 
   // ---- stages, each only enqueues on the group's stream (names follow hetu_gpu_table.h:82-97) ----
   void swap_batches() { std::swap(cur, prev); }
+  void check_batch(const int64_t *keys, size_t n) const; // refuses what no batch can be
   void preprocess_index(const int64_t *keys, size_t n) {
     ingest_keys(keys, n);
     index_batch();
@@ -344,6 +346,8 @@ class Group {
  private:
   void exchange_shapes();
   void push_pull_steps(const float *const *grads, float *const *dsts, uint32_t bag); // the body of push_pull_all
+  void preprocess_steps(const int64_t *const *keys, const size_t *n, bool &taken); // the body of preprocess_all
+  void stop_work();
   void finish_lists();
   bool lists_running_ = false; // a preprocess has launched the run lists of the previous batch on the main stream
   bool index_joining_ = false; // push_pull has taken a pending index over and not yet read its results

@@ -85,6 +85,13 @@ void Batch::clear(hipStream_t s, int nrank) {
   cleared = true;
 }
 
+void Batch::drop() {
+  n = U = 0;
+  idx_map_valid = planned = tile_sorted = one_block = direct_gather = comp_valid = keys_made = cleared = false;
+  lists_ready = true;
+  for (auto *c : {&send_cnt, &recv_cnt, &push_cnt, &pushrecv_cnt}) std::fill(c->begin(), c->end(), 0);
+}
+
 BatchView Batch::view() const {
   BatchView v;
   v.n = n;
@@ -218,6 +225,9 @@ Shard::~Shard() {
   if (mirror) (void)hipHostFree(mirror);
 }
 
+// four words per tile in the refresh of a group
+static size_t scan_scratch_bytes(size_t n) { return (scan_blocks(n) + 2) * 16; }
+
 void Shard::reserve_batch_scratch(uint32_t n) {
   const size_t m = std::max<uint32_t>(n, 1);
   const size_t ks = kl.wide ? 8 : 4;
@@ -226,7 +236,7 @@ void Shard::reserve_batch_scratch(uint32_t n) {
   vtmp0.reserve(m * 4);
   vtmp1.reserve(m * 4);
   sortws.reserve(index_table_words(m) * 4);
-  block_sums.reserve((scan_blocks(m) + 2) * 16); // four words per tile in the refresh of a group
+  block_sums.reserve(scan_scratch_bytes(m));
   headws.reserve(head_chunk_words(m) * 4);
   sp.ktmp0 = ktmp0.p;
   sp.ktmp1 = ktmp1.p;
@@ -256,10 +266,13 @@ void Shard::use_scratch_area(void *area, uint32_t n) {
   sp.headws = (uint32_t *)take(head_chunk_words(m) * 4);
 }
 
-// csrc/core/preprocess.cu:92-141
-void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scratch_area) {
+void Shard::check_batch(const int64_t *keys, size_t n) const {
   HCTR_CHECK(n < 0xfffffff0ull, "a batch holds fewer than 2^32 keys");
   HCTR_CHECK(keys != nullptr || n == 0, "null key pointer");
+}
+
+// csrc/core/preprocess.cu:92-141
+void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *scratch_area) {
   hipStream_t s = group->stream;
   cur.n = (uint32_t)n;
   cur.U = 0;
@@ -692,7 +705,9 @@ bool Shard::pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *
   }
   HCTR_CHECK(dst == nullptr || cur.n % bag == 0, "pooled pull: the batch is not a whole number of bags");
   // sized for the batch's keys: how many of them are unique the kernels read on the device (the host has not
-  // waited for the index); the scan scratch is the one the batch's index was given, its kernels are through
+  // waited for the index); the scan scratch is the one the batch's index was given, its kernels are through (and the
+  // batch may have become the current one again after a preprocess that failed for want of memory, scratch included)
+  block_sums.reserve(scan_scratch_bytes(cur.n));
   ret_i.reserve((size_t)cur.n * 4);
   src_row.reserve((size_t)cur.n * 4);
   o.t = tv;
@@ -707,7 +722,7 @@ bool Shard::pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *
   o.delta = delta;
   o.q_idx = group->rq_idx_all.as<index_t>();
   o.q_ver = group->rq_ver_all.as<version_t>();
-  o.tile_counts = sp.block_sums;
+  o.tile_counts = block_sums.as<uint32_t>();
   o.host_stats = mirror->stats;
   o.unique_guess = prev.U ? prev.U : cur.n;
   return true;
@@ -1181,8 +1196,47 @@ void Group::finish_lists() {
 void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
   HCTR_CHECK(complete(), "the loopback group named by (ip, port) is missing ranks");
   HCTR_HIP(hipSetDevice(device_id));
+  // a call that its arguments refuse leaves every batch as it found it
+  for (Shard *m : members) m->check_batch(keys[m->cfg.rank], n[m->cfg.rank]);
   flush_index(); // preprocess twice in a row: the earlier batch is indexed before it becomes the previous one
   finish_lists();
+  for (Shard *m : members) m->swap_batches();
+  bool taken = false;
+  try {
+    preprocess_steps(keys, n, taken);
+  } catch (...) {
+    // Taken: an error of the batch's own, a key outside the table.  Otherwise something failed on the way (an allocation,
+    // say), and nothing may be done with batches that have keys and no index, not even by the next call, which lists the
+    // runs of the batch before: they become empty, and the batches the call found current are that again.  (Those before
+    // them are lost, as in a call that succeeds: their buffers were the new batches'.)
+    if (!taken) {
+      stop_work();
+      index_pending = index_rest_pending = lists_running_ = false;
+      (void)hipGetLastError(); // a failed allocation is not the next launch's error
+      for (Shard *m : members) {
+        m->mirror->key_err = 0;
+        (void)hipMemsetAsync(m->err_ptr(), 0, 4, stream);
+        m->cur.drop();
+        m->swap_batches();
+      }
+    }
+    throw;
+  }
+}
+
+// after a failure: nothing runs any more, and nobody asks for the times of what ran
+void Group::stop_work() {
+  (void)hipStreamSynchronize(index_stream);
+  (void)hipStreamSynchronize(stream);
+  for (auto &mk : marks) {
+    event_pool.push_back(mk.a);
+    event_pool.push_back(mk.b);
+  }
+  marks.clear();
+}
+
+// The body of preprocess_all.  taken: the batches are whole, or will be when the launches that are left have run.
+void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &taken) {
   if (defer_index && !stage_timing && nrank == 1) {
     // One shard: everything is enqueued on the second stream, and the call returns as soon as the caller's ids have
     // been read.  Sorting and deduplicating them does not depend on the pending gradient push, which the next
@@ -1193,7 +1247,6 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     Shard *m = members[0];
     StreamSwitch on(*this, index_stream);
     if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
-    m->swap_batches();
     m->ingest_keys(keys[0], n[0], &m->mirror->key_err); // the flag lives in pinned host memory the kernel can write
     if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
     if (!m->read_.word) HCTR_HIP(hipEventRecord(ev_keys, stream));
@@ -1208,6 +1261,7 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
       lists_running_ = true;
     }
     const bool bad_key = wait_ids_read();
+    taken = true;
     if (time_calls) {
       float ms = 0.f;
       HCTR_HIP(hipEventSynchronize(ev1));
@@ -1224,7 +1278,6 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     // waits for the index before it builds the queries, which are the first thing that needs it.  The push plan of the
     // previous batches was made at the end of the step before.
     std::vector<Shard *> late;
-    for (Shard *m : members) m->swap_batches();
     // a previous batch that no push_pull has seen yet (two preprocess calls in a row) is planned here, on the main
     // stream, and waited for (the plan sizes the push buffers)
     for (Shard *m : members)
@@ -1245,6 +1298,7 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     const bool bad_key = wait_ids_read(); // the callers may reuse their buffers
     if (!late.empty()) sync_stream();
     for (Shard *m : late) m->finish_plan(m->prev);
+    taken = true;
     float ms = 0.f;
     if (time_calls) {
       HCTR_HIP(hipEventSynchronize(ev1));
@@ -1258,7 +1312,6 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
   if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
   std::vector<Shard *> unplanned;
   for (Shard *m : members) {
-    m->swap_batches();
     m->preprocess_index(keys[m->cfg.rank], n[m->cfg.rank]);
     if (!m->prev.planned) unplanned.push_back(m);
   }
@@ -1267,6 +1320,7 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
   for (Shard *m : members) m->enqueue_readback_preprocess();
   if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
   sync_stream();
+  taken = true;
   float ms = 0.f;
   if (time_calls) HCTR_HIP(hipEventElapsedTime(&ms, ev0, ev1));
   collect_marks();
@@ -1344,13 +1398,7 @@ void Group::push_pull_all(const float *const *grads, float *const *dsts, size_t 
     // Something failed after work was enqueued (a runtime error, a device-side check).  Nothing may still be running
     // when the caller sees the error, and an index that this call started to join is handed back to the next call
     // that needs it (flush_index takes its results over) instead of being dropped with its batch.
-    (void)hipStreamSynchronize(index_stream);
-    (void)hipStreamSynchronize(stream);
-    for (auto &mk : marks) {
-      event_pool.push_back(mk.a);
-      event_pool.push_back(mk.b);
-    }
-    marks.clear();
+    stop_work();
     if (index_joining_) index_pending = true;
     index_joining_ = false;
     throw;

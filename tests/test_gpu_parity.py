@@ -780,3 +780,58 @@ def test_run_lengths_around_the_chunks_of_the_push(width, nrank):
         p.compare_state(1e-5, "step %d" % step)
         prev_n = [k.shape[0] for k in keys]
     p.close()
+
+
+@pytest.mark.parametrize("nrank", [1, 2])
+@pytest.mark.parametrize("defer", [True, False])
+def test_a_refused_preprocess_leaves_the_batches_alone(defer, nrank):
+    say("refused preprocess", defer, nrank)
+    rng = np.random.default_rng(5)
+    length, width, n = 3_000, 8, 2_000
+    root = (np.arange(length) % nrank).astype(np.uint8)
+    p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    p.tables[0].defer_index(defer)
+    for step in range(4):
+        p.preprocess([rng.integers(0, length, n) for _ in range(nrank)], device_keys=True)
+        if step:
+            with pytest.raises(RuntimeError, match="null key pointer"):
+                capi.group_preprocess(p.tables, [d.data_ptr() for d in p.keep[:-1]] + [0], p.n)
+        g = [rng.normal(0, 1e-3, size=(n, width)).astype(np.float32) if step else None for _ in range(nrank)]
+        out, ref = p.push_pull(g)
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+    p.compare_state(1e-5, "end")
+    p.compare_ints([capi.VERSION, capi.STATS, capi.SIZES], "end")
+    p.close()
+
+
+@pytest.mark.parametrize("nrank", [1, 2])
+def test_preprocess_without_memory_for_its_batch(nrank):
+    # no room for the last shard's buffers: that batch is dropped, the one before is the current one again, and what the
+    # next calls do with it is what they do without the call between
+    import torch
+    say("no memory for a batch", nrank)
+    rng = np.random.default_rng(6)
+    length, width, n, huge = 5_000, 8, 20_000, 64 << 20
+    root = (np.arange(length) % nrank).astype(np.uint8)
+    p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    ids = torch.zeros(huge, dtype=torch.int64, device="cuda")
+    prev = 0
+    for step in range(5):
+        k = n - 1000 * step
+        p.preprocess([rng.integers(0, length, k) for _ in range(nrank)], device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(prev, width)).astype(np.float32) if prev else None for _ in range(nrank)])
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        prev = k
+        if step in (1, 2):
+            torch.cuda.empty_cache()
+            hold = torch.empty(torch.cuda.mem_get_info()[0] - (1 << 30), dtype=torch.uint8, device="cuda")
+            with pytest.raises(RuntimeError, match="out of memory"):
+                capi.group_preprocess(p.tables, [d.data_ptr() for d in p.keep[:-1]] + [ids.data_ptr()], p.n[:-1] + [huge])
+            del hold
+            torch.cuda.empty_cache()
+    p.compare_state(1e-5, "end")
+    p.close()
