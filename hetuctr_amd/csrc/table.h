@@ -57,6 +57,7 @@ struct Batch {
   bool idx_map_valid = false;
   bool cleared = false; // the device side reads as an empty batch (U = 0, no buckets, no runs) since clear()
   bool planned = false; // the push plan (need, prefix, push_cnt) has been computed for the batch as it stands
+  int early_sort_steps = 0; // three-launch passes: the launches that preprocess enqueues before it returns
   bool lists_ready = true;  // the run lists of the batch's push have been built (or the batch is empty)
   bool tile_sorted = false; // indexed by the tile-sorted passes (tile_sort.h)
   bool one_block = false;   // indexed by one block in one launch (tile_sort.h)
@@ -110,6 +111,15 @@ class Group;
 #define HCTR_EARLY_TILE_PASSES 1
 #endif
 constexpr int kEarlySortSteps = HCTR_EARLY_SORT_STEPS, kEarlyTilePasses = HCTR_EARLY_TILE_PASSES;
+// ... and where the run lists of the batch before are built meanwhile, the column scan alone.  The push follows those lists
+// within a few microseconds, and a scatter launched early would be holding the CUs then, two blocks each: the long runs'
+// blocks, which start first, would land two by two on the few it leaves, and the push of 4.16 M keys of 16 floats, Zipf 1.4
+// (508 blocks of the scatter on 512 places), takes 391 us instead of 269.  Two training steps with the scatter early and
+// behind the push: those 1116 and 865 us (903 with the lists in front of the push), 1.6 M keys 410 and 393, 2.6 M 586 and
+// 569; pooled, 64 floats, 4.15 M keys 1013 and 832, 8.4 M 1584 and 1598 (no difference: runs differ by 2 %); keys held in 64
+// bits, one block per CU, 2 M 701 and 497, 3 M 772 and 688, with exponent 1.05 741 and 760.  A push that follows without
+// such lists comes a little later; 3 M keys of 32 floats are 4 % slower this way.
+constexpr int kEarlySortStepsBesideLists = 2;
 // One shard: a batch whose output rows take up to this many bytes is gathered in batch order straight from its keys
 // (Batch::direct_gather).  Measured on an MI355X with 512-byte rows: 107 k keys 78 us per step against 92 with the gather
 // in sorted order behind the index, 426 k keys 165 against 174, 852 k keys 316 against 279 -- in batch order the

@@ -282,6 +282,7 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
   cur.direct_gather = false;
   cur.comp_valid = false;
   cur.one_block = cur.tile_sorted = false;
+  cur.early_sort_steps = kEarlySortSteps;
   ids_ = nullptr;
   key_flag_ = flag ? flag : err_ptr();
   read_ = ReadSignal();
@@ -450,8 +451,8 @@ void Group::index_batches(Shard *const *shards, size_t count, uint32_t *u_out, i
         const int passes = launch_tile_sort_passes(s, kl, r, m, from, to);
         for (int k = 0; k < m; k++) unique[k].sorted_keys = r[k].b.keys[passes & 1];
       } else {
-        const int from = part == 2 ? kEarlySortSteps : 0, to = part == 1 ? kEarlySortSteps : (1 << 30);
         Batch &cur = f.cur;
+        const int from = part == 2 ? cur.early_sort_steps : 0, to = part == 1 ? cur.early_sort_steps : (1 << 30);
         SortScratch sc;
         sc.words = f.sp.sortws;
         sc.n_cap = cur.n;
@@ -1250,9 +1251,11 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
     m->ingest_keys(keys[0], n[0], &m->mirror->key_err); // the flag lives in pinned host memory the kernel can write
     if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
     if (!m->read_.word) HCTR_HIP(hipEventRecord(ev_keys, stream));
+    const bool lists = m->trains_ && m->prev.n != 0 && !m->prev.lists_ready;
+    if (lists) m->cur.early_sort_steps = kEarlySortStepsBesideLists;
     enqueue_index(m, 1);
     index_rest_pending = true;
-    if (m->trains_ && m->prev.n != 0 && !m->prev.lists_ready) {
+    if (lists) {
       // The next push_pull will probably push the previous batch, whose gather worked from the keys: its run lists are
       // built now, on the main stream, while the host waits for the ids to be read (built in front of the push they
       // are 4 us of kernel and a launch gap of a 53 k-key step; of 8.5 M keys 12 us).

@@ -835,3 +835,31 @@ def test_preprocess_without_memory_for_its_batch(nrank):
             torch.cuda.empty_cache()
     p.compare_state(1e-5, "end")
     p.close()
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n", [3_000, 140_000, 1_572_865])
+def test_index_cut_behind_the_column_scan(n, wide, monkeypatch):
+    # three-launch passes whose scatters all follow the push, because run lists were built while preprocess waited for the
+    # ids: training steps, a second preprocess and look-ups in between, and batches cut the other way after those
+    say("index cut behind the column scan", n, wide)
+    monkeypatch.setenv("HETUCTR_TILE_SORT", "0")
+    if wide:
+        monkeypatch.setenv("HETUCTR_FORCE_WIDE_KEYS", "1")
+    rng = np.random.default_rng(n)
+    length, width = 40_000, 4
+    p = single(length, width, lr=0.05)
+    draw = zipf_sampler(length, 1.2, rng)
+    prev = 0
+    for step, (batches, train) in enumerate([(1, False), (1, True), (1, True), (2, True), (1, False), (1, True), (1, True)]):
+        for b in range(batches):
+            k = n - 7 * (step + b)
+            p.preprocess([draw(k)], device_keys=True)
+            prev, last = (last if step or b else 0), k
+        g = rng.normal(0, 1e-3, size=(prev, width)).astype(np.float32) if train else None
+        out, ref = p.push_pull([g])
+        assert_close(out[0], ref[0], 1e-5, "dst step %d" % step)
+        p.compare_ints([capi.UNIQUE, capi.SORTED_ARG, capi.RUN_START, capi.OFFSET], "step %d" % step)
+    p.compare_state(1e-5, "end")
+    p.compare_ints([capi.VERSION], "end")
+    p.close()
