@@ -863,3 +863,33 @@ def test_index_cut_behind_the_column_scan(n, wide, monkeypatch):
     p.compare_state(1e-5, "end")
     p.compare_ints([capi.VERSION], "end")
     p.close()
+
+
+@pytest.mark.parametrize("n", [300, 60_000])
+def test_ids_overwritten_where_a_push_follows_the_three_launch_passes(n, monkeypatch):
+    # lists built by the gather, the index in three launches per pass: such a preprocess waits behind the kernel that reads
+    # the ids, and reports a bad one, whatever the size of the batch
+    import torch
+    say("ids overwritten in front of a push", n)
+    monkeypatch.setenv("HETUCTR_TILE_SORT", "0")
+    monkeypatch.setenv("HETUCTR_DIRECT_GATHER_MAX", "0")
+    rng = np.random.default_rng(n)
+    length, width = 9_000, 8
+    p = single(length, width, lr=0.05)
+    side = torch.cuda.Stream()
+    prev = 0
+    for step in range(6):
+        k = n - step
+        p.preprocess([rng.integers(0, length, k)], device_keys=True)
+        with torch.cuda.stream(side):
+            p.keep[0].fill_(7)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(prev, width)).astype(np.float32) if prev else None])
+        assert_close(out[0], ref[0], 1e-5, "dst step %d" % step)
+        prev = k
+    p.compare_state(1e-5, "end")
+    bad = torch.full((n,), 3, dtype=torch.int64, device="cuda")
+    bad[n // 2] = length
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="outside"):
+        p.tables[0].preprocess(bad.data_ptr(), n)
+    p.close()
