@@ -81,14 +81,14 @@ struct TableView {
 //          width from four on, and rows at pointers that are not 16-byte aligned.  The last lane of a row starts at
 //          column W - 4, so it shares up to three columns with the lane before: both read them, and where a row is
 //          updated in place only the lane before writes them,
-//   1      rows of less than four floats, and the few widths in the millions that no slice of the push's long role fits.
+//   1      rows of less than four floats.
 // Against one float per lane (what every width but multiples of four took before), rows of 37 floats, 195 k keys of 39
 // Zipf fields on an MI355X: a training step 148 -> 86 us (the push alone was 103 us of
 // the 148).
 constexpr int kOdd4 = -4;
 template <int VEC> constexpr uint32_t kCols = VEC < 0 ? (uint32_t)-VEC : (uint32_t)VEC;
 inline int row_vec(uint32_t width, const void *p) {
-  return width < 4 ? 1 : (width % 4 == 0 && (uintptr_t)p % 16 == 0) ? 4 : slices_hold_overlap(width) ? kOdd4 : 1;
+  return width < 4 ? 1 : (width % 4 == 0 && (uintptr_t)p % 16 == 0) ? 4 : kOdd4;
 }
 // the column a lane that is due at column c < width really starts at
 template <int VEC> __device__ __forceinline__ uint32_t lane_col(uint32_t c, uint32_t width) {

@@ -741,13 +741,12 @@ inline int lanes_for(uint32_t width, int vec) {
   return lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
 }
 
-// expands F<VEC, LPR>(args...) over the (VEC, LPR) pairs; rows that move one float per lane have less than four or millions
+// expands F<VEC, LPR>(args...) over the (VEC, LPR) pairs; rows that move one float per lane have less than four
 #define HCTR_DISPATCH_ROW(vec, lpr, CALL)         \
   do {                                            \
     if ((vec) == 4) HCTR_DISPATCH_LPR(4, lpr, CALL); \
     else if ((vec) == kOdd4) HCTR_DISPATCH_LPR(kOdd4, lpr, CALL); \
-    else if ((lpr) == 4) CALL(1, 4);              \
-    else CALL(1, 64);                             \
+    else CALL(1, 4);                              \
   } while (0)
 #define HCTR_DISPATCH_LPR(V, lpr, CALL) \
   do {                                  \

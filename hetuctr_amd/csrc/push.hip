@@ -45,15 +45,11 @@ constexpr int kBatch = HCTR_TILE_BATCH;   // short role: gradient rows in flight
 constexpr int kInFlight = 16;             // long role: rows in flight per loader thread
 constexpr int kSlice = kSliceColumns;     // long role: columns per block
 constexpr int kLongBlocks = HCTR_LONG_BLOCKS;
-#ifndef HCTR_GIANT_SLICE
-#define HCTR_GIANT_SLICE 32
-#endif
 #ifndef HCTR_GIANT_CLASSES
 #define HCTR_GIANT_CLASSES 6
 #endif
-constexpr int kGiantSlice = HCTR_GIANT_SLICE;     // long role: the longest runs are cut into slices of this many columns;
-constexpr int kGiantClasses = HCTR_GIANT_CLASSES; // they are the runs of the first length classes (>= 4096)
-static_assert(kSlice % kGiantSlice == 0, "tiers of the long role");
+constexpr int kGiantClasses = HCTR_GIANT_CLASSES; // long role: the runs cut into slices of kGiantSlice columns are those of the
+                                                  // first length classes (>= 4096)
 constexpr int kMedBlocks = HCTR_MED_BLOCKS;
 
 namespace {
@@ -428,8 +424,9 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
 // summed in 290 us.  Bags of 10 ids x 64 floats, Zipf 1.4 (8.5 M keys): two steps 1757 -> 1580 us with what follows here; rows
 // of 37 floats, 195 k keys of 39 Zipf fields: 154 -> 140 us, since such widths take this path too.  More blocks at once do not
 // help (128 / 192 / 256: 1570 / 1584 / 1589 us, and rows of 37 floats 140 / 145 / 169).
-// Generic path (CSC 0; rows of less than four floats, and widths that leave one to three columns over): seven loader waves
-// and one that reads and adds, eight rows at a time, three slots.
+// Generic path (CSC 0; rows of less than four floats): seven loader waves and one that reads and adds, eight rows at a time,
+// three slots.  Widths that leave one to three columns over took it too: two steps of 213 k keys, Zipf 1.4, 65 floats 226
+// us there and 181 here, 129 floats 276 and 258.
 constexpr int kTable = 16;     // runs per bundle at most
 constexpr int kHeldRows = 96;  // rows a lane of a summing wave holds
 constexpr int kSlotsFast = 2, kSlotsGeneric = 3; // LDS slots
@@ -460,10 +457,9 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
   constexpr int kSummers = CSC ? 2 : 1;
   constexpr int kLoaders = kPushBlock - kSummers * kWave;
   const uint32_t W = t.width;
-  uint32_t CS = CSC ? (uint32_t)CSC : min((uint32_t)kSlice, (W + C - 1) / C * C);
-  if (VEC == kOdd4 && !CSC) CS = overlap_slice(W, CS); // row_vec() has made sure that one of them holds the last lane
-  uint32_t lanes = (CS + C - 1) / C; // loader lanes per row slice, rounded up to a power of two
-  lanes = lanes <= 1 ? 1 : lanes <= 2 ? 2 : lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
+  static_assert((CSC == 0) == (VEC == 1), "the generic path is for rows of less than four floats, one slice each");
+  const uint32_t CS = CSC ? (uint32_t)CSC : W;
+  const uint32_t lanes = CSC ? CS / C : W <= 2 ? W : 4; // loader lanes per row slice, a power of two
   const uint32_t RPL = CSC ? (uint32_t)(kLoaders / (CSC / C)) : kLoaders / lanes;
   constexpr int kSliceLanes = CSC ? CSC / (int)C : 1;
   constexpr int kRPT = CSC ? kChunkRows<CSC> / (kLoaders / kSliceLanes) : 2; // rows per loader thread and chunk
@@ -671,7 +667,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
         // this wave's chunks are every other one of the bundle
         constexpr uint32_t kHeld = kHeldRows;
         // where the column lies in a row of the ring: the last lane of a row at any address starts at column W - 4
-        const uint32_t due = mycol / 4 * 4, at = !col_ok ? 0 : place + (VEC == kOdd4 && due + 4 > W ? due + 4 - W : 0);
+        const uint32_t at = !col_ok ? 0 : VEC == kOdd4 ? overlapped_place(place, mycol, W) : place;
         float x[kHeld];
         uint32_t j = 0, c = wave, passed = 0; // chunk c of run j of the bundle is next
         uint32_t rank, L, off;                // of that run
@@ -773,16 +769,6 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
   }
 }
 
-// How many classes of long runs, from the longest on, are cut into slices of kGiantSlice columns, the others being cut into
-// slices of kSlice; negative: the width leaves one to three columns over in either, which no lane of four columns can serve.
-// Slices of kSlice columns are not worth it where the last one would be half empty.
-__device__ __forceinline__ int narrow_classes(uint32_t width) {
-  const uint32_t wide = width % kSlice, narrow = width % kGiantSlice;
-  const bool in_wide = wide == 0 || wide >= 4, in_narrow = narrow == 0 || narrow >= 4;
-  if (in_narrow && wide && wide <= kSlice / 2) return kLongBuckets;
-  return !in_wide ? -1 : in_narrow ? kGiantClasses : 0;
-}
-
 // all roles in one launch: the long chains start first, medium and short blocks fill the machine behind them, the
 // version counters of a single shard come last
 template <int VEC, int LPR, typename K, bool kSingle, bool kPooled>
@@ -791,7 +777,7 @@ __device__ __forceinline__ void push_block(const TableView &t, int id_bits, cons
   // one LDS area for whichever role the block plays: the row ring of the long role or the index staging of the
   // medium role (one slice of kLongRun indices per group)
   constexpr int kRingWords = VEC == 1 ? kSlotsGeneric * 2 * kPushBlock
-                                      : std::max({ring_floats(64), ring_floats(32), ring_floats(16), kSlotsGeneric * 2 * kPushBlock * 4});
+                                      : std::max({ring_floats(64), ring_floats(32), ring_floats(16)});
   constexpr int kStageWords = (kPushBlock / LPR) * (int)kLongRun;
   __shared__ __align__(16) float lds[kRingWords > kStageWords ? kRingWords : kStageWords];
   __shared__ uint4 run_table[2 * kTable];
@@ -807,19 +793,14 @@ __device__ __forceinline__ void push_block(const TableView &t, int id_bits, cons
       long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, sums_at_hand, c_lo, c_hi, block,
                                                        kLongBlocks, counters);
     };
-    constexpr int kOneSlice = VEC != 1 && LPR <= 8 ? LPR * 4 : 0, kNarrow = VEC != 1 && LPR > 8 ? kGiantSlice : 0;
-    if constexpr (kOneSlice != 0) { // rows of up to 16 or 32 floats
-      runs(std::integral_constant<int, kOneSlice>(), 0, kLongBuckets, tk);
-    } else if constexpr (kNarrow != 0) {
-      const int narrow = narrow_classes(t.width);
-      if (narrow >= 0) {
-        if (narrow > 0) runs(std::integral_constant<int, kNarrow>(), 0, narrow, tk);
-        if (narrow < kLongBuckets) runs(std::integral_constant<int, kSlice>(), narrow, kLongBuckets, tk + kTicketLanes);
-      } else {
-        runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);
-      }
-    } else {
+    if constexpr (VEC == 1) {
       runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);
+    } else if constexpr (LPR <= 8) { // rows of up to 16 or 32 floats
+      runs(std::integral_constant<int, LPR * 4>(), 0, kLongBuckets, tk);
+    } else {
+      const int narrow = narrow_slices(t.width) ? kLongBuckets : kGiantClasses;
+      runs(std::integral_constant<int, kGiantSlice>(), 0, narrow, tk);
+      if (narrow < kLongBuckets) runs(std::integral_constant<int, kSlice>(), narrow, kLongBuckets, tk + kTicketLanes);
     }
   } else if (block < kLongBlocks + kMedBlocks) { // medium runs take long per block: they start early
     medium_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, (uint32_t *)lds, block - kLongBlocks, kMedBlocks);
@@ -909,9 +890,8 @@ void launch_push_t(hipStream_t st, int id_bits, PushShards &shards, int count) {
 
 template <int VEC, typename K, bool kPooled>
 void launch_push_p(hipStream_t st, int id_bits, PushShards &shards, int count) {
-  if constexpr (VEC == 1) { // rows of less than four floats, or of millions (row_vec)
-    if (shards.s[0].t.width < 4) launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
-    else launch_push_t<VEC, 64, K, kPooled>(st, id_bits, shards, count);
+  if constexpr (VEC == 1) { // rows of less than four floats
+    launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);
   } else {
     const uint32_t lanes = (shards.s[0].t.width + kCols<VEC> - 1) / kCols<VEC>;
     if (lanes <= 4) launch_push_t<VEC, 4, K, kPooled>(st, id_bits, shards, count);

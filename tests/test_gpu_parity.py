@@ -759,7 +759,7 @@ def test_preprocess_again_while_the_run_lists_are_built(n):
 @pytest.mark.parametrize("width", [12, 16, 21, 32, 37, 64, 66, 80, 97, 128])
 def test_run_lengths_around_the_chunks_of_the_push(width, nrank):
     # runs that end just before, at and behind the chunks of 96 and 192 rows, their halves and groups of four, in slices of 16,
-    # 32 and 64 columns, whole and partly filled, and (width 66) in the generic layout; sums bit for bit
+    # 32 and 64 columns, whole and partly filled (width 66: two columns in the last one); sums bit for bit
     say("runs around chunks", width, nrank)
     rng = np.random.default_rng(13)
     lens = [129, 130, 131, 159, 160, 189, 191, 192, 193, 194, 195, 196, 203, 287, 288, 289, 290, 383, 384, 385, 387, 575, 576,
