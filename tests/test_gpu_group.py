@@ -406,3 +406,34 @@ def test_pushes_of_unequal_length_to_one_owner(sizes):
         p.compare_ints(INT_ITEMS_POST, "step %d" % step)
         prev = list(sizes)
     p.close()
+
+
+@pytest.mark.parametrize("large", [0, 1])
+def test_one_shard_reads_its_ids_by_word_and_the_other_by_event(large):
+    # 2^21 + 1 keys are one block too many for the word that says the ids are read, so the call waits for one shard by an
+    # event and for the other by the word; either may hold a bad id, and both buffers are the caller's when the call returns
+    say("ids read by word and by event, large batch at", large)
+    rng = np.random.default_rng(11)
+    length, width, ns = 5_000, 1, [700, 700]
+    ns[large] = (1 << 21) + 1
+    root = rng.integers(0, 2, size=length).astype(np.uint8)
+    p = Pair(2, length, width, root, [np.flatnonzero(root == r).astype(np.int64) for r in range(2)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    side = torch.cuda.Stream()
+    bad = [None, large, None, 1 - large, None]
+    for step, where in enumerate(bad):
+        if where is not None:
+            ids = [torch.full((n,), 3, dtype=torch.int64, device="cuda") for n in ns]
+            ids[where][-1] = length
+            torch.cuda.synchronize()
+            with pytest.raises(RuntimeError, match="outside"):
+                capi.group_preprocess(p.tables, [d.data_ptr() for d in ids], ns)
+            continue
+        p.preprocess([rng.integers(0, length, n) for n in ns], device_keys=True)
+        with torch.cuda.stream(side):
+            for d in p.keep:
+                d.fill_(7)
+        out, ref = p.push_pull([None, None])
+        for r in range(2):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+    p.close()
