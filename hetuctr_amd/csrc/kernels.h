@@ -144,6 +144,10 @@ void launch_one_or_records(int count, uint32_t threads, Make &&make, Blocks &&bl
 // zero and stores seq << 1 | (an id was out of range) in *word, which lies in pinned memory and is polled.  A launch and
 // the wait for it then take 8.3 us for 52 blocks of a batch and 9.7 for 191, where an event behind the kernel takes 11.8;
 // the count is one atomic per block, served one after the other, and eats that up between 256 and 416 blocks.
+// There is no release in this: what makes the keys visible is what gfx950 does with the instructions, not the memory model.  A
+// store at agent scope (sc1) writes through the XCD's cache, s_waitcnt vmcnt(0) returns when such stores are done, the barrier
+// orders every wave's wait before the count, and the kernel that reads the keys begins with an acquire of its own launch.  A
+// release would write back the whole cache of the XCD once per block.  A port to another chip has to put one there.
 constexpr uint32_t kReadSignalBlocks = 256;
 struct ReadSignal {
   uint32_t *count = nullptr, *word = nullptr; // word == nullptr: nobody polls

@@ -21,7 +21,7 @@ constexpr int kTile = kBlock * kItems; // 2048: scan_blocks(n) sizes the scratch
 // ids -> sort keys (owner << id_bits | id; they are the batch's copy of the ids as well), the range check, the reset
 // of the batch's run counters, and the per-tile counts of the first sort pass' digit: a block works on one sort tile, so the sort
 // needs no counting launch of its own for that pass.  This is the one kernel that reads the caller's buffer: the
-// call may return when it is through.
+// call may return when it has said that it has them all (ReadSignal), or is through.
 template <typename K, int ITEMS, int M> // M: records of the launch
 __global__ __launch_bounds__(kSortBlock) void make_keys(Records<KeyShard, M> shards, int id_bits, int dbits) {
   uint32_t tile, tiles;

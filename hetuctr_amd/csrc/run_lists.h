@@ -1,7 +1,7 @@
 // The run lists of a batch for the push that sums its gradients one step later: runs longer than kLongRun by length
 // class, runs of medium length in one list (the lists' layout is with BatchView in kernels.h).  They are built after the
 // unique pass by whichever kernel comes next anyway -- the gather of the step, whose first blocks take a chunk of unique
-// ranks each before their own work -- or by a launch of their own where no gather follows.
+// ranks each before their own work -- or by a launch of their own where no gather follows or the gather works from the keys (Shard::list_runs).
 #pragma once
 #include "kernels.h"
 

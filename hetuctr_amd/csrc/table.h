@@ -62,11 +62,10 @@ struct Batch {
   bool tile_sorted = false; // indexed by the tile-sorted passes (tile_sort.h)
   bool one_block = false;   // indexed by one block in one launch (tile_sort.h)
   bool direct_gather = false; // one shard, small batch: the step's gather works from `comp` in batch order and does not
-                              // wait for the index (the run lists are then built in front of the batch's push)
-  bool comp_valid = false;    // comp holds the batch's sort keys in batch order
-  bool keys_made = false;   // comp holds the batch's sort keys (a kernel of its own made them); else the first launch
-                            // of the tile-sorted passes read the ids itself and no copy in batch order exists: the ids
-                            // of the batch are read back through the index when somebody asks for them
+                              // wait for the index (the run lists are then built while the next preprocess waits for
+                              // its ids, or in front of the batch's push)
+  bool keys_made = false;   // the ids are read by a kernel that makes the sort keys alone; else by the first launch of the
+                            // tile-sorted passes.  Either leaves the sort keys in comp
   // comp: the batch's sort keys in batch order (id and owner of every position); staged: ids that arrived in
   // pageable host memory, on their way to the key kernel
   DeviceBuf comp, staged, sorted_arg, rank_sorted, idx_map, ukey, run_start, uoff, bucket_lo, dU, long_list, dnlong, med_list;

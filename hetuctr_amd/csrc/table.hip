@@ -87,7 +87,7 @@ void Batch::clear(hipStream_t s, int nrank) {
 
 void Batch::drop() {
   n = U = 0;
-  idx_map_valid = planned = tile_sorted = one_block = direct_gather = comp_valid = keys_made = cleared = false;
+  idx_map_valid = planned = tile_sorted = one_block = direct_gather = keys_made = cleared = false;
   lists_ready = true;
   for (auto *c : {&send_cnt, &recv_cnt, &push_cnt, &pushrecv_cnt}) std::fill(c->begin(), c->end(), 0);
 }
@@ -280,7 +280,6 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
   cur.planned = false;
   cur.lists_ready = n == 0;
   cur.direct_gather = false;
-  cur.comp_valid = false;
   cur.one_block = cur.tile_sorted = false;
   cur.early_sort_steps = kEarlySortSteps;
   ids_ = nullptr;
@@ -326,7 +325,6 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
       cur.direct_gather = cfg.nrank == 1 && flag != nullptr && cur.n <= direct_gather_max;
       cur.one_block = tile_sort_mode == 1 && cur.n <= kOneBlockKeys && kl.max_digit_bits == 0;
       cur.keys_made = !cur.tile_sorted || cur.one_block;
-      cur.comp_valid = true; // either kernel leaves the sort keys in batch order (a gather from the keys reads them)
       ids_ = ids;
       narrowed_ = narrowed;
       // Not in front of the three-launch passes if the push follows at once, its run lists having been built by a gather:
@@ -480,8 +478,8 @@ void Group::index_batches(Shard *const *shards, size_t count, uint32_t *u_out, i
     if (part == 1) return;
     StageScope st(*this, S_UNIQUE);
     launch_unique(s, kl, unique, m, !f.cur.tile_sorted);
-    // the run lists follow in the gather of the step, or before the batch's push if that gather did not look at the
-    // index or never came (lists_ready)
+    // the run lists follow in the gather of the step; if that gather did not look at the index or never came (lists_ready),
+    // while the next preprocess waits for its ids, or before the batch's push
     // (built behind the index instead, they make the index the longer of a small step's two chains: 78 us against 64)
   });
 }
@@ -682,7 +680,7 @@ void Shard::finish_handle_query() {
 // whether this step's gather works from the keys in batch order (and the step does not wait for the index)
 // (bags: a pooled gather walks the batch in its own order anyway, so it always works from the keys when they are there)
 bool Shard::direct_now(uint32_t bag) const {
-  if (cfg.nrank != 1 || !cur.comp_valid || cur.n == 0) return false;
+  if (cfg.nrank != 1 || cur.n == 0) return false;
   return bag == 1 ? cur.direct_gather : pooled_from_keys;
 }
 
@@ -837,11 +835,7 @@ size_t Shard::fetch(int which, void *out, size_t cap) {
     case HCTR_F_STORE_IDS: return put64(download<index_t>(store_ids.p, tv.n_stored), tv.n_stored, out, cap);
     case HCTR_F_KEYS: { // the ids of the batch as its sort keys hold them (an id outside the table reads as 0)
       std::vector<uint64_t> k(cur.n);
-      if (!cur.comp_valid) { // no copy in batch order was kept: position sorted_arg[j] holds the key of rank_sorted[j]
-        const auto uk = ukeys(cur);
-        const auto pos = download<uint32_t>(cur.sorted_arg.p, cur.n), rk = download<uint32_t>(cur.rank_sorted.p, cur.n);
-        for (size_t j = 0; j < cur.n; j++) k[pos[j]] = uk[rk[j]] & id_mask;
-      } else if (kl.wide) {
+      if (kl.wide) {
         auto h = download<uint64_t>(cur.comp.p, cur.n);
         for (size_t i = 0; i < cur.n; i++) k[i] = h[i] & id_mask;
       } else {
@@ -1282,7 +1276,7 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
   }
   if (defer_index && !stage_timing) {
     // Several shards: as with one, the ids are read by a kernel on the second stream and the call returns when that
-    // kernel is through; the index of the current batches follows on that stream (no event between the two streams:
+    // kernel has read them; the index of the current batches follows on that stream (no event between the two streams:
     // waiting for one costs the host 15-20 us), next to the pushes that the next push_pull queues first.  push_pull
     // waits for the index before it builds the queries, which are the first thing that needs it.  The push plan of the
     // previous batches was made at the end of the step before.

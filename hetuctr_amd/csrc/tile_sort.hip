@@ -153,7 +153,7 @@ __device__ __forceinline__ void store_sorted_tile(const uint32_t *area, const ui
 
 // Launch 0: ids -> sort keys (owner << id_bits | id), the range check, the reset of the batch's run counters, and the
 // tile sorted by the first digit.  This is the one kernel that reads the caller's buffer: the call may return when it
-// is through.  (csrc/core/preprocess.cu:11-20 builds the reference's sort key.)
+// has said that it has them all (ReadSignal), or is through.  (csrc/core/preprocess.cu:11-20 builds the reference's sort key.)
 struct KeysJob {
   const index_t *ids;
   uint32_t n, pitch;
@@ -212,8 +212,8 @@ __global__ __launch_bounds__(kSortBlock) void keys_tile_sort(Records<KeysJob, M>
   for (int r = 0; r < ITEMS; r++) {
     key[r] = (K)((owner[r] << id_bits) | id[r]);
     val[r] = tile_lo + w * S::kSub + r * kWave + lane;
-    // the sort keys in batch order as well, for a caller that works on the batch before it is sorted (optional)
-    if (keys_out && w * S::kSub + r * kWave + lane < tile_n) store_key(keys_out + val[r], key[r], J.read);
+    // the sort keys in batch order as well, for whoever works on the batch before it is sorted
+    if (w * S::kSub + r * kWave + lane < tile_n) store_key(keys_out + val[r], key[r], J.read);
   }
   tell_ids_read(J.read, tile_blocks, bad, err); // the caller need not wait for the sort
   tile_sort_by_digit<K, ITEMS, DBITS>(key, val, tile_n, 0, dbits, area, bin_start, sm);
