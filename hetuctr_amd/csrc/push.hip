@@ -439,6 +439,11 @@ __device__ __forceinline__ float from_lower_half(float x) {
   return __uint_as_float(__builtin_amdgcn_permlane32_swap(v, v, false, false)[0]);
 }
 
+// This wave's LDS operations are done.  A barrier waits for them by itself, but where it is the first thing in a loop the compiler
+// of ROCm 7.2 drops that wait, having seen nothing outstanding in front of the loop: what comes around the loop is
+// outstanding.  (tests/test_kernel_resources.py looks for such barriers in every kernel.)
+__device__ __forceinline__ void lds_done() { __builtin_amdgcn_s_waitcnt(0xc07f); } // lgkmcnt(0), nothing else
+
 // a value that is the same in every lane, moved to a scalar register
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
@@ -686,6 +691,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
         settle();
         if (wave) __syncthreads(), passed++;
         for (uint32_t g = wave; g < G; g += 2) {
+          lds_done();      // the sum in `hand`: without the wait the other wave now and then took the sum of two chunks before
           __syncthreads(); // chunk g is in the ring
           const uint32_t rows = min(CR, L - c * CR);
           const float *sp = lds + (g % slots) * slot_floats + at;
