@@ -331,8 +331,9 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
       // returning later it finds the first scatter nearly done instead of on the CUs of its long runs (as beside
       // kEarlySortStepsBesideLists).  Two steps with the word and without: rows of 64 floats, Zipf 1.4, 1.58 M keys 599 and
       // 547 us, 1.7 M 637 and 569, of exponent 1.05 599 and 591 (no difference); where lists are built in between the
-      // word is the faster: pooled, 64 floats, 1.6 M keys 385 and 402.
-      const bool push_at_once = !cur.tile_sorted && !cur.one_block && trains_ && prev.n != 0 && prev.lists_ready;
+      // word is the faster: pooled, 64 floats, 1.6 M keys 385 and 402.  Ids from pageable memory, which arrive in front of the
+      // key kernel: 1.7 M keys, Zipf 1.4, with the word 984 and without 1024.
+      const bool push_at_once = visible && !cur.tile_sorted && !cur.one_block && trains_ && prev.n != 0 && prev.lists_ready;
       if (flag != nullptr && !push_at_once && (cur.keys_made ? sort_tiles(n) : tile_count(n)) <= kReadSignalBlocks) {
         read_.count = &dst_->read_count;
         read_.word = &mirror->ids_read;
