@@ -323,8 +323,9 @@ __global__ __launch_bounds__(kBlock) void scan_positions(const OwnerShard *__res
 
 // What comes back per unique key of the step, in two roles over tiles of kRTile keys.  They need the owners' flags only, so they
 // share the launches of place_returns and pack_rows, the flags and offsets being requested before the number of unique keys is
-// here.  (In launches of their own behind pack_rows they took 14 us and two gaps of a step of four shards of 53 k keys; two
-// steps 355 -> 337 us.)
+// here.  (In launches of their own behind pack_rows they took 14 us and two gaps of a step of four shards of 53 k keys.  Beside the
+// owners' work remote_emit still takes what it took -- with 1.7 M keys the two launches 44 + 14 us, the one 60 -- so the gaps
+// are what is gained: two steps 355 -> 337 us in one pair, 364 -> 347 in another, where runs differ by up to 10 %.)
 //  count_returned  returned rows per tile, and the counts of the step: keys cached and fresh enough, not stored here, cached
 //                  and refreshed; and whether an owned row came back as outdated (it never may)
 //  remote_emit     ret_i[u] = index of u's row among the returned rows (exclusive scan of the flags; a tile adds up the

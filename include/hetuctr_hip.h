@@ -59,7 +59,9 @@ int hctr_destroy(hctr_table *t);
  * next (hctr_push_pull, a second hctr_preprocess, hctr_debug_fetch).  This is the one deviation from the reference,
  * whose call returns when all of its work is done (hetu_gpu_table.cu:64): hctr_defer_index(t, 0), or
  * HETUCTR_DEFER_INDEX=0 in the environment, restores exactly that.  The details of the early return are with
- * hctr_defer_index below.  With nrank > 1 the call completes when every shard of the group has made it. */
+ * hctr_defer_index below.  With nrank > 1 the call completes when every shard of the group has made it.
+ * A call refused for its arguments leaves every batch as it was.  After one that fails on the way (no memory for the batch, say)
+ * the batch that was current is current again, and none lies before it; a bad key is an error of a batch that is there. */
 int hctr_preprocess(hctr_table *t, const int64_t *keys, size_t n);
 
 /* hctr_preprocess for callers that cannot allocate device memory (tight serving loops, harnesses that forbid
