@@ -16,9 +16,9 @@
 // One launch, three ranges of blocks, one per class of run length (the long chains are dispatched first and the
 // other blocks fill the machine behind them):
 //  * long (> kLongRun duplicates): bundles of runs are streamed by whole blocks, one column slice at a time.  Six
-//    loader waves keep 16 vectors of gradient rows in flight per lane and stage them through two LDS slots; two waves
-//    take turns at adding the staged rows in order, one column per lane, each reading its rows from LDS into registers
-//    while the other one adds.  The serial chain costs one add per duplicate.
+//    loader waves keep 16 vectors of gradient rows in flight per lane and stage them through two LDS slots; one wave
+//    adds the staged rows in order, one column per lane, and one draws the work and applies the sums.  The serial chain
+//    costs one add per duplicate.
 //    The longest runs are started first and cut into narrower slices, i.e. fed by more blocks.
 //  * medium (kTinyRun < duplicates <= kLongRun): one group of LPR lanes per run, kBatch rows in flight.
 //  * short (<= kTinyRun): a group of LPR lanes (LPR*VEC floats = one row) owns a few consecutive unique keys
@@ -46,10 +46,13 @@ constexpr int kInFlight = 16;             // long role: rows in flight per loade
 constexpr int kSlice = kSliceColumns;     // long role: columns per block
 constexpr int kLongBlocks = HCTR_LONG_BLOCKS;
 #ifndef HCTR_GIANT_CLASSES
-#define HCTR_GIANT_CLASSES 6
+#define HCTR_GIANT_CLASSES 4
 #endif
-constexpr int kGiantClasses = HCTR_GIANT_CLASSES; // long role: the runs cut into slices of kGiantSlice columns are those of the
-                                                  // first length classes (>= 4096)
+// Long role: the runs cut into slices of kGiantSlice columns are those of the first length classes (>= 16384).  Such a slice costs a
+// block 3.4 ns per row, one of 64 columns 6: only of the longest runs does the chain matter more than the work.  (From 4096 on,
+// the long runs of 8.5 M pooled keys, Zipf 1.4, were done after 451 us instead of 435; from 32768 or 65536 on 434 and 428, but runs
+// of 8 k rows of a batch of 1.7 M keys then took as long as its longest.)
+constexpr int kGiantClasses = HCTR_GIANT_CLASSES;
 constexpr int kMedBlocks = HCTR_MED_BLOCKS;
 
 namespace {
@@ -409,34 +412,46 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
 // A block works on ONE column slice (CS columns) of a bundle of long runs at a time and treats the bundle as one
 // stream of chunks, so that the loads of the next run are in flight while the current one is summed.  Runs are
 // listed by length class, longest first; a bundle is 1..kTable runs of one class holding at least ~2048
-// occurrences.  Tickets (bundle, slice) are handed out through one counter per group of blocks that share slices;
-// the first wave draws the next ticket and fetches its run descriptors while the loaders of the current bundle wait
-// for their first rows, so a change of bundle costs only the refill of the load pipeline.
-// Fast path (slices of 16, 32 or 64 columns, CSC).  Two waves sum; the other six ("loaders") only move gradient rows global ->
-// registers -> LDS.  A row slice is read by CSC / 4 loader lanes, a chunk is 96 rows, or 192 where a slice has at most 32
-// columns and the two halves of a wave hold 96 rows each (chunks never span two runs).  Everyone meets at one barrier per
-// chunk: while chunk g - 1 is added by the wave that has it in registers, the other wave reads chunk g from its slot and the
-// loaders fill the other slot with chunk g + 1; the sums pass from wave to wave in LDS.  What bounds it: the chain of adds, 4.6
-// cycles per row (a lone wave's dependent v_add_f32), and per chunk a barrier, the hand-over and the change of halves, about
-// 400 cycles; with every block of a batch at it, the rows coming out of the last-level cache.  One wave that reads and
-// adds by turns spends 4 cycles per row on each.  Why rows lie in a slot as they come: written column by column, in 4-byte pieces, they
-// took the LDS longer than the adds (a chunk of 192 rows 1600 cycles with the adds left out).  A chain of 106 k rows is
-// summed in 290 us.  Bags of 10 ids x 64 floats, Zipf 1.4 (8.5 M keys): two steps 1757 -> 1580 us with what follows here; rows
-// of 37 floats, 195 k keys of 39 Zipf fields: 154 -> 140 us, since such widths take this path too.  More blocks at once do not
-// help (128 / 192 / 256: 1570 / 1584 / 1589 us, and rows of 37 floats 140 / 145 / 169).
+// occurrences.  Tickets (bundle, slice) are handed out through one counter per group of blocks that share slices.
+//
+// Fast path (slices of 16, 32 or 64 columns, CSC).  One wave sums, one draws the tickets and applies the sums, the other six
+// ("loaders") move gradient rows global -> registers -> LDS.
+//  * The lanes of the summing wave are kSets sets of one lane per column of the slice, and a chunk is 96 rows for each set.  The
+//    wave reads a chunk in two halves of 12 x 16 bytes per lane, four rows of the lane's column at a time, and adds one half
+//    while the next one is on its way.  A sum never leaves its wave (it goes from set to set by a swap of lanes).
+//  * For that, four neighbouring rows of a column lie side by side in LDS.  A loader lane has just these rows (four columns of
+//    four neighbouring rows of the chunk) in its registers and stores one column of them at a time; where a column lies in a
+//    group of rows (column_slot) makes both sides touch every bank equally often.
+//  * The waves never meet at a barrier.  Loaders count the parts of a chunk they have written, the summing wave the chunks it has
+//    read, and whoever needs a slot full or empty looks at the count.
+//  * The rows the sums are added to (with several shards also the plan's words and the pending rows) are requested by the wave that
+//    draws, when a bundle begins, and are there when its sums arrive.  It draws the next ticket kDrawAhead chunks before a bundle
+//    ends: drawn at its beginning, tickets lay with the blocks that had the longest runs while others ran out of work.
+// What bounds it: the chain.  Adds alone take 4.3 cycles per row, the 24 reads of a chunk of 192 rows 6 to 12 cycles each, the
+// counts about 150 per chunk; 7.4 cycles per row in all at 2.3 GHz, 2.5 more where the rows come from HBM and not from the
+// last-level cache.  Two waves that took turns at reading and adding, with a barrier per chunk, took 7.6 and 9.9; what is gained
+// beyond the chain is the end of the launch, where blocks now finish together.  The push of 8.5 M keys of 64 floats, Zipf 1.4:
+// pooled by tens 480 -> 425 us, plain 624 -> 565; of 1.7 M keys of 128 floats 247 -> 240.  Steps of those batches 3 to 7 %
+// shorter, of 195 k keys of 37 floats 5 %.  Measured without gain: one read between every few adds (14 cycles each), a raised
+// priority for the summing wave, 20 instead of 16 vectors in flight, 192 blocks, barriers instead of counts.
 // Generic path (CSC 0; rows of less than four floats): seven loader waves and one that reads and adds, eight rows at a time,
-// three slots.  Widths that leave one to three columns over took it too: two steps of 213 k keys, Zipf 1.4, 65 floats 226
-// us there and 181 here, 129 floats 276 and 258.
-constexpr int kTable = 16;     // runs per bundle at most
-constexpr int kHeldRows = 96;  // rows a lane of a summing wave holds
+// three slots.
+constexpr int kTable = 16;      // runs per bundle at most
+constexpr int kHalfGroups = 12; // groups of four rows a lane of the summing wave holds of half a chunk
+constexpr int kSlotVectors = 2 * kHalfGroups * kWave; // 16-byte vectors of a slot of the ring: a chunk, whatever the slice
 constexpr int kSlotsFast = 2, kSlotsGeneric = 3; // LDS slots
-template <int CSC> constexpr int kRowSets = CSC == kWave ? 1 : 2;         // sets of rows in the lanes of a summing wave
-template <int CSC> constexpr int kChunkRows = kHeldRows * kRowSets<CSC>; // rows per chunk of the fast path
-constexpr int ring_floats(int cs) { return kSlotsFast * cs * (cs == kWave ? kHeldRows : 2 * kHeldRows + 1); }
-// the value of lane i in lane i + 32
-__device__ __forceinline__ float from_lower_half(float x) {
+constexpr uint32_t kDrawAhead = 16; // chunks before the end of a bundle at which the next ticket is drawn
+// the value of the lanes 16 / 32 below (up) or above (!up), for the lanes of the other half of a pair of halves
+template <int D, bool up> __device__ __forceinline__ float from_half(float x) {
   const uint32_t v = __float_as_uint(x);
-  return __uint_as_float(__builtin_amdgcn_permlane32_swap(v, v, false, false)[0]);
+  if constexpr (D == 32) return __uint_as_float(__builtin_amdgcn_permlane32_swap(v, v, false, false)[up ? 0 : 1]);
+  else return __uint_as_float(__builtin_amdgcn_permlane16_swap(v, v, false, false)[up ? 0 : 1]);
+}
+// The sets of a summing wave in the order in which they hold the rows of the first half of a chunk; the second half goes back.
+// Neighbours differ in one bit, so that a swap of halves of the wave moves a sum on.
+__host__ __device__ constexpr uint32_t set_at(uint32_t t, bool second, int sets) {
+  const uint32_t k = second ? sets - 1 - t : t;
+  return k ^ (k >> 1);
 }
 
 // This wave's LDS operations are done.  A barrier waits for them by itself, but where it is the first thing in a loop the compiler
@@ -444,8 +459,31 @@ __device__ __forceinline__ float from_lower_half(float x) {
 // outstanding.  (tests/test_kernel_resources.py looks for such barriers in every kernel.)
 __device__ __forceinline__ void lds_done() { __builtin_amdgcn_s_waitcnt(0xc07f); } // lgkmcnt(0), nothing else
 
+// the value of lane Q of the quad
+template <int Q> __device__ __forceinline__ uint64_t of_quad(uint64_t v) {
+  constexpr int kPerm = Q * 0x55;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, kPerm, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), kPerm, 0xf, 0xf, true);
+  return (uint64_t)hi << 32 | lo;
+}
 // a value that is the same in every lane, moved to a scalar register
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// Counts in LDS that the waves of a block poll instead of meeting at a barrier.  What a count stands for is done when it moves
+// (the caller waits for its LDS operations first), and what follows it is not begun before it is seen.
+__device__ __forceinline__ uint32_t peek(const uint32_t *count) { return __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+__device__ __forceinline__ void wait_until(const uint32_t *count, uint32_t at_least) {
+  while ((int)(uni(peek(count)) - at_least) < 0) __builtin_amdgcn_s_sleep(1);
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void tell(uint32_t *count, uint32_t value) {
+  asm volatile("" ::: "memory");
+  if (threadIdx.x % kWave == 0) __hip_atomic_store(count, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void tell_add(uint32_t *count) {
+  asm volatile("" ::: "memory");
+  if (threadIdx.x % kWave == 0) (void)__hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 // runs per bundle: classes halve in length -- one run of 2048 or more, 2 of 1024.., 4, 8, 16; `shrink` halves that
 // (down to single runs) for batches with few long runs
@@ -455,31 +493,25 @@ __device__ __forceinline__ uint32_t bundle_runs(int cls, uint32_t shrink) {
 
 template <int VEC, typename K, int CSC, bool kPooled> // CSC: columns per slice if known at compile time, else 0
 __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
-                                          float *lds, uint4 *tables, uint32_t *shared, float *row_stash, float *hand, int c_lo,
+                                          float *lds, uint4 *tables, uint32_t *shared, float *sums, int c_lo,
                                           int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
   typedef typename Vec<VEC>::T V;
   constexpr uint32_t C = kCols<VEC>;
-  constexpr int kSummers = CSC ? 2 : 1;
-  constexpr int kLoaders = kPushBlock - kSummers * kWave;
+  constexpr uint32_t kOthers = CSC ? 2 : 1; // waves that do not load
+  constexpr int kLoaders = kPushBlock - kOthers * kWave;
   const uint32_t W = t.width;
   static_assert((CSC == 0) == (VEC == 1), "the generic path is for rows of less than four floats, one slice each");
   const uint32_t CS = CSC ? (uint32_t)CSC : W;
   const uint32_t lanes = CSC ? CS / C : W <= 2 ? W : 4; // loader lanes per row slice, a power of two
-  const uint32_t RPL = CSC ? (uint32_t)(kLoaders / (CSC / C)) : kLoaders / lanes;
-  constexpr int kSliceLanes = CSC ? CSC / (int)C : 1;
-  constexpr int kRPT = CSC ? kChunkRows<CSC> / (kLoaders / kSliceLanes) : 2; // rows per loader thread and chunk
-  constexpr int kDepth = kInFlight / kRPT;  // chunks in flight per loader thread
-  const uint32_t CR = RPL * kRPT;             // rows per chunk
-  static_assert(!CSC || kChunkRows<CSC> == kRPT * (kLoaders / kSliceLanes), "a chunk of the fast path is whole loads");
+  constexpr int kSets = CSC ? kWave / CSC : 1;
+  constexpr int kRPT = CSC ? 4 : 2;        // rows per loader thread and chunk
+  constexpr int kDepth = kInFlight / kRPT; // chunks in flight per loader thread
+  const uint32_t CR = kLoaders / lanes * kRPT; // rows per chunk
+  constexpr uint32_t kHalfRows = 4 * kHalfGroups * kSets;
+  static_assert(!CSC || 2 * kHalfRows == kLoaders / (CSC / C) * kRPT, "a chunk of the fast path is whole loads");
   const uint32_t slices = (W + CS - 1) / CS;
-  // A ring slot holds the rows of a chunk one after the other.  On the fast path the second set of rows lies one row further:
-  // the lanes that read it use the other half of the banks.
-  constexpr uint32_t kPad = CSC && kRowSets<CSC> > 1 ? 1 : 0;
-  const uint32_t slot_floats = (CR + kPad) * CS;
-  constexpr uint32_t slots = CSC ? kSlotsFast : kSlotsGeneric;
   const float neg_lr = t.neg_lr;
   const uint32_t wave = uni(threadIdx.x / kWave);
-  const bool summer = wave < (uint32_t)kSummers, lead = wave == 0; // the lead also draws the tickets
   const uint32_t *__restrict__ sorted_arg = p.sorted_arg;
 
   // tickets of this block's group: (bundle, slice) with the bundle changing slowest, so the longest runs go first
@@ -504,19 +536,20 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
   if (!nbundles) return;
   const uint32_t tickets = nbundles * n_sl;
 
-  // the lead wave draws a ticket and leaves its bundle in set `to`: descriptors of the runs (one lane per run), number of
-  // runs, chunks and the slice
-  auto draw = [&](uint32_t to) {
+  // one wave draws a ticket and leaves its bundle in set `to`: descriptors of the runs (one lane per run, which keeps its own
+  // in `mine`), number of runs, chunks and the slice
+  auto draw = [&](uint32_t to, uint4 &mine) {
+    const uint32_t lane = threadIdx.x % kWave;
     uint32_t tk = 0;
-    if (threadIdx.x == 0) tk = atomicAdd(counters + lane_id, 1u);
+    if (lane == 0) tk = atomicAdd(counters + lane_id, 1u);
     tk = (uint32_t)__builtin_amdgcn_readfirstlane((int)tk);
     if (tk >= tickets) {
       // Every block of the group draws exactly one ticket past the end.  The block that draws the last of them
       // knows that nobody will touch the counter again in this launch and puts it back to zero, so that the same
       // batch can be pushed again (push_pull twice without a preprocess in between applies the gradient twice,
       // csrc/core/hetu_gpu_table.cu:9-41).
-      if (threadIdx.x == 0 && tk == tickets + group_blocks - 1) atomicExch(counters + lane_id, 0u);
-      if (threadIdx.x == 0) shared[to * 4] = 0;
+      if (lane == 0 && tk == tickets + group_blocks - 1) atomicExch(counters + lane_id, 0u);
+      if (lane == 0) shared[to * 4] = 0;
       return;
     }
     uint32_t bundle = tk / n_sl;
@@ -538,222 +571,481 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
       }
     }
     uint32_t chunks = 0;
-    if (threadIdx.x < runs) {
-      const uint4 m = p.long_list[(size_t)cls * p.long_cap + run0 + threadIdx.x]; // rank, first position, length, offset
-      chunks = (m.z + CR - 1) / CR;
-      tables[to * kTable + threadIdx.x] = m;
+    if (lane < runs) {
+      mine = p.long_list[(size_t)cls * p.long_cap + run0 + lane]; // rank, first position, length, offset
+      chunks = (mine.z + CR - 1) / CR;
+      tables[to * kTable + lane] = mine;
     }
 #pragma unroll
     for (int d = kTable / 2; d; d >>= 1) chunks += __shfl_down(chunks, d);
-    if (threadIdx.x == 0) {
+    if (lane == 0) {
       shared[to * 4] = runs;
       shared[to * 4 + 1] = chunks;
       shared[to * 4 + 2] = lane_id + (tk % n_sl) * share;
     }
   };
 
-  __syncthreads(); // of the runs before these
-  if (lead) draw(0);
-  __syncthreads();
-  for (uint32_t cur = 0;; cur ^= 1) {
-    const uint4 *table = tables + cur * kTable;
-    const uint32_t J = uni(shared[cur * 4]), G = uni(shared[cur * 4 + 1]), slice = uni(shared[cur * 4 + 2]); // runs, chunks and slice of this bundle
-    if (!J) break;
-    if (lead) draw(cur ^ 1); // while the loaders wait for the first rows of this bundle
+  // Whole rounds run without a condition inside: with one, the compiler must assume that loads may have been
+  // skipped and waits for nearly everything in flight before each use.
+  auto rounds = [&](uint32_t G, auto &&step) {
+    uint32_t g0 = 0;
+    for (; g0 + kDepth <= G; g0 += kDepth) {
+#pragma unroll
+      for (int k = 0; k < kDepth; k++) step(k);
+    }
+#pragma unroll
+    for (int k = 0; k < kDepth; k++)
+      if (g0 + k < G) step(k); // uniform over the block: all waves make the same number of barriers
+  };
 
-    if (!summer) {
+  __syncthreads(); // of the runs before these
+  if constexpr (CSC != 0) {
+    f32x4 *const ring = (f32x4 *)lds;
+    constexpr uint32_t kColVecs = CSC / 4; // column vectors of a row slice
+    // Where in a group of four rows the vector of column 4 * v + k of the slice lies: neighbours in v side by side, and the k turned
+    // by the group's number where the group is shorter than a round of all banks.
+    auto column_slot = [](uint32_t v, uint32_t k, uint32_t group) { return (k ^ (group & (kSets - 1))) * kColVecs + v; };
+    // the column of the slice that lane position `pl` of a set sums
+    auto column_of = [](uint32_t pl) { return pl % kColVecs * 4 + pl / kColVecs; };
+    // What the waves tell each other, all of it counted from the start of the role: bundles drawn, bundles summed, bundles whose sums
+    // have been fetched, chunks read, and per slot the loader waves that have written their part of a chunk there.  (One count for both slots would not do: a wave may
+    // be done with the next chunk while another is not with this one.)  Bundle number b is in set b % 2, chunk number c in
+    // slot c % 2.
+    uint32_t *const drawn = shared + 8, *const summed = shared + 9, *const fetched = shared + 10, *const taken = shared + 11,
+                   *const written = shared + 12;
+    constexpr uint32_t kLoaderWaves = kLoaders / kWave;
+    auto all_wrote = [](uint32_t chunk) { return (chunk / 2 + 1) * kLoaderWaves; };
+    if (threadIdx.x < 6) shared[8 + threadIdx.x] = 0;
+    lds_done();
+    __syncthreads();
+    if (wave % 4) {
       // ---------------- loaders ----------------
-      uint32_t lt = threadIdx.x - kSummers * kWave; // loader thread number
-      asm volatile("" : "+v"(lt)); // what follows from it is worked out here and takes no registers of the summing waves
-      const uint32_t my_row = lt / lanes, my_lane = lt % lanes;
-      const uint32_t due = slice * CS + my_lane * C;   // first column of this lane's vector
-      const bool in_slice = CSC ? true : my_lane * C < CS && my_row < RPL;
-      const uint32_t col = due < W ? lane_col<VEC>(due, W) : due;
-      const uint32_t lcol = col - slice * CS;          // ... inside the slice
-      // Loads are unconditional and branch-free so that kDepth chunks stay in flight per thread: positions
-      // past the end of a run re-read its last row (never summed), lanes outside the slice read column 0.
-      const embed_t *gbase = a.grad + ((in_slice && due < W) ? col : 0);
-      // The bag of a position is worked out here and not where the position is read: there it would wait for it.
-      auto row_load = [&](uint32_t pos) -> V {
-        return grad_load<Vec<VEC>, kPooled>((const embed_t *)((const char *)gbase + (uint64_t)grad_row<kPooled>(pos, a.bag) * (W * 4)));
-      };
-      // cursor of the index stage, 2 * kDepth chunks ahead of the LDS stage; past the end of the stream it
-      // stays on the last run
-      uint32_t cj = 0, first = 0; // the run, and the first row of the next chunk in it
-      uint32_t clo, len;
+      uint32_t lt = threadIdx.x - (wave < 4 ? 1 : 2) * kWave; // loader thread number
+      asm volatile("" : "+v"(lt)); // what follows from it is worked out here and takes no registers of the other waves
+      const uint32_t group = lt / kColVecs, my_lane = lt % kColVecs; // the group of four rows of a chunk, the column vector
+      uint32_t slot_of[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; k++) slot_of[k] = group * CSC + column_slot(my_lane, k, group);
+      // Every quad of lanes works out where its group's four rows lie, one row per lane: in every lane for itself that kept the
+      // loaders' SIMDs busy longer than the adds take.
+      const uint32_t my_row = group * 4 + lt % 4;
+      uint32_t idx[kDepth];
+      V val[kDepth][kRPT];
+      // The cursor of the index stage, 2 * kDepth chunks ahead of the LDS stage.  Loads are unconditional, so that kDepth chunks stay
+      // in flight per thread: positions past the end of a run re-read its last row (never summed), and so do the chunks past the
+      // end of the bundle.
+      uint32_t runs = 0, run = 0, clo = 0, len = 0, first = 0, at = 0; // at: chunks written, in all bundles
+      const uint4 *table = tables;
+      const embed_t *base = a.grad;
       auto open_run = [&]() {
-        const uint4 m = table[cj];
+        const uint4 m = table[run];
         clo = uni(m.y), len = uni(m.z), first = 0;
       };
-      open_run();
-      auto next_chunk = [&](uint32_t(&dst)[kRPT]) {
+      auto read_index = [&](int k) {
         const uint32_t from = min(first, len - 1), last = min(CR, len - from) - 1;
-        const uint32_t *pos = sorted_arg + clo + from;
-#pragma unroll
-        for (int q = 0; q < kRPT; q++) dst[q] = pos[min(q * RPL + my_row, last)];
+        idx[k] = sorted_arg[clo + from + min(my_row, last)];
         first += CR;
         if (first >= len) {
-          if (cj + 1 < J) {
-            cj++;
-            open_run();
-          } else {
-            first = len;
-          }
+          if (run + 1 < runs) run++, open_run();
+          else first = len;
         }
       };
-      uint32_t idx[kDepth][kRPT];
-      V val[kDepth][kRPT];
-#pragma unroll
-      for (int k = 0; k < kDepth; k++) next_chunk(idx[k]);
-#pragma unroll
-      for (int k = 0; k < kDepth; k++)
-#pragma unroll
-        for (int q = 0; q < kRPT; q++) val[k][q] = row_load(idx[k][q]);
-#pragma unroll
-      for (int k = 0; k < kDepth; k++) next_chunk(idx[k]);
-      // invariant at step k of a round: val[k] holds chunk g0+k, idx[k] the row indices of chunk g0+k+kDepth
-      uint32_t slot = 0;
-      auto step = [&](int k) {
-        float *sp = lds + slot * slot_floats;
-        slot = slot + 1 == slots ? 0 : slot + 1;
-#pragma unroll
-        for (int q = 0; q < kRPT; q++) {
-          if (in_slice) {
-            // the fast path's lanes write where they are due, also the last one of a row, which starts before that
-            if (CSC) *(V *)(sp + (q * RPL + (q >= kRPT / 2 ? kPad : 0) + my_row) * CS + my_lane * C) = val[k][q];
-            else Vec<VEC>::store_all(sp + (q * RPL + my_row) * CS + lcol, val[k][q]);
-          }
-          val[k][q] = row_load(idx[k][q]); // chunk + kDepth
-        }
-        next_chunk(idx[k]); // chunk + 2 * kDepth
-        __syncthreads();    // barrier of this chunk
+      auto find_rows = [&](int k, const embed_t *(&from)[kRPT]) { // (the bag of a position where it is read would wait for it)
+        const uint64_t off = (uint64_t)grad_row<kPooled>(idx[k], a.bag) * (W * 4);
+        from[0] = (const embed_t *)((const char *)base + of_quad<0>(off));
+        from[1] = (const embed_t *)((const char *)base + of_quad<1>(off));
+        from[2] = (const embed_t *)((const char *)base + of_quad<2>(off));
+        from[3] = (const embed_t *)((const char *)base + of_quad<3>(off));
       };
-      // Whole rounds run without a condition inside: with one, the compiler must assume that loads may have been
-      // skipped and waits for nearly everything in flight before each use.
-      uint32_t g0 = 0;
-      for (; g0 + kDepth <= G; g0 += kDepth) {
+      auto read_rows = [&](int k, const embed_t *const (&from)[kRPT]) {
 #pragma unroll
-        for (int k = 0; k < kDepth; k++) step(k);
+        for (int q = 0; q < kRPT; q++) val[k][q] = grad_load<Vec<VEC>, kPooled>(from[q]);
+      };
+      for (uint32_t bundle = 0;; bundle++) {
+        wait_until(drawn, bundle + 1);
+        const uint32_t cur = bundle & 1, G = uni(shared[cur * 4 + 1]);
+        runs = uni(shared[cur * 4]);
+        if (!runs) break;
+        const uint32_t due = uni(shared[cur * 4 + 2]) * CSC + my_lane * C; // first column of this lane's vector
+        base = a.grad + (due < W ? lane_col<VEC>(due, W) : 0u);
+        table = tables + cur * kTable, run = 0;
+        open_run();
+#pragma unroll
+        for (int k = 0; k < kDepth; k++) read_index(k);
+#pragma unroll
+        for (int k = 0; k < kDepth; k++) {
+          const embed_t *from[kRPT];
+          find_rows(k, from);
+          read_rows(k, from);
+          read_index(k); // in the order of the rounds below: the compiler waits for what either way into them has in flight
+        }
+        // val[k] holds the chunk that is written next and idx[k] the row indices of the one kDepth behind it
+        rounds(G, [&](int k) {
+          const embed_t *from[kRPT];
+          find_rows(k, from);
+          wait_until(taken, at - 1); // the chunk that was in this slot has been read (before the first two: -1 and 0)
+          f32x4 *sp = ring + (at & 1) * kSlotVectors;
+#pragma unroll
+          for (int c = 0; c < 4; c++) sp[slot_of[c]] = f32x4{val[k][0][c], val[k][1][c], val[k][2][c], val[k][3][c]};
+          read_rows(k, from);
+          lds_done();
+          tell_add(written + (at & 1)); // this wave's part of the chunk is in its slot
+          at++;
+          read_index(k);
+        });
       }
-#pragma unroll
-      for (int k = 0; k < kDepth; k++)
-        if (g0 + k < G) step(k); // uniform over the block: the summing waves make the same number of barriers
-      if (CSC) __syncthreads();  // the last chunk is added behind this one
-    } else {
-      // ---------------- summing waves: rows strictly in order ----------------
+    } else if (wave == 0) {
+      // ---------------- the summing wave: rows strictly in order ----------------
       uint32_t lane = threadIdx.x % kWave;
       asm volatile("" : "+v"(lane)); // what follows from it is worked out here and takes no registers of the loaders
-      constexpr uint32_t kHalves = CSC ? kRowSets<CSC> : 1;
-      // the place of the column this lane sums, and which rows of a chunk the lane holds
-      const uint32_t place = lane % (kWave / kHalves), half = lane / (kWave / kHalves);
-      const uint32_t mycol = slice * CS + place;
-      const bool col_ok = place < CS && mycol < W;
-      const bool direct = t.nrank == 1; // every key is owned and resident; the version counters move elsewhere
-      if (direct && wave == kSummers - 1) {
-        // The table rows the sums are added to, for every run of the bundle at once and parked in LDS: requested
-        // run by run, each would arrive a memory round trip after its run had been summed (a run of a few hundred
-        // occurrences is summed in a fraction of one), and the loaders would wait behind the full ring meanwhile.
-        // This wait happens once per bundle, while the loaders' first rows are on their way.
-        float rows[kTable / kHalves];
+      const uint32_t set = lane / CSC, pl = lane % CSC;
+      // where this lane's rows of either half start, and the t-th set of each
+      uint32_t turn = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < kTable / kHalves; j++) {
-          rows[j] = 0.f;
-          if (j * kHalves + half < J && col_ok) rows[j] = t.emb[(size_t)table[j * kHalves + half].w * W + mycol];
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kTable / kHalves; j++) row_stash[(j * kHalves + half) * kWave + place] = rows[j];
-      }
-      auto finish = [&](uint32_t u, uint32_t off, uint32_t j, float acc) { // the sum of run j of the bundle is complete
-        const float scaled = acc * neg_lr;
-        if (direct) t.emb[(size_t)off * W + mycol] = row_stash[j * kWave + place] + scaled;
-        else apply_row<Vec<1>, K>(t, id_bits, p, a, u, scaled, mycol);
+      for (uint32_t k = 0; k < (uint32_t)kSets; k++)
+        if (set_at(k, false, kSets) == set) turn = k;
+      const uint32_t base0 = turn * (kHalfGroups * CSC), base1 = (kHalfGroups * kSets + (kSets - 1 - turn) * kHalfGroups) * CSC;
+      typedef f32x4 Half[kHalfGroups];
+      auto add4 = [](const f32x4 &v, float &acc) { acc += v[0], acc += v[1], acc += v[2], acc += v[3]; };
+      auto pass = [](auto from, auto second, float &acc) { // the sum goes on to the next set
+        constexpr bool kSecond = decltype(second)::value;
+        constexpr uint32_t s = set_at(decltype(from)::value, kSecond, kSets), to = set_at(decltype(from)::value + 1, kSecond, kSets);
+        acc = from_half<(s ^ to) * CSC, (s < to)>(acc);
       };
-      if constexpr (CSC != 0) {
-        // this wave's chunks are every other one of the bundle
-        constexpr uint32_t kHeld = kHeldRows;
-        // where the column lies in a row of the ring: the last lane of a row at any address starts at column W - 4
-        const uint32_t at = !col_ok ? 0 : VEC == kOdd4 ? overlapped_place(place, mycol, W) : place;
-        float x[kHeld];
-        uint32_t j = 0, c = wave, passed = 0; // chunk c of run j of the bundle is next
-        uint32_t rank, L, off;                // of that run
-        auto open_run = [&]() {
-          const uint4 m = table[j];
-          rank = uni(m.x), L = uni(m.z), off = uni(m.w);
-        };
-        auto settle = [&]() {
-          while (c * CR >= L && j + 1 < J) {
-            c -= (L + CR - 1) / CR;
-            j++;
-            open_run();
-          }
-        };
-        open_run();
-        settle();
-        if (wave) __syncthreads(), passed++;
-        for (uint32_t g = wave; g < G; g += 2) {
-          lds_done();      // the sum in `hand`: without the wait the other wave now and then took the sum of two chunks before
-          __syncthreads(); // chunk g is in the ring
-          const uint32_t rows = min(CR, L - c * CR);
-          const float *sp = lds + (g % slots) * slot_floats + at;
-          if (rows % 4) { // a last group of less than four rows is put aside
+      // adds the n rows of half a chunk; returns the set that then holds the sum
+      auto add_half = [&](auto second, const Half &x, uint32_t n, const f32x4 &rest, float &acc) -> uint32_t {
+        auto pass_on = [&](auto from) { pass(from, second, acc); };
+        auto add_set = [&]() {
 #pragma unroll
-            for (uint32_t q = 0; q < 3; q++) {
-              const uint32_t r = min(rows / 4 * 4 + q, CR - 1);
-              hand[(1 + wave * 3 + q) * kWave + lane] = sp[(r + (r >= kHeld ? kPad : 0)) * CS];
+          for (int i = 0; i < kHalfGroups; i++) add4(x[i], acc);
+        };
+        auto add_first = [&](uint32_t m) { // the first m < 4 * kHalfGroups rows of the set; the last m % 4 lie apart
+#pragma unroll
+          for (int i = 0; i < kHalfGroups - 1; i++)
+            if (m >= 4u * (i + 1)) add4(x[i], acc);
+          if (m % 4 > 0) acc += rest[0];
+          if (m % 4 > 1) acc += rest[1];
+          if (m % 4 > 2) acc += rest[2];
+        };
+        constexpr uint32_t kSetRows = 4 * kHalfGroups;
+        uint32_t done = 0; // sets whose rows have all been added
+        if (n >= kSetRows) {
+          add_set(), done = 1;
+          if constexpr (kSets > 1) {
+            if (n >= 2 * kSetRows) {
+              pass_on(std::integral_constant<uint32_t, 0>()), add_set(), done = 2;
+              if constexpr (kSets > 2) {
+                if (n >= 3 * kSetRows) {
+                  pass_on(std::integral_constant<uint32_t, 1>()), add_set(), done = 3;
+                  if (n == 4 * kSetRows) pass_on(std::integral_constant<uint32_t, 2>()), add_set(), done = 4;
+                }
+              }
             }
           }
-#pragma unroll
-          for (uint32_t q = 0; q < kHeld; q++) x[q] = sp[(half * (kHeld + kPad) + q) * CS];
-          __syncthreads(); // the other wave has added chunk g - 1; chunk g is in registers
-          float acc = 0.f; // the reference starts every sum from 0
-          if (c) acc = hand[place];
-          auto add4 = [&](uint32_t q) { acc += x[q], acc += x[q + 1], acc += x[q + 2], acc += x[q + 3]; };
-          auto add_held = [&](uint32_t n) { // the first n rows the lane holds, without those behind the last four
-#pragma unroll
-            for (uint32_t q = 0; q < kHeld; q += 4)
-              if (n >= q + 4) add4(q);
-          };
-          auto add_all = [&]() {
-#pragma unroll
-            for (uint32_t q = 0; q < kHeld; q += 4) add4(q);
-          };
-          if (rows < kHeld) {
-            add_held(rows);
-          } else {
-            add_all();
-            if (kHalves > 1 && rows > kHeld) {
-              acc = from_lower_half(acc);
-              if (rows == CR) add_all();
-              else add_held(rows - kHeld);
-            }
-          }
-          if (rows % 4) {
-            const float *rest = hand + (1 + wave * 3) * kWave + lane;
-            acc += rest[0];
-            if (rows % 4 > 1) acc += rest[kWave];
-            if (rows % 4 > 2) acc += rest[2 * kWave];
-          }
-          // the lanes that have added the last rows
-          const bool have = half == (rows > kHeld ? 1u : 0u);
-          if (c * CR + rows < L) {
-            if (have) hand[place] = acc;
-          } else if (have && col_ok) {
-            finish(rank, off, j, acc);
-          }
-          passed += 2;
-          c += 2;
-          settle();
         }
-        if (passed < G + 1) __syncthreads();
-      } else {
+        const uint32_t over = n - done * kSetRows;
+        if (over) {
+          if constexpr (kSets > 1) {
+            if (done == 1) pass_on(std::integral_constant<uint32_t, 0>());
+            if constexpr (kSets > 2) {
+              if (done == 2) pass_on(std::integral_constant<uint32_t, 1>());
+              if (done == 3) pass_on(std::integral_constant<uint32_t, 2>());
+            }
+          }
+          add_first(over);
+          done++;
+        }
+        return set_at(done - 1, decltype(second)::value, kSets);
+      };
+      uint32_t at_chunk = 0; // chunks read, in all bundles
+      for (uint32_t bundle = 0;; bundle++) {
+        wait_until(drawn, bundle + 1);
+        const uint32_t cur = bundle & 1;
+        const uint32_t runs = uni(shared[cur * 4]), G = uni(shared[cur * 4 + 1]), slice = uni(shared[cur * 4 + 2]);
+        if (!runs) break;
+        const uint4 *table = tables + cur * kTable;
+        // Where the lane's column lies: where it is due, but for the columns of the last lane of a row at any address, which starts
+        // at column W - 4.
+        const uint32_t place = column_of(pl), mycol = slice * CSC + place;
+        const uint32_t at = VEC == kOdd4 && mycol < W ? overlapped_place(place, mycol, W) : place;
+        uint32_t col[kSets]; // in the groups of number 0, 1, ... mod kSets
+#pragma unroll
+        for (uint32_t k = 0; k < (uint32_t)kSets; k++) col[k] = column_slot(at / 4, at % 4, k);
+        auto read_half = [&](Half &x, const f32x4 *sp) {
+          const f32x4 *from[kSets];
+#pragma unroll
+          for (int k = 0; k < kSets; k++) {
+            uint32_t first = (uint32_t)(sp - ring) + col[k];
+            asm volatile("" : "+v"(first)); // one address and 12 offsets, not 12 addresses kept in registers for the next time
+            from[k] = ring + first;
+          }
+#pragma unroll
+          for (int i = 0; i < kHalfGroups; i++) x[i] = from[i % kSets][i * CSC];
+        };
+        // a whole half is added from x while the next one is read into y
+        auto add_reading = [&](auto second, const Half &x, Half &y, const f32x4 *sp, float &acc, auto &&late) {
+          auto one_set = [&](auto turn) {
+            constexpr int t = decltype(turn)::value;
+#pragma unroll
+            for (int i = 0; i < kHalfGroups; i++) {
+              add4(x[i], acc);
+              if (t * kHalfGroups + i + 1 == kSets * kHalfGroups * 3 / 4) { // what was read has come by now
+                asm volatile("" : "+v"(acc));
+                late();
+                __builtin_amdgcn_sched_barrier(0);
+              }
+            }
+            if constexpr (t + 1 < kSets) pass(turn, second, acc);
+          };
+          read_half(y, sp);
+          __builtin_amdgcn_sched_barrier(0);
+          one_set(std::integral_constant<uint32_t, 0>());
+          if constexpr (kSets > 1) one_set(std::integral_constant<uint32_t, 1>());
+          if constexpr (kSets > 2) one_set(std::integral_constant<uint32_t, 2>()), one_set(std::integral_constant<uint32_t, 3>());
+          asm volatile("" : "+v"(acc)); // the adds stay in front of what follows
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        Half x0, x1;
+        f32x4 rest = {0.f, 0.f, 0.f, 0.f};
+        float acc = 0.f; // the reference starts every sum from 0
+        uint32_t j = 0, left = uni(table[0].z); // the run, and its rows that have not been read
+        uint32_t n1 = 0, j1 = 0;  // rows of the second half that wait in x1, and their run ...
+        bool ends1 = false;       // ... which they end
+        auto finish = [&](uint32_t run, uint32_t holder) { // the sum of a run is complete
+          if (set == holder) sums[run * CSC + pl] = acc;
+          acc = 0.f;
+        };
+        auto slot = [&]() { return ring + (at_chunk & 1) * kSlotVectors; };
+        auto chunk_taken = [&]() { // both halves are in registers, or will be in a moment
+          at_chunk++;
+          lds_done();
+          tell(taken, at_chunk);
+        };
+        wait_until(fetched, bundle); // the sums of the bundle before (this one's first rows are on their way)
+        const uint32_t end = at_chunk + G;
+        while (at_chunk != end) {
+          if (n1 == kHalfRows && !ends1) { // whole chunks that follow a whole one
+            const uint32_t whole = left / CR;
+            uint32_t seen = peek(written + (at_chunk & 1));
+            for (uint32_t k = 0; k < whole; k++) {
+              if ((int)(uni(seen) - all_wrote(at_chunk)) < 0) wait_until(written + (at_chunk & 1), all_wrote(at_chunk));
+              asm volatile("" ::: "memory");
+              const f32x4 *sp = slot();
+              add_reading(std::true_type(), x1, x0, sp + base0, acc, []() {});
+              add_reading(std::false_type(), x0, x1, sp + base1, acc, [&]() {
+                chunk_taken(); // the loaders have to fill the slot before the chunk after the next is due
+                seen = peek(written + (at_chunk & 1)); // here when the next chunk is due
+              });
+            }
+            left -= whole * CR;
+            if (!left) {
+              ends1 = true;
+              if (j + 1 < runs) left = uni(table[++j].z);
+            }
+            if (at_chunk == end) break;
+          }
+          wait_until(written + (at_chunk & 1), all_wrote(at_chunk));
+          const f32x4 *sp = slot();
+          const uint32_t rows = min(CR, left), n0 = min(rows, kHalfRows);
+          read_half(x0, sp + base0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (n1) {
+            const uint32_t holder = add_half(std::true_type(), x1, n1, rest, acc);
+            if (ends1) finish(j1, holder);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          const uint32_t last_group = min(rows / 4, CR / 4 - 1); // of which the chunk may have less than four rows
+          rest = sp[last_group * CSC + column_slot(at / 4, at % 4, last_group)];
+          read_half(x1, sp + base1);
+          __builtin_amdgcn_sched_barrier(0);
+          const uint32_t holder = add_half(std::false_type(), x0, n0, rest, acc);
+          n1 = rows - n0, j1 = j, ends1 = rows == left;
+          if (ends1 && !n1) finish(j, holder);
+          left -= rows;
+          if (!left && j + 1 < runs) left = uni(table[++j].z);
+          chunk_taken();
+        }
+        if (n1) finish(j1, add_half(std::true_type(), x1, n1, rest, acc));
+        lds_done();
+        tell(summed, bundle + 1);
+      }
+    } else {
+      // ---------------- the wave that draws the tickets and applies the sums ----------------
+      uint32_t lane = threadIdx.x % kWave;
+      asm volatile("" : "+v"(lane));
+      const uint32_t set = lane / CSC, pl = lane % CSC;
+      constexpr int kRuns = kTable / kSets; // runs per set: number j * kSets + set of the bundle
+      const bool direct = t.nrank == 1;     // every key is owned and resident; the version counters move elsewhere
+      uint4 next = {0, 0, 0, 0};
+      draw(0, next);
+      lds_done();
+      tell(drawn, 1);
+      uint32_t end = 0; // chunks of the bundles up to this one
+      for (uint32_t bundle = 0;; bundle++) {
+        const uint32_t cur = bundle & 1;
+        const uint32_t runs = uni(shared[cur * 4]), slice = uni(shared[cur * 4 + 2]);
+        if (!runs) break;
+        end += uni(shared[cur * 4 + 1]);
+        const uint4 mine = next; // of run `lane` of the bundle
+        const uint32_t mycol = slice * CSC + column_of(pl);
+        const bool col_ok = mycol < W;
+        // the rows the sums will be added to, all of them at once; they are here long before the sums
+        uint32_t need = 0, q = 0;
+        if (!direct && lane < runs) need = a.need[mine.x], q = a.prefix[mine.x];
+        float row[kRuns], pend[kRuns];
+        auto off_of = [&](int j) { return (slot_t)__shfl((int)mine.w, j * kSets + set); };
+        auto works = [&](int j) { return col_ok && j * kSets + set < runs; };
+        auto type_of = [&](int j) { // the update type of generate_query.cu:18-25
+          const slot_t o = off_of(j);
+          const bool nd = __shfl((int)need, j * kSets + set) != 0;
+          return direct ? 1 : o == kNoSlot ? 0 : ((uint32_t)o >= t.n_cached ? 1 : (nd ? 2 : 3));
+        };
+#pragma unroll
+        for (int j = 0; j < kRuns; j++) {
+          row[j] = 0.f;
+          const slot_t o = off_of(j);
+          if (works(j) && (direct || o != kNoSlot)) row[j] = t.emb[(size_t)o * W + mycol];
+        }
+        if (!direct) {
+#pragma unroll
+          for (int j = 0; j < kRuns; j++) {
+            pend[j] = 0.f;
+            const slot_t o = off_of(j);
+            if (works(j) && o != kNoSlot && (uint32_t)o < t.n_cached) pend[j] = t.pend[(size_t)o * W + mycol];
+          }
+        }
+        // The next ticket is drawn when this bundle is nearly through: drawn at once, it would lie here while blocks with shorter
+        // bundles run out of work.
+        wait_until(taken, end - min(end, kDrawAhead));
+        draw(cur ^ 1, next);
+        lds_done();
+        tell(drawn, bundle + 2);
+        wait_until(summed, bundle + 1);
+        float sum[kRuns];
+#pragma unroll
+        for (int j = 0; j < kRuns; j++) sum[j] = sums[(j * kSets + set) * CSC + pl];
+        lds_done();
+        tell(fetched, bundle + 1);
+#pragma unroll
+        for (int j = 0; j < kRuns; j++) {
+          const slot_t o = off_of(j);
+          const int type = type_of(j);
+          const uint32_t at = (uint32_t)__shfl((int)q, j * kSets + set);
+          if (!works(j)) continue;
+          const float scaled = sum[j] * neg_lr;
+          if (type != 0) t.emb[(size_t)o * W + mycol] = row[j] + scaled;
+          else Vec<1>::store_away(a.g_val + (size_t)at * W + mycol, scaled, 0);
+          if (type >= 2) {
+            float g = pend[j] + scaled;
+            if (type == 2) {
+              Vec<1>::store_away(a.g_val + (size_t)at * W + mycol, g, 0);
+              g = 0.f;
+            }
+            t.pend[(size_t)o * W + mycol] = g;
+          }
+        }
+      }
+    }
+    lds_done();
+  } else {
+    // cursor of a loader's index stage, 2 * kDepth chunks ahead of its LDS stage; past the end of the stream it stays on the
+    // last run
+    uint32_t bundle_set = 0, J = 0, cj = 0, first = 0; // the run, and the first row of the next chunk in it
+    uint32_t clo = 0, len = 1;
+    auto open_run = [&]() {
+      const uint4 m = tables[bundle_set * kTable + cj];
+      clo = uni(m.y), len = uni(m.z), first = 0;
+    };
+    // read(positions of the next chunk, its last row): loads are unconditional, so that kDepth chunks stay in flight per thread, and
+    // rows past the end of a run re-read its last one (never summed)
+    auto next_chunk = [&](auto &&read) {
+      const uint32_t from = min(first, len - 1), last = min(CR, len - from) - 1;
+      read(sorted_arg + clo + from, last);
+      first += CR;
+      if (first >= len) {
+        if (cj + 1 < J) {
+          cj++;
+          open_run();
+        } else {
+          first = len;
+        }
+      }
+    };
+    auto open_cursor = [&](uint32_t set, uint32_t runs) {
+      bundle_set = set, J = runs, cj = 0;
+      open_run();
+    };
+    uint4 mine;
+    if (wave == 0) draw(0, mine);
+    __syncthreads();
+    for (uint32_t cur = 0;; cur ^= 1) {
+      const uint4 *table = tables + cur * kTable;
+      const uint32_t runs = uni(shared[cur * 4]), G = uni(shared[cur * 4 + 1]), slice = uni(shared[cur * 4 + 2]);
+      if (!runs) break;
+      if (wave == 0) draw(cur ^ 1, mine); // while the loaders wait for the first rows of this bundle
+      const uint32_t slot_floats = CR * CS;
+      if (wave != 0) {
+        const uint32_t lt = threadIdx.x - kWave, my_row = lt / lanes, my_lane = lt % lanes, step = kLoaders / lanes;
+        const bool in_slice = my_lane < CS && my_row < step;
+        const uint32_t col = slice * CS + my_lane;
+        const embed_t *gbase = a.grad + (in_slice && col < W ? col : 0u); // lanes outside the slice read column 0
+        uint32_t idx[kDepth][kRPT];
+        V val[kDepth][kRPT];
+        auto read_index = [&](int k) {
+          next_chunk([&](const uint32_t *pos, uint32_t last) {
+#pragma unroll
+            for (int q = 0; q < kRPT; q++) idx[k][q] = pos[min(q * step + my_row, last)];
+          });
+        };
+        auto row_load = [&](uint32_t pos) -> V { // (the bag of a position where it is read would wait for it)
+          return grad_load<Vec<VEC>, kPooled>((const embed_t *)((const char *)gbase + (uint64_t)grad_row<kPooled>(pos, a.bag) * (W * 4)));
+        };
+        // val[k] holds chunk k and idx[k] the row indices of chunk k + kDepth
+        open_cursor(cur, runs);
+#pragma unroll
+        for (int k = 0; k < kDepth; k++) read_index(k);
+#pragma unroll
+        for (int k = 0; k < kDepth; k++)
+#pragma unroll
+          for (int q = 0; q < kRPT; q++) val[k][q] = row_load(idx[k][q]);
+#pragma unroll
+        for (int k = 0; k < kDepth; k++) read_index(k);
         uint32_t slot = 0;
-        for (uint32_t j = 0; j < J; j++) {
+        rounds(G, [&](int k) {
+          float *sp = lds + slot * slot_floats;
+          slot = slot + 1 == kSlotsGeneric ? 0 : slot + 1;
+#pragma unroll
+          for (int q = 0; q < kRPT; q++) {
+            if (in_slice) Vec<VEC>::store_all(sp + (q * step + my_row) * CS + my_lane, val[k][q]);
+            val[k][q] = row_load(idx[k][q]); // chunk + kDepth
+          }
+          read_index(k); // chunk + 2 * kDepth
+          lds_done();
+          __syncthreads(); // barrier of this chunk
+        });
+      } else {
+        const uint32_t place = threadIdx.x % kWave, mycol = slice * CS + place;
+        const bool col_ok = place < CS && mycol < W;
+        const bool direct = t.nrank == 1;
+        if (direct) { // the table rows the sums are added to, for every run of the bundle at once and parked in LDS
+          float rows[kTable];
+#pragma unroll
+          for (uint32_t j = 0; j < kTable; j++) {
+            rows[j] = 0.f;
+            if (j < runs && col_ok) rows[j] = t.emb[(size_t)table[j].w * W + mycol];
+          }
+#pragma unroll
+          for (uint32_t j = 0; j < kTable; j++) sums[j * kWave + place] = rows[j];
+        }
+        uint32_t slot = 0;
+        for (uint32_t j = 0; j < runs; j++) {
           const uint4 m = table[j];
           float acc = 0.f; // the reference starts every sum from 0
           for (uint32_t c = 0; c * CR < m.z; c++) {
+            lds_done();
             __syncthreads(); // barrier of this chunk
             const float *sp = lds + slot * slot_floats + place;
-            slot = slot + 1 == slots ? 0 : slot + 1;
+            slot = slot + 1 == kSlotsGeneric ? 0 : slot + 1;
             if (place < CS) {
               const uint32_t rows = min(CR, m.z - c * CR);
               uint32_t r = 0;
@@ -767,11 +1059,15 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
               for (; r < rows; r++) acc += sp[r * CS];
             }
           }
-          if (col_ok) finish(m.x, m.w, j, acc);
+          if (col_ok) { // the sum of run j of the bundle is complete
+            const float scaled = acc * neg_lr;
+            if (direct) t.emb[(size_t)m.w * W + mycol] = sums[j * kWave + place] + scaled;
+            else apply_row<Vec<1>, K>(t, id_bits, p, a, m.x, scaled, mycol);
+          }
         }
       }
+      __syncthreads(); // everybody is done with the table and the ring
     }
-    __syncthreads(); // everybody is done with the table and the ring
   }
 }
 
@@ -782,22 +1078,19 @@ __device__ __forceinline__ void push_block(const TableView &t, int id_bits, cons
                                            uint32_t block) {
   // one LDS area for whichever role the block plays: the row ring of the long role or the index staging of the
   // medium role (one slice of kLongRun indices per group)
-  constexpr int kRingWords = VEC == 1 ? kSlotsGeneric * 2 * kPushBlock
-                                      : std::max({ring_floats(64), ring_floats(32), ring_floats(16)});
+  constexpr int kRingWords = VEC == 1 ? kSlotsGeneric * 2 * kPushBlock : kSlotsFast * kSlotVectors * 4;
   constexpr int kStageWords = (kPushBlock / LPR) * (int)kLongRun;
   __shared__ __align__(16) float lds[kRingWords > kStageWords ? kRingWords : kStageWords];
   __shared__ uint4 run_table[2 * kTable];
-  __shared__ uint32_t run_totals[2 * 4];
-  __shared__ float sums_at_hand[7 * kWave];  // long role: the sums one wave leaves to the other; up to three rows of each
-  __shared__ float row_stash[kTable * kWave]; // long role: the table rows of a bundle's runs (one slice, one lane each)
+  __shared__ uint32_t run_totals[4 * 4];
+  __shared__ float sums[kTable * kWave]; // long role: the sums of a bundle's runs (generic path: the rows they are added to)
   if (block < kLongBlocks) {
     // Every block first takes tickets of the longest runs, which are cut into narrower column slices so that more
     // blocks feed each of them (the blocks of a saturated memory system get equal shares of it, and a chain
     // advances with the share of the block that feeds it), then tickets of the other long runs.
     uint32_t *tk = p.d_nlong + kTicketBase;
     auto runs = [&](auto csc, int c_lo, int c_hi, uint32_t *counters) {
-      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, row_stash, sums_at_hand, c_lo, c_hi, block,
-                                                       kLongBlocks, counters);
+      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, sums, c_lo, c_hi, block, kLongBlocks, counters);
     };
     if constexpr (VEC == 1) {
       runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);

@@ -783,6 +783,33 @@ def test_run_lengths_around_the_chunks_of_the_push(width, nrank):
 
 
 @pytest.mark.parametrize("nrank", [1, 2])
+@pytest.mark.parametrize("width,lens", [(64, "giants"), (128, "giants"), (130, "giants"), (64, "bundles"), (256, "bundles"), (16, "bundles")])
+def test_long_runs_of_many_bundles_and_of_the_narrow_slices(width, lens, nrank):
+    # giants: runs around 16384 rows, from where on rows are cut into slices of 32 columns, ending inside either half of a chunk of 192;
+    # bundles: several tickets per block, one after the other, of runs a chunk or two long.  Sums bit for bit
+    say("narrow slices / many bundles", width, lens, nrank)
+    rng = np.random.default_rng(17)
+    count = np.array([16383, 16384, 16385, 16387, 16416, 16512, 16575, 16576, 16577, 18001] if lens == "giants" else
+                     rng.integers(129, 260, size=1200))
+    length = 2 * len(count)
+    root = (np.arange(length) % nrank).astype(np.uint8)
+    p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    prev_n = [0] * nrank
+    for step in range(2):
+        keys = [np.repeat(rng.permutation(length)[:len(count)].astype(np.int64), count) for _ in range(nrank)]
+        for k in keys:
+            rng.shuffle(k)
+        p.preprocess(keys, device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(n, width)).astype(np.float32) for n in prev_n])
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        p.compare_state(1e-5, "step %d" % step)
+        prev_n = [k.shape[0] for k in keys]
+    p.close()
+
+
+@pytest.mark.parametrize("nrank", [1, 2])
 @pytest.mark.parametrize("defer", [True, False])
 def test_a_refused_preprocess_leaves_the_batches_alone(defer, nrank):
     say("refused preprocess", defer, nrank)
