@@ -94,6 +94,25 @@ def test_pooled_rows_of_odd_widths_and_unaligned_pointers(bag, width, off, nrank
     p.close()
 
 
+@pytest.mark.parametrize("nrank", [1, 2])
+@pytest.mark.parametrize("width", [3, 12, 30, 37, 64, 128, 132, 300])
+def test_bags_around_the_rounds_of_the_pooled_gather(width, nrank):
+    # the lanes of a group find the rows of a bag together, one position each, and read them eight at a time: bags that end before,
+    # at and behind a round and the group's lanes, in rows of every number of lanes and of two rounds of columns
+    print("pooled look-ups, width", width, "shards", nrank, flush=True)
+    rng = np.random.default_rng(300 + width)
+    length = 3_000
+    root = (np.arange(length) % nrank).astype(np.uint8)
+    p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    for bag in (2, 4, 7, 8, 9, 15, 16, 17, 31, 33, 64, 65, 129):
+        keys = [rng.integers(0, length, size=bag * (37 - 5 * r)).astype(np.int64) for r in range(nrank)]
+        out, ref = pooled_step(p, keys, [None] * nrank, bag)
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "bag %d rank %d" % (bag, r))
+    p.close()
+
+
 def test_pooled_matches_the_plain_call_with_replicated_gradients():
     # the definition itself, on the GPU alone: same table state as hctr_push_pull with every bag's gradient repeated,
     # pooled rows = the plain rows added up in key order
