@@ -348,14 +348,16 @@ struct QueryArea {
 void launch_place_queries(hipStream_t s, OwnerShard *shards_dev, const OwnerShard *shards_host, int nsrc,
                           const QueryArea &area);
 // shards_dev: the array in device memory.  nshards == nsrc: every shard of the group is in the array, in rank order (an
-// owner looks its requesters up there).  push_blocks: the most blocks a shard's received pushes need; queries_max: no
-// shard receives more queries than this; queries_guess: what the busiest shard probably receives (the grids are cut
+// owner looks its requesters up there).
+// The received pushes; push_blocks: the most blocks a shard's need.  Nothing of it depends on the batches that are current: it
+// does not wait for their index.
+void launch_apply_pushes(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width, uint32_t push_blocks);
+// The received queries, behind launch_apply_pushes; queries_max: no shard receives more queries than this; queries_guess: what the busiest shard probably receives (the grids are cut
 // from it; what a shard does receive, the kernels read from the records and stride over).
 // pulls: the requesters; their launches' share is the index of every returned row per unique key (a.ret_i), where the gather
 // reads each key's row (a.src_row) and the counts of the step.
 struct PullShard;
-void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width,
-                       uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess, const PullShard *pulls, int npulls);
+void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width, uint32_t queries_max, uint32_t queries_guess, const PullShard *pulls, int npulls);
 // requester: refresh cached rows that came back, then gather every key's row into dst
 struct PullArgs {
   const uint32_t *got;       // [U] or nullptr: nothing came back (nrank == 1)

@@ -807,18 +807,23 @@ static uint32_t guessed_blocks(uint32_t guess, uint32_t most, uint32_t per_block
   return std::max(1u, div_up(std::min<uint64_t>(g, most), per_block));
 }
 
-void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width,
-                       uint32_t push_blocks, uint32_t queries_max, uint32_t queries_guess, const PullShard *pulls, int npulls) {
+void launch_apply_pushes(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width, uint32_t push_blocks) {
+  if (!push_blocks) return;
+  const int vec = row_vec(width, nullptr);
+  const int lpr = lanes_for(width, vec);
+  const uint32_t rpb = owner_push_rows_per_block(width);
+#define CALL(V, L) \
+  hipLaunchKernelGGL((apply_remote_all<V, L>), dim3(push_blocks, nshards), dim3(kBlock), 0, s, shards_dev, nsrc, rpb)
+  HCTR_DISPATCH_ROW(vec, lpr, CALL);
+#undef CALL
+  HCTR_HIP(hipGetLastError());
+}
+
+void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards, int nsrc, uint32_t width, uint32_t queries_max,
+                       uint32_t queries_guess, const PullShard *pulls, int npulls) {
   const uint32_t tiles = guessed_blocks(queries_guess, queries_max, kBlock);
   const int vec = row_vec(width, nullptr);
   const int lpr = lanes_for(width, vec);
-  if (push_blocks) {
-    const uint32_t rpb = owner_push_rows_per_block(width);
-#define CALL(V, L) \
-  hipLaunchKernelGGL((apply_remote_all<V, L>), dim3(push_blocks, nshards), dim3(kBlock), 0, s, shards_dev, nsrc, rpb)
-    HCTR_DISPATCH_ROW(vec, lpr, CALL);
-#undef CALL
-  }
   hipLaunchKernelGGL(decide_count, dim3(tiles, nshards), dim3(kBlock), 0, s, shards_dev, nsrc);
   hipLaunchKernelGGL(scan_positions, dim3(tiles, nshards), dim3(kBlock), 0, s, shards_dev, nsrc);
   // the launches of several groups of requesters, the first of them with the owners' work

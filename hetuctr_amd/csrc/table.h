@@ -300,16 +300,21 @@ class Group {
   // enqueues the push plans of one batch of each of the shards; the counts reach the host when the stream has run it
   void plan_batches(const std::vector<Shard *> &shards, Batch Shard::*which);
   void flush_index();                    // waits for a pending index and takes its results over
-  // owner-side arguments of every shard: pinned staging and the device copy the kernels read
+  // owner-side arguments of every shard: pinned staging and the device copy the kernels read (owner_host: the records behind
+  // the distances of the pushed rows in one staging area, because both go to the device in front of the push)
   OwnerShard *owner_host = nullptr;
   DeviceBuf owner_dev, ret_delta_dev;    // ret_delta_dev: nrank words per owner, see OwnerShard::ret_delta
+  uint64_t fill_owners();
+  void apply_pushes();
   void owner_side(uint64_t queries_max, const std::vector<PullShard> &pulls);
   // Where every shard's pushed rows go: one receive area for the whole group (ids, counts, rows), cut into one piece
   // per owner and, inside it, per source; sized from the plans before any push kernel runs.  Every sender gets, per
   // owner, the distance between a row's place in its own plan and its place in the area (nrank words per sender).
-  void place_pushes();
+  uint64_t place_pushes(); // and fills the owners' records; returns the most queries there can be
   DeviceBuf rg_idx_all, rg_cnt_all, rg_val_all, push_delta_dev;
-  uint32_t *push_delta_host = nullptr;   // pinned staging of the distances
+  uint32_t *push_delta_host = nullptr;   // pinned staging of the distances and, owner_offset() bytes in, of the records
+  size_t owner_offset() const { return ((size_t)nrank * nrank * sizeof(uint32_t) + 255) / 256 * 256; }
+  bool pushes_placed_ = false;           // the step has pushed rows: push_delta_dev holds its distances and records
   // The same for the queries of a step: one receive area (ids, versions, and what the owners keep per query), nrank
   // distances per requester.  How many queries go where is known on the device only: reserve_queries() sizes the area
   // for the most there can be, launch_place_queries (behind the upload of the owners' records) cuts it.

@@ -904,7 +904,6 @@ Group::~Group() {
   if (ev_push) (void)hipEventDestroy(ev_push);
   if (ev_pushed) (void)hipEventDestroy(ev_pushed);
   if (ev_plan) (void)hipEventDestroy(ev_plan);
-  if (owner_host) (void)hipHostFree(owner_host);
   if (push_delta_host) (void)hipHostFree(push_delta_host);
 }
 
@@ -962,15 +961,23 @@ void Group::collect_marks() {
   marks.clear();
 }
 
-// handleGradient + handleQuery of every shard (csrc/core/hetu_gpu_table.cu:27-31): one set of launches for the group
-void Group::owner_side(uint64_t queries_max, const std::vector<PullShard> &pulls) {
+// handleGradient of every shard (csrc/core/hetu_gpu_table.cu:27): right behind the pushes.  The records it reads came with the
+// distances of the pushed rows; the array the query kernels read is filled beside the pushes (place_queries writes into it).
+void Group::apply_pushes() {
+  if (!pushes_placed_) return;
   uint32_t push_blocks = 0;
   for (int r = 0; r < nrank; r++) push_blocks = std::max(push_blocks, owner_host[r].push_blocks);
   StageScope st(*this, S_OWNER);
+  launch_apply_pushes(stream, (const OwnerShard *)(push_delta_dev.as<char>() + owner_offset()), nrank, nrank, members[0]->cfg.width, push_blocks);
+}
+
+// handleQuery of every shard (csrc/core/hetu_gpu_table.cu:28-31): one set of launches for the group
+void Group::owner_side(uint64_t queries_max, const std::vector<PullShard> &pulls) {
+  StageScope st(*this, S_OWNER);
   // the grids of the query kernels: from what the busiest owner received in the step before (the first step: the most)
   const uint32_t guess = queries_seen_ ? queries_guess_ : (uint32_t)queries_max;
-  launch_owner_side(stream, owner_dev.as<OwnerShard>(), nrank, nrank, members[0]->cfg.width, push_blocks, (uint32_t)queries_max,
-                    guess, pulls.data(), (int)pulls.size());
+  launch_owner_side(stream, owner_dev.as<OwnerShard>(), nrank, nrank, members[0]->cfg.width, (uint32_t)queries_max, guess,
+                    pulls.data(), (int)pulls.size());
 }
 
 void Group::set_defer_index(bool on) {
@@ -1001,13 +1008,16 @@ void Group::set_stage_timing(bool on) {
 // every owner is known from the plans before any push kernel starts, so the area is sized and cut here: one piece per
 // owner, inside it one per source, both in rank order.  In one process the area is one allocation; between GPUs every
 // owner would hold its piece and hand its address to the others.
-void Group::place_pushes() {
+uint64_t Group::place_pushes() {
   const int R = nrank;
-  if (R == 1) return;
+  if (R == 1) return 0;
+  pushes_placed_ = false;
+  const size_t staged = owner_offset() + (size_t)R * sizeof(OwnerShard);
   if (!push_delta_host) {
-    HCTR_HIP(hipHostMalloc((void **)&push_delta_host, (size_t)R * R * sizeof(uint32_t), hipHostMallocDefault));
-    push_delta_dev.reserve((size_t)R * R * sizeof(uint32_t));
+    HCTR_HIP(hipHostMalloc((void **)&push_delta_host, staged, hipHostMallocDefault));
+    owner_host = (OwnerShard *)((char *)push_delta_host + owner_offset());
   }
+  push_delta_dev.reserve(staged);
   uint64_t total = 0;
   for (int d = 0; d < R; d++) {
     Shard &dst = *members[d];
@@ -1023,7 +1033,7 @@ void Group::place_pushes() {
   HCTR_CHECK(total < 0xfffffff0ull, "more than 2^32 rows are pushed in one step");
   bool any = false;
   for (const Shard *m : members) any |= m->prev_active;
-  if (!any) return;
+  if (!any) return fill_owners();
   const size_t W = members[0]->cfg.width;
   rg_idx_all.reserve(total * sizeof(index_t));
   rg_cnt_all.reserve(total * sizeof(version_t));
@@ -1038,7 +1048,9 @@ void Group::place_pushes() {
       if (src.prev_active) glo += src.prev.push_cnt[d];
     }
   }
-  HCTR_HIP(hipMemcpyAsync(push_delta_dev.p, push_delta_host, (size_t)R * R * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+  const uint64_t queries_max = fill_owners();
+  HCTR_HIP(hipMemcpyAsync(push_delta_dev.p, push_delta_host, staged, hipMemcpyHostToDevice, stream));
+  pushes_placed_ = true;
   // plan position -> position in the area, for every shard's push kernel
   std::vector<PlaceShard> v;
   for (Shard *m : members)
@@ -1049,6 +1061,15 @@ void Group::place_pushes() {
     }
   StageScope st(*this, S_PUSH);
   launch_place_rows(stream, members[0]->kl, v.data(), (int)v.size());
+  return queries_max;
+}
+
+uint64_t Group::fill_owners() {
+  owner_dev.reserve((size_t)nrank * sizeof(OwnerShard));
+  ret_delta_dev.reserve((size_t)nrank * nrank * sizeof(uint32_t));
+  const uint64_t queries_max = reserve_queries();
+  for (Shard *m : members) m->fill_owner_args(owner_host[m->cfg.rank], queries_max);
+  return queries_max;
 }
 
 // csrc/core/all2all.cu:18-46: every owner's receive buffer is the requesters' buckets for it, in source order.  The
@@ -1412,7 +1433,7 @@ void Group::push_pull_all(const float *const *grads, float *const *dsts, size_t 
 void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint32_t bag) {
   if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
   for (Shard *m : members) m->begin_push(grads[m->cfg.rank], bag);
-  place_pushes();
+  const uint64_t queries_max = place_pushes();
   {
     std::vector<PushShard> pushes;
     PushShard r;
@@ -1423,21 +1444,14 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   }
   if (time_calls) HCTR_HIP(hipEventRecord(ev_push, stream));
   if (nrank > 1) HCTR_HIP(hipEventRecord(ev_pushed, stream));
+  apply_pushes();       // (a small batch's push is over before its index: the owners' rows are updated meanwhile)
   enqueue_index_rest(); // the pushes are in their queue, now the rest of the current batches' index
   // One shard and a small batch: the gather works from the batch's keys and needs nothing of its index, which is
   // longer than the push of such a batch.  The step then leaves the index pending: whatever needs it next (the next
   // preprocess, which makes this batch the previous one; a fetch) waits for it, by then long done.
   const bool index_not_needed = nrank == 1 && (dsts[0] == nullptr || members[0]->direct_now(bag));
   const bool join_index = index_pending && !index_not_needed;
-  uint64_t queries_max = 0;
   if (nrank > 1) {
-    if (!owner_host) {
-      HCTR_HIP(hipHostMalloc((void **)&owner_host, (size_t)nrank * sizeof(OwnerShard), hipHostMallocDefault));
-      owner_dev.reserve((size_t)nrank * sizeof(OwnerShard));
-      ret_delta_dev.reserve((size_t)nrank * nrank * sizeof(uint32_t));
-    }
-    queries_max = reserve_queries();
-    for (Shard *m : members) m->fill_owner_args(owner_host[m->cfg.rank], queries_max);
     {
       // Behind the index, on its stream and beside the pushes: the owners' records go to the device and the receive
       // area of the queries is cut there from the counts the index left (nothing of this needs the host to know them).
