@@ -36,7 +36,7 @@ template <int VEC> __device__ __forceinline__ void store_own(embed_t *row, typen
 }
 
 // The queries of a step (csrc/core/generate_query.cu:91-106): per unique key its id and the version of the local copy
-// (invalid if the key is not resident here), written where the key's owner reads its queries: place u + delta[owner]
+// (invalid if the key is not cached here), written where the key's owner reads its queries: place u + delta[owner]
 // of a receive area all owners share.
 // (This and the other kernels of a shard's own batch: see kShardsPerLaunch.)
 typedef Records<PullShard, kShardsPerLaunch> PullShards;
@@ -51,7 +51,8 @@ __global__ __launch_bounds__(kBlock) void build_queries(PullShards shards, int i
   const K key = ((const K *)c.ukey)[u];
   const uint32_t pos = u + S.delta[(uint32_t)(key >> id_bits)];
   S.q_idx[pos] = (index_t)(key & (K)(((uint64_t)1 << id_bits) - 1));
-  S.q_ver[pos] = o != kNoSlot ? S.t.ver[o] : kInvalidVersion;
+  // (of rows the shard owns none: no owner asks whether its own copy is outdated, and it may be moving the version just now)
+  S.q_ver[pos] = o != kNoSlot && (uint32_t)o < S.t.n_cached ? S.t.ver[o] : kInvalidVersion;
 }
 
 // ---- owner side: every kernel below serves ALL shards of a loopback group in one launch (blockIdx.y = shard), the

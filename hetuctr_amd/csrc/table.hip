@@ -1451,7 +1451,15 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   // preprocess, which makes this batch the previous one; a fetch) waits for it, by then long done.
   const bool index_not_needed = nrank == 1 && (dsts[0] == nullptr || members[0]->direct_now(bag));
   const bool join_index = index_pending && !index_not_needed;
+  std::vector<PullShard> pulls;
+  std::vector<Shard *> pulling;
   if (nrank > 1) {
+    PullShard r;
+    for (Shard *m : members)
+      if (m->pull_record(r, dsts[m->cfg.rank], bag, query_delta_dev.as<uint32_t>() + (size_t)nrank * m->cfg.rank)) {
+        pulls.push_back(r);
+        pulling.push_back(m);
+      }
     {
       // Behind the index, on its stream and beside the pushes: the owners' records go to the device and the receive
       // area of the queries is cut there from the counts the index left (nothing of this needs the host to know them).
@@ -1461,10 +1469,16 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
         StageScope st(*this, S_QUERY);
         launch_place_queries(stream, owner_dev.as<OwnerShard>(), owner_host, nrank, query_area());
       }
+      HCTR_HIP(hipStreamWaitEvent(stream, ev_pushed, 0));
+      {
+        // csrc/core/generate_query.cu:91-106: every query is written where its owner reads it (Group::reserve_queries); the
+        // versions in it are those of cached rows, which the pushes moved and the owners, who are applying them, do not
+        StageScope st(*this, S_QUERY);
+        launch_build_queries(stream, members[0]->kl, pulls.data(), (int)pulls.size());
+      }
       HCTR_HIP(hipEventRecord(ev_index, stream));
       // the push plans of the current batches, for the step in which they are the previous ones: after the pushes of
       // this step (they move the update counters the plan reads), beside everything else the step still does
-      HCTR_HIP(hipStreamWaitEvent(stream, ev_pushed, 0));
       plan_batches(members, &Shard::cur);
       HCTR_HIP(hipEventRecord(ev_plan, stream));
     }
@@ -1480,19 +1494,6 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   }
   if (join_index || nrank > 1) HCTR_HIP(hipStreamWaitEvent(stream, ev_index, 0));
   if (nrank > 1) {
-    std::vector<PullShard> pulls;
-    std::vector<Shard *> pulling;
-    PullShard r;
-    for (Shard *m : members)
-      if (m->pull_record(r, dsts[m->cfg.rank], bag, query_delta_dev.as<uint32_t>() + (size_t)nrank * m->cfg.rank)) {
-        pulls.push_back(r);
-        pulling.push_back(m);
-      }
-    {
-      // csrc/core/generate_query.cu:91-106: every query is written where its owner reads it (Group::reserve_queries)
-      StageScope st(*this, S_QUERY);
-      launch_build_queries(stream, members[0]->kl, pulls.data(), (int)pulls.size());
-    }
     owner_side(queries_max, pulls);
     // the reference waits here for the return counts (hetu_gpu_table.cu:33); they stay on the device
     {
