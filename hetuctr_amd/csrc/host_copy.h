@@ -18,7 +18,8 @@ class HostStager {
   // been read (the caller may reuse it).  The staging buffer is reused by the next call on this object, which first
   // waits for the transfers enqueued here.
   // narrow_ids: `src` holds 64-bit ids and `dst` receives bytes / 2 bytes of 32-bit ones, half the bytes on the bus;
-  // an id that does not fit (a negative one too) arrives as 0xffffffff.
+  // an id that does not fit (a negative one too) arrives as 0xffffffff.  What is narrowed is looked at on the way:
+  // largest() says afterwards how large an id arrived.
   void copy(void *dst, const void *src, size_t bytes, hipStream_t s, bool narrow_ids = false);
 
   // The same without the transfer, for kLendUpTo bytes at most: returns the staging buffer, filled, at the address a kernel
@@ -28,8 +29,10 @@ class HostStager {
   // it need be: lent as well, 426 k ids took 201 us instead of 247 and 1.7 M 635 instead of 651.
   static constexpr size_t kLendUpTo = 2 << 20;
   const void *lend(const void *src, size_t bytes, hipStream_t s, bool narrow_ids);
+  uint32_t largest() const { return largest_; } // of the ids the last call narrowed, as 32-bit ones
 
  private:
+  uint32_t largest_ = 0;
   void reserve(size_t bytes, hipStream_t reader);
   unsigned char *pinned_ = nullptr;
   size_t cap_ = 0;

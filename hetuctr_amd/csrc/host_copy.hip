@@ -1,6 +1,7 @@
 // Pageable host memory -> device through a pinned staging buffer filled by a crew of threads.  Host code only.
 #include "host_copy.h"
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -26,6 +27,7 @@ struct Job {
   size_t bytes, pieces; // of the source
   bool narrow;          // the source is 64-bit ids, the staging buffer gets 32-bit ones
   std::atomic<size_t> next{0};
+  std::atomic<uint32_t> largest{0}; // of the narrowed ids of all finished pieces
   std::unique_ptr<std::atomic<unsigned char>[]> done;
 
   Job(const void *s, void *d, size_t n, bool narrow_ids)
@@ -39,19 +41,26 @@ struct Job {
     const size_t i = next.fetch_add(1, std::memory_order_relaxed);
     if (i >= pieces) return false;
     const size_t lo = i * kPiece, len = std::min(kPiece, bytes - lo);
-    if (narrow) narrow_ids(dst + lo / 2, src + lo, len / sizeof(int64_t));
-    else std::memcpy(dst + lo, src + lo, len);
+    if (narrow) {
+      const uint32_t here = narrow_ids(dst + lo / 2, src + lo, len / sizeof(int64_t));
+      uint32_t seen = largest.load(std::memory_order_relaxed);
+      while (here > seen && !largest.compare_exchange_weak(seen, here, std::memory_order_relaxed)) {
+      }
+    } else std::memcpy(dst + lo, src + lo, len);
     done[i].store(1, std::memory_order_release);
     return true;
   }
-  // an id that does not fit 32 bits (negative ones included) becomes 0xffffffff
-  static void narrow_ids(unsigned char *to, const unsigned char *from, size_t n) {
+  // an id that does not fit 32 bits (negative ones included) becomes 0xffffffff; returns the largest
+  static uint32_t narrow_ids(unsigned char *to, const unsigned char *from, size_t n) {
     const uint64_t *__restrict__ in = (const uint64_t *)from;
     uint32_t *__restrict__ out = (uint32_t *)to;
+    uint32_t largest = 0;
     for (size_t k = 0; k < n; k++) {
       const uint64_t v = in[k];
       out[k] = (v >> 32) ? 0xffffffffu : (uint32_t)v;
+      largest = std::max(largest, out[k]);
     }
+    return largest;
   }
 };
 
@@ -159,6 +168,7 @@ const void *HostStager::lend(const void *src, size_t bytes, hipStream_t s, bool 
   }
   for (size_t i = 0; i < job->pieces; i++) // pieces other threads are still copying
     while (!job->done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
+  largest_ = job->largest.load(std::memory_order_relaxed);
   return pinned_;
 }
 
@@ -192,6 +202,7 @@ void HostStager::copy(void *dst, const void *src, size_t bytes, hipStream_t s, b
   };
   try {
     stage(true);
+    largest_ = job->largest.load(std::memory_order_relaxed);
     send(true);
     HCTR_HIP(hipEventRecord(sent_, s));
   } catch (...) {

@@ -96,6 +96,7 @@ struct HostMirror {
   // written by the kernel that reads the caller's ids when preprocess returns early (no copy): an id out of range, or
   // the two at once (ReadSignal)
   uint32_t key_err, ids_read;
+  uint32_t key_err_known; // where the kernel's range check reports what the host has found already
 };
 
 class Group;
@@ -167,6 +168,11 @@ class Shard {
   uint32_t *key_flag_ = nullptr; // ... and where it reports a key out of range
   ReadSignal read_;              // ... or how it says that it has read them all
   bool wait_ids_read(hipStream_t on); // waits for that, if it does say so; true: a key was out of range
+  // One shard, ids narrowed on their way through pinned memory: the caller's buffer is free and the ids' range known when they
+  // are staged, so preprocess waits for no kernel (ids_bad_ is what it reports).  Whoever reads the sort keys outside the index
+  // stream waits first: a step's gather from the keys (keys_unread_).
+  bool staged_ = false, ids_bad_ = false, keys_unread_ = false;
+  void wait_keys();
   TileSortBuffers tile_sort_buffers() const; // the index scratch as the tile-sorted passes take it
   HostStager stager;                         // ids that arrive in pageable host memory go through its pinned buffer
   bool pooled_from_keys = true;   // HETUCTR_POOLED_FROM_KEYS=0: pooled gathers of one shard go through the inverse index

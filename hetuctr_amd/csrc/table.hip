@@ -285,6 +285,7 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
   ids_ = nullptr;
   key_flag_ = flag ? flag : err_ptr();
   read_ = ReadSignal();
+  staged_ = ids_bad_ = keys_unread_ = false;
   if (!scratch_area) cur.reserve(cur.n, cfg.nrank, kl.wide); // else: the caller has checked that the buffers hold n keys
   if (n == 0) { // :93-95
     cur.clear(s, cfg.nrank);
@@ -314,6 +315,13 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
           cur.staged.reserve(n * sizeof(index_t));
           stager.copy(cur.staged.p, keys, n * sizeof(index_t), s, narrowed);
           ids = cur.staged.as<index_t>();
+        }
+        // Nothing of the caller's is needed any more.  (The transfer of 1.7 M ids takes 95 us longer than their staging, and the
+        // next push can run meanwhile: two steps of 128 floats 1403 -> 1268 us; of 53 k ids 125.6 -> 123.8.)
+        if (narrowed && flag != nullptr && cfg.nrank == 1) {
+          staged_ = keys_unread_ = true;
+          ids_bad_ = stager.largest() >= tv.id_max;
+          key_flag_ = &mirror->key_err_known;
         }
       }
       cur.tile_sorted = tile_sort_mode == 2 ? tile_sort_possible(cur.n) : (tile_sort_mode == 1 && tile_sort_fits(cur.n));
@@ -598,6 +606,14 @@ void Shard::begin_push(const float *grad, uint32_t bag) {
   HCTR_CHECK(prev.n % bag == 0, "pooled push: the previous batch is not a whole number of bags");
 }
 
+// the sort keys of the batch are about to be read on the main stream by a kernel that does not wait for the index
+void Shard::wait_keys() {
+  if (!keys_unread_) return;
+  keys_unread_ = false;
+  if (read_.word) (void)wait_ids_read(group->index_stream); // (by the time a push has been queued they are there)
+  else HCTR_HIP(hipStreamWaitEvent(group->stream, group->ev_keys, 0));
+}
+
 // the run lists of the batch that is pushed next, if no gather has built them
 void Shard::list_runs() {
   if (prev.n == 0 || prev.lists_ready) return;
@@ -742,6 +758,7 @@ void Shard::write_back(float *dst, uint32_t bag) {
   StageScope st(*group, S_GATHER);
   HCTR_CHECK(cur.n % bag == 0, "pooled pull: the batch is not a whole number of bags");
   if (direct_now(bag)) {
+    wait_keys();
     if (bag > 1) launch_gather_pooled_direct(s, tv, kl, cur.comp.p, cur.n, dst, bag);
     else launch_gather_direct(s, tv, kl, cur.comp.p, cur.n, dst, a.stream_stores);
     return;
@@ -1238,6 +1255,7 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
       (void)hipGetLastError(); // a failed allocation is not the next launch's error
       for (Shard *m : members) {
         m->mirror->key_err = 0;
+        m->keys_unread_ = false; // (and no kernel may have been launched that would say otherwise)
         (void)hipMemsetAsync(m->err_ptr(), 0, 4, stream);
         m->cur.drop();
         m->swap_batches();
@@ -1285,7 +1303,7 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
       m->list_runs();
       lists_running_ = true;
     }
-    const bool bad_key = wait_ids_read();
+    const bool bad_key = m->staged_ ? m->ids_bad_ : wait_ids_read();
     taken = true;
     if (time_calls) {
       float ms = 0.f;

@@ -459,6 +459,41 @@ def test_large_batches_of_ids_in_pageable_host_memory():
     p.close()
 
 
+@pytest.mark.parametrize("bag", [1, 5])
+@pytest.mark.parametrize("n", [5, 8_190, 60_000, 262_140, 262_150, 700_000])
+def test_steps_from_ids_still_on_their_way(n, bag):
+    # preprocess of ids in pageable memory returns when they are staged: the caller's buffer is overwritten at once, and nothing but
+    # push_pull waits for the kernel that reads them -- its gather from the keys by word, by event, or with the index
+    import torch
+    say("ids on their way", n, bag)
+    rng = np.random.default_rng(41)
+    length, width = 40_000, 16
+    p = single(length, width, init=("Uniform", -0.01, 0.01), lr=0.05)
+    buf, prev = np.zeros(n + 10, np.int64), 0
+    for step in range(6):
+        k = n - 5 * step if n > 30 else n
+        want = rng.integers(0, length, size=k).astype(np.int64)
+        buf[:k] = want
+        if step == 4:                                       # reported by the call itself, treated as id 0
+            buf[k - 1], want[k - 1] = length, 0
+            with pytest.raises(RuntimeError, match="outside"):
+                p.tables[0].preprocess(buf.ctypes.data, k)
+        else:
+            p.tables[0].preprocess(buf.ctypes.data, k)
+        buf[:] = -1
+        p.oracle.preprocess([want])
+        g = rng.normal(0, 1e-3, size=(prev // bag, width)).astype(np.float32) if prev and step != 2 else None
+        dst = torch.full((k // bag, width), float("nan"), device="cuda")
+        dg = torch.from_numpy(g).cuda() if g is not None else None
+        torch.cuda.synchronize()
+        p.tables[0].push_pull_pooled(dg.data_ptr() if g is not None else 0, dst.data_ptr(), bag)
+        ref = p.oracle.push_pull_pooled([g], bag)[0] if bag > 1 else p.oracle.push_pull([g])[0]
+        assert_close(dst.cpu().numpy(), ref, 1e-5, "dst step %d" % step)
+        prev = k
+    p.compare_state(1e-5, "end")
+    p.close()
+
+
 def test_host_ids_from_two_threads_at_once():
     # two tables, each fed large host batches by a thread of its own: the threads that stage host ids are shared by
     # the process, a copy posted while another is under way must leave both batches intact
