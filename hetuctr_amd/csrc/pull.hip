@@ -463,14 +463,14 @@ __global__ __launch_bounds__(kBlock) void place_returns(const OwnerShard *__rest
   shards[d].ret_delta[s] = before - shards[d].seg_dev[s];
 }
 
-// kPackAhead rows to return per group of LPR lanes; which rows, scan_positions has listed.  A row goes straight into
+// kPackAhead rows to return per group of LPR lanes (two, four of many rows); which rows, scan_positions has listed.  A row goes straight into
 // the buffers of the shard that asked for it (in one process a plain device address, between GPUs peer memory).
-#ifndef HCTR_PACK_AHEAD
-#define HCTR_PACK_AHEAD 2
-#endif
-constexpr int kPackAhead = HCTR_PACK_AHEAD;
+// Four where that leaves kPackBlocks blocks at least: what a block does before its first row -- two tables, a barrier, the list --
+// is then shared by more rows (rows of 128 floats, 16 k for each of seven owners: 58.6 -> 47.7 us); a small launch is as long as its
+// longest block (rows of 32 floats, four owners of 5 k: 8.2 us with two, 10.4 with four).
+constexpr uint32_t kPackBlocks = 4096;
 // The launch has a row of blocks per owner, the first pack_blocks of which do this; the rows behind them do remote_emit.
-template <int VEC, int LPR>
+template <int VEC, int LPR, int kPackAhead>
 __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict__ shards, int nseg, PullShards pulls, uint32_t pack_blocks) {
   if (blockIdx.y >= (uint32_t)nseg) {
     const uint32_t block = (blockIdx.y - nseg) * gridDim.x + blockIdx.x;
@@ -527,33 +527,58 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
 }
 
 
-// One group per unique rank of the current batch, kRefreshRows of them after one another where the batch is large: a block's
-// start -- its record, how many keys there are -- costs as much as a row.  Four batches of 100 k unique keys, 128 floats: 18
-// to 20 us, with two rows per group 23, with one 32.  A batch whose blocks run at once anyway (kRefreshBlocks of them)
-// takes fewer rows per group: four of 20 k unique keys, 32 floats, took 7.3 us with four, 5 with one.
-constexpr int kRefreshRows = 4;
-constexpr uint32_t kRefreshBlocks = 512;
+// The cached rows that came back.  A wave looks at the flags of kWave unique keys at a time, one per lane, lists those that have
+// something to do and copies their rows, a group of LPR lanes per row, four rows on their way at a time.  A group per key, which
+// looked at its flags by itself, took 11.2 us for 314 k unique keys of which none came back into a cached row (now 4.6), 18.8 for
+// four batches of 70 k where some did (17.4), 26.9 where nearly all did (29.2), and 5.2 for four small ones (5.8).
 template <int VEC, int LPR>
 __global__ __launch_bounds__(kBlock) void refresh(PullShards shards) {
   typedef typename RowVec<VEC>::T V;
+  __shared__ uint2 todo[kBlock]; // {resident offset, returned row}, kWave of every wave
   uint32_t block, blocks;
   const PullShard &S = my_record(shards, block, blocks);
   const TableView &t = S.t;
   const BatchView &b = S.b;
   const PullArgs &a = S.a;
-  constexpr int kGroups = kBlock / LPR;
-  const uint32_t U = *b.d_U, gl = threadIdx.x % LPR, W = t.width;
-  for (uint32_t u = block * kGroups + threadIdx.x / LPR; u < U; u += blocks * kGroups) {
-    const slot_t o = b.uoff[u];
-    const bool got = a.got[u] != 0;
-    if (!got || o == kNoSlot || (uint32_t)o >= t.n_cached) continue; // (an owned row that came back is reported by remote_emit)
-    const uint32_t k = a.ret_i[u];
-    if (gl == 0) t.ver[o] = a.in_ver[k];
-    for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
-      const uint32_t col = lane_col<VEC>(c, W);
-      *(V *)(t.emb + (size_t)o * W + col) =
-          *(const V *)(a.in_val + (size_t)k * W + col) + *(const V *)(t.pend + (size_t)o * W + col);
+  constexpr uint32_t kGroups = kWave / LPR; // of a wave
+  const uint32_t U = *b.d_U, lane = threadIdx.x % kWave, gl = lane % LPR, W = t.width;
+  uint2 *const mine = todo + threadIdx.x / kWave * kWave;
+  for (uint32_t u0 = (block * kBlock + threadIdx.x) / kWave * kWave; u0 < U; u0 += blocks * kBlock) {
+    const uint32_t u = u0 + lane, at = min(u, U - 1);
+    const slot_t o = b.uoff[at];
+    const bool work = u < U && a.got[at] != 0 && o != kNoSlot && (uint32_t)o < t.n_cached; // (an owned row that came back is reported by remote_emit)
+    const uint64_t all = __ballot(work);
+    if (!all) continue;
+    if (work) {
+      const uint32_t k = a.ret_i[u];
+      t.ver[o] = a.in_ver[k];
+      mine[__popcll(all & (((uint64_t)1 << lane) - 1))] = make_uint2((uint32_t)o, k);
     }
+    // a wave's LDS operations are done in its own order; the fences keep the compiler from moving them
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t rows = __popcll(all);
+    constexpr uint32_t kAhead = 4; // rows of a group under way together
+    for (uint32_t r = lane / LPR; r < rows; r += kGroups * kAhead) {
+      uint2 w[kAhead];
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) w[k] = mine[min(r + k * kGroups, rows - 1)];
+      for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+        const uint32_t col = lane_col<VEC>(c, W);
+        V in[kAhead], pend[kAhead];
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; k++) {
+          in[k] = *(const V *)(a.in_val + (size_t)w[k].y * W + col);
+          pend[k] = *(const V *)(t.pend + (size_t)w[k].x * W + col);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; k++)
+          if (r + k * kGroups < rows) *(V *)(t.emb + (size_t)w[k].x * W + col) = in[k] + pend[k];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier(); // the list is written again for the next keys
   }
 }
 
@@ -841,12 +866,15 @@ void launch_owner_side(hipStream_t s, const OwnerShard *shards_dev, int nshards,
     hipLaunchKernelGGL(place_returns, dim3(place_blocks + p.cut.total), dim3(kBlock), 0, s, shards_dev, nsrc, p, place_blocks);
   });
   with_requesters(queries_max != 0, [&](const PullShards &p, bool owners) {
-#define CALL(V, L)                                                                                                     \
-  do {                                                                                                                 \
-    const uint32_t pack = owners ? guessed_blocks(queries_guess, queries_max, kPackAhead * (kBlock / L)) : 0u;         \
-    const uint32_t across = std::max(pack, 64u); /* few rows to pack: few idle blocks, and few rows of requesters */   \
-    hipLaunchKernelGGL((pack_rows<V, L>), dim3(across, nshards + div_up(p.cut.total, across)), dim3(kBlock), 0, s,     \
-                       shards_dev, nsrc, p, pack);                                                                     \
+    auto blocks = [&](int ahead) { return owners ? guessed_blocks(queries_guess, queries_max, ahead * (kBlock / lpr)) : 0u; };
+    const bool four = (uint64_t)blocks(4) * nshards >= kPackBlocks;
+    const uint32_t pack = blocks(four ? 4 : 2);
+    const uint32_t across = std::max(pack, 64u); // few rows to pack: few idle blocks, and few rows of requesters
+    const dim3 grid(across, nshards + div_up(p.cut.total, across));
+#define CALL(V, L)                                                                                             \
+  do {                                                                                                         \
+    if (four) hipLaunchKernelGGL((pack_rows<V, L, 4>), grid, dim3(kBlock), 0, s, shards_dev, nsrc, p, pack);    \
+    else hipLaunchKernelGGL((pack_rows<V, L, 2>), grid, dim3(kBlock), 0, s, shards_dev, nsrc, p, pack);         \
   } while (0)
     HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
@@ -858,11 +886,7 @@ void launch_refresh(hipStream_t s, const PullShard *shards, int count) {
   if (!count) return;
   const uint32_t width = shards[0].t.width;
   const int vec = row_vec(width, nullptr), lpr = lanes_for(width, vec);
-  const uint32_t groups = kBlock / lpr;
-  auto blocks = [&](const PullShard &o) {
-    return std::max(guessed_blocks(o.unique_guess, o.b.n, groups * kRefreshRows),
-                    std::min(kRefreshBlocks, guessed_blocks(o.unique_guess, o.b.n, groups)));
-  };
+  auto blocks = [&](const PullShard &o) { return guessed_blocks(o.unique_guess, o.b.n, kBlock); };
   for_shards(shards, count, blocks, [&](const PullShards &p, int) {
 #define CALL(V, L) hipLaunchKernelGGL((refresh<V, L>), grid_of(p), dim3(kBlock), 0, s, p)
     HCTR_DISPATCH_ROW(vec, lpr, CALL);
