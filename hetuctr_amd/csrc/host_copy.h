@@ -23,10 +23,12 @@ class HostStager {
   void copy(void *dst, const void *src, size_t bytes, hipStream_t s, bool narrow_ids = false);
 
   // The same without the transfer, for kLendUpTo bytes at most: returns the staging buffer, filled, at the address a kernel
-  // launched on `s` reads it through the bus.  The caller waits for that kernel before the next call on this object.
+  // launched on `s` reads it through the bus.  The caller waits for that kernel before the next call on this object (preprocess
+  // does: for the whole index of the batch before).
   // A training step whose ids arrive this way against one with the transfer (rows of 64 floats, MI355X): 53 k ids 73 us
   // instead of 110, 213 k 129 (168), 262 k -- the most that are lent -- 146 (184).  The line is lower than
-  // it need be: lent as well, 426 k ids took 201 us instead of 247 and 1.7 M 635 instead of 651.
+  // it need be: lent as well, 426 k ids took 201 us instead of 247 and 1.7 M 635 instead of 651.  (All of it while
+  // preprocess still waited for the kernel that reads the ids.)
   static constexpr size_t kLendUpTo = 2 << 20;
   const void *lend(const void *src, size_t bytes, hipStream_t s, bool narrow_ids);
   uint32_t largest() const { return largest_; } // of the ids the last call narrowed, as 32-bit ones
