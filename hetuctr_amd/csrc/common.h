@@ -26,12 +26,16 @@ struct Error : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
 
+// The runtime keeps an error of this thread until somebody asks for it: what is thrown here is not to be found again by the
+// caller's next launch, or this library's.
 #define HCTR_HIP(expr)                                                                              \
   do {                                                                                              \
     hipError_t e__ = (expr);                                                                        \
-    if (e__ != hipSuccess)                                                                          \
+    if (e__ != hipSuccess) {                                                                        \
+      (void)hipGetLastError();                                                                      \
       throw ::hctr::Error(std::string(#expr) + " failed: " + hipGetErrorString(e__) + " (" + __FILE__ + \
                           ":" + std::to_string(__LINE__) + ")");                                   \
+    }                                                                                               \
   } while (0)
 
 #define HCTR_CHECK(cond, msg)                                   \

@@ -1252,7 +1252,6 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
     if (!taken) {
       stop_work();
       index_pending = index_rest_pending = lists_running_ = false;
-      (void)hipGetLastError(); // a failed allocation is not the next launch's error
       for (Shard *m : members) {
         m->mirror->key_err = 0;
         m->keys_unread_ = false; // (and no kernel may have been launched that would say otherwise)

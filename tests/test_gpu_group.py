@@ -437,3 +437,62 @@ def test_one_shard_reads_its_ids_by_word_and_the_other_by_event(large):
         for r in range(2):
             assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
     p.close()
+
+
+def fill_the_gpu(leave):
+    # holds of device memory after which at most `leave` bytes are free
+    held = []
+    torch.cuda.empty_cache()
+    torch.cuda.synchronize()
+    for piece in (1 << 30, 16 << 20):
+        while torch.cuda.mem_get_info()[0] > leave + piece // 2:
+            free = torch.cuda.mem_get_info()[0]
+            try:
+                held.append(torch.empty(max(free - (1 << 30), piece), dtype=torch.uint8, device="cuda"))
+            except torch.OutOfMemoryError:
+                break
+    assert torch.cuda.mem_get_info()[0] <= leave + (16 << 20)
+    return held
+
+
+@pytest.mark.parametrize("repeats", [2])
+def test_step_without_memory_for_its_push_plan(repeats):
+    # The first step of a pair of batch buffers plans their push last, behind everything else it allocates.  No room for that plan:
+    # the step fails, and the steps after it do what they do where there was room (nothing is pushed in the step that
+    # fails and no row is cached: the tables are the same either way).
+    n, width, leave = 20_000_000, 4, 48 << 20        # the plan asks for 90 MB at a time
+    length = n // repeats
+    say("no memory for a push plan", repeats)
+    gen = torch.Generator(device="cuda")
+    tables = []
+    for short in (True, False):
+        gen.manual_seed(repeats)
+        root = (np.arange(length) % 2).astype(np.uint8)
+        p = Pair(2, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(2)],
+                 init=("Uniform", -0.01, 0.01), lr=0.05, with_oracle=False)
+        tables.append(p.tables)
+        dst = torch.empty((n, width), device="cuda")
+        prev = 0
+        for step in range(4):
+            k = n if step < 2 else n // 4
+            ids = torch.randperm(n, device="cuda", generator=gen)[:k] % length
+            grad = torch.randn((prev, width), device="cuda", generator=gen) if step > 1 else None
+            torch.cuda.synchronize()
+            capi.group_preprocess(p.tables, [ids.data_ptr(), 0], [k, 0])
+            args = (p.tables, [grad.data_ptr() if grad is not None else 0, 0], [dst.data_ptr(), 0])
+            if short and step == 1:
+                held = fill_the_gpu(leave)
+                with pytest.raises(RuntimeError, match="out of memory"):
+                    capi.group_push_pull(*args)
+                del held
+                torch.cuda.empty_cache()
+            else:
+                capi.group_push_pull(*args)
+            prev = k
+        del ids, grad, dst
+    for r in range(2):
+        for item in (capi.EMBEDDING, capi.VERSION):
+            a, b = (t[r].fetch(item) for t in tables)
+            assert np.array_equal(a, b), "shard %d item %d: %d of %d entries differ" % (r, item, (a != b).sum(), a.size)
+    for t in tables[0] + tables[1]:
+        t.close()
