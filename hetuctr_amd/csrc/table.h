@@ -199,6 +199,7 @@ class Shard {
   bool pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *delta);
   PullArgs pull_args(float *dst) const;
   uint32_t take_list_chunks();
+  void forget_lists();
   void gather_bags(const PullArgs &a, uint32_t bag);
   void write_back(float *dst, uint32_t bag = 1); // one shard
   bool direct_now(uint32_t bag) const; // this step's gather works from the keys and does not wait for the index

@@ -719,6 +719,14 @@ uint32_t Shard::take_list_chunks() {
   return run_list_chunks(cur.n);
 }
 
+// A step that was to build the batch's run lists has failed, and whether its gather was launched nobody knows (it is not at
+// work any more): the lists are empty again, and whoever needs them next builds all of them.
+void Shard::forget_lists() {
+  if (cur.n == 0) return;
+  (void)hipMemsetAsync(cur.dnlong.p, 0, 4 * kRunCounters, group->stream);
+  cur.lists_ready = false;
+}
+
 // several shards: this shard's part of the launches on the requesters' own batches; false: its batch is empty
 bool Shard::pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *delta) {
   if (cur.n == 0) {
@@ -1441,6 +1449,7 @@ void Group::push_pull_all(const float *const *grads, float *const *dsts, size_t 
     // when the caller sees the error, and an index that this call started to join is handed back to the next call
     // that needs it (flush_index takes its results over) instead of being dropped with its batch.
     stop_work();
+    for (Shard *m : members) m->forget_lists();
     if (index_joining_) index_pending = true;
     index_joining_ = false;
     throw;

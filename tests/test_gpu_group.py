@@ -455,7 +455,7 @@ def fill_the_gpu(leave):
     return held
 
 
-@pytest.mark.parametrize("repeats", [2])
+@pytest.mark.parametrize("repeats", [2, 20, 400])
 def test_step_without_memory_for_its_push_plan(repeats):
     # The first step of a pair of batch buffers plans their push last, behind everything else it allocates.  No room for that plan:
     # the step fails, and the steps after it do what they do where there was room (nothing is pushed in the step that
