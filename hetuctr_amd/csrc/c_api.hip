@@ -198,7 +198,10 @@ int hctr_last_times(hctr_table *t, float *preprocess_ms, float *push_pull_ms) {
   return guarded([&] {
     HCTR_CHECK(t && t->shard, "null table");
     HCTR_CHECK(t->shard->group->time_calls, "call timing is off: switch it on with hctr_call_timing(t, 1) first");
-    if (preprocess_ms) *preprocess_ms = t->shard->last_pre_ms;
+    if (preprocess_ms) {
+      t->shard->group->take_pre_time();
+      *preprocess_ms = t->shard->last_pre_ms;
+    }
     if (push_pull_ms) *push_pull_ms = t->shard->last_pp_ms;
   });
 }

@@ -289,7 +289,7 @@ class Group {
   const int device_id;
   const std::string key;
   hipStream_t stream = nullptr;          // the stream the stages enqueue on (see StreamSwitch)
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_pre0 = nullptr, ev_pre1 = nullptr; // call timing: of push_pull, of preprocess
   // Single shard: preprocess enqueues its work on a second stream and returns once the caller's ids are consumed;
   // sorting and deduplicating them has no dependence on the pending gradient push, so the next push_pull starts the
   // push on the main stream right away and only the gather waits for both.
@@ -332,6 +332,7 @@ class Group {
   bool queries_seen_ = false;
   DeviceBuf rq_idx_all, rq_ver_all, rq_outdated_all, rq_slot_all, rq_ret_all, query_delta_dev;
   bool time_calls = false;               // bracket the two calls with events (hctr_call_timing)
+  bool pre_timed_ = false;               // the events of the last preprocess are recorded and nobody has asked for the time
   std::vector<Shard *> members;
   double wait_seconds = 120.0;
   void sync_stream();
@@ -348,6 +349,7 @@ class Group {
   void collect_marks();                  // after a stream sync
   void set_defer_index(bool on);         // switches the early return of preprocess; waits for a pending index first
   void set_call_timing(bool on);         // events around the two calls; the times of earlier calls are forgotten
+  void take_pre_time();                  // last_pre_ms of every shard, waiting for the kernels of the call if need be
   void set_stage_timing(bool on);        // resets the accumulators; waits for a pending index under the group's lock
 
   void join(Shard *s);

@@ -907,8 +907,7 @@ Group::Group(int nr, int dev, std::string k) : nrank(nr), device_id(dev), key(st
   HCTR_HIP(hipEventCreateWithFlags(&ev_plan, hipEventDisableTiming));
   const char *defer = getenv("HETUCTR_DEFER_INDEX");
   defer_index = !(defer && atoi(defer) == 0);
-  HCTR_HIP(hipEventCreate(&ev0));
-  HCTR_HIP(hipEventCreate(&ev1));
+  for (hipEvent_t *e : {&ev0, &ev1, &ev_pre0, &ev_pre1}) HCTR_HIP(hipEventCreate(e));
   a_keys_.resize(nr);
   a_n_.resize(nr);
   a_grad_.resize(nr);
@@ -918,8 +917,8 @@ Group::Group(int nr, int dev, std::string k) : nrank(nr), device_id(dev), key(st
 }
 
 Group::~Group() {
-  if (ev0) (void)hipEventDestroy(ev0);
-  if (ev1) (void)hipEventDestroy(ev1);
+  for (hipEvent_t e : {ev0, ev1, ev_pre0, ev_pre1})
+    if (e) (void)hipEventDestroy(e);
   for (auto &m : marks) { (void)hipEventDestroy(m.a); (void)hipEventDestroy(m.b); }
   for (auto e : event_pool) (void)hipEventDestroy(e);
   if (stream) (void)hipStreamDestroy(stream);
@@ -1014,8 +1013,21 @@ void Group::set_defer_index(bool on) {
 void Group::set_call_timing(bool on) {
   std::lock_guard<std::mutex> lk(mu_);
   time_calls = on;
+  pre_timed_ = false;
   for (Shard *m : members)
     if (m) m->last_pre_ms = m->last_pp_ms = m->last_push_ms = 0.f;
+}
+
+// The device time of the last preprocess, taken over when it is asked for: the call may have returned before its kernels ran.
+void Group::take_pre_time() {
+  std::lock_guard<std::mutex> lk(mu_);
+  if (!pre_timed_) return;
+  float ms = 0.f;
+  HCTR_HIP(hipEventSynchronize(ev_pre1));
+  HCTR_HIP(hipEventElapsedTime(&ms, ev_pre0, ev_pre1));
+  for (Shard *m : members)
+    if (m) m->last_pre_ms = ms;
+  pre_timed_ = false;
 }
 
 void Group::set_stage_timing(bool on) {
@@ -1249,6 +1261,7 @@ void Group::preprocess_all(const int64_t *const *keys, const size_t *n) {
   flush_index(); // preprocess twice in a row: the earlier batch is indexed before it becomes the previous one
   finish_lists();
   for (Shard *m : members) m->swap_batches();
+  pre_timed_ = false;
   bool taken = false;
   try {
     preprocess_steps(keys, n, taken);
@@ -1294,9 +1307,9 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
     // follows from push_pull once the push kernel is in its queue.
     Shard *m = members[0];
     StreamSwitch on(*this, index_stream);
-    if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
+    if (time_calls) HCTR_HIP(hipEventRecord(ev_pre0, stream));
     m->ingest_keys(keys[0], n[0], &m->mirror->key_err); // the flag lives in pinned host memory the kernel can write
-    if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
+    if (time_calls) HCTR_HIP(hipEventRecord(ev_pre1, stream));
     if (!m->read_.word) HCTR_HIP(hipEventRecord(ev_keys, stream));
     const bool lists = m->trains_ && m->prev.n != 0 && !m->prev.lists_ready;
     if (lists) m->cur.early_sort_steps = kEarlySortStepsBesideLists;
@@ -1312,12 +1325,7 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
     }
     const bool bad_key = m->staged_ ? m->ids_bad_ : wait_ids_read();
     taken = true;
-    if (time_calls) {
-      float ms = 0.f;
-      HCTR_HIP(hipEventSynchronize(ev1));
-      HCTR_HIP(hipEventElapsedTime(&ms, ev0, ev1));
-      m->last_pre_ms = ms;
-    }
+    pre_timed_ = time_calls;
     if (bad_key) throw Error("hetuCTR: preprocess: a key lies outside [0, length) (it was treated as id 0)");
     return;
   }
@@ -1335,10 +1343,10 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
     plan_batches(late, &Shard::prev);
     {
       StreamSwitch on(*this, index_stream);
-      if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
+      if (time_calls) HCTR_HIP(hipEventRecord(ev_pre0, stream));
       for (Shard *m : members) m->prepare_keys(keys[m->cfg.rank], n[m->cfg.rank], &m->mirror->key_err);
       launch_keys(members.data(), members.size());
-      if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
+      if (time_calls) HCTR_HIP(hipEventRecord(ev_pre1, stream));
       HCTR_HIP(hipEventRecord(ev_keys, stream));
     }
     // Only the first launches of the index go out here (they keep the GPU busy until the pushes arrive); the rest
@@ -1349,17 +1357,12 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
     if (!late.empty()) sync_stream();
     for (Shard *m : late) m->finish_plan(m->prev);
     taken = true;
-    float ms = 0.f;
-    if (time_calls) {
-      HCTR_HIP(hipEventSynchronize(ev1));
-      HCTR_HIP(hipEventElapsedTime(&ms, ev0, ev1));
-    }
-    for (Shard *m : members) m->last_pre_ms = ms;
+    pre_timed_ = time_calls;
     exchange_shapes();
     if (bad_key) throw Error("hetuCTR: preprocess: a key lies outside [0, length) (it was treated as id 0)");
     return;
   }
-  if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
+  if (time_calls) HCTR_HIP(hipEventRecord(ev_pre0, stream));
   std::vector<Shard *> unplanned;
   for (Shard *m : members) {
     m->preprocess_index(keys[m->cfg.rank], n[m->cfg.rank]);
@@ -1368,15 +1371,13 @@ void Group::preprocess_steps(const int64_t *const *keys, const size_t *n, bool &
   enqueue_bucket_sizes(true);
   plan_batches(unplanned, &Shard::prev);
   for (Shard *m : members) m->enqueue_readback_preprocess();
-  if (time_calls) HCTR_HIP(hipEventRecord(ev1, stream));
+  if (time_calls) HCTR_HIP(hipEventRecord(ev_pre1, stream));
   sync_stream();
   taken = true;
-  float ms = 0.f;
-  if (time_calls) HCTR_HIP(hipEventElapsedTime(&ms, ev0, ev1));
+  pre_timed_ = time_calls;
   collect_marks();
   std::string first_error;
   for (Shard *m : members) {
-    m->last_pre_ms = ms;
     try {
       m->finish_preprocess();
     } catch (const Error &e) {

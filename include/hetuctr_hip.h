@@ -147,7 +147,8 @@ int hctr_stream(hctr_table *t, void **stream_out);
 /* Device time of the last preprocess and push_pull calls in milliseconds, measured with HIP events on
  * that stream around the launched work (host-side waits excluded).  The events cost host time in every call, so they
  * are recorded only while hctr_call_timing(t, 1) is in force (off when a table is created; switching it either way
- * zeroes the stored times).  While it is off hctr_last_times and hctr_last_push_ms fail with an error instead of
+ * zeroes the stored times).  Neither call waits for an event of its own: the time of a preprocess whose kernels have not run
+ * yet is waited for by hctr_last_times.  While it is off hctr_last_times and hctr_last_push_ms fail with an error instead of
  * returning stale or zero times.  No counterpart in the reference. */
 int hctr_call_timing(hctr_table *t, int on);
 int hctr_last_times(hctr_table *t, float *preprocess_ms, float *push_pull_ms);
@@ -157,8 +158,10 @@ int hctr_last_times(hctr_table *t, float *preprocess_ms, float *push_pull_ms);
  * seen, e.g. after two hctr_preprocess calls in a row, is planned, and waited for, in this call).  The sort / unique
  * stages of the new batch keep running on a
  * second stream, next to the gradient push that the following hctr_push_pull starts, and are waited for before the
- * rows are gathered (several shards: before the queries are built).  preprocess_ms above is then the time up to
- * that return, push_pull_ms covers the rest.  Anything that needs the batch's index earlier (a second hctr_preprocess,
+ * rows are gathered (several shards: before the queries are built).  preprocess_ms above is then the device time from
+ * the start of the call to the end of the kernel that reads the ids, push_pull_ms covers the rest.  One shard, a table of
+ * less than 2^32 rows and ids in pageable host memory: the call returns when the ids are staged in pinned memory, and that
+ * kernel, for larger batches behind a transfer, may end after the next push_pull has begun (the two times then overlap).  Anything that needs the batch's index earlier (a second hctr_preprocess,
  * hctr_debug_fetch, hctr_stage_timing) waits for it.  HETUCTR_DEFER_INDEX=0 in the environment restores a
  * preprocess that returns only when all its work is done (hetu_gpu_table.cu:64); with stage timing on it always is.
  * hctr_last_push_ms (needs hctr_call_timing, like hctr_last_times): device time from the start of the last hctr_push_pull to the end of its push stage, i.e. the

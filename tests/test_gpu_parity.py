@@ -955,3 +955,39 @@ def test_ids_overwritten_where_a_push_follows_the_three_launch_passes(n, monkeyp
     with pytest.raises(RuntimeError, match="outside"):
         p.tables[0].preprocess(bad.data_ptr(), n)
     p.close()
+
+
+@pytest.mark.parametrize("n", [5_000, 300_000])
+def test_timed_preprocess_of_staged_ids_returns_as_early(n):
+    # ids in pageable memory, lent to the key kernel and sent by a transfer: with call timing on preprocess returns when they are
+    # staged as well, and the time of its kernels is waited for by whoever asks.  The caller's default stream, which the library's
+    # streams come behind, is kept busy: what the call enqueues cannot have run when it returns.
+    import torch
+    say("timed preprocess of staged ids", n)
+    length, width = 40_000, 8
+    rng = np.random.default_rng(n)
+    p = single(length, width, lr=0.05)
+    t = p.tables[0]
+    t.call_timing(True)
+    a = torch.randn(8192, 8192, device="cuda")
+    b = torch.empty_like(a)
+    dst = torch.empty((n, width), device="cuda")
+    busy = torch.cuda.Event()
+    for step in range(4):
+        keys = rng.integers(0, length, n).astype(np.int64)
+        torch.mm(a, a, out=b)                             # (its first launch loads code)
+        torch.cuda.synchronize()
+        for _ in range(10):
+            torch.mm(a, a, out=b)
+        busy.record()
+        t.preprocess(keys.ctypes.data, n)
+        if step > 1:                                      # either batch has its buffers (allocating them may wait)
+            assert not busy.query(), "preprocess waited for its kernels"
+        if step == 2:
+            assert t.last_times()[0] > 0 and busy.query() # asked for in between
+        t.push_pull(0, dst.data_ptr())
+        assert t.last_times()[0] > 0
+        p.oracle.preprocess([keys])
+        assert_close(dst.cpu().numpy(), p.oracle.push_pull([None])[0], 1e-5, "dst step %d" % step)
+    t.call_timing(False)
+    p.close()
