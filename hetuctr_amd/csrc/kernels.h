@@ -382,7 +382,9 @@ struct PullShard {
   // refresh: scratch of 4 * scan_blocks(n) words; four words the device can write (hit / miss / refreshed counts of the step,
   // error bits)
   uint32_t *tile_counts, *host_stats;
-  uint32_t unique_guess;     // the grid of the row kernel is cut from it (how many keys are unique the kernels read)
+  // what the step before had: unique keys (the grid of the refresh is cut from it; how many there are the kernels read), cached
+  // rows that came back
+  uint32_t unique_guess, refreshed_guess;
 };
 void launch_build_queries(hipStream_t s, const KeyLayout &kl, const PullShard *shards, int count);
 // The refresh of the cached rows that came back.

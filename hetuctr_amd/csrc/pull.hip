@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kBlock) void build_queries(PullShards shards, int i
 // receive buffer is ascending in id (it is a slice of the sender's sorted unique keys), block b takes the ids
 // between two splitters drawn from the longest segment, finds that id range in every other segment by binary search,
 // and walks the sources in order with a barrier between them.  Inside a source ids are distinct, so its rows are
-// applied in parallel, kAhead rows per group of LPR lanes at a time.
+// applied in parallel, kRefreshAhead rows per group of LPR lanes at a time.
 //
 // A search is done by kProbes lanes at once, which cut what is left into kProbes + 1 pieces per round, and both ends of all ranges
 // are searched for side by side: 3 or 4 dependent loads for segments of 5 k rows where one lane per source, one end after the
@@ -131,37 +131,37 @@ __global__ __launch_bounds__(kBlock) void apply_remote_all(const OwnerShard *__r
   }
   __syncthreads();
   const uint32_t gl = threadIdx.x % LPR;
-  constexpr int kAhead = kApplyAhead;
+  constexpr int kRefreshAhead = kApplyAhead;
   bool bad = false;
   for (int s = 0; s < nsrc; s++) {
     const uint32_t end = hi[s];
-    for (uint32_t k0 = lo[s] + threadIdx.x / LPR; k0 < end; k0 += kGroups * kAhead) {
-      slot_t o[kAhead];
-      uint64_t id[kAhead];
+    for (uint32_t k0 = lo[s] + threadIdx.x / LPR; k0 < end; k0 += kGroups * kRefreshAhead) {
+      slot_t o[kRefreshAhead];
+      uint64_t id[kRefreshAhead];
 #pragma unroll
-      for (int a = 0; a < kAhead; a++) id[a] = (uint64_t)rg_idx[min(k0 + a * kGroups, end - 1)];
+      for (int a = 0; a < kRefreshAhead; a++) id[a] = (uint64_t)rg_idx[min(k0 + a * kGroups, end - 1)];
 #pragma unroll
-      for (int a = 0; a < kAhead; a++) {
+      for (int a = 0; a < kRefreshAhead; a++) {
         o[a] = owned_slot(slot, id[a], id_max, n_cached);
         if (k0 + a * kGroups >= end) o[a] = kNoSlot;
         else if (o[a] == kNoSlot) bad = true;
       }
       if (gl == 0) {
 #pragma unroll
-        for (int a = 0; a < kAhead; a++)
+        for (int a = 0; a < kRefreshAhead; a++)
           if (o[a] != kNoSlot) ver[o[a]] += load_once(rg_cnt + k0 + a * kGroups);
       }
       for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
         const uint32_t col = lane_col<VEC>(c, W);
-        V cur[kAhead], add[kAhead];
+        V cur[kRefreshAhead], add[kRefreshAhead];
 #pragma unroll
-        for (int a = 0; a < kAhead; a++) {
+        for (int a = 0; a < kRefreshAhead; a++) {
           if (o[a] == kNoSlot) continue;
           cur[a] = *(const V *)(emb + (size_t)o[a] * W + col);
           add[a] = __builtin_nontemporal_load((const V *)(rg_val + (size_t)(k0 + a * kGroups) * W + col)); // read once: keep it out of the caches
         }
 #pragma unroll
-        for (int a = 0; a < kAhead; a++)
+        for (int a = 0; a < kRefreshAhead; a++)
           if (o[a] != kNoSlot) store_own<VEC>(emb + (size_t)o[a] * W + col, cur[a] + add[a], c - col);
       }
     }
@@ -463,14 +463,14 @@ __global__ __launch_bounds__(kBlock) void place_returns(const OwnerShard *__rest
   shards[d].ret_delta[s] = before - shards[d].seg_dev[s];
 }
 
-// kPackAhead rows to return per group of LPR lanes (two, four of many rows); which rows, scan_positions has listed.  A row goes straight into
+// kPackRefreshAhead rows to return per group of LPR lanes (two, four of many rows); which rows, scan_positions has listed.  A row goes straight into
 // the buffers of the shard that asked for it (in one process a plain device address, between GPUs peer memory).
 // Four where that leaves kPackBlocks blocks at least: what a block does before its first row -- two tables, a barrier, the list --
 // is then shared by more rows (rows of 128 floats, 16 k for each of seven owners: 58.6 -> 47.7 us); a small launch is as long as its
 // longest block (rows of 32 floats, four owners of 5 k: 8.2 us with two, 10.4 with four).
 constexpr uint32_t kPackBlocks = 4096;
 // The launch has a row of blocks per owner, the first pack_blocks of which do this; the rows behind them do remote_emit.
-template <int VEC, int LPR, int kPackAhead>
+template <int VEC, int LPR, int kPackRefreshAhead>
 __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict__ shards, int nseg, PullShards pulls, uint32_t pack_blocks) {
   if (blockIdx.y >= (uint32_t)nseg) {
     const uint32_t block = (blockIdx.y - nseg) * gridDim.x + blockIdx.x;
@@ -488,15 +488,15 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
   const uint32_t total = sseg[nseg]; // rows this shard returns: known on the device only, the grid is cut for the most
   const embed_t *__restrict__ emb = S.t.emb;
   const uint32_t gl = threadIdx.x % LPR, W = S.t.width;
-  for (uint32_t k0 = blockIdx.x * (kGroups * kPackAhead) + threadIdx.x / LPR; k0 < total; k0 += pack_blocks * (kGroups * kPackAhead)) {
-  slot_t o[kPackAhead];
+  for (uint32_t k0 = blockIdx.x * (kGroups * kPackRefreshAhead) + threadIdx.x / LPR; k0 < total; k0 += pack_blocks * (kGroups * kPackRefreshAhead)) {
+  slot_t o[kPackRefreshAhead];
 #pragma unroll
-  for (int a = 0; a < kPackAhead; a++) o[a] = k0 + a * kGroups < total ? S.ret_slot[k0 + a * kGroups] : kNoSlot;
+  for (int a = 0; a < kPackRefreshAhead; a++) o[a] = k0 + a * kGroups < total ? S.ret_slot[k0 + a * kGroups] : kNoSlot;
   // the requester of every row: the segment of the return order it lies in (segments may be empty)
-  embed_t *dst_val[kPackAhead];
-  version_t *dst_ver[kPackAhead];
+  embed_t *dst_val[kPackRefreshAhead];
+  version_t *dst_ver[kPackRefreshAhead];
 #pragma unroll
-  for (int a = 0; a < kPackAhead; a++) {
+  for (int a = 0; a < kPackRefreshAhead; a++) {
     const uint32_t k = min(k0 + a * kGroups, total - 1);
     uint32_t lo = 0, hi = nseg - 1;
     while (lo < hi) { // the first segment that ends behind k
@@ -510,29 +510,67 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
   }
   if (gl == 0) {
 #pragma unroll
-    for (int a = 0; a < kPackAhead; a++)
+    for (int a = 0; a < kPackRefreshAhead; a++)
       if (o[a] != kNoSlot) *dst_ver[a] = S.t.ver[o[a]];
   }
   for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
     const uint32_t col = lane_col<VEC>(c, W);
-    V v[kPackAhead];
+    V v[kPackRefreshAhead];
 #pragma unroll
-    for (int a = 0; a < kPackAhead; a++)
+    for (int a = 0; a < kPackRefreshAhead; a++)
       if (o[a] != kNoSlot) v[a] = *(const V *)(emb + (size_t)o[a] * W + col);
 #pragma unroll
-    for (int a = 0; a < kPackAhead; a++)
+    for (int a = 0; a < kPackRefreshAhead; a++)
       if (o[a] != kNoSlot) __builtin_nontemporal_store(v[a], (V *)(dst_val[a] + col)); // read next by another shard's kernels
   }
   }
 }
 
 
-// The cached rows that came back.  A wave looks at the flags of kWave unique keys at a time, one per lane, lists those that have
-// something to do and copies their rows, a group of LPR lanes per row, four rows on their way at a time.  A group per key, which
-// looked at its flags by itself, took 11.2 us for 314 k unique keys of which none came back into a cached row (now 4.6), 18.8 for
-// four batches of 70 k where some did (17.4), 26.9 where nearly all did (29.2), and 5.2 for four small ones (5.8).
+// The cached rows that came back, in one of three ways.  What bounds them: a chain of three loads (flags, where the row came
+// back, the row), and where many rows came back the memory.
+//  * A group of LPR lanes per unique key, up to kRefreshEachBlocks blocks of those: they run at once, and nothing is as short.
+//  * A wave looks at the flags of `flags` unique keys, one per lane, lists those that have something to do and copies their rows, a
+//    group per row, kRefreshAhead rows on their way at a time: at as many keys as its groups copy in one go, where most
+//    rows come back (in the step before they did) or ...
+//  * ... at kWave keys, where few do and that makes kRefreshSparseBlocks blocks at least: most of the work is then to look.
+// us on an MI355X, four shards, by unique keys of each shard; none / three quarters of them came back into a cached row:
+//     rows of 32 floats       first way      second        third       | of 128: first       second          third
+//     3.7 k / 2.3 k           2.4 /  4.5     2.8 /  5.3    2.8 /  6.8  |    3.8 /   5.7     2.3 /   6.6    2.7 /  14.1
+//      25 k / 15.5 k          3.2 /  7.3     2.5 /  7.2    2.5 /  8.6  |    7.6 /  17.3     3.9 /  15.5    4.2 /  22.3
+//     125 k / 78 k            9.1 / 21.5     4.9 / 19.1    4.3 / 21.6  |   28.2 /  73.9    12.2 /  65.6    4.6 /  76.7
+//     500 k / 310 k          28.4 / 80.1    13.5 / 71.4    9.0 / 73.5  |  103.7 / 295.4    39.4 / 278.4    9.3 / 289.1
+// Half of them: the second way 41.0, the third 44.0 (78 k, 128 floats), 45.0 and 44.5 (310 k, 32 floats); a quarter: 30.7 and 28.2,
+// 33.6 and 28.8.  A group per key that goes on to the next key, four in a row, took 16.5 / 70.6 us (78 k, 128 floats)
+// and 55.3 / 274.8 (310 k).
+constexpr uint32_t kRefreshAhead = 4;
+constexpr uint64_t kRefreshEachBlocks = 1536, kRefreshSparseBlocks = 512;
 template <int VEC, int LPR>
-__global__ __launch_bounds__(kBlock) void refresh(PullShards shards) {
+__global__ __launch_bounds__(kBlock) void refresh_each(PullShards shards) {
+  typedef typename RowVec<VEC>::T V;
+  uint32_t block, blocks;
+  const PullShard &S = my_record(shards, block, blocks);
+  const TableView &t = S.t;
+  const BatchView &b = S.b;
+  const PullArgs &a = S.a;
+  constexpr uint32_t kGroups = kBlock / LPR;
+  const uint32_t U = *b.d_U, gl = threadIdx.x % LPR, W = t.width;
+  for (uint32_t u = block * kGroups + threadIdx.x / LPR; u < U; u += blocks * kGroups) {
+    const slot_t o = b.uoff[u];
+    const bool got = a.got[u] != 0;
+    if (!got || o == kNoSlot || (uint32_t)o >= t.n_cached) continue; // (an owned row that came back is reported by remote_emit)
+    const uint32_t k = a.ret_i[u];
+    if (gl == 0) t.ver[o] = a.in_ver[k];
+    for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
+      const uint32_t col = lane_col<VEC>(c, W);
+      *(V *)(t.emb + (size_t)o * W + col) =
+          *(const V *)(a.in_val + (size_t)k * W + col) + *(const V *)(t.pend + (size_t)o * W + col);
+    }
+  }
+}
+
+template <int VEC, int LPR>
+__global__ __launch_bounds__(kBlock) void refresh(PullShards shards, uint32_t flags) {
   typedef typename RowVec<VEC>::T V;
   __shared__ uint2 todo[kBlock]; // {resident offset, returned row}, kWave of every wave
   uint32_t block, blocks;
@@ -543,10 +581,10 @@ __global__ __launch_bounds__(kBlock) void refresh(PullShards shards) {
   constexpr uint32_t kGroups = kWave / LPR; // of a wave
   const uint32_t U = *b.d_U, lane = threadIdx.x % kWave, gl = lane % LPR, W = t.width;
   uint2 *const mine = todo + threadIdx.x / kWave * kWave;
-  for (uint32_t u0 = (block * kBlock + threadIdx.x) / kWave * kWave; u0 < U; u0 += blocks * kBlock) {
+  for (uint32_t u0 = (block * kBlock + threadIdx.x) / kWave * flags; u0 < U; u0 += blocks * (kBlock / kWave) * flags) {
     const uint32_t u = u0 + lane, at = min(u, U - 1);
     const slot_t o = b.uoff[at];
-    const bool work = u < U && a.got[at] != 0 && o != kNoSlot && (uint32_t)o < t.n_cached; // (an owned row that came back is reported by remote_emit)
+    const bool work = lane < flags && u < U && a.got[at] != 0 && o != kNoSlot && (uint32_t)o < t.n_cached; // (an owned row that came back is reported by remote_emit)
     const uint64_t all = __ballot(work);
     if (!all) continue;
     if (work) {
@@ -559,21 +597,20 @@ __global__ __launch_bounds__(kBlock) void refresh(PullShards shards) {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const uint32_t rows = __popcll(all);
-    constexpr uint32_t kAhead = 4; // rows of a group under way together
-    for (uint32_t r = lane / LPR; r < rows; r += kGroups * kAhead) {
-      uint2 w[kAhead];
+    for (uint32_t r = lane / LPR; r < rows; r += kGroups * kRefreshAhead) {
+      uint2 w[kRefreshAhead];
 #pragma unroll
-      for (uint32_t k = 0; k < kAhead; k++) w[k] = mine[min(r + k * kGroups, rows - 1)];
+      for (uint32_t k = 0; k < kRefreshAhead; k++) w[k] = mine[min(r + k * kGroups, rows - 1)];
       for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
         const uint32_t col = lane_col<VEC>(c, W);
-        V in[kAhead], pend[kAhead];
+        V in[kRefreshAhead], pend[kRefreshAhead];
 #pragma unroll
-        for (uint32_t k = 0; k < kAhead; k++) {
+        for (uint32_t k = 0; k < kRefreshAhead; k++) {
           in[k] = *(const V *)(a.in_val + (size_t)w[k].y * W + col);
           pend[k] = *(const V *)(t.pend + (size_t)w[k].x * W + col);
         }
 #pragma unroll
-        for (uint32_t k = 0; k < kAhead; k++)
+        for (uint32_t k = 0; k < kRefreshAhead; k++)
           if (r + k * kGroups < rows) *(V *)(t.emb + (size_t)w[k].x * W + col) = in[k] + pend[k];
       }
     }
@@ -886,9 +923,24 @@ void launch_refresh(hipStream_t s, const PullShard *shards, int count) {
   if (!count) return;
   const uint32_t width = shards[0].t.width;
   const int vec = row_vec(width, nullptr), lpr = lanes_for(width, vec);
-  auto blocks = [&](const PullShard &o) { return guessed_blocks(o.unique_guess, o.b.n, kBlock); };
+  auto blocks_of = [&](const PullShard &o, uint32_t keys) { return guessed_blocks(o.unique_guess, o.b.n, keys); }; // keys per block
+  uint64_t unique = 0, refreshed = 0, each_blocks = 0, sparse_blocks = 0;
+  for (int k = 0; k < count; k++) {
+    unique += shards[k].unique_guess;
+    refreshed += shards[k].refreshed_guess;
+    each_blocks += blocks_of(shards[k], kBlock / lpr);
+    sparse_blocks += blocks_of(shards[k], kBlock);
+  }
+  const bool each = each_blocks <= kRefreshEachBlocks;
+  const bool sparse = 2 * refreshed < unique && sparse_blocks >= kRefreshSparseBlocks;
+  const uint32_t flags = sparse ? kWave : std::min<uint32_t>(kWave, kRefreshAhead * (kWave / lpr));
+  auto blocks = [&](const PullShard &o) { return blocks_of(o, each ? kBlock / lpr : kBlock / kWave * flags); };
   for_shards(shards, count, blocks, [&](const PullShards &p, int) {
-#define CALL(V, L) hipLaunchKernelGGL((refresh<V, L>), grid_of(p), dim3(kBlock), 0, s, p)
+#define CALL(V, L)                                                                            \
+  do {                                                                                        \
+    if (each) hipLaunchKernelGGL((refresh_each<V, L>), grid_of(p), dim3(kBlock), 0, s, p);    \
+    else hipLaunchKernelGGL((refresh<V, L>), grid_of(p), dim3(kBlock), 0, s, p, flags);       \
+  } while (0)
     HCTR_DISPATCH_ROW(vec, lpr, CALL);
 #undef CALL
     HCTR_HIP(hipGetLastError());

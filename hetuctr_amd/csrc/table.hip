@@ -755,6 +755,7 @@ bool Shard::pull_record(PullShard &o, float *dst, uint32_t bag, const uint32_t *
   o.tile_counts = block_sums.as<uint32_t>();
   o.host_stats = mirror->stats;
   o.unique_guess = prev.U ? prev.U : cur.n;
+  o.refreshed_guess = (uint32_t)last_stats[2];
   return true;
 }
 

@@ -496,3 +496,27 @@ def test_step_without_memory_for_its_push_plan(repeats):
             assert np.array_equal(a, b), "shard %d item %d: %d of %d entries differ" % (r, item, (a != b).sum(), a.size)
     for t in tables[0] + tables[1]:
         t.close()
+
+
+@pytest.mark.parametrize("width,n", [(32, 9_000), (1, 90_000), (16, 110_000), (37, 40_000), (64, 12_301), (300, 5_000)])
+def test_cached_rows_come_back_in_every_way_of_the_refresh(width, n):
+    # a group of lanes per key (the first); a wave per 64 keys, or, where most rows came back in the step before or the batch is of
+    # medium size, per as many keys as its groups copy in one go: every shard caches everything, and what the others
+    # push comes back in the next step; look-ups, where nothing does, behind those
+    say("refresh", width, n)
+    rng = np.random.default_rng(width)
+    length = n
+    root = rng.integers(0, 2, length).astype(np.uint8)
+    everything = np.arange(length, dtype=np.int64)
+    p = Pair(2, length, width, root, [everything, everything], init=("Uniform", -0.01, 0.01), lr=0.05)
+    for step in range(6):
+        k = [n - 3 * step, n - 7 * step]
+        p.preprocess([rng.integers(0, length, m) for m in k], device_keys=True)
+        train = 0 < step < 4
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(m, width)).astype(np.float32) if train else None for m in prev] if step else [None] * 2)
+        for r in range(2):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        prev = k
+    p.compare_state(1e-5, "end")
+    p.compare_ints([capi.VERSION, capi.UPDATES, capi.STATS], "end")
+    p.close()
