@@ -45,14 +45,6 @@ constexpr int kBatch = HCTR_TILE_BATCH;   // short role: gradient rows in flight
 constexpr int kInFlight = 16;             // long role: rows in flight per loader thread
 constexpr int kSlice = kSliceColumns;     // long role: columns per block
 constexpr int kLongBlocks = HCTR_LONG_BLOCKS;
-#ifndef HCTR_GIANT_CLASSES
-#define HCTR_GIANT_CLASSES 4
-#endif
-// Long role: the runs cut into slices of kGiantSlice columns are those of the first length classes (>= 16384).  Such a slice costs a
-// block 3.4 ns per row, one of 64 columns 6: only of the longest runs does the chain matter more than the work.  (From 4096 on,
-// the long runs of 8.5 M pooled keys, Zipf 1.4, were done after 451 us instead of 435; from 32768 or 65536 on 434 and 428, but runs
-// of 8 k rows of a batch of 1.7 M keys then took as long as its longest.)
-constexpr int kGiantClasses = HCTR_GIANT_CLASSES;
 constexpr int kMedBlocks = HCTR_MED_BLOCKS;
 
 namespace {
@@ -485,16 +477,18 @@ __device__ __forceinline__ void tell_add(uint32_t *count) {
   if (threadIdx.x % kWave == 0) (void)__hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// runs per bundle: classes halve in length -- one run of 2048 or more, 2 of 1024.., 4, 8, 16; `shrink` halves that
+// the number of long runs of class c, of which lane c has it
+__device__ __forceinline__ uint32_t count_of(uint32_t counts, int c) { return (uint32_t)__builtin_amdgcn_readlane((int)counts, c); }
+
+// log2 of the runs per bundle: classes halve in length -- one run of 2048 or more, 2 of 1024.., 4, 8, 16; `shrink` halves that
 // (down to single runs) for batches with few long runs
-__device__ __forceinline__ uint32_t bundle_runs(int cls, uint32_t shrink) {
-  return cls <= 6 ? 1u : max(min(1u << (cls - 6), (uint32_t)kTable) >> shrink, 1u);
-}
+__device__ __forceinline__ int bundle_log(int cls, int shrink) { return max(min(cls - 6, 4) - shrink, 0); }
+static_assert(kTable == 1 << 4, "the most runs per bundle");
 
 template <int VEC, typename K, int CSC, bool kPooled> // CSC: columns per slice if known at compile time, else 0
 __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
-                                          float *lds, uint4 *tables, uint32_t *shared, float *sums, int c_lo,
-                                          int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
+                                          float *lds, uint4 *tables, uint32_t *shared, float *sums,
+                                          uint32_t counts, int c_lo, int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
   typedef typename Vec<VEC>::T V;
   constexpr uint32_t C = kCols<VEC>;
   constexpr uint32_t kOthers = CSC ? 2 : 1; // waves that do not load
@@ -519,21 +513,24 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
   const uint32_t lane_id = bidx % share;
   const uint32_t n_sl = (slices - lane_id + share - 1) / share; // slices lane_id, lane_id + share, ...
   const uint32_t group_blocks = (nblk - lane_id + share - 1) / share; // blocks drawing from this counter
-  uint32_t cnt[kLongBuckets];
-#pragma unroll
-  for (int c = 0; c < kLongBuckets; c++) cnt[c] = (c >= c_lo && c < c_hi) ? uni(p.d_nlong[c]) : 0u;
+  // Lane c looks after class c of the runs.  (In scalar registers, twelve of them, some of the loaders' were spilled.)
+  const int class_of_lane = threadIdx.x % kWave;
+  counts = class_of_lane >= c_lo && class_of_lane < c_hi ? counts : 0u;
+  if (!__ballot(counts != 0)) return;
   // A block streams a bundle at the pace its rows in flight allow (a few ns per occurrence), whatever the other
   // blocks do: a small batch, whose long runs make fewer tickets than there are blocks to draw them, gets smaller
   // bundles until every block has work or every bundle is a single run.  Every block computes the same value.
-  uint32_t shrink = 0, nbundles;
+  uint32_t nbundles, of_class; // bundles; of this lane's class
+  int shrink = 0;
   for (;;) {
+    const int lg = bundle_log(class_of_lane, shrink);
+    of_class = (counts + (1u << lg) - 1) >> lg;
     nbundles = 0;
 #pragma unroll
-    for (int c = 0; c < kLongBuckets; c++) nbundles += (cnt[c] + bundle_runs(c, shrink) - 1) / bundle_runs(c, shrink);
+    for (int c = 0; c < kLongBuckets; c++) nbundles += count_of(of_class, c);
     if (shrink == 4 || nbundles * slices >= 2 * nblk) break;
     shrink++;
   }
-  if (!nbundles) return;
   const uint32_t tickets = nbundles * n_sl;
 
   // one wave draws a ticket and leaves its bundle in set `to`: descriptors of the runs (one lane per run, which keeps its own
@@ -555,16 +552,16 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
     uint32_t bundle = tk / n_sl;
     int cls = 0;
     uint32_t run0 = 0, runs = 0;
-    bool found = false;
+    asm volatile("" : "+v"(of_class)); // asked anew, not kept in scalar registers
 #pragma unroll
     for (int c = 0; c < kLongBuckets; c++) {
-      const uint32_t bs = bundle_runs(c, shrink), nb = (cnt[c] + bs - 1) / bs;
-      if (!found) {
+      const uint32_t nb = count_of(of_class, c);
+      if (!runs) {
         if (bundle < nb) {
-          found = true;
+          const int lg = bundle_log(c, shrink);
           cls = c;
-          run0 = bundle * bs;
-          runs = min(bs, cnt[c] - run0);
+          run0 = bundle << lg;
+          runs = min(1u << lg, count_of(counts, c) - run0);
         } else {
           bundle -= nb;
         }
@@ -1089,15 +1086,20 @@ __device__ __forceinline__ void push_block(const TableView &t, int id_bits, cons
     // blocks feed each of them (the blocks of a saturated memory system get equal shares of it, and a chain
     // advances with the share of the block that feeds it), then tickets of the other long runs.
     uint32_t *tk = p.d_nlong + kTicketBase;
+    uint32_t counts = p.d_nlong[min(threadIdx.x % kWave, (uint32_t)kLongBuckets - 1)]; // long runs by length class, one per lane
     auto runs = [&](auto csc, int c_lo, int c_hi, uint32_t *counters) {
-      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, sums, c_lo, c_hi, block, kLongBlocks, counters);
+      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, sums, counts, c_lo, c_hi, block, kLongBlocks, counters);
     };
     if constexpr (VEC == 1) {
       runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);
     } else if constexpr (LPR <= 8) { // rows of up to 16 or 32 floats
       runs(std::integral_constant<int, LPR * 4>(), 0, kLongBuckets, tk);
     } else {
-      const int narrow = narrow_slices(t.width) ? kLongBuckets : kGiantClasses;
+      uint64_t rows = 0; // of all long runs, roughly: by the middle of their classes
+#pragma unroll
+      for (int c = 0; c < kLongBuckets; c++) rows += (uint64_t)count_of(counts, c) * (3u << 16 >> c);
+      const int narrow = narrow_slices(t.width) ? kLongBuckets : narrow_classes(t.width, rows, kLongBlocks);
+      asm volatile("" : "+v"(counts)); // read again from here on, not kept in twelve scalar registers
       runs(std::integral_constant<int, kGiantSlice>(), 0, narrow, tk);
       if (narrow < kLongBuckets) runs(std::integral_constant<int, kSlice>(), narrow, kLongBuckets, tk + kTicketLanes);
     }

@@ -818,13 +818,15 @@ def test_run_lengths_around_the_chunks_of_the_push(width, nrank):
 
 
 @pytest.mark.parametrize("nrank", [1, 2])
-@pytest.mark.parametrize("width,lens", [(64, "giants"), (128, "giants"), (130, "giants"), (64, "bundles"), (256, "bundles"), (16, "bundles")])
+@pytest.mark.parametrize("width,lens", [(64, "giants"), (128, "giants"), (130, "giants"), (64, "bundles"), (256, "bundles"), (16, "bundles"), (256, "share")])
 def test_long_runs_of_many_bundles_and_of_the_narrow_slices(width, lens, nrank):
     # giants: runs around 16384 rows, from where on rows are cut into slices of 32 columns, ending inside either half of a chunk of 192;
-    # bundles: several tickets per block, one after the other, of runs a chunk or two long.  Sums bit for bit
+    # bundles: several tickets per block, one after the other, of runs a chunk or two long; share: so many rows in all that runs of 6000
+    # stay in slices of 64 columns, behind those of 9000, which do not.  Sums bit for bit
     say("narrow slices / many bundles", width, lens, nrank)
     rng = np.random.default_rng(17)
     count = np.array([16383, 16384, 16385, 16387, 16416, 16512, 16575, 16576, 16577, 18001] if lens == "giants" else
+                     list(range(5900, 6000, 2)) + list(range(9000, 9010)) if lens == "share" else
                      rng.integers(129, 260, size=1200))
     length = 2 * len(count)
     root = (np.arange(length) % nrank).astype(np.uint8)

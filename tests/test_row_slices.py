@@ -61,3 +61,28 @@ def test_every_width_stays_inside_its_slice(tmp_path):
     out = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
     # half of the widths below 2^24, without 0
     assert (out.returncode, out.stdout) == (0, "ok %d\n" % (2 ** 23 - 1)), out.stdout
+
+
+def test_the_longest_runs_are_cut_narrower_where_they_outlast_a_block_s_share(tmp_path):
+    # the rule in python: classes down to 4096 rows whose runs are half a block's share long at least (four thirds of it, where a row is
+    # one slice of less than 64 columns)
+    src, exe = tmp_path / "classes.cpp", tmp_path / "classes"
+    src.write_text(r"""
+#include <cstdio>
+#include <initializer_list>
+#include "row_slices.h"
+using namespace hctr;
+int main() {
+  for (uint32_t w : {33u, 48u, 63u, 64u, 65u, 128u, 1000u, 1u << 24})
+    for (int e = 0; e < 34; e++)
+      for (uint64_t rows : {1ull << e, (1ull << e) - 1, 3ull << e}) printf("%u %llu %d\n", w, (unsigned long long)rows, narrow_classes(w, rows, 128));
+}
+""")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I" + CSRC, str(src), "-o", str(exe)], check=True)
+    lines = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, check=True).stdout.split("\n")[:-1]
+    assert len(lines) == 8 * 34 * 3
+    for line in lines:
+        w, rows, got = map(int, line.split())
+        share = rows * -(-w // 64) // 128
+        want = [c for c in range(6) if (3 * 2 ** (17 - c) >= 4 * share if w < 64 else 2 * 2 ** (17 - c) >= share)]
+        assert got == len(want), line
