@@ -738,13 +738,15 @@ __device__ __forceinline__ void pool_bag(uint32_t W, uint32_t i0, uint32_t bag, 
       uint32_t row[kPer];
 #pragma unroll
       for (int j = 0; j < kPer; j++) row[j] = row_of(i0 + min(h0 + j * LPR + gl, bag - 1));
-#pragma unroll
-      for (int r = 0; r < kFound; r += kPoolAhead) {
+// Not unrolled: that took 82 registers with 32 lanes, 116 with 64, and half the waves fitted (213 k bags of eight rows of 160 floats
+// 139 us, as a loop 98; of 128 floats 73 and 66).
+#pragma unroll 1
+      for (int r = 0; r < kFound; r += kPoolAhead) { // once, where a lane has several positions
         const uint32_t h = h0 + r;
         if (h >= bag) break;
         const uint32_t n = min(bag - h, (uint32_t)kPoolAhead);
         V v[kPoolAhead];
-        auto fetch = [&](int k) { v[k] = *(const V *)(row_at((uint32_t)__shfl((int)row[(r + k) / LPR], (r + k) % LPR, LPR)) + col); };
+        auto fetch = [&](int k) { v[k] = *(const V *)(row_at((uint32_t)__shfl((int)row[k / LPR], kPer > 1 ? k % LPR : r + k, LPR)) + col); };
         if (n == kPoolAhead) {
 #pragma unroll
           for (int k = 0; k < kPoolAhead; k++) fetch(k);
