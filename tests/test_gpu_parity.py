@@ -1,5 +1,8 @@
 """Parity of the HIP path (through the C ABI) against the CPU oracle on the same seeded inputs.
 Integers bit-exact; fp32 table values and pulled rows within 1e-5 relative (see gpu_util.assert_close)."""
+import os
+import re
+
 import numpy as np
 import pytest
 
@@ -460,33 +463,58 @@ def test_large_batches_of_ids_in_pageable_host_memory():
 
 
 @pytest.mark.parametrize("bag", [1, 5])
-@pytest.mark.parametrize("n", [5, 8_190, 60_000, 262_140, 262_150, 700_000])
-def test_steps_from_ids_still_on_their_way(n, bag):
+@pytest.mark.parametrize("n,way", [(5, "word"), (8_190, "word"), (60_000, "word"), (262_140, "word"), (262_150, "word"), (262_300, "word"), (700_000, "word"),
+                                   (2_200_000, "event"), (60_000, "index"), (300_000, "index")])
+def test_steps_from_ids_still_on_their_way(n, way, bag, monkeypatch):
     # preprocess of ids in pageable memory returns when they are staged: the caller's buffer is overwritten at once, and nothing but
-    # push_pull waits for the kernel that reads them -- its gather from the keys by word, by event, or with the index
+    # push_pull, which follows at once, waits for the kernel that reads them -- its gather from the keys by word, by event (of
+    # more blocks than count themselves), or its sorted gather with the index.  The default stream is kept busy in front
+    # of the two calls: nothing that they enqueue has run before the second one has enqueued all of it.
     import torch
-    say("ids on their way", n, bag)
+    say("ids on their way", n, way, bag)
+    length, width = 40_000, 16 if n < 1 << 20 else 4
+    csrc = os.path.join(os.path.dirname(capi.__file__), "csrc")
+    limit = lambda f, name: int(re.search(name + r"\D*(\d+)", open(os.path.join(csrc, f)).read()).group(1))
+    blocks, tile = limit("kernels.h", "kReadSignalBlocks ="), 16 * limit("radix_sort.h", "HCTR_SORT_BLOCK")
+    # up to 2^20 keys every pass has at most kReadSignalBlocks tiles, from there on of 16 keys per thread (and batches of any kind
+    # go through the three-launch passes)
+    assert (-(-(n - 25) // tile) > blocks) if way == "event" else n < 1 << 20
+    if way == "index":
+        monkeypatch.setenv("HETUCTR_DIRECT_GATHER_MAX", "0")
+        monkeypatch.setenv("HETUCTR_POOLED_FROM_KEYS", "0")
     rng = np.random.default_rng(41)
-    length, width = 40_000, 16
     p = single(length, width, init=("Uniform", -0.01, 0.01), lr=0.05)
     buf, prev = np.zeros(n + 10, np.int64), 0
+    a = torch.randn(8192, 8192, device="cuda")
+    b = torch.mm(a, a)
+    with pytest.raises(RuntimeError, match="null key pointer"):
+        p.tables[0].preprocess(0, 5)                        # (the first exception of a process takes a while to be thrown)
     for step in range(6):
         k = n - 5 * step if n > 30 else n
         want = rng.integers(0, length, size=k).astype(np.int64)
         buf[:k] = want
-        if step == 4:                                       # reported by the call itself, treated as id 0
-            buf[k - 1], want[k - 1] = length, 0
-            with pytest.raises(RuntimeError, match="outside"):
-                p.tables[0].preprocess(buf.ctypes.data, k)
-        else:
-            p.tables[0].preprocess(buf.ctypes.data, k)
-        buf[:] = -1
-        p.oracle.preprocess([want])
         g = rng.normal(0, 1e-3, size=(prev // bag, width)).astype(np.float32) if prev and step != 2 else None
         dst = torch.full((k // bag, width), float("nan"), device="cuda")
         dg = torch.from_numpy(g).cuda() if g is not None else None
         torch.cuda.synchronize()
+        for _ in range(6):
+            torch.mm(a, a, out=b)
+        busy = torch.cuda.Event()
+        busy.record()
+        if step == 4:                                       # reported by the call itself, treated as id 0
+            buf[k - 1], want[k - 1] = length, 0
+        error = ""
+        try:
+            p.tables[0].preprocess(buf.ctypes.data, k)
+        except RuntimeError as e:
+            error = str(e)
+        early = not busy.query()
+        buf[:] = -1
         p.tables[0].push_pull_pooled(dg.data_ptr() if g is not None else 0, dst.data_ptr(), bag)
+        # (the first two allocate their batch's buffers, and from 2^18 keys down the sort needs larger tables)
+        assert early or step < 2 or n == 262_150, "preprocess waited for its kernels"
+        assert ("outside" in error) == (step == 4) and bool(error) == (step == 4), error
+        p.oracle.preprocess([want])
         ref = p.oracle.push_pull_pooled([g], bag)[0] if bag > 1 else p.oracle.push_pull([g])[0]
         assert_close(dst.cpu().numpy(), ref, 1e-5, "dst step %d" % step)
         prev = k
