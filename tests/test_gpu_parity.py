@@ -463,15 +463,50 @@ def test_large_batches_of_ids_in_pageable_host_memory():
 
 
 @pytest.mark.parametrize("bag", [1, 5])
+@pytest.mark.parametrize("n", [5, 8_190, 60_000, 262_140, 262_150, 700_000])
+def test_steps_from_ids_still_on_their_way(n, bag):
+    # preprocess of ids in pageable memory returns when they are staged: the caller's buffer is overwritten at once, and nothing but
+    # push_pull waits for the kernel that reads them -- its gather from the keys by word, by event, or with the index
+    import torch
+    say("ids on their way", n, bag)
+    rng = np.random.default_rng(41)
+    length, width = 40_000, 16
+    p = single(length, width, init=("Uniform", -0.01, 0.01), lr=0.05)
+    buf, prev = np.zeros(n + 10, np.int64), 0
+    for step in range(6):
+        k = n - 5 * step if n > 30 else n
+        want = rng.integers(0, length, size=k).astype(np.int64)
+        buf[:k] = want
+        if step == 4:                                       # reported by the call itself, treated as id 0
+            buf[k - 1], want[k - 1] = length, 0
+            with pytest.raises(RuntimeError, match="outside"):
+                p.tables[0].preprocess(buf.ctypes.data, k)
+        else:
+            p.tables[0].preprocess(buf.ctypes.data, k)
+        buf[:] = -1
+        p.oracle.preprocess([want])
+        g = rng.normal(0, 1e-3, size=(prev // bag, width)).astype(np.float32) if prev and step != 2 else None
+        dst = torch.full((k // bag, width), float("nan"), device="cuda")
+        dg = torch.from_numpy(g).cuda() if g is not None else None
+        torch.cuda.synchronize()
+        p.tables[0].push_pull_pooled(dg.data_ptr() if g is not None else 0, dst.data_ptr(), bag)
+        ref = p.oracle.push_pull_pooled([g], bag)[0] if bag > 1 else p.oracle.push_pull([g])[0]
+        assert_close(dst.cpu().numpy(), ref, 1e-5, "dst step %d" % step)
+        prev = k
+    p.compare_state(1e-5, "end")
+    p.close()
+
+
+@pytest.mark.parametrize("bag", [1, 5])
 @pytest.mark.parametrize("n,way", [(5, "word"), (8_190, "word"), (60_000, "word"), (262_140, "word"), (262_150, "word"), (262_300, "word"), (700_000, "word"),
                                    (2_200_000, "event"), (60_000, "index"), (300_000, "index")])
-def test_steps_from_ids_still_on_their_way(n, way, bag, monkeypatch):
+def test_push_pull_right_behind_a_preprocess_of_staged_ids(n, way, bag, monkeypatch):
     # preprocess of ids in pageable memory returns when they are staged: the caller's buffer is overwritten at once, and nothing but
     # push_pull, which follows at once, waits for the kernel that reads them -- its gather from the keys by word, by event (of
     # more blocks than count themselves), or its sorted gather with the index.  The default stream is kept busy in front
     # of the two calls: nothing that they enqueue has run before the second one has enqueued all of it.
     import torch
-    say("ids on their way", n, way, bag)
+    say("push_pull right behind staged ids", n, way, bag)
     length, width = 40_000, 16 if n < 1 << 20 else 4
     csrc = os.path.join(os.path.dirname(capi.__file__), "csrc")
     limit = lambda f, name: int(re.search(name + r"\D*(\d+)", open(os.path.join(csrc, f)).read()).group(1))
@@ -846,16 +881,39 @@ def test_run_lengths_around_the_chunks_of_the_push(width, nrank):
 
 
 @pytest.mark.parametrize("nrank", [1, 2])
-@pytest.mark.parametrize("width,lens", [(64, "giants"), (128, "giants"), (130, "giants"), (64, "bundles"), (256, "bundles"), (16, "bundles"), (256, "share")])
+@pytest.mark.parametrize("width,lens", [(64, "giants"), (128, "giants"), (130, "giants"), (64, "bundles"), (256, "bundles"), (16, "bundles")])
 def test_long_runs_of_many_bundles_and_of_the_narrow_slices(width, lens, nrank):
     # giants: runs around 16384 rows, from where on rows are cut into slices of 32 columns, ending inside either half of a chunk of 192;
-    # bundles: several tickets per block, one after the other, of runs a chunk or two long; share: so many rows in all that runs of 6000
-    # stay in slices of 64 columns, behind those of 9000, which do not.  Sums bit for bit
+    # bundles: several tickets per block, one after the other, of runs a chunk or two long.  Sums bit for bit
     say("narrow slices / many bundles", width, lens, nrank)
     rng = np.random.default_rng(17)
     count = np.array([16383, 16384, 16385, 16387, 16416, 16512, 16575, 16576, 16577, 18001] if lens == "giants" else
-                     list(range(5900, 6000, 2)) + list(range(9000, 9010)) if lens == "share" else
                      rng.integers(129, 260, size=1200))
+    length = 2 * len(count)
+    root = (np.arange(length) % nrank).astype(np.uint8)
+    p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
+             init=("Uniform", -0.01, 0.01), lr=0.05)
+    prev_n = [0] * nrank
+    for step in range(2):
+        keys = [np.repeat(rng.permutation(length)[:len(count)].astype(np.int64), count) for _ in range(nrank)]
+        for k in keys:
+            rng.shuffle(k)
+        p.preprocess(keys, device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(n, width)).astype(np.float32) for n in prev_n])
+        for r in range(nrank):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        p.compare_state(1e-5, "step %d" % step)
+        prev_n = [k.shape[0] for k in keys]
+    p.close()
+
+
+@pytest.mark.parametrize("nrank", [1, 2])
+def test_long_runs_around_a_block_s_share(nrank):
+    # so many rows in all that runs of 6000 stay in slices of 64 columns, behind those of 9000, which do not.  Sums bit for bit
+    width = 256
+    say("runs around a block's share", nrank)
+    rng = np.random.default_rng(17)
+    count = np.array(list(range(5900, 6000, 2)) + list(range(9000, 9010)))
     length = 2 * len(count)
     root = (np.arange(length) % nrank).astype(np.uint8)
     p = Pair(nrank, length, width, root, [np.nonzero(root == r)[0].astype(np.int64) for r in range(nrank)],
