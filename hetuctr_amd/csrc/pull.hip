@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kBlock) void build_queries(PullShards shards, int i
 // receive buffer is ascending in id (it is a slice of the sender's sorted unique keys), block b takes the ids
 // between two splitters drawn from the longest segment, finds that id range in every other segment by binary search,
 // and walks the sources in order with a barrier between them.  Inside a source ids are distinct, so its rows are
-// applied in parallel, kRefreshAhead rows per group of LPR lanes at a time.
+// applied in parallel, kAhead rows per group of LPR lanes at a time.
 //
 // A search is done by kProbes lanes at once, which cut what is left into kProbes + 1 pieces per round, and both ends of all ranges
 // are searched for side by side: 3 or 4 dependent loads for segments of 5 k rows where one lane per source, one end after the
@@ -131,37 +131,37 @@ __global__ __launch_bounds__(kBlock) void apply_remote_all(const OwnerShard *__r
   }
   __syncthreads();
   const uint32_t gl = threadIdx.x % LPR;
-  constexpr int kRefreshAhead = kApplyAhead;
+  constexpr int kAhead = kApplyAhead;
   bool bad = false;
   for (int s = 0; s < nsrc; s++) {
     const uint32_t end = hi[s];
-    for (uint32_t k0 = lo[s] + threadIdx.x / LPR; k0 < end; k0 += kGroups * kRefreshAhead) {
-      slot_t o[kRefreshAhead];
-      uint64_t id[kRefreshAhead];
+    for (uint32_t k0 = lo[s] + threadIdx.x / LPR; k0 < end; k0 += kGroups * kAhead) {
+      slot_t o[kAhead];
+      uint64_t id[kAhead];
 #pragma unroll
-      for (int a = 0; a < kRefreshAhead; a++) id[a] = (uint64_t)rg_idx[min(k0 + a * kGroups, end - 1)];
+      for (int a = 0; a < kAhead; a++) id[a] = (uint64_t)rg_idx[min(k0 + a * kGroups, end - 1)];
 #pragma unroll
-      for (int a = 0; a < kRefreshAhead; a++) {
+      for (int a = 0; a < kAhead; a++) {
         o[a] = owned_slot(slot, id[a], id_max, n_cached);
         if (k0 + a * kGroups >= end) o[a] = kNoSlot;
         else if (o[a] == kNoSlot) bad = true;
       }
       if (gl == 0) {
 #pragma unroll
-        for (int a = 0; a < kRefreshAhead; a++)
+        for (int a = 0; a < kAhead; a++)
           if (o[a] != kNoSlot) ver[o[a]] += load_once(rg_cnt + k0 + a * kGroups);
       }
       for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
         const uint32_t col = lane_col<VEC>(c, W);
-        V cur[kRefreshAhead], add[kRefreshAhead];
+        V cur[kAhead], add[kAhead];
 #pragma unroll
-        for (int a = 0; a < kRefreshAhead; a++) {
+        for (int a = 0; a < kAhead; a++) {
           if (o[a] == kNoSlot) continue;
           cur[a] = *(const V *)(emb + (size_t)o[a] * W + col);
           add[a] = __builtin_nontemporal_load((const V *)(rg_val + (size_t)(k0 + a * kGroups) * W + col)); // read once: keep it out of the caches
         }
 #pragma unroll
-        for (int a = 0; a < kRefreshAhead; a++)
+        for (int a = 0; a < kAhead; a++)
           if (o[a] != kNoSlot) store_own<VEC>(emb + (size_t)o[a] * W + col, cur[a] + add[a], c - col);
       }
     }
@@ -463,14 +463,14 @@ __global__ __launch_bounds__(kBlock) void place_returns(const OwnerShard *__rest
   shards[d].ret_delta[s] = before - shards[d].seg_dev[s];
 }
 
-// kPackRefreshAhead rows to return per group of LPR lanes (two, four of many rows); which rows, scan_positions has listed.  A row goes straight into
+// kPackAhead rows to return per group of LPR lanes (two, four of many rows); which rows, scan_positions has listed.  A row goes straight into
 // the buffers of the shard that asked for it (in one process a plain device address, between GPUs peer memory).
 // Four where that leaves kPackBlocks blocks at least: what a block does before its first row -- two tables, a barrier, the list --
 // is then shared by more rows (rows of 128 floats, 16 k for each of seven owners: 58.6 -> 47.7 us); a small launch is as long as its
 // longest block (rows of 32 floats, four owners of 5 k: 8.2 us with two, 10.4 with four).
 constexpr uint32_t kPackBlocks = 4096;
 // The launch has a row of blocks per owner, the first pack_blocks of which do this; the rows behind them do remote_emit.
-template <int VEC, int LPR, int kPackRefreshAhead>
+template <int VEC, int LPR, int kPackAhead>
 __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict__ shards, int nseg, PullShards pulls, uint32_t pack_blocks) {
   if (blockIdx.y >= (uint32_t)nseg) {
     const uint32_t block = (blockIdx.y - nseg) * gridDim.x + blockIdx.x;
@@ -488,15 +488,15 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
   const uint32_t total = sseg[nseg]; // rows this shard returns: known on the device only, the grid is cut for the most
   const embed_t *__restrict__ emb = S.t.emb;
   const uint32_t gl = threadIdx.x % LPR, W = S.t.width;
-  for (uint32_t k0 = blockIdx.x * (kGroups * kPackRefreshAhead) + threadIdx.x / LPR; k0 < total; k0 += pack_blocks * (kGroups * kPackRefreshAhead)) {
-  slot_t o[kPackRefreshAhead];
+  for (uint32_t k0 = blockIdx.x * (kGroups * kPackAhead) + threadIdx.x / LPR; k0 < total; k0 += pack_blocks * (kGroups * kPackAhead)) {
+  slot_t o[kPackAhead];
 #pragma unroll
-  for (int a = 0; a < kPackRefreshAhead; a++) o[a] = k0 + a * kGroups < total ? S.ret_slot[k0 + a * kGroups] : kNoSlot;
+  for (int a = 0; a < kPackAhead; a++) o[a] = k0 + a * kGroups < total ? S.ret_slot[k0 + a * kGroups] : kNoSlot;
   // the requester of every row: the segment of the return order it lies in (segments may be empty)
-  embed_t *dst_val[kPackRefreshAhead];
-  version_t *dst_ver[kPackRefreshAhead];
+  embed_t *dst_val[kPackAhead];
+  version_t *dst_ver[kPackAhead];
 #pragma unroll
-  for (int a = 0; a < kPackRefreshAhead; a++) {
+  for (int a = 0; a < kPackAhead; a++) {
     const uint32_t k = min(k0 + a * kGroups, total - 1);
     uint32_t lo = 0, hi = nseg - 1;
     while (lo < hi) { // the first segment that ends behind k
@@ -510,17 +510,17 @@ __global__ __launch_bounds__(kBlock) void pack_rows(const OwnerShard *__restrict
   }
   if (gl == 0) {
 #pragma unroll
-    for (int a = 0; a < kPackRefreshAhead; a++)
+    for (int a = 0; a < kPackAhead; a++)
       if (o[a] != kNoSlot) *dst_ver[a] = S.t.ver[o[a]];
   }
   for (uint32_t c = gl * kCols<VEC>; c < W; c += LPR * kCols<VEC>) {
     const uint32_t col = lane_col<VEC>(c, W);
-    V v[kPackRefreshAhead];
+    V v[kPackAhead];
 #pragma unroll
-    for (int a = 0; a < kPackRefreshAhead; a++)
+    for (int a = 0; a < kPackAhead; a++)
       if (o[a] != kNoSlot) v[a] = *(const V *)(emb + (size_t)o[a] * W + col);
 #pragma unroll
-    for (int a = 0; a < kPackRefreshAhead; a++)
+    for (int a = 0; a < kPackAhead; a++)
       if (o[a] != kNoSlot) __builtin_nontemporal_store(v[a], (V *)(dst_val[a] + col)); // read next by another shard's kernels
   }
   }
