@@ -1458,6 +1458,15 @@ void Group::push_pull_all(const float *const *grads, float *const *dsts, size_t 
   }
 }
 
+// The queries of a step are built on the index stream, while the owners apply the pushes, or behind both on the main stream.  Beside
+// them the launch costs the step nothing once the owners take longer than the rest of the index -- they go through one
+// shard's rows after another's, so that both the rows and the shards they come from count -- but the index stream then waits for
+// the pushes and the main stream for the queries.  Two steps on an MI355X, us, beside / behind, by floats of the gradient
+// rows times shards that push: 0.9 M 275 / 265, 2.2 M 307 / 293, 27 M 321 / 316 and 318 / 312, 54 M from one shard 505 / 492,
+// from two 544 / 534, from four 331 / 335, 62 M 399 / 410, 109 M 426 / 435, 533 / 539 and 725 / 737, 218 M (one shard)
+// 1574 / 1590, 436 M 899 / 904 and 1309 / 1320.
+constexpr uint64_t kQueriesBeside = 56ull << 20;
+
 void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint32_t bag) {
   if (time_calls) HCTR_HIP(hipEventRecord(ev0, stream));
   for (Shard *m : members) m->begin_push(grads[m->cfg.rank], bag);
@@ -1481,6 +1490,16 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   const bool join_index = index_pending && !index_not_needed;
   std::vector<PullShard> pulls;
   std::vector<Shard *> pulling;
+  // csrc/core/generate_query.cu:91-106: every query is written where its owner reads it (Group::reserve_queries).  The versions in
+  // it are those of cached rows, which the pushes moved and the owners, who may be applying them, do not.
+  auto build_queries = [&] {
+    StageScope st(*this, S_QUERY);
+    launch_build_queries(stream, members[0]->kl, pulls.data(), (int)pulls.size());
+  };
+  uint64_t pushed = 0, pushing = 0; // floats of the gradient rows, shards they come from
+  for (const Shard *m : members)
+    if (m->prev_active) pushed += (uint64_t)m->prev.n * m->cfg.width, pushing++;
+  const bool queries_beside = pushed * pushing >= kQueriesBeside;
   if (nrank > 1) {
     PullShard r;
     for (Shard *m : members)
@@ -1497,16 +1516,14 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
         StageScope st(*this, S_QUERY);
         launch_place_queries(stream, owner_dev.as<OwnerShard>(), owner_host, nrank, query_area());
       }
-      HCTR_HIP(hipStreamWaitEvent(stream, ev_pushed, 0));
-      {
-        // csrc/core/generate_query.cu:91-106: every query is written where its owner reads it (Group::reserve_queries); the
-        // versions in it are those of cached rows, which the pushes moved and the owners, who are applying them, do not
-        StageScope st(*this, S_QUERY);
-        launch_build_queries(stream, members[0]->kl, pulls.data(), (int)pulls.size());
+      if (queries_beside) {
+        HCTR_HIP(hipStreamWaitEvent(stream, ev_pushed, 0));
+        build_queries();
       }
       HCTR_HIP(hipEventRecord(ev_index, stream));
       // the push plans of the current batches, for the step in which they are the previous ones: after the pushes of
       // this step (they move the update counters the plan reads), beside everything else the step still does
+      if (!queries_beside) HCTR_HIP(hipStreamWaitEvent(stream, ev_pushed, 0));
       plan_batches(members, &Shard::cur);
       HCTR_HIP(hipEventRecord(ev_plan, stream));
     }
@@ -1522,6 +1539,7 @@ void Group::push_pull_steps(const float *const *grads, float *const *dsts, uint3
   }
   if (join_index || nrank > 1) HCTR_HIP(hipStreamWaitEvent(stream, ev_index, 0));
   if (nrank > 1) {
+    if (!queries_beside) build_queries();
     owner_side(queries_max, pulls);
     // the reference waits here for the return counts (hetu_gpu_table.cu:33); they stay on the device
     {

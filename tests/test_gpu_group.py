@@ -520,3 +520,24 @@ def test_cached_rows_come_back_in_every_way_of_the_refresh(width, n):
     p.compare_state(1e-5, "end")
     p.compare_ints([capi.VERSION, capi.UPDATES, capi.STATS], "end")
     p.close()
+
+
+@pytest.mark.parametrize("bound", [0, 5])
+def test_queries_built_beside_the_owners_and_behind_them(bound):
+    # two shards that push n x 128 floats each: 56 Mi floats times shards are reached at 114,688 keys of each.  Steps on either side
+    # of that take turns, with a third of the other shard's rows cached, so that the queries carry versions the pushes move
+    say("queries beside the owners", bound)
+    rng = np.random.default_rng(bound)
+    length, width = 50_000, 128
+    p, root = update_pair(2, length, width, bounds=(bound, bound), init=("Uniform", -0.01, 0.01), lr=0.05, cache="third", seed=3)
+    prev = None
+    for step, n in enumerate([114_688, 114_687, 120_000, 114_680, 114_688, 5_000, 300]):
+        k = [n, n]
+        p.preprocess([rng.integers(0, length, m) for m in k], device_keys=True)
+        out, ref = p.push_pull([rng.normal(0, 1e-3, size=(m, width)).astype(np.float32) for m in prev] if prev else [None] * 2)
+        for r in range(2):
+            assert_close(out[r], ref[r], 1e-5, "dst step %d rank %d" % (step, r))
+        prev = k
+    p.compare_state(1e-5, "end")
+    p.compare_ints([capi.VERSION, capi.UPDATES, capi.STATS], "end")
+    p.close()
