@@ -130,9 +130,10 @@ template <typename T4> struct Vec<1, T4> {
 };
 
 // A gradient row is read exactly once per step: it is loaded past the caches.  With sum-pooled bags (kPooled) a row
-// is read once per key of its bag, so there it is loaded the ordinary way and the repeats hit the cache.
-template <typename R, bool kPooled> __device__ __forceinline__ typename R::T grad_load(const embed_t *p) { // R: a Vec
-  return HCTR_GRAD_NT && !kPooled ? R::load_once(p) : R::load(p);
+// is read once per key of its bag, so there it is loaded the ordinary way and the repeats hit the cache; and so it is
+// in the long role (kAgain) where it shares its lines with its neighbours, see push_block.
+template <typename R, bool kAgain> __device__ __forceinline__ typename R::T grad_load(const embed_t *p) { // R: a Vec
+  return HCTR_GRAD_NT && !kAgain ? R::load_once(p) : R::load(p);
 }
 
 // The version / update counters of unique rank u and its entry among the pushed rows (gradient_index_kernel,
@@ -485,7 +486,8 @@ __device__ __forceinline__ uint32_t count_of(uint32_t counts, int c) { return (u
 __device__ __forceinline__ int bundle_log(int cls, int shrink) { return max(min(cls - 6, 4) - shrink, 0); }
 static_assert(kTable == 1 << 4, "the most runs per bundle");
 
-template <int VEC, typename K, int CSC, bool kPooled> // CSC: columns per slice if known at compile time, else 0
+// CSC: columns per slice if known at compile time, else 0; kAgain: the lines a gradient row lies in are read again
+template <int VEC, typename K, int CSC, bool kPooled, bool kAgain>
 __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const BatchView &p, const PushArgs &a,
                                           float *lds, uint4 *tables, uint32_t *shared, float *sums,
                                           uint32_t counts, int c_lo, int c_hi, uint32_t bidx, uint32_t nblk, uint32_t *counters) {
@@ -656,7 +658,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
       };
       auto read_rows = [&](int k, const embed_t *const (&from)[kRPT]) {
 #pragma unroll
-        for (int q = 0; q < kRPT; q++) val[k][q] = grad_load<Vec<VEC>, kPooled>(from[q]);
+        for (int q = 0; q < kRPT; q++) val[k][q] = grad_load<Vec<VEC>, kAgain>(from[q]);
       };
       for (uint32_t bundle = 0;; bundle++) {
         wait_until(drawn, bundle + 1);
@@ -995,7 +997,7 @@ __device__ __forceinline__ void long_role(const TableView &t, int id_bits, const
           });
         };
         auto row_load = [&](uint32_t pos) -> V { // (the bag of a position where it is read would wait for it)
-          return grad_load<Vec<VEC>, kPooled>((const embed_t *)((const char *)gbase + (uint64_t)grad_row<kPooled>(pos, a.bag) * (W * 4)));
+          return grad_load<Vec<VEC>, kAgain>((const embed_t *)((const char *)gbase + (uint64_t)grad_row<kPooled>(pos, a.bag) * (W * 4)));
         };
         // val[k] holds chunk k and idx[k] the row indices of chunk k + kDepth
         open_cursor(cur, runs);
@@ -1087,21 +1089,29 @@ __device__ __forceinline__ void push_block(const TableView &t, int id_bits, cons
     // advances with the share of the block that feeds it), then tickets of the other long runs.
     uint32_t *tk = p.d_nlong + kTicketBase;
     uint32_t counts = p.d_nlong[min(threadIdx.x % kWave, (uint32_t)kLongBuckets - 1)]; // long runs by length class, one per lane
-    auto runs = [&](auto csc, int c_lo, int c_hi, uint32_t *counters) {
-      long_role<VEC, K, decltype(csc)::value, kPooled>(t, id_bits, p, a, lds, run_table, run_totals, sums, counts, c_lo, c_hi, block, kLongBlocks, counters);
+    auto runs = [&](auto csc, auto again, int c_lo, int c_hi, uint32_t *counters) {
+      long_role<VEC, K, decltype(csc)::value, kPooled, kPooled || decltype(again)::value>(t, id_bits, p, a, lds, run_table, run_totals, sums, counts, c_lo, c_hi, block, kLongBlocks, counters);
     };
     if constexpr (VEC == 1) {
-      runs(std::integral_constant<int, 0>(), 0, kLongBuckets, tk);
+      runs(std::integral_constant<int, 0>(), std::false_type(), 0, kLongBuckets, tk);
     } else if constexpr (LPR <= 8) { // rows of up to 16 or 32 floats
-      runs(std::integral_constant<int, LPR * 4>(), 0, kLongBuckets, tk);
+      // A row that is no whole line shares one with its neighbour, whose key is often the same one (several ids per field), and a
+      // lane reads neighbours in four loads: they are to find the line in the cache.  Loaded past it / not, 5.3 M keys of 18 ids
+      // per field, Zipf 1.2, the push alone on an MI355X: 12 floats 449 / 373 us, 17 floats 540 / 446, 31 floats 702 / 636; 3 ids
+      // per field, 24 floats, 1.6 M keys 124 / 97; one id per field, 20 floats, 2.6 M keys 158 / 132.  Of 32 floats,
+      // which are a line, 432 / 439, and two steps 1370 / 1411: their rows push out what the gather reads.
+      constexpr int kLineFloats = 32;
+      if (LPR * 4 == kLineFloats && t.width == kLineFloats && !kPooled)
+        runs(std::integral_constant<int, LPR * 4>(), std::false_type(), 0, kLongBuckets, tk);
+      else runs(std::integral_constant<int, LPR * 4>(), std::true_type(), 0, kLongBuckets, tk);
     } else {
       uint64_t rows = 0; // of all long runs, roughly: by the middle of their classes
 #pragma unroll
       for (int c = 0; c < kLongBuckets; c++) rows += (uint64_t)count_of(counts, c) * (3u << 16 >> c);
       const int narrow = narrow_slices(t.width) ? kLongBuckets : narrow_classes(t.width, rows, kLongBlocks);
       asm volatile("" : "+v"(counts)); // read again from here on, not kept in twelve scalar registers
-      runs(std::integral_constant<int, kGiantSlice>(), 0, narrow, tk);
-      if (narrow < kLongBuckets) runs(std::integral_constant<int, kSlice>(), narrow, kLongBuckets, tk + kTicketLanes);
+      runs(std::integral_constant<int, kGiantSlice>(), std::false_type(), 0, narrow, tk);
+      if (narrow < kLongBuckets) runs(std::integral_constant<int, kSlice>(), std::false_type(), narrow, kLongBuckets, tk + kTicketLanes);
     }
   } else if (block < kLongBlocks + kMedBlocks) { // medium runs take long per block: they start early
     medium_role<VEC, LPR, K, kSingle, kPooled>(t, id_bits, p, a, (uint32_t *)lds, block - kLongBlocks, kMedBlocks);
