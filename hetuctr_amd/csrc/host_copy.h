@@ -26,9 +26,9 @@ class HostStager {
   // launched on `s` reads it through the bus.  The caller waits for that kernel before the next call on this object (preprocess
   // does: for the whole index of the batch before).
   // A training step whose ids arrive this way against one with the transfer (rows of 64 floats, MI355X): 53 k ids 73 us
-  // instead of 110, 213 k 129 (168), 262 k -- the most that are lent -- 146 (184).  The line is lower than
-  // it need be: lent as well, 426 k ids took 201 us instead of 247 and 1.7 M 635 instead of 651.  (All of it while
-  // preprocess still waited for the kernel that reads the ids.)
+  // instead of 110, 213 k 129 (168), 262 k -- the most that are lent -- 146 (184), all while preprocess still waited for the kernel
+  // that reads the ids.  Since it returns when they are staged, two steps lent and transferred: 426 k ids 340 and 378 us, 852 k
+  // 564 and 554, 1.7 M 1016 and 955, of 128 floats 1425 and 1335.  The line could be half a million ids.
   static constexpr size_t kLendUpTo = 2 << 20;
   const void *lend(const void *src, size_t bytes, hipStream_t s, bool narrow_ids);
   uint32_t largest() const { return largest_; } // of the ids the last call narrowed, as 32-bit ones

@@ -467,7 +467,9 @@ __global__ __launch_bounds__(kBlock) void place_returns(const OwnerShard *__rest
 // the buffers of the shard that asked for it (in one process a plain device address, between GPUs peer memory).
 // Four where that leaves kPackBlocks blocks at least: what a block does before its first row -- two tables, a barrier, the list --
 // is then shared by more rows (rows of 128 floats, 16 k for each of seven owners: 58.6 -> 47.7 us); a small launch is as long as its
-// longest block (rows of 32 floats, four owners of 5 k: 8.2 us with two, 10.4 with four).
+// longest block (rows of 32 floats, four owners of 5 k: 8.2 us with two, 10.4 with four).  Two and four on either side of the line:
+// four owners that all ask, 106 k keys of 64 floats each 36.2 and 31.6, eight, 53 k of 128 68.6 and 62.5 (four is taken); one of four asking,
+// 426 k of 128, 18.1 and 15.9, both of two, 426 k of 32, 35.7 and 24.2 (two is): in the middle the line could be lower.
 constexpr uint32_t kPackBlocks = 4096;
 // The launch has a row of blocks per owner, the first pack_blocks of which do this; the rows behind them do remote_emit.
 template <int VEC, int LPR, int kPackAhead>

@@ -424,8 +424,8 @@ __device__ __forceinline__ void medium_role(const TableView &t, int id_bits, con
 // counts about 150 per chunk; 7.4 cycles per row in all at 2.3 GHz, 2.5 more where the rows come from HBM and not from the
 // last-level cache.  Two waves that took turns at reading and adding, with a barrier per chunk, took 7.6 and 9.9; what is gained
 // beyond the chain is the end of the launch, where blocks now finish together.  The push of 8.5 M keys of 64 floats, Zipf 1.4:
-// pooled by tens 480 -> 425 us, plain 624 -> 565; of 1.7 M keys of 128 floats 247 -> 240.  Steps of those batches 3 to 7 %
-// shorter, of 195 k keys of 37 floats 5 %.  Measured without gain: one read between every few adds (14 cycles each), a raised
+// pooled by tens 480 -> 425 us, plain 624 -> 565; of 1.7 M keys of 128 floats 247 -> 240.  Steps of the first two
+// 7 and 6 % shorter, of the last within their spread (2 %) the same, of 195 k keys of 37 floats 5 %.  Measured without gain: one read between every few adds (14 cycles each), a raised
 // priority for the summing wave, 20 instead of 16 vectors in flight, 192 blocks, barriers instead of counts.
 // Generic path (CSC 0; rows of less than four floats): seven loader waves and one that reads and adds, eight rows at a time,
 // three slots.
@@ -433,7 +433,9 @@ constexpr int kTable = 16;      // runs per bundle at most
 constexpr int kHalfGroups = 12; // groups of four rows a lane of the summing wave holds of half a chunk
 constexpr int kSlotVectors = 2 * kHalfGroups * kWave; // 16-byte vectors of a slot of the ring: a chunk, whatever the slice
 constexpr int kSlotsFast = 2, kSlotsGeneric = 3; // LDS slots
-constexpr uint32_t kDrawAhead = 16; // chunks before the end of a bundle at which the next ticket is drawn
+// Chunks before the end of a bundle at which the next ticket is drawn.  4, 16 and 64: the push of 195 k keys of 37 floats, Zipf 1.4, 23.8,
+// 23.3 and 27.4 us, of 1.04 M of 64 floats, 1.1, 96, 93 and 95, of 5.3 M of 17 floats, 1.2, 539, 538 and 539.
+constexpr uint32_t kDrawAhead = 16;
 // the value of the lanes 16 / 32 below (up) or above (!up), for the lanes of the other half of a pair of halves
 template <int D, bool up> __device__ __forceinline__ float from_half(float x) {
   const uint32_t v = __float_as_uint(x);

@@ -317,7 +317,8 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
           ids = cur.staged.as<index_t>();
         }
         // Nothing of the caller's is needed any more.  (The transfer of 1.7 M ids takes 95 us longer than their staging, and the
-        // next push can run meanwhile: two steps of 128 floats 1403 -> 1268 us; of 53 k ids 125.6 -> 123.8.)
+        // next push can run meanwhile: two steps of 128 floats 1.04 to 1.10 times shorter in four comparisons, 1376 -> 1318 and 1454 -> 1318
+        // us the outermost; of 53 k ids 125.6 -> 123.8.)
         if (narrowed && flag != nullptr && cfg.nrank == 1) {
           staged_ = keys_unread_ = true;
           ids_bad_ = stager.largest() >= tv.id_max;
@@ -339,8 +340,9 @@ void Shard::prepare_keys(const int64_t *keys, size_t n, uint32_t *flag, void *sc
       // returning later it finds the first scatter nearly done instead of on the CUs of its long runs (as beside
       // kEarlySortStepsBesideLists).  Two steps with the word and without: rows of 64 floats, Zipf 1.4, 1.58 M keys 599 and
       // 547 us, 1.7 M 637 and 569, of exponent 1.05 599 and 591 (no difference); where lists are built in between the
-      // word is the faster: pooled, 64 floats, 1.6 M keys 385 and 402.  Ids from pageable memory, which arrive in front of the
-      // key kernel: 1.7 M keys, Zipf 1.4, with the word 984 and without 1024.
+      // word is the faster: pooled, 64 floats, 1.6 M keys 385 and 402.  Ids from pageable memory,
+      // for which preprocess waits no longer than their staging: 1.7 M keys, 64 floats, with the word and without, Zipf 1.4 901 and
+      // 919, 1.05 955 and 971, 128 floats 1339 and 1339.
       const bool push_at_once = visible && !cur.tile_sorted && !cur.one_block && trains_ && prev.n != 0 && prev.lists_ready;
       if (flag != nullptr && !push_at_once && (cur.keys_made ? sort_tiles(n) : tile_count(n)) <= kReadSignalBlocks) {
         read_.count = &dst_->read_count;
